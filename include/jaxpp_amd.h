@@ -94,7 +94,8 @@ int jpp_graph_destroy(void* graph_exec);
  * algorithmic FLOPs / HBM bytes the launchers declared.  Class names:
  *   gemm_<nn|nt|tn>_<bf16|gelu|dgelu|accf32|f32>_<BM>x<BN>   (nn: y = x W,
  *       nt: dx = dy W^T, tn: dW = x^T dy)
- *   (+ "w8" for 8-wave tiles, "s3"/"s4" for 3 or 4 LDS stages),
+ *   (+ "w8" for 8-wave tiles, "s3" - "s5" for 3 to 5 LDS stages, "k2" for tiles shared by two
+ *   wave groups, "_multi" for several products in one launch),
  *   attn_fwd, attn_bwd_dq, attn_bwd_dkv, norm_fwd, norm_bwd, swiglu_fwd,
  *   swiglu_bwd, rope, grad_accum, colsum, adam */
 int jpp_probe_begin(const char* kernel_class);
@@ -146,7 +147,8 @@ typedef struct {
   int gelu_tanh;     /* 0: erf form, 1: tanh approximation */
   int tile;          /* 0: choose (may run the last, half-empty round of 256x256 tiles as a second
                         launch of 128x256 tiles); 1: 128x128; 2: 256x128; 3: 128x256; 4: 256x256
-                        (8 waves each) */
+                        (8 waves each); 5: 64x64 (two groups of 4 waves that take the K-steps in
+                        turn: the even and the odd steps are summed apart, then added) */
   /* grouped GEMM over experts (0 = plain).  seg: device int32 [n_seg + 1], row
    * offsets of the expert groups in the token-permuted buffers, multiples of 256.
    *   JPP_GROUP_M: rows of A and C are grouped; group e multiplies b + e * stride_b.
@@ -173,9 +175,9 @@ typedef struct {
    * dimensions - as if the pairs were concatenated along the contraction index.  The
    * weight gradients of several microbatches accumulate this way with one read and one write
    * of the fp32 accumulator instead of one per microbatch.  0 or 1: one pair.  Built for
-   * trans_a = trans_b = 1 with JPP_EPI_ACC_F32 on the 256-wide tiles: N a multiple of 256,
-   * `tile` 0 (the library then takes 256x256, or 128x256 when M is not a multiple of 256),
-   * 3 or 4; anything else is JPP_ERR_INVALID. */
+   * trans_a = trans_b = 1 with JPP_EPI_ACC_F32, on every tile but 256x128 (`tile` 0 takes
+   * 256x256, or 128x256 when M is not a multiple of 256; a grouped contraction goes by its
+   * size); anything else is JPP_ERR_INVALID. */
   const void* a_more[3];
   const void* b_more[3];
   int k_parts;
@@ -201,15 +203,16 @@ enum { JPP_GROUP_NONE = 0, JPP_GROUP_M = 1, JPP_GROUP_K = 2 };
 int jpp_gemm_bf16(void* stream, const jpp_gemm_args* args);
 
 /* Up to four independent accumulated weight gradients - every problem with trans_a = trans_b =
- * 1, JPP_EPI_ACC_F32, no groups, M and N multiples of 256, the same k and k_parts - as ONE
- * grid of 256x256 tiles, problem after problem.  Stands where the reference's weight-gradient
- * task holds several independent dot_generals (one per parameter of the layer,
- * src/jaxpp/jaxpr_utils.py:138-167 puts them all into BWD_W): launched one by one, each leaves
- * its last round of tiles partly empty (a 6144 x 4096 gradient is 384 tiles on 256 CUs);
- * together they close up.  Every output element is computed by one workgroup in a fixed order
- * (deterministic), the same order as in a single launch on 256x256 tiles; a single launch that
- * runs its last round on 128x256 tiles adds the old accumulator value at another point of the
- * sum there, so the two agree to fp32 rounding.  n_problems = 1 is jpp_gemm_bf16. */
+ * 1, JPP_EPI_ACC_F32, no groups, the same k and k_parts - as ONE grid of tiles, problem after
+ * problem.  Stands where the reference's weight-gradient task holds several independent
+ * dot_generals (one per parameter of the layer, src/jaxpp/jaxpr_utils.py:138-167 puts them all
+ * into BWD_W): launched one by one, each leaves its last round of tiles partly empty (a 6144 x
+ * 4096 gradient is 384 tiles on 256 CUs), small ones most of the device; together they close up.
+ * Tiles are 256x256 when M and N are multiples of 256 and the problems are most of a round of
+ * them, else 128x128 or 64x64.  Every output element is computed by one workgroup in a fixed
+ * order (deterministic), the same order as in a single launch on the same tile; a single launch
+ * that runs its last round on 128x256 tiles adds the old accumulator value at another point of
+ * the sum there, so the two agree to fp32 rounding.  n_problems = 1 is jpp_gemm_bf16. */
 int jpp_gemm_bf16_multi(void* stream, const jpp_gemm_args* problems, int n_problems);
 
 /* ---- fused attention (softmax(QK^T/sqrt(d)) V), forward and backward -------

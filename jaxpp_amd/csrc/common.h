@@ -176,15 +176,22 @@ __device__ __forceinline__ void lds_wait_all() { asm volatile("s_waitcnt lgkmcnt
 
 // Chunk permutation of row k of an MC tile.  A transpose read has lanes 0-15 on rows
 // k .. k+3 and lanes 16-31 on rows k+8 .. k+11 (8 rows are a multiple of the bank span
-// apart): bits 0-1 of k move a chunk by 64 bytes, bit 3 by 32, so those 32 lanes touch
-// every bank once.
-__device__ __forceinline__ int mc_swz(int k) { return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1); }
+// apart), 32 bytes each.  Rows of 256 bytes and more: bits 0-1 of k move a chunk by 64 bytes,
+// bit 3 by 32, so those 32 lanes touch every bank once.  Rows of 128 bytes (a 64-row tile, 8
+// chunks): two rows span the banks, so bit 0 needs no help; bit 1 of k moves a chunk by 32
+// bytes, bit 3 by 64.
+template <int ROWS>
+__device__ __forceinline__ int mc_swz(int k) {
+  if constexpr (ROWS == 64) return (((k >> 1) & 1) << 1) ^ (((k >> 3) & 1) << 2);
+  return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1);
+}
 
 template <int ROWS, bool MC, int NW = 4>
 struct DmaTile {
   static constexpr int BYTES = ROWS * 128;
   static constexpr int INSTS = ROWS / (8 * NW);  // wave-level loads per wave (NW waves share a tile)
   static_assert(INSTS >= 1, "tile too small for this many waves");
+  static_assert(ROWS == 64 || ROWS >= 128, "the chunk permutations stay inside rows of these lengths");
   typedef uint32_t Offsets[INSTS];
 
   // per-lane byte offsets (from the tile's first element) of this wave's loads;
@@ -199,7 +206,7 @@ struct DmaTile {
       } else {
         constexpr int CPR = ROWS / 8, RPI = 64 / CPR;
         const int k = inst * RPI + lane / CPR;
-        off[i] = (uint32_t)(((long)k * ld + (((lane % CPR) ^ mc_swz(k)) << 3)) * 2);
+        off[i] = (uint32_t)(((long)k * ld + (((lane % CPR) ^ mc_swz<ROWS>(k)) << 3)) * 2);
       }
     }
   }
@@ -233,7 +240,7 @@ struct DmaTile {
       // two transpose reads of 4 contraction rows x 16 operand rows per 16-lane group
       const int n = row0 + ((s & 3) << 2);
       const int k = k32 * 32 + (g << 3) + (s >> 2);
-      const uint8_t* p = tile + k * (ROWS * 2) + (((n >> 3) ^ mc_swz(k)) << 4) + ((n & 7) << 1);
+      const uint8_t* p = tile + k * (ROWS * 2) + (((n >> 3) ^ mc_swz<ROWS>(k)) << 4) + ((n & 7) << 1);
       const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
           (__attribute__((address_space(3))) s16x4*)JPP_LDS_PTR(p));
       const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(

@@ -32,6 +32,12 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
+// output tiles (jpp_gemm_args.tile)
+enum { kTile128 = 1, kTile256x128 = 2, kTile128x256 = 3, kTile256 = 4, kTile64 = 5,
+       kTile64x128 = 6 /* the library's own choice only */ };
+constexpr long kCus = 256;
+constexpr long kMostCus = 192;  // 256x256 tiles from which a grid of them is taken without asking
+
 struct GemmParams {
   const bf16_t* a;
   const bf16_t* b;
@@ -211,8 +217,9 @@ __device__ __forceinline__ int group_steps(const int* seg, const int* seg_rows, 
   return (rows + 63) / 64;
 }
 
-template <int BM, int BN, bool TA, bool TB, int EPI, int NW, int NS, bool KP = false, bool MP = false>
-__global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
+template <int BM, int BN, bool TA, bool TB, int EPI, int NW, int NS, bool KP = false, bool MP = false,
+          int KG = 1>
+__global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
   GemmParams p = args.p;
   int bid = blockIdx.x;  // this workgroup's tile within its problem
   if constexpr (MP) {
@@ -262,7 +269,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
 
   const int tid = threadIdx.x, lane = tid & 63;
   // (wave-uniform where the waves differ in what they do: a scalar branch around the copies)
-  const int wave = DW == NW ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_all = DW == NW && KG == 1 ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
+  // KG > 1: the workgroup is KG groups of NW waves that share the output tile and take the
+  // K-steps in turn (group g steps g, g + KG, ...), each with LDS stages of its own
+  // - small tiles, whose K-step is a chain of latencies (barrier, fragment reads, copies) and
+  // not work: at 512 x 1024 x 4096 (128 tiles of 64x64) one group takes 670 cycles a step with
+  // eight stages, two groups 900 a pair of steps with four (22 -> 15.5 us; four groups with the
+  // two stages that then fit 19 us: the copies land too late; five stages instead of four
+  // change nothing).  Larger tiles gain nothing (128x128: 28 us one group, 35 us two).
+  const int grp = KG == 1 ? 0 : wave_all / NW, wave = KG == 1 ? wave_all : wave_all % NW;
   const bool dma_wave = wave < DW;
   const int wm = wave / WN, wn = wave % WN;
   int tm, tn;
@@ -354,7 +369,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
   // loops too short for that add the old values in the epilogue, where rows are whole too.
   static_assert(BN * 4 <= 1024, "a row of the fp32 tile is one 64-lane copy");
   constexpr int NBT = BM / NW, C_LDS = NS * (BM + BN) * 128, C_PITCH = 1024 + 16;  // a copy is 1 KB
-  const bool stream_c = EPI == JPP_EPI_ACC_F32 && kt_n >= NBT + NS;
+  const bool stream_c = KG == 1 && NS <= 4 && EPI == JPP_EPI_ACC_F32 && kt_n >= NBT + NS;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -363,7 +378,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
   // (lanes past the end of a narrow row repeat its last piece)
   const uint32_t c_off0 =
       (uint32_t)(((m0 + wave) * p.ldc + n0 + min(lane, BN / 4 - 1) * 4) * 4);
-  const uint32_t lds0 = lds_address(smem);
+  uint8_t* const stages = smem + grp * (NS * STAGE);
+  const uint32_t lds0 = lds_address(stages);
+  // iteration t of a group is K-step t KG + grp of the contraction; the groups meet at every
+  // iteration's barrier, so those that have run out of steps take part without multiplying
+  const int it_n = KG == 1 ? kt_n : (kt_n + KG - 1) / KG;
+  auto k_step = [&](int t) { return KG == 1 ? t : min(t * KG + grp, kt_n - 1); };
   typename TileA::Offsets offa;
   typename TileB::Offsets offb;
   TileA::offsets(offa, p.lda, wave, lane);
@@ -388,7 +408,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
   if (kt_n > 0) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const int k = min(s, kt_n - 1);
+      const int k = k_step(min(s, it_n - 1));
       if (dma_wave) {
         TileA::template issue<0, IA>(uniform_ptr(a_at(k)), offa, lds0 + s * STAGE, wave);
         TileB::template issue<0, IB>(uniform_ptr(b_at(k)), offb, lds0 + s * STAGE + A_BYTES, wave);
@@ -398,9 +418,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < TN; ++j) fw[0][j] = TileB::frag16(smem + A_BYTES, row_w + j * 16, 0, lane);
+  for (int j = 0; j < TN; ++j) fw[0][j] = TileB::frag16(stages + A_BYTES, row_w + j * 16, 0, lane);
 #pragma unroll
-  for (int i = 0; i < TMH; ++i) fx[0][i] = TileA::frag16(smem, row_x + i * 16, 0, lane);
+  for (int i = 0; i < TMH; ++i) fx[0][i] = TileA::frag16(stages, row_x + i * 16, 0, lane);
 
   int st = 0;   // stage of K-step kt: kt % NS
   int cbi = 0;  // accumulator-row buffer of K-step kt: kt % (NS + 1)
@@ -417,13 +437,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
   const bf16_t* ga_late = nullptr;
   const bf16_t* gb_late = nullptr;
   int st_late = 0;
-  for (int kt = 0; kt < kt_n; ++kt) {
+  for (int kt = 0; kt < it_n; ++kt) {
     const int nst = st + 1 == NS ? 0 : st + 1;
-    const uint8_t* sa = smem + st * STAGE;
+    const uint8_t* sa = stages + st * STAGE;
     const uint8_t* sb = sa + A_BYTES;
-    const uint8_t* na = smem + nst * STAGE;
+    const uint8_t* na = stages + nst * STAGE;
+    const bool live = KG == 1 || kt * KG + grp < kt_n;
     // past the end the last K-step is fetched again, unused
-    const int kn = min(kt + NS, kt_n - 1);
+    const int kn = k_step(min(kt + NS, it_n - 1));
     const bf16_t* ga = uniform_ptr(a_at(kn));
     const bf16_t* gb = uniform_ptr(b_at(kn));
 #pragma unroll
@@ -449,7 +470,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
           else if (cin == 1) dma_wait<(NS - 2) * OPB + 1>();
           else if (cin == 2) dma_wait<(NS - 2) * OPB + 2>();
           else dma_wait<(NS - 2) * OPB + 3>();
-          static_assert(NS <= 4, "the wait above distinguishes up to three rows in flight");
+          
         }
         lds_wait_all();
         __syncthreads();
@@ -517,6 +538,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
                                                    lds0 + st_late * STAGE + A_BYTES, wave);
           }
         }
+        if (KG > 1 && !live) continue;
         // a walk over the 2 x TN tiles of this pair of rows, the next pair taking the columns in
         // the opposite direction
 #pragma unroll
@@ -545,22 +567,49 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
   }
   dma_wait_all();   // the refetches of the last two K-steps must not outlive the block's LDS
 
+  // the groups' sums, in group order: wave w of every group holds the same elements, so they
+  // change hands through LDS lane by lane, 16 bytes at a time
+  if constexpr (KG > 1) {
+    __syncthreads();
+    uint8_t* const mine = smem + ((grp - 1) * NW + wave) * (TM * TN * 1024) + lane * 16;
+    if (grp > 0) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) *(f32x4*)(mine + (i * TN + j) * 1024) = acc[i][j];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int g = 1; g < KG; ++g)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[i][j] += *(const f32x4*)(mine + (g * NW * TM * TN + i * TN + j) * 1024);
+    }
+  }
+  // tile rows that pass through LDS at a time in the epilogues below: of a tile shared by
+  // several wave groups (a small one) all
+  constexpr bool WHOLE = KG > 1;
+
   if constexpr (EPI == JPP_EPI_ACC_F32 || EPI == JPP_EPI_F32) {
     // fp32 outputs leave through LDS as well (see below), a quarter of the tile per pass:
     // 16-byte stores of contiguous rows instead of 32-byte pieces of 32 rows
-    constexpr int IPP = TM / 2, RP = IPP * 16, PITCH = BN * 4 + 16, NT = NW * 64;
+    constexpr int IPP = WHOLE ? TM : TM / 2, RP = WHOLE ? BM : IPP * 16, PITCH = BN * 4 + 16,
+                  NT = NW * KG * 64;
     constexpr int TPR = BN / 4, RPI = NT / TPR;
 #pragma unroll 1
-    for (int pass = 0; pass < 2 * (TM / IPP); ++pass) {
+    for (int pass = 0; pass < (WHOLE ? 1 : 2 * (TM / IPP)); ++pass) {
       const int half = pass / (TM / IPP), i0 = (pass % (TM / IPP)) * IPP;
       __syncthreads();
-      if (wm == half) {
+      if (WHOLE ? grp == 0 : wm == half) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
           if (i >= i0 && i < i0 + IPP) {
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-              *(f32x4*)(smem + ((i - i0) * 16 + (lane & 15)) * PITCH +
+              *(f32x4*)(smem + ((WHOLE ? row_x : 0) + (i - i0) * 16 + (lane & 15)) * PITCH +
                         (wn * (BN / WN) + j * 16 + (lane >> 4) * 4) * 4) = acc[i][j];
           }
       }
@@ -605,17 +654,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
     // - and is taken back out by rows: a thread owns 8 consecutive columns of a row, so
     // every global access of the epilogue (output, residual, pre-activation, gate/up) is a
     // 16-byte piece of a contiguous run, and the arithmetic runs in fp32 exactly as before.
-    constexpr int HALF = BM / 2, PITCH = BN * 4 + 16, NT = NW * 64;
+    constexpr int HALF = WHOLE ? BM : BM / 2, PITCH = BN * 4 + 16, NT = NW * KG * 64;
     const bf16_t* bias = p.bias;
 #pragma unroll 1
-    for (int half = 0; half < 2; ++half) {
+    for (int half = 0; half < BM / HALF; ++half) {
       __syncthreads();  // fragments of the last K-step / the previous half are out of LDS
-      if (wm == half) {
+      if (WHOLE ? grp == 0 : wm == half) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            *(f32x4*)(smem + (i * 16 + (lane & 15)) * PITCH +
+            *(f32x4*)(smem + ((WHOLE ? row_x : 0) + i * 16 + (lane & 15)) * PITCH +
                       (wn * (BN / WN) + j * 16 + (lane >> 4) * 4) * 4) = acc[i][j];
       }
       __syncthreads();
@@ -738,7 +787,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_kernel(GemmArgs<MP> args) {
 #undef a_at
 #undef b_at
 
-template <int BM, int BN, bool TA, bool TB, int EPI, int NW, int NS>
+template <int BM, int BN, bool TA, bool TB, int EPI, int NW, int NS, int KG = 1>
 const char* class_name() {
   // built once per instantiation; the initialisation of a function-local static is
   // thread-safe
@@ -748,30 +797,30 @@ const char* class_name() {
     const char* epi = EPI == JPP_EPI_BF16 ? "bf16" : EPI == JPP_EPI_GELU ? "gelu"
                     : EPI == JPP_EPI_DGELU ? "dgelu" : EPI == JPP_EPI_ACC_F32 ? "accf32"
                     : EPI == JPP_EPI_SWIGLU ? "swiglu" : EPI == JPP_EPI_DSWIGLU ? "dswiglu" : "f32";
-    snprintf(buf, sizeof(buf), "gemm_%s_%s_%dx%d%s%s", lay, epi, BM, BN, NW == 8 ? "w8" : "",
-             NS == 2 ? "" : NS == 3 ? "s3" : "s4");
+    snprintf(buf, sizeof(buf), "gemm_%s_%s_%dx%d%s%s%s", lay, epi, BM, BN, NW == 8 ? "w8" : "",
+             NS == 2 ? "" : NS == 3 ? "s3" : NS == 4 ? "s4" : "s5", KG == 1 ? "" : "k2");
     return std::string(buf);
   }();
   return name.c_str();
 }
 
-template <int BM, int BN, bool TA, bool TB, int EPI, int NW = 4, int NS = 2, bool KP = false>
+template <int BM, int BN, bool TA, bool TB, int EPI, int NW = 4, int NS = 2, bool KP = false, int KG = 1>
 int launch(hipStream_t stream, GemmParams& p) {
   // two operand stages; the bf16 epilogues stage half a tile in fp32 with padded rows
-  constexpr int SMEM_LOOP = NS * (BM + BN) * 128, SMEM_EPI = (BM / 2) * (BN * 4 + 16);
+  constexpr int SMEM_LOOP = KG * NS * (BM + BN) * 128,
+                SMEM_EPI = (KG > 1 ? BM : BM / 2) * (BN * 4 + 16);
   // + NS+1 buffers of NW rows of the fp32 tile (padded) for C += A B
-  constexpr int SMEM = EPI == JPP_EPI_ACC_F32 ? SMEM_LOOP + (NS + 1) * NW * (1024 + 16)
+  constexpr int SMEM = EPI == JPP_EPI_ACC_F32 && KG == 1 && NS <= 4 ? SMEM_LOOP + (NS + 1) * NW * (1024 + 16)
                        : (EPI == JPP_EPI_F32 || SMEM_LOOP > SMEM_EPI) ? SMEM_LOOP : SMEM_EPI;
   if constexpr (!KP) {
-    // several operand pairs: only the accumulating weight-gradient kernels on 256-wide tiles
-    // are built for that
+    // several operand pairs: only the accumulating weight-gradient kernels are built for that
     if (p.k_parts > 1) {
-      if constexpr (TA && TB && EPI == JPP_EPI_ACC_F32 && BN == 256 && NW == 8 && NS == 2)
-        return launch<BM, BN, TA, TB, EPI, NW, NS, true>(stream, p);
+      if constexpr (TA && TB && EPI == JPP_EPI_ACC_F32 && !(BM == 256 && BN == 128))
+        return launch<BM, BN, TA, TB, EPI, NW, NS, true, KG>(stream, p);
       else
         return jpp_set_error(JPP_ERR_INVALID, "gemm: several operand pairs are supported for "
-                             "accumulated weight gradients (tn, JPP_EPI_ACC_F32) on 256x256 and "
-                             "128x256 tiles");
+                             "accumulated weight gradients (tn, JPP_EPI_ACC_F32), not on 256x128 "
+                             "tiles");
     }
   }
   // algorithmic extent: grouped launches count the non-padding rows when the caller gave them
@@ -785,10 +834,10 @@ int launch(hipStream_t stream, GemmParams& p) {
   // of its 256x256 launch, which declares the whole product's work)
   const bool tail = p.tail_split >= 2;
   ProbeScope probe(stream, tail ? class_name<256, 256, TA, TB, EPI, 8, 2>()
-                                : class_name<BM, BN, TA, TB, EPI, NW, NS>(),
+                                : class_name<BM, BN, TA, TB, EPI, NW, NS, KG>(),
                    tail ? 0.0 : 2.0 * am * p.n * ak,
                    tail ? 0.0 : 2.0 * am * ak + b_bytes + copies * am * p.n * cb);
-  auto kern = gemm_kernel<BM, BN, TA, TB, EPI, NW, NS, KP>;
+  auto kern = gemm_kernel<BM, BN, TA, TB, EPI, NW, NS, KP, false, KG>;
   static_assert(SMEM <= 160 * 1024, "LDS of one CU");
   // the LDS limit of a kernel is sticky: set once per instantiation, by whichever host
   // thread launches it first (the others wait for that call and see its result)
@@ -802,18 +851,20 @@ int launch(hipStream_t stream, GemmParams& p) {
   p.tiles_m = p.m / BM;
   p.tiles_n = p.n / BN;
   const int blocks = p.tiles_m * p.tiles_n * (p.group_mode == JPP_GROUP_K ? p.n_seg : 1);
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(NW * 64), SMEM, stream, GemmArgs<false>{p});
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(NW * KG * 64), SMEM, stream, GemmArgs<false>{p});
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
 
-// Several accumulated weight gradients (C_i += sum_j A_ij^T B_ij) as one grid of 256x256
+// Several accumulated weight gradients (C_i += sum_j A_ij^T B_ij) as one grid of BM x BN
 // tiles: problem i's tiles follow problem i-1's, so the half-filled last rounds of the single
 // launches (384 or 896 tiles on 256 CUs) close up - the four weight gradients of a
-// Llama-3-8B-shaped layer are 13 full rounds together.
+// Llama-3-8B-shaped layer are 13 full rounds together - and small ones share the device.
+template <int BM, int BN, int NW, int NS, int KG = 1>
 int launch_multi(hipStream_t stream, GemmParams* ps, int n) {
-  constexpr int BM = 256, BN = 256, NW = 8, NS = 2;
-  constexpr int SMEM = NS * (BM + BN) * 128 + (NS + 1) * NW * (1024 + 16);
+  constexpr bool STREAM_C = KG == 1 && NS <= 4;
+  constexpr int SMEM = KG * NS * (BM + BN) * 128 + (STREAM_C ? (NS + 1) * NW * (1024 + 16) : 0);
+  static_assert(SMEM <= 160 * 1024, "LDS of one CU");
   GemmArgs<true> args;
   args.p = ps[0];
   int first = 0;
@@ -840,8 +891,10 @@ int launch_multi(hipStream_t stream, GemmParams* ps, int n) {
     memset(&args.more[i - 1], 0, sizeof(GemmProblem));
     args.more[i - 1].first = 0x7fffffff;
   }
-  ProbeScope probe(stream, "gemm_tn_accf32_256x256w8_multi", flops, bytes);
-  auto kern = gemm_kernel<BM, BN, true, true, JPP_EPI_ACC_F32, NW, NS, true, true>;
+  static const std::string cls =
+      std::string(class_name<BM, BN, true, true, JPP_EPI_ACC_F32, NW, NS, KG>()) + "_multi";
+  ProbeScope probe(stream, cls.c_str(), flops, bytes);
+  auto kern = gemm_kernel<BM, BN, true, true, JPP_EPI_ACC_F32, NW, NS, true, true, KG>;
   static std::once_flag configured;
   static hipError_t configure_rc = hipSuccess;
   std::call_once(configured, [&] {
@@ -849,44 +902,109 @@ int launch_multi(hipStream_t stream, GemmParams* ps, int n) {
                                        hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
   });
   JPP_CHECK_HIP(configure_rc);
-  hipLaunchKernelGGL(kern, dim3(first), dim3(NW * 64), SMEM, stream, args);
+  hipLaunchKernelGGL(kern, dim3(first), dim3(NW * KG * 64), SMEM, stream, args);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
 
+// The 128x128 tile runs with five LDS stages (one workgroup per CU) when every CU has at most
+// one tile, else with two (two workgroups per CU); the 64x64 tile, whose two wave groups share
+// it, with four or two by the same rule.
+bool deep_stages(long tiles, long ksteps, int tile) {
+  return tiles <= kCus && (tile == kTile128 || ksteps > 8);
+}
+
 template <bool TA, bool TB, int EPI>
 int launch_tiled(hipStream_t stream, GemmParams& p, int tile) {
+  const int bm = tile == kTile64 ? 64 : 128;
+  const long tiles = (long)(p.m / bm) * (p.n / bm) * (p.group_mode == JPP_GROUP_K ? p.n_seg : 1);
+  const bool deep = deep_stages(tiles, p.k / 64, tile);
   switch (tile) {
-    case 2:  // 8 waves of 128x32; three stages where the accumulator rows leave room
+    case kTile256x128:  // 8 waves of 128x32; three stages where the accumulator rows leave room
       return launch<256, 128, TA, TB, EPI, 8, EPI == JPP_EPI_ACC_F32 ? 2 : 3>(stream, p);
-    case 3:  // 8 waves of 64x64
+    case kTile128x256:  // 8 waves of 64x64
       return launch<128, 256, TA, TB, EPI, 8, EPI == JPP_EPI_ACC_F32 ? 2 : 3>(stream, p);
-    case 4: return launch<256, 256, TA, TB, EPI, 8>(stream, p);
-    default:
-      // 128x128: 8 waves (64x32 each); the SwiGLU epilogues, which no measured workload
-      // reaches at this tile size, keep the plain 4-wave form.  With more tiles than two per
-      // CU, two stages and two workgroups per CU; with fewer (and a K loop long enough to pay
-      // for the longer prologue) the one workgroup a CU gets prefetches deeper instead (4
-      // stages, 3 where the accumulator rows need room too).
-      if constexpr (EPI == JPP_EPI_SWIGLU || EPI == JPP_EPI_DSWIGLU) {
-        return launch<128, 128, TA, TB, EPI>(stream, p);
-      } else {
-        const long tiles = (long)(p.m / 128) * (p.n / 128) *
-                           (p.group_mode == JPP_GROUP_K ? p.n_seg : 1);
-        if (tiles > 2 * 256 || p.k < 2048) return launch<128, 128, TA, TB, EPI, 8>(stream, p);
-        return launch<128, 128, TA, TB, EPI, 8, EPI == JPP_EPI_ACC_F32 ? 3 : 4>(stream, p);
-      }
+    case kTile256: return launch<256, 256, TA, TB, EPI, 8>(stream, p);
+    case kTile64x128:
+      // the 64x64 form for products that rotate heads of 128: the same sums in the same order
+      // (two wave groups), so the rotated product is the plain one's bits rotated
+      if constexpr (!TA && TB && EPI == JPP_EPI_BF16)
+        return launch<64, 128, TA, TB, EPI, 4, 3, false, 2>(stream, p);
+      else
+        return jpp_set_error(JPP_ERR_INVALID, "gemm: unknown tile %d", tile);
+    case kTile64:  // two groups of 4 waves (32x32 each) that take the K-steps in turn
+      return deep ? launch<64, 64, TA, TB, EPI, 4, 4, false, 2>(stream, p)
+                  : launch<64, 64, TA, TB, EPI, 4, 2, false, 2>(stream, p);
+    default:  // 128x128: 8 waves (64x32 each)
+      return deep ? launch<128, 128, TA, TB, EPI, 8, 5>(stream, p)
+                  : launch<128, 128, TA, TB, EPI, 8, 2>(stream, p);
   }
 }
 
-// 256 CUs.  The 256x256 tile run by 8 waves (two per SIMD, so one wave's LDS
-// reads hide under the other's MFMAs) is the fastest whenever it gives most CUs
-// a tile; smaller problems take 128x128 tiles, two workgroups per CU.
-int choose_tile(long m, long n) {
-  const long t256 = (m % 256 == 0 && n % 256 == 0) ? (m / 256) * (n / 256) : 0;
-  return t256 >= 192 ? 4 : 1;
+// Expected time of a product of `tiles` tiles, `ksteps` K-steps of 64 each, in us:
+//   start + w * (tile_cost + ksteps * step),   w = tiles of the busiest of the 256 CUs
+// (two workgroups fit on a CU in the two-stage forms: their steps overlap, so a CU's lone
+// workgroup takes a step cost of its own).  The constants are least-squares fits to 208 random
+// shapes (M, N 128 .. 8192, K 128 .. 8192) timed alone, 7 tile forms each, mean error 4 - 10 %;
+// choosing the smallest estimate costs 1.8 % against always choosing the measured best, where
+// the rule before (256x256 from 192 tiles on, else 128x128) cost 37 %: a 512 x 1024 x 4096
+// input gradient has 32 tiles of 128x128 for 256 CUs and took 28 us, 15 us as 128 tiles of
+// 64x64 with two wave groups each.
+struct TileForm {
+  int tile, bm, bn;
+  bool deep;              // which of the tile's two forms (kTile128, kTile64)
+  float start, tile_cost, lone_step, step;
+};
+constexpr TileForm kForward[] = {
+    {kTile64, 64, 64, true, 1.5f, 2.8f, 0.19f, 0.19f},    {kTile64, 64, 64, false, 2.1f, 1.4f, 0.285f, 0.19f},
+    {kTile128, 128, 128, true, 0.f, 5.2f, 0.41f, 0.41f},  {kTile128, 128, 128, false, 1.2f, 2.6f, 0.60f, 0.45f},
+    {kTile128x256, 128, 256, true, 0.f, 6.1f, 0.65f, 0.65f}, {kTile256, 256, 256, true, 0.f, 7.9f, 1.07f, 1.07f}};
+constexpr TileForm kWeightGrad[] = {
+    {kTile64, 64, 64, true, 1.0f, 3.2f, 0.23f, 0.23f},    {kTile64, 64, 64, false, 1.7f, 1.8f, 0.31f, 0.21f},
+    {kTile128, 128, 128, true, 0.f, 6.0f, 0.46f, 0.46f},  {kTile128, 128, 128, false, 0.f, 4.5f, 0.75f, 0.81f},
+    {kTile128x256, 128, 256, true, 0.f, 6.6f, 0.95f, 0.95f}, {kTile256, 256, 256, true, 0.f, 10.f, 1.28f, 1.28f}};
+
+struct Extent { long m, n; };
+
+// tile with the smallest estimate for products of these extents in one grid; *us: the estimate
+int cheapest_tile(const Extent* e, int n, long ksteps, bool wgrad, bool may_64, bool may_128x256, float* us) {
+  int best = kTile128;
+  float best_us = 0.f;
+  for (const TileForm& f : wgrad ? kWeightGrad : kForward) {
+    if ((f.tile == kTile64 && !may_64) || (f.tile == kTile128x256 && !may_128x256)) continue;
+    long tiles = 0;
+    for (int i = 0; i < n && tiles >= 0; ++i)
+      tiles = e[i].m % f.bm || e[i].n % f.bn ? -1 : tiles + (e[i].m / f.bm) * (e[i].n / f.bn);
+    if (tiles < 0) continue;
+    if ((f.tile == kTile64 || f.tile == kTile128) && f.deep != deep_stages(tiles, ksteps, f.tile)) continue;
+    const long w = (tiles + kCus - 1) / kCus;
+    const float t = f.start + w * (f.tile_cost + ksteps * (w == 1 ? f.lone_step : f.step));
+    if (best_us == 0.f || t < best_us) { best_us = t; best = f.tile; }
+  }
+  if (us) *us = best_us;
+  return best;
 }
 
+// The 256x256 tile run by 8 waves (two per SIMD, so one wave's LDS reads hide under the other's
+// MFMAs) is the fastest whenever it gives most CUs a tile; smaller problems go by the estimate.
+// Grouped problems (whole 256-row segments) are estimated from the rows that hold data.
+int choose_tile(const jpp_gemm_args* a) {
+  const bool group_m = a->group_mode == JPP_GROUP_M, group_k = a->group_mode == JPP_GROUP_K;
+  Extent e = {a->m, a->n};
+  long ksteps = a->k / 64;
+  if (group_m && a->group_rows)   // half of a segment's last 256 rows are padding on average
+    e.m = std::min<long>(a->m, (a->group_rows + 128L * a->n_seg + 255) / 256 * 256);
+  if (group_k) {
+    e.m *= a->n_seg;              // an output per group
+    if (a->group_rows) ksteps = a->group_rows / (64L * a->n_seg) + 1;
+    else return kTile256;
+  }
+  const long t256 = e.m % 256 == 0 && e.n % 256 == 0 ? (e.m / 256) * (e.n / 256) : 0;
+  if (t256 >= kMostCus || (group_m && !a->group_rows)) return kTile256;
+  const int tile = cheapest_tile(&e, 1, ksteps, a->trans_a && a->trans_b, true, true, nullptr);
+  // (a rotated head lies inside one tile)
+  return tile == kTile64 && a->rope_cos && a->rope_head_dim > 64 ? (int)kTile64x128 : tile;
+}
 
 // sub-problem whose first row / column is (m_off, n_off) of the full one
 void shift_origin(GemmParams& p, bool ta, bool tb, int epi, long m_off, long n_off) {
@@ -1036,16 +1154,13 @@ extern "C" int jpp_gemm_bf16(void* stream_, const jpp_gemm_args* a) {
   hipStream_t stream = (hipStream_t)stream_;
   GemmParams p;
   if (int rc = prepare(a, p)) return rc;
-  int tile = a->tile ? a->tile : choose_tile(a->m, a->n);
-  // row groups come in 256-row segments; a contraction split into groups takes any tile
-  if (a->group_mode == JPP_GROUP_M || (a->group_mode == JPP_GROUP_K && !a->tile)) tile = 4;
-  // several operand pairs exist on the 256-wide tiles only: a tile left to the library goes
-  // there whatever the problem's size (N not a multiple of 256 is refused below, with the
-  // kernel's message)
-  if (a->k_parts > 1 && !a->tile) tile = 4;
-  JPP_REQUIRE(tile >= 1 && tile <= 4, "gemm: unknown tile %d", tile);
-  if ((tile == 2 || tile == 4) && a->m % 256) tile = a->n % 256 ? 1 : 3;
-  if ((tile == 3 || tile == 4) && a->n % 256) tile = a->m % 256 ? 1 : 2;
+  int tile = a->tile ? a->tile : choose_tile(a);
+  // several operand pairs of an ungrouped product: the 256-wide tiles whatever its size
+  // (jpp_gemm_bf16_multi is the way to run small ones)
+  if (a->k_parts > 1 && !a->tile && a->group_mode == JPP_GROUP_NONE) tile = kTile256;
+  JPP_REQUIRE(a->tile >= 0 && a->tile <= 5, "gemm: unknown tile %d", a->tile);
+  if ((tile == kTile256x128 || tile == kTile256) && a->m % 256) tile = a->n % 256 ? kTile128 : kTile128x256;
+  if ((tile == kTile128x256 || tile == kTile256) && a->n % 256) tile = a->m % 256 ? kTile128 : kTile256x128;
 
   // A grid of 256x256 tiles whose last round fills at most half of the 256 CUs runs that
   // round as a separate launch of 128x256 tiles over the last rows or columns: a full round
@@ -1097,7 +1212,9 @@ extern "C" int jpp_gemm_bf16_multi(void* stream_, const jpp_gemm_args* problems,
   JPP_REQUIRE(problems && n_problems >= 1 && n_problems <= 4, "gemm_multi: 1 to 4 problems");
   if (n_problems == 1) return jpp_gemm_bf16(stream_, problems);
   GemmParams ps[4];
-  long tiles = 0;
+  Extent e[4];
+  long tiles = 0, t256 = 0;
+  bool whole = true;
   for (int i = 0; i < n_problems; ++i) {
     const jpp_gemm_args* a = problems + i;
     if (int rc = prepare(a, ps[i])) return rc;
@@ -1105,13 +1222,22 @@ extern "C" int jpp_gemm_bf16_multi(void* stream_, const jpp_gemm_args* problems,
                     a->group_mode == JPP_GROUP_NONE && !a->bias && !a->resid && !a->tile,
                 "gemm_multi: problem %d is not a plain accumulated weight gradient (trans_a = "
                 "trans_b = 1, JPP_EPI_ACC_F32, no groups, bias, residual or tile choice)", i);
-    JPP_REQUIRE(a->m % 256 == 0 && a->n % 256 == 0,
-                "gemm_multi: problem %d: M and N must be multiples of 256, got %ldx%ld", i,
-                (long)a->m, (long)a->n);
     JPP_REQUIRE(a->k == problems[0].k && ps[i].k_parts == ps[0].k_parts,
                 "gemm_multi: problem %d differs from problem 0 in k or k_parts", i);
-    tiles += (a->m / 256) * (a->n / 256);
+    e[i] = {a->m, a->n};
+    whole = whole && a->m % 256 == 0 && a->n % 256 == 0;
+    t256 += (a->m / 256) * (a->n / 256);
+    tiles += (a->m / 64) * (a->n / 64);
   }
   JPP_REQUIRE(tiles < (1L << 30), "gemm_multi: too many tiles");
-  return launch_multi(stream, ps, n_problems);
+  const long ksteps = (long)ps[0].k / 64 * ps[0].k_parts;
+  const int tile = whole && t256 >= kMostCus ? (int)kTile256
+                   : cheapest_tile(e, n_problems, ksteps, true, true, false, nullptr);
+  const bool deep = deep_stages(tile == kTile64 ? tiles : tiles / 4, ksteps, tile);
+  if (tile == kTile256) return launch_multi<256, 256, 8, 2>(stream, ps, n_problems);
+  if (tile == kTile64)
+    return deep ? launch_multi<64, 64, 4, 4, 2>(stream, ps, n_problems)
+                : launch_multi<64, 64, 4, 2, 2>(stream, ps, n_problems);
+  return deep ? launch_multi<128, 128, 8, 5>(stream, ps, n_problems)
+              : launch_multi<128, 128, 8, 2>(stream, ps, n_problems);
 }

@@ -90,7 +90,7 @@ struct jpp_stage {
   // layer l+1 read set (l+1)%3 while layer l's input-gradient chain writes set l%3 and
   // hands its result to layer l-1 in set (l-1)%3.
   LayerStash wsets[3];
-  Buf s_dx[2], s_t1, s_t2, s_t3, s_t4, s_partial, s_partial_side, s_delta, s_wg, s_split, s_cos,
+  Buf s_dx[2], s_t1, s_t2, s_t3, s_t4, s_partial, s_partial_side, s_delta, s_wg, s_cos,
       s_sin, s_moework;
   size_t total_bytes = 0;
   // second stream (two_streams): weight gradients trail the input-gradient chain
@@ -206,31 +206,8 @@ int bias_grads4(jpp_stage* s, hipStream_t st, const jpp_colsum_item* items, floa
 int wgrad(jpp_stage* s, hipStream_t st, const void* x, int64_t ldx, const void* dy, int64_t lddy,
           float* acc, int64_t rows, int64_t cols) {
   if (s->f32()) return gemm(s, st, x, ldx, 1, dy, lddy, 1, acc, cols, rows, cols, s->T, JPP_EPI_ACC_F32);
-  if (s->d.fused_wgrad_accum) {
-    // A weight matrix of at most 128 tiles of 128x128 leaves half of the CUs without work:
-    // the contraction over the tokens is then split over `parts` workgroups per tile, which
-    // leave f32 partial products in scratch, and an ordered sum adds them to the accumulator
-    // (the order is fixed, so the result does not depend on timing).
-    const int64_t tiles = (rows / 128) * (cols / 128);
-    int parts = 1;
-    while (parts < 8 && tiles * parts * 2 <= 256 && s->T % (parts * 2 * 64) == 0 &&
-           s->T / (parts * 2) >= 512)
-      parts *= 2;
-    if (parts > 1 && (size_t)parts * rows * cols * 4 <= s->s_wg.bytes) {
-      float* ws = s->S<float>(s->s_wg);
-      jpp_gemm_args g;
-      memset(&g, 0, sizeof(g));
-      g.a = x; g.b = dy; g.c = ws; g.m = rows; g.n = cols; g.k = 0;
-      g.lda = ldx; g.ldb = lddy; g.ldc = cols; g.trans_a = 1; g.trans_b = 1;
-      g.epilogue = JPP_EPI_F32; g.tile = 1;
-      g.seg = s->S<int32_t>(s->s_split) + 16 * (parts == 2 ? 0 : parts == 4 ? 1 : 2);
-      g.n_seg = parts; g.group_mode = JPP_GROUP_K; g.stride_c = rows * cols;
-      g.group_rows = s->T;
-      RC(jpp_gemm_bf16(st, &g));
-      return jpp_sum_accum_f32(st, acc, ws, parts, rows * cols);
-    }
+  if (s->d.fused_wgrad_accum)
     return gemm(s, st, x, ldx, 1, dy, lddy, 1, acc, cols, rows, cols, s->T, JPP_EPI_ACC_F32);
-  }
   void* g = s->S<>(s->s_wg);
   RC(gemm(s, st, x, ldx, 1, dy, lddy, 1, g, cols, rows, cols, s->T, JPP_EPI_BF16));
   return jpp_grad_accum_f32(st, acc, g, rows * cols, 0);
@@ -275,26 +252,27 @@ struct WgradBatch {
   }
 };
 
-// Runs a layer's gathered weight gradients: as one grid of 256x256 tiles when that takes
-// fewer rounds of the 256 CUs than the launches one by one (whose last rounds stay partly
-// empty: a round of 128x256 tiles for a rest of at most 128 tiles costs about 0.77 of a full
-// one), else one by one.  Which way is taken depends on the shapes only.
+// Runs a layer's gathered weight gradients.  As one grid of 256x256 tiles when that takes fewer
+// rounds of the 256 CUs than the launches one by one (whose last rounds stay partly empty: a
+// round of 128x256 tiles for a rest of at most 128 tiles costs about 0.77 of a full one).  When
+// together they are less than a round (kFullGrid tiles), or not all a multiple of 256 in both
+// directions, always: one by one each would leave most of the device idle - four products of
+// 768 .. 3072 x 768 on 1152 tokens were 80 us in six launches, BERT-large's four (192 tiles of
+// 256x256 together) 3.3 % of that stage's step.  Which way is taken depends on the shapes only.
 int run_wgrads(jpp_stage* s, hipStream_t st, WgradBatch& w) {
-  bool multi = w.n >= 2 && !s->f32() && s->d.fused_wgrad_accum;
+  constexpr long kFullGrid = 192;
+  const bool multi = w.n >= 2 && !s->f32() && s->d.fused_wgrad_accum;
+  bool whole = true;
   long total = 0;
   double apart = 0;
-  for (int i = 0; i < w.n && multi; ++i) {
+  for (int i = 0; i < w.n; ++i) {
     const jpp_gemm_args& q = w.g[i];
-    if (q.m % 256 || q.n % 256) { multi = false; break; }
+    whole = whole && q.m % 256 == 0 && q.n % 256 == 0;
     const long t = (q.m / 256) * (q.n / 256), rest = t % 256;
     total += t;
     apart += (double)(t / 256) + (rest == 0 ? 0.0 : (rest <= 128 && t > 256 ? 0.77 : 1.0));
   }
-  // (matrices of fewer than 192 tiles would run one by one on 128x128 tiles, each launch
-  // leaving most of the device idle: BERT-large's four are 192 tiles of 256x256 together,
-  // one round, -3.3 % step time; below half a round in total the single launches, which
-  // split the contraction over workgroups, keep the device busier)
-  if (multi && total >= 128 && (double)((total + 255) / 256) < apart - 0.25) {
+  if (multi && (!whole || total < kFullGrid || (double)((total + 255) / 256) < apart - 0.25)) {
     // smallest first: measured 1 % faster than largest first at the Llama-3-8B shapes
     jpp_gemm_args order[4];
     for (int i = 0; i < w.n; ++i) order[i] = w.g[i];
@@ -929,10 +907,7 @@ int jpp_stage_create(const jpp_stage_desc* d, jpp_stage** out) {
   s->s_delta = sc.take((size_t)2 * d->batch * d->n_heads * d->seq * 4);
   size_t max_w = 0;
   for (auto& p : s->pinfo) max_w = std::max(max_w, (size_t)(p.rows * p.cols));
-  // unfused path: a bf16 weight gradient; fused path: partial products of a split contraction
-  // (at most 256 tiles of 128x128 in all)
-  s->s_wg = sc.take(d->fused_wgrad_accum ? (size_t)256 * 128 * 128 * 4 : max_w * e);
-  s->s_split = sc.take(3 * 16 * 4);  // token offsets of a contraction split in 2, 4, 8
+  s->s_wg = sc.take(d->fused_wgrad_accum ? 256 : max_w * e);  // unfused path: a bf16 weight gradient
   s->s_cos = sc.take((size_t)d->seq * (hd / 2) * 4);
   s->s_sin = sc.take((size_t)d->seq * (hd / 2) * 4);
   s->scratch_bytes = sc.total;
@@ -967,12 +942,6 @@ int jpp_stage_create(const jpp_stage_desc* d, jpp_stage** out) {
   keep(hipMemset(s->params, 0, n_layers * s->layer_elems * s->es));
   keep(hipMemset(s->grads, 0, n_layers * s->layer_elems * 4));
 
-  {
-    int32_t split[3 * 16] = {};
-    for (int k = 0; k < 3; ++k)
-      for (int i = 0; i <= (2 << k); ++i) split[16 * k + i] = (int32_t)(T / (2 << k) * i);
-    keep(hipMemcpy(s->S<>(s->s_split), split, sizeof(split), hipMemcpyHostToDevice));
-  }
   if (d->family == JPP_FAMILY_LLAMA || d->family == JPP_FAMILY_MIXTRAL) {
     // cos/sin of pos * theta^(-2i/d): evaluated in double, stored as f32
     const int half = hd / 2;

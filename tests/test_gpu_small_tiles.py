@@ -1,0 +1,123 @@
+"""Products with fewer tiles than the device has CUs: the 64x64 tile whose two wave groups take
+the K-steps in turn, its 64x128 form for rotated heads of 128, the five-stage 128x128 tile, and
+several weight gradients in one grid of small tiles - at the sizes where they can go wrong: one
+K-step (a group without work), odd numbers of steps, fewer steps than LDS stages, more tiles than
+one round.  Against numpy in float64; the bar for fp32 outputs is 1e-4 sqrt(K) of N(0, 1) x
+N(0, 0.3) products (fp32 accumulation errs by 6e-8 sqrt(K) of terms of size 0.3), for bf16 ones
+1e-2 (an ulp is 4e-3 of the element)."""
+import math
+
+import numpy as np
+import pytest
+
+from jaxpp_amd import runtime as rt
+from test_gpu_kernels import close, dev_bf16, rnd
+from oracle import layers as L
+
+pytestmark = pytest.mark.gpu
+
+LAYOUT = {"nn": (0, 1), "nt": (0, 0), "tn": (1, 1)}
+SIZES = [(128, 128, 64), (128, 256, 192), (256, 128, 320), (128, 384, 1088),  # 64x64, deep stages
+         (1152, 1280, 128), (1152, 1280, 448),                                  # more than 256 of them
+         (384, 128, 64)]
+
+
+@pytest.mark.parametrize("tile", [1, 5])
+@pytest.mark.parametrize("lay", LAYOUT)
+@pytest.mark.parametrize("m,n,k", SIZES)
+def test_small_tiles(lay, m, n, k, tile):
+    print(f"small tile {tile} {lay} {m}x{n}x{k}", flush=True)
+    ta, tb = LAYOUT[lay]
+    rng = np.random.default_rng(m + n + k + tile)
+    a, b = rnd(rng, m, k), rnd(rng, n, k, scale=0.3)
+    want = a.astype(np.float64) @ b.astype(np.float64).T
+    a_h, b_h = (np.ascontiguousarray(x.T) if t else x for x, t in ((a, ta), (b, tb)))
+    da, db = dev_bf16(a_h), dev_bf16(b_h)
+    args = (da.ptr, db.ptr)
+    dims = (m, n, k, a_h.shape[1], b_h.shape[1], n, ta, tb)
+    if lay != "nt":
+        prev = rng.standard_normal((m, n)).astype(np.float32)
+        dc = rt.DeviceBuffer.from_numpy(prev)
+        rt.gemm(*args, dc.ptr, *dims, rt.EPI_ACC_F32, tile=tile)
+        rt.sync()
+        close(dc.download(np.float32, (m, n)), prev + want, 1e-4 * math.sqrt(k), "accumulated")
+    dc = rt.DeviceBuffer(2 * m * n)
+    rt.gemm(*args, dc.ptr, *dims, rt.EPI_BF16, tile=tile)
+    rt.sync()
+    close(dc.download_bf16((m, n)), want, 1e-2, "bf16")
+
+
+@pytest.mark.parametrize("k", [64, 448])
+def test_rotated_heads_of_128_on_small_tiles(k):
+    """The rotated product is the plain one's bits rotated, whichever tile either takes."""
+    batch, seq, heads, rot, d = 1, 128, 5, 3, 128
+    rng = np.random.default_rng(k)
+    m, n = batch * seq, heads * d
+    da, dw = dev_bf16(rnd(rng, m, k)), dev_bf16(rnd(rng, k, n, scale=0.1))
+    cos, sin = (rt.DeviceBuffer.from_numpy(t) for t in L.rope_tables(seq, d, 5e5, np.float32))
+    plain, fused = rt.DeviceBuffer(2 * m * n), rt.DeviceBuffer(2 * m * n)
+    rt.gemm(da.ptr, dw.ptr, plain.ptr, m, n, k, k, n, n, 0, 1)
+    rt.check(rt.load().jpp_rope(None, plain.ptr, n, cos.ptr, sin.ptr, batch, seq, rot, d, 0))
+    rt.gemm(da.ptr, dw.ptr, fused.ptr, m, n, k, k, n, n, 0, 1, rope=(cos.ptr, sin.ptr, rot * d, seq, d))
+    rt.sync()
+    np.testing.assert_array_equal(fused.download_bf16((m, n)), plain.download_bf16((m, n)))
+
+
+@pytest.mark.parametrize("parts,k,shapes", [
+    (1, 64, [(128, 384), (128, 128), (128, 256), (256, 128)]),          # 28 tiles of 64x64
+    (3, 192, [(384, 128), (128, 640)]),                                  # nine steps over three pairs
+    (2, 128, [(768, 2304), (768, 768), (3072, 768)]),                    # more than 256 of 64x64
+    (1, 128, [(1408, 1408), (1408, 2816), (2816, 1408), (640, 1408)])])  # 128x128
+def test_small_weight_gradients_in_one_launch(parts, k, shapes):
+    rng = np.random.default_rng(parts + k)
+    probs, keep, wants = [], [], []
+    for m, n in shapes:
+        As = [rnd(rng, k, m) for _ in range(parts)]
+        Bs = [rnd(rng, k, n, scale=0.3) for _ in range(parts)]
+        prev = rng.standard_normal((m, n)).astype(np.float32)
+        wants.append(prev + sum(a.astype(np.float64).T @ b.astype(np.float64) for a, b in zip(As, Bs)))
+        dA, dB, dc = [dev_bf16(a) for a in As], [dev_bf16(b) for b in Bs], rt.DeviceBuffer.from_numpy(prev)
+        keep.append((dA, dB, dc))
+        probs.append(dict(a=dA[0].ptr, b=dB[0].ptr, c=dc.ptr, m=m, n=n, k=k, lda=m, ldb=n, ldc=n,
+                          more=[(a.ptr, b.ptr) for a, b in zip(dA[1:], dB[1:])]))
+    print(f"multi {parts} x {k} {shapes}", flush=True)
+    rt.gemm_multi(probs)
+    rt.sync()
+    for (_, _, dc), want, shape in zip(keep, wants, shapes):
+        close(dc.download(np.float32, shape), want, 1e-4 * math.sqrt(k * parts), f"multi {shape}")
+
+
+@pytest.mark.parametrize("counts", [[70, 0, 256, 3], [300, 1, 64, 129]])
+def test_small_grouped_products(counts):
+    """Row-grouped and contraction-grouped products that state how many rows hold data: small
+    ones leave the 256x256 tile."""
+    print(f"small groups {counts}", flush=True)
+    E, h, f = len(counts), 256, 512
+    rng = np.random.default_rng(sum(counts))
+    seg = np.concatenate([[0], np.cumsum([(c + 255) // 256 * 256 for c in counts])]).astype(np.int32)
+    cap = int(seg[-1]) + 256
+    x, dy = np.zeros((cap, h), np.float32), np.zeros((cap, f), np.float32)
+    for e, c in enumerate(counts):
+        x[seg[e]:seg[e] + c], dy[seg[e]:seg[e] + c] = rnd(rng, c, h), rnd(rng, c, f)
+    w = rnd(rng, E * h, f, scale=0.1)
+    b_seg = rt.DeviceBuffer.from_numpy(seg)
+    b_rows = rt.DeviceBuffer.from_numpy(np.asarray(counts, np.int32))
+    dx, ddy, dw, dc = dev_bf16(x), dev_bf16(dy), dev_bf16(w), rt.DeviceBuffer(2 * cap * f)
+    dc.zero()
+    rt.gemm(dx.ptr, dw.ptr, dc.ptr, cap, f, h, h, f, f, 0, 1, seg=b_seg.ptr, n_seg=E, group_mode=1,
+            stride_b=h * f, group_rows=sum(counts), seg_rows=b_rows.ptr)
+    acc = rng.standard_normal((E, h, f)).astype(np.float32)
+    dacc = rt.DeviceBuffer.from_numpy(acc)
+    rt.gemm(dx.ptr, ddy.ptr, dacc.ptr, h, f, 0, h, f, f, 1, 1, rt.EPI_ACC_F32, seg=b_seg.ptr, n_seg=E,
+            group_mode=2, stride_c=h * f, group_rows=2 * sum(counts), seg_rows=b_rows.ptr,
+            more=[(dx.ptr, ddy.ptr)], more_seg=[(b_seg.ptr, b_rows.ptr)])
+    rt.sync()
+    got = dc.download_bf16((cap, f))
+    assert not got[seg[E]:].any(), "rows past the last group are not written"
+    for e, c in enumerate(counts):
+        rows = slice(seg[e], seg[e] + c)
+        want = x[rows].astype(np.float64) @ w[e * h:(e + 1) * h].astype(np.float64)
+        if c:
+            close(got[rows], want, 1e-2, f"rows of group {e}")
+        want = acc[e] + 2 * x[rows].astype(np.float64).T @ dy[rows].astype(np.float64)
+        close(dacc.download(np.float32, (E, h, f))[e], want, 1e-4 * math.sqrt(2 * max(c, 1)), f"dW of group {e}")
