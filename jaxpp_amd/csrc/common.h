@@ -57,6 +57,9 @@ struct ProbeScope {
   }
 };
 
+// jpp_colsum_accum_f32 of up to four matrices with the same rows in one launch (f32_ops.hip)
+int jpp_colsum_f32_items(hipStream_t stream, int n, const jpp_colsum_item* items, int64_t rows);
+
 // -- bf16 <-> f32 -------------------------------------------------------------
 __device__ __forceinline__ float bf16_to_f32(bf16_t b) {
   return __uint_as_float(((uint32_t)b) << 16);

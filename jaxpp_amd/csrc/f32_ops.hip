@@ -3,9 +3,9 @@
 // float32, tests/test_transformations.py:42-93 builds its model in float32 too).  Same
 // argument structs as the bf16 entry points with every bf16 tensor replaced by an f32 one.
 //
-// These kernels serve small problems whose results must hold 1e-4 against an fp32 CPU run;
-// they are written for plain fp32 arithmetic in a fixed summation order (FMA chains over
-// the contraction index, row and column sums in index order), not for the matrix cores.
+// These kernels serve small problems whose results must hold 1e-4 against an fp32 CPU run:
+// fp32 arithmetic throughout, the contractions on the fp32 matrix instruction, every sum in an
+// order that the shapes fix.
 #include <math.h>
 
 #include "common.h"
@@ -63,11 +63,70 @@ struct SgemmParams {
   long stride_b, stride_c;
 };
 
-// 64x64 output tile, 16x16 threads of 4x4 outputs each, K in steps of 16 through LDS
+// operand vectors: 16 (8) bytes from addresses of which 4-byte alignment is known
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
+
+// One wave's fragments of an operand for 16 contraction elements: T subtiles of 16 rows, for
+// v_mfma_f32_16x16x4_f32.  Lane l (c = l % 16, g = l / 16) supplies row c of subtile i with
+// contraction element 4 g + s to MFMA s; any order serves as long as both operands share it,
+// and this one makes every load a vector of the operand's contiguous index:
+//   SLOW = false  [rows][k]: row 16 i + c, elements 4 g .. 4 g + 3 in one load per subtile
+//   SLOW = true   [k][rows]: rows T c .. T c + T - 1 (row T c + i belongs to subtile i) of
+//                 contraction element 4 g + s in one load per s
+template <int T, bool SLOW>
+struct Frag32 {
+  float v[T][4];
+  __device__ __forceinline__ void load(const float* p, long ld) {
+    if constexpr (!SLOW) {
+#pragma unroll
+      for (int i = 0; i < T; ++i) {
+        const f32x4_u q = *(const f32x4_u*)(p + 16 * i * ld);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) v[i][s] = q[s];
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if constexpr (T == 4) {
+          const f32x4_u q = *(const f32x4_u*)(p + s * ld);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i][s] = q[i];
+        } else if constexpr (T == 2) {
+          const f32x2_u q = *(const f32x2_u*)(p + s * ld);
+          v[0][s] = q[0];
+          v[1][s] = q[1];
+        } else {
+          v[0][s] = p[s * ld];
+        }
+      }
+    }
+  }
+  // this lane's first element of the tile whose first row and contraction element are `p`
+  static __device__ __forceinline__ const float* lane_ptr(const float* p, long ld, int c, int g) {
+    return SLOW ? p + 4 * g * ld + T * c : p + c * ld + 4 * g;
+  }
+};
+
+// A workgroup owns BM x 64 outputs; its four waves each multiply the whole tile over every
+// fourth step of 16 contraction elements, and their four sums meet in LDS in wave order.
+// These products are small (512 x 256 x 256 and a few times that): what bounds them is latency,
+// so the work is spread over as many CUs as the tile allows and inside a CU over the
+// contraction, and operands go from L2 straight into MFMA fragments - no barrier and no LDS
+// before the sums, D steps of loads in flight per wave.  v_mfma_f32_16x16x4_f32 accumulates as
+// a chain of fused multiply-adds does, at twice the rate of v_fma_f32; the four shorter chains
+// halve the distance to a float64 sum (5.7e-7 -> 2.9e-7 at k = 1024).  512 x 256 x 256 takes
+// 6.5 us, 512 x 256 x 1024 9.7 us; the 64 x 64 tile of 16 x 16 threads in its place, one barrier
+// pair per 16 contraction elements on 32 CUs, and attention with a pair of lanes per row made a
+// two-layer row of eight microbatches of 512 tokens 30.0 ms, now 2.30 ms.
+template <int BM, bool TA, bool TB>
 __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
-  __shared__ float As[16][68], Bs[16][68];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const long m0 = (long)blockIdx.y * 64, n0 = (long)blockIdx.x * 64;
+  constexpr int TM = BM / 16, TN = 4, D = BM == 64 ? 2 : 4, PITCH = 68;
+  __shared__ float part[2][4][16 * PITCH];
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tiles_n = p.n / 64;
+  const long m0 = (long)(blockIdx.x / tiles_n) * BM, n0 = (long)(blockIdx.x % tiles_n) * 64;
   if (p.group_mode == JPP_GROUP_M) {
     // rows of A and C are grouped by expert; each group multiplies its own B
     if (m0 >= p.seg[p.n_seg]) return;
@@ -83,86 +142,127 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
     p.b += r0 * p.ldb;
     p.c += (long)e * p.stride_c;
   }
-  float acc[4][4];
+  // the epilogue's 16 rows at a time: pass i holds subtile i, a thread four columns of a row
+  const int er = tid >> 4, eq = (tid & 15) * 4;
+  const long col = n0 + eq;
+  auto out_row = [&](int i) { return m0 + (TA ? TM * er + i : 16 * i + er); };
+  // what the epilogue adds or multiplies with arrives during the contraction
+  const float* pre_src = p.epi == JPP_EPI_ACC_F32 ? p.c : p.epi == JPP_EPI_DGELU ? p.aux
+                         : p.epi == JPP_EPI_BF16 ? p.resid : nullptr;
+  const long pre_ld = p.epi == JPP_EPI_ACC_F32 ? p.ldc : p.epi == JPP_EPI_DGELU ? p.ldaux : p.ldresid;
+  f32x4 pre[TM];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < TM; ++i)
+    pre[i] = pre_src ? (f32x4)*(const f32x4_u*)(pre_src + out_row(i) * pre_ld + col) : f32x4{0.f, 0.f, 0.f, 0.f};
+
+  typedef Frag32<TM, TA> FA;
+  typedef Frag32<TN, TB> FB;
+  f32x4 acc[TM][TN];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-  for (int k0 = 0; k0 < p.k; k0 += 16) {
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int e = tid + 256 * i;
-      // consecutive threads follow the operand's contiguous index
-      if (p.ta) {
-        const int mm = e & 63, kk = e >> 6;
-        As[kk][mm] = p.a[(long)(k0 + kk) * p.lda + m0 + mm];
-      } else {
-        const int kk = e & 15, mm = e >> 4;
-        As[kk][mm] = p.a[(m0 + mm) * p.lda + k0 + kk];
-      }
-      if (p.tb) {
-        const int nn = e & 63, kk = e >> 6;
-        Bs[kk][nn] = p.b[(long)(k0 + kk) * p.ldb + n0 + nn];
-      } else {
-        const int kk = e & 15, nn = e >> 4;
-        Bs[kk][nn] = p.b[(n0 + nn) * p.ldb + k0 + kk];
-      }
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = (p.k / 16 - wave + 3) / 4;   // wave, wave + 4, ...
+  if (steps > 0) {
+    const long step_a = TA ? 64 * p.lda : 64, step_b = TB ? 64 * p.ldb : 64;
+    const float* pa = FA::lane_ptr(p.a + (TA ? m0 : m0 * p.lda), p.lda, c, g) + wave * (step_a / 4);
+    const float* pb = FB::lane_ptr(p.b + (TB ? n0 : n0 * p.ldb), p.ldb, c, g) + wave * (step_b / 4);
+    FA fa[D];
+    FB fb[D];
+#pragma unroll
+    for (int u = 0; u < D - 1; ++u) {
+      fa[u].load(pa + min(u, steps - 1) * step_a, p.lda);
+      fb[u].load(pb + min(u, steps - 1) * step_b, p.ldb);
     }
-    __syncthreads();
+    for (int t = 0; t < steps; t += D) {
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const float4 av = *(const float4*)&As[kk][ty * 4];
-      const float4 bv = *(const float4*)&Bs[kk][tx * 4];
-      const float a4[4] = {av.x, av.y, av.z, av.w}, b4[4] = {bv.x, bv.y, bv.z, bv.w};
+      for (int u = 0; u < D; ++u) {
+        // (past the end the last step is fetched again, unused)
+        const long nt = min(t + u + D - 1, steps - 1);
+        fa[(u + D - 1) % D].load(pa + nt * step_a, p.lda);
+        fb[(u + D - 1) % D].load(pb + nt * step_b, p.ldb);
+        if (t + u < steps) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+          for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a4[i], b4[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const long row = m0 + ty * 4 + i;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const long col = n0 + tx * 4 + j;
-      float v = acc[i][j];
-      if (p.epi == JPP_EPI_ACC_F32) {
-        p.c[row * p.ldc + col] += v;
-        continue;
+              for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[u].v[j][s], fa[u].v[i][s], acc[i][j], 0, 0, 0);
+        }
       }
-      if (p.epi == JPP_EPI_SWIGLU) {
-        // a 64-column tile is one block of the interleaved layout: gate features in its first
-        // 32 columns (threads tx < 8), the matching up features 32 columns on (thread tx + 8,
-        // lane + 8 of the same wave)
-        p.c[row * p.ldc + col] = v;
-        const float other = __shfl_xor(v, 8);
-        if (tx < 8) p.c2[row * p.ldc2 + n0 / 2 + tx * 4 + j] = swiglu32(v, other);
-        continue;
-      }
-      if (p.epi == JPP_EPI_DSWIGLU) {
-        // v = d s of feature `col`; gate / up of that feature sit at 64 q + w and 64 q + 32 + w
-        const long q = col >> 5, w = col & 31;
-        const float* arow = p.aux + row * p.ldaux + 64 * q + w;
-        float dg, du;
-        swiglu_grad32(arow[0], arow[32], v, dg, du);
-        float* crow = p.c + row * p.ldc + 64 * q + w;
-        crow[0] = dg;
-        crow[32] = du;
-        continue;
-      }
-      if (p.bias) v += p.bias[col];
-      if (p.epi == JPP_EPI_GELU) {
-        p.c2[row * p.ldc2 + col] = gelu32(v, p.gelu_tanh);
-      } else if (p.epi == JPP_EPI_DGELU) {
-        v *= gelu_grad32(p.aux[row * p.ldaux + col], p.gelu_tanh);
-      } else if (p.resid) {
-        v += p.resid[row * p.ldresid + col];
-      }
-      p.c[row * p.ldc + col] = v;
     }
   }
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    // lane (c, g): row c of subtile i and, of column subtile j, the four indices 4 g + r
+    float* mine = &part[i & 1][wave][c * PITCH];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *(f32x4*)(mine + 16 * (TB ? g : j) + 4 * (TB ? j : g)) =
+          TB ? f32x4{acc[i][0][j], acc[i][1][j], acc[i][2][j], acc[i][3][j]} : acc[i][j];
+    __syncthreads();
+    const float* src = &part[i & 1][0][er * PITCH + eq];
+    f32x4 v = *(const f32x4*)src;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) v += *(const f32x4*)(src + w * 16 * PITCH);
+    const long row = out_row(i);
+    float* const dst = p.c + row * p.ldc + col;
+    if (p.epi == JPP_EPI_ACC_F32) {
+      *(f32x4_u*)dst = pre[i] + v;
+      continue;
+    }
+    if (p.epi == JPP_EPI_SWIGLU) {
+      // a 64-column tile is one block of the interleaved layout: gate features in its first
+      // 32 columns (threads eq < 32), the matching up features 32 columns on (lane + 8)
+      *(f32x4_u*)dst = v;
+      f32x4 s;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] = swiglu32(v[e], __shfl_xor(v[e], 8));
+      if (eq < 32) *(f32x4_u*)(p.c2 + row * p.ldc2 + n0 / 2 + eq) = s;
+      continue;
+    }
+    if (p.epi == JPP_EPI_DSWIGLU) {
+      // v = d s of features col .. col + 3; gate / up of feature f sit at 64 (f / 32) + f % 32
+      // and 32 behind it
+      const long at = 64 * (col >> 5) + (col & 31);
+      const f32x4 gate = *(const f32x4_u*)(p.aux + row * p.ldaux + at);
+      const f32x4 up = *(const f32x4_u*)(p.aux + row * p.ldaux + at + 32);
+      f32x4 dg, du;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float x, y;
+        swiglu_grad32(gate[e], up[e], v[e], x, y);
+        dg[e] = x;
+        du[e] = y;
+      }
+      *(f32x4_u*)(p.c + row * p.ldc + at) = dg;
+      *(f32x4_u*)(p.c + row * p.ldc + at + 32) = du;
+      continue;
+    }
+    if (p.bias) v += (f32x4)*(const f32x4_u*)(p.bias + col);
+    if (p.epi == JPP_EPI_GELU) {
+      f32x4 s;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] = gelu32(v[e], p.gelu_tanh);
+      *(f32x4_u*)(p.c2 + row * p.ldc2 + col) = s;
+    } else if (p.epi == JPP_EPI_DGELU) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] *= gelu_grad32(pre[i][e], p.gelu_tanh);
+    } else if (p.resid) {
+      v += p.epi == JPP_EPI_BF16 ? pre[i] : (f32x4)*(const f32x4_u*)(p.resid + row * p.ldresid + col);
+    }
+    *(f32x4_u*)dst = v;
+  }
+}
+
+template <int BM>
+void sgemm_launch(hipStream_t st, const SgemmParams& p) {
+  const dim3 grid((unsigned)(p.m / BM * (p.n / 64)), 1u, p.group_mode == JPP_GROUP_K ? (unsigned)p.n_seg : 1u);
+  if (p.ta && p.tb) hipLaunchKernelGGL((sgemm_kernel<BM, true, true>), grid, dim3(256), 0, st, p);
+  else if (p.ta) hipLaunchKernelGGL((sgemm_kernel<BM, true, false>), grid, dim3(256), 0, st, p);
+  else if (p.tb) hipLaunchKernelGGL((sgemm_kernel<BM, false, true>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((sgemm_kernel<BM, false, false>), grid, dim3(256), 0, st, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -200,15 +300,80 @@ __global__ __launch_bounds__(256) void norm_fwd32_kernel(const float* __restrict
   }
 }
 
-__global__ __launch_bounds__(256) void norm_bwd32_kernel(const float* __restrict__ dy,
-                                                         const float* __restrict__ x,
-                                                         const float* mean_in,
-                                                         const float* __restrict__ rstd_in,
-                                                         const float* __restrict__ gamma,
-                                                         const float* resid, float* __restrict__ dx,
-                                                         long rows, int cols) {
+// Column sums of 16 adjacent columns over all rows by one workgroup of 1024 threads: thread
+// (rg, c) = (tid / 16, tid % 16) adds rows rg, rg + 64, ... of column c, the 64 sums of a column
+// meet first inside a wave (4 of them), then in wave order.  These sums are latency and nothing
+// else: one thread per column walks its rows one load after another, 4 to 16 waves on the whole
+// device.  Spread like this a thread's loads are in flight together: the four bias gradients of
+// a layer of hidden 256 on 512 tokens 4.8 us in one launch, a norm's backward 4.9 us.
+struct ColSum {
+  float a, b;
+};
+template <typename Load>
+__device__ __forceinline__ ColSum column_sums(long rows, Load load) {
+  __shared__ ColSum red[16][16];
+  const int tid = threadIdx.x, c = tid & 15, wave = tid >> 6;
+  ColSum s = {0.f, 0.f};
+  long r = tid >> 4;
+  for (; r + 7 * 64 < rows; r += 8 * 64) {
+    ColSum v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = load(r + i * 64);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      s.a += v[i].a;
+      s.b += v[i].b;
+    }
+  }
+  for (; r < rows; r += 64) {
+    const ColSum v = load(r);
+    s.a += v.a;
+    s.b += v.b;
+  }
+#pragma unroll
+  for (int o = 16; o < 64; o <<= 1) {
+    s.a += __shfl_xor(s.a, o);
+    s.b += __shfl_xor(s.b, o);
+  }
+  if ((tid & 63) < 16) red[wave][c] = s;
+  __syncthreads();
+  ColSum t = {0.f, 0.f};
+  if (tid < 16)
+    for (int w = 0; w < 16; ++w) {
+      t.a += red[w][c].a;
+      t.b += red[w][c].b;
+    }
+  return t;   // (threads 0 .. 15)
+}
+
+// Both halves of a norm's backward in one launch (they read the same tensors and neither reads
+// what the other writes): the first `row_blocks` workgroups take 16 rows each, one wave per
+// row, for dx; each of the others the parameter gradients of 16 columns,
+// dgamma[c] += sum_r dy[r,c] xhat[r,c], dbeta[c] += sum_r dy[r,c].
+__global__ __launch_bounds__(1024) void norm_bwd32_kernel(const float* __restrict__ dy,
+                                                          const float* __restrict__ x,
+                                                          const float* mean_in,
+                                                          const float* __restrict__ rstd_in,
+                                                          const float* __restrict__ gamma,
+                                                          const float* resid, float* __restrict__ dx,
+                                                          float* dgamma, float* dbeta, long rows,
+                                                          int cols, int row_blocks) {
+  if ((int)blockIdx.x >= row_blocks) {
+    const int col = ((int)blockIdx.x - row_blocks) * 16 + (threadIdx.x & 15);
+    const bool in = col < cols;
+    const ColSum s = column_sums(in ? rows : 0, [&](long r) {
+      const float d = dy[r * cols + col];
+      const float mean = mean_in ? mean_in[r] : 0.f;
+      return ColSum{d * (x[r * cols + col] - mean) * rstd_in[r], d};
+    });
+    if (threadIdx.x < 16 && in) {
+      dgamma[col] += s.a;
+      if (dbeta) dbeta[col] += s.b;
+    }
+    return;
+  }
   const int lane = threadIdx.x & 63;
-  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long row = (long)blockIdx.x * 16 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const float rstd = rstd_in[row], mean = mean_in ? mean_in[row] : 0.f;
   const float* xr = x + row * cols;
@@ -229,53 +394,56 @@ __global__ __launch_bounds__(256) void norm_bwd32_kernel(const float* __restrict
   }
 }
 
-// dgamma[c] += sum_r dy[r,c] xhat[r,c]; dbeta[c] += sum_r dy[r,c]: a thread per column, rows
-// in index order
-__global__ __launch_bounds__(64) void norm_wgrad32_kernel(const float* __restrict__ dy,
-                                                          const float* __restrict__ x,
-                                                          const float* mean_in,
-                                                          const float* __restrict__ rstd_in,
-                                                          float* dgamma, float* dbeta, long rows,
-                                                          int cols) {
-  const int c = blockIdx.x * 64 + threadIdx.x;
-  if (c >= cols) return;
-  float g = 0.f, b = 0.f;
-  for (long r = 0; r < rows; ++r) {
-    const float d = dy[r * cols + c];
-    const float mean = mean_in ? mean_in[r] : 0.f;
-    g += d * (x[r * cols + c] - mean) * rstd_in[r];
-    b += d;
-  }
-  dgamma[c] += g;
-  if (dbeta) dbeta[c] += b;
-}
-
-// acc[c] += sum_r x[r,c]
-__global__ __launch_bounds__(64) void colsum32_kernel(const float* __restrict__ x, long ld,
-                                                      long rows, int cols, float* acc) {
-  const int c = blockIdx.x * 64 + threadIdx.x;
-  if (c >= cols) return;
-  float s = 0.f;
-  for (long r = 0; r < rows; ++r) s += x[r * ld + c];
-  acc[c] += s;
+// acc[c] += sum_r x[r,c] of up to four matrices with the same rows; `first[i]`: first workgroup
+// of matrix i (past the grid where there is none)
+struct ColItems32 {
+  const float* x[4];
+  float* acc[4];
+  long ld[4];
+  int cols[4], first[4];
+};
+__global__ __launch_bounds__(1024) void colsum32_kernel(ColItems32 p, long rows) {
+  const int blk = blockIdx.x;
+  const bool s1 = blk >= p.first[1], s2 = blk >= p.first[2], s3 = blk >= p.first[3];
+#define JPP_PICK(field) (s3 ? p.field[3] : s2 ? p.field[2] : s1 ? p.field[1] : p.field[0])
+  const float* const x = JPP_PICK(x);
+  float* const acc = JPP_PICK(acc);
+  const long ld = JPP_PICK(ld);
+  const int cols = JPP_PICK(cols), col = (blk - JPP_PICK(first)) * 16 + (threadIdx.x & 15);
+#undef JPP_PICK
+  const bool in = col < cols;
+  const ColSum s = column_sums(in ? rows : 0, [&](long r) { return ColSum{x[r * ld + col], 0.f}; });
+  if (threadIdx.x < 16 && in) acc[col] += s.a;
 }
 
 // loss = scale * mean((out - target)^2), dout = scale * 2 (out - target) / count: one
-// workgroup, partial sums per thread in index order, then a fixed tree
-__global__ __launch_bounds__(256) void mse32_kernel(const float* __restrict__ out,
-                                                    const float* __restrict__ target, long count,
-                                                    float scale, float* loss, float* dout) {
-  __shared__ float red[256];
+// workgroup, partial sums per thread in index order (eight elements' loads in flight), then a
+// fixed tree
+__global__ __launch_bounds__(1024) void mse32_kernel(const float* __restrict__ out,
+                                                     const float* __restrict__ target, long count,
+                                                     float scale, float* loss, float* dout) {
+  __shared__ float red[1024];
   float s = 0.f;
   const float k = scale * 2.0f / (float)count;
-  for (long i = threadIdx.x; i < count; i += 256) {
+  long i = threadIdx.x;
+  for (; i + 7 * 1024 < count; i += 8 * 1024) {
+    float d[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) d[e] = out[i + e * 1024] - target[i + e * 1024];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      s += d[e] * d[e];
+      if (dout) dout[i + e * 1024] = k * d[e];
+    }
+  }
+  for (; i < count; i += 1024) {
     const float d = out[i] - target[i];
     s += d * d;
     if (dout) dout[i] = k * d;
   }
   red[threadIdx.x] = s;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
+  for (int w = 512; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
     __syncthreads();
   }
@@ -305,9 +473,17 @@ __global__ __launch_bounds__(256) void rope32_kernel(float* __restrict__ x, long
 }
 
 // ---------------------------------------------------------------------------
-// Attention.  A row (query or key) belongs to a pair of adjacent lanes, each holding half
-// of the head dimension; dot products over the head dimension are the sum of the pair's
-// halves.  The other side's rows pass through LDS 32 at a time.
+// Attention on the fp32 matrix instruction, 16 rows of one side per workgroup: its waves take
+// the other side's tiles of 16 rows in turn and meet in LDS, in wave order, at the end.  Sizes
+// here are small (16 sequences and heads of 128 positions), so a workgroup per 16 rows and the
+// split over its waves are what fills the device; operands go from L2 straight into MFMA
+// fragments.  With c = lane % 16 and g = lane / 16, three layouts fit each other unchanged:
+//   row fragment   row c, elements 16 t + 4 g .. + 3 of the head dimension: operand of a
+//                  product over the head dimension
+//   score tile     its result: row 4 g + r of the A side, row c of the B side in register r -
+//                  which is the B operand of a product over the A side's rows
+//   column frag.   row 4 g + r, elements 64 t + 4 c .. + 3: the A operand of that product; its
+//                  result holds elements 64 t + 16 g + 4 r + j of row c (tile 4 t + j, register r)
 // ---------------------------------------------------------------------------
 struct Attn32 {
   const float *q, *k, *v, *d_o;
@@ -317,170 +493,246 @@ struct Attn32 {
   float scale;
 };
 
-__device__ __forceinline__ float pair_sum(float v) { return v + __shfl_xor(v, 1); }
+// (eight waves where their partial results and fragments have room, two per SIMD)
+template <int D>
+constexpr int kAttnWaves32 = D == 64 ? 8 : 4;
 
 template <int D>
-__global__ __launch_bounds__(128) void attn_fwd32_kernel(Attn32 p) {
-  constexpr int H = D / 2;
-  __shared__ float Ks[32][D], Vs[32][D];
-  const int tid = threadIdx.x, r = tid >> 1, half = tid & 1;
-  const int h = blockIdx.y, b = blockIdx.z, hk = h / (p.n_heads / p.n_kv_heads);
-  const int qi = blockIdx.x * 64 + r;
-  const long row0 = (long)b * p.seq;
-  float q[H], o[H];
+struct Rows32 {   // row fragments of 16 rows
+  f32x4 v[D / 16];
+  __device__ __forceinline__ void load(const float* p, long ld, int c, int g) {
 #pragma unroll
-  for (int d = 0; d < H; ++d) {
-    q[d] = p.q[(row0 + qi) * p.ldq + h * D + half * H + d];
-    o[d] = 0.f;
+    for (int t = 0; t < D / 16; ++t) v[t] = *(const f32x4_u*)(p + c * ld + 16 * t + 4 * g);
   }
-  float m = -INFINITY, l = 0.f;
-  const int kend = p.causal ? blockIdx.x * 64 + 64 : p.seq;
-  for (int k0 = 0; k0 < kend; k0 += 32) {
-    __syncthreads();
-    for (int e = tid; e < 32 * D; e += 128) {
-      const int kr = e / D, d = e % D;
-      Ks[kr][d] = p.k[(row0 + k0 + kr) * p.ldk + hk * D + d];
-      Vs[kr][d] = p.v[(row0 + k0 + kr) * p.ldv + hk * D + d];
+};
+template <int D>
+struct Cols32 {   // column fragments of 16 rows
+  f32x4 v[4][D / 64];
+  __device__ __forceinline__ void load(const float* p, long ld, int c, int g) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < D / 64; ++t) v[r][t] = *(const f32x4_u*)(p + (4 * g + r) * ld + 64 * t + 4 * c);
+  }
+};
+// score tile of two sets of 16 rows
+template <int D>
+__device__ __forceinline__ f32x4 score32(const Rows32<D>& a, const Rows32<D>& b) {
+  // two chains: an MFMA's result is the next one's input after 8 passes
+  f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+  for (int t = 0; t < D / 16; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f32x4& s = e & 1 ? s1 : s0;
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[t][e], b.v[t][e], s, 0, 0, 0);
     }
-    __syncthreads();
-    float s[32];
+  return s0 + s1;
+}
+// acc += (columns of the A side's 16 rows)^T (score tile)
+template <int D>
+__device__ __forceinline__ void outer32(f32x4 (&acc)[D / 16], const Cols32<D>& a, const f32x4& s) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int t = 0; t < D / 64; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[4 * t + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[r][t][j], s[r], acc[4 * t + j], 0, 0, 0);
+}
+// sum and maximum over the four lanes that share c
+__device__ __forceinline__ float quad_sum(float v) {
+  v += __shfl_xor(v, 16);
+  return v + __shfl_xor(v, 32);
+}
+__device__ __forceinline__ float quad_max(float v) {
+  v = fmaxf(v, __shfl_xor(v, 16));
+  return fmaxf(v, __shfl_xor(v, 32));
+}
+// The waves' accumulators, added in wave order, to 16 rows of `out`; `buf`: W x 16 x D floats of
+// LDS that no wave reads any more.  Register r of tile 4 t + j, lane (c, g) is element
+// 64 t + 16 g + 4 r + j of row c.
+template <int D, int W>
+__device__ __forceinline__ void store_sum32(const f32x4 (&acc)[D / 16], float* buf, float* out, long ld) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < D / 64; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *(f32x4*)(buf + ((wave * (D / 64) + t) * 4 + r) * 256 + lane * 4) =
+          f32x4{acc[4 * t][r], acc[4 * t + 1][r], acc[4 * t + 2][r], acc[4 * t + 3][r]};
+  __syncthreads();
+  // piece (t, r) of lane (c, g) is out[c][64 t + 16 g + 4 r ..]
+  for (int i = tid; i < 16 * D / 4; i += 64 * W) {
+    const int row = i / (D / 4), piece = i % (D / 4), t = piece / 16, pg = (piece >> 2) & 3, r = piece & 3;
+    const float* src = buf + (t * 4 + r) * 256 + (pg * 16 + row) * 4;
+    f32x4 v = *(const f32x4*)src;
+#pragma unroll
+    for (int w = 1; w < W; ++w) v += *(const f32x4*)(src + w * 16 * D);
+    *(f32x4_u*)(out + row * ld + piece * 4) = v;
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_fwd32_kernel(Attn32 p) {
+  constexpr int W = kAttnWaves32<D>;
+  __shared__ float buf[W * 16 * D];
+  __shared__ float ms[W][16], ls[W][16];
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = blockIdx.y, b = blockIdx.z, hk = h / (p.n_heads / p.n_kv_heads);
+  const int q0 = blockIdx.x * 16;
+  const long row0 = (long)b * p.seq;
+  Rows32<D> q;
+  q.load(p.q + (row0 + q0) * p.ldq + h * D, p.ldq, c, g);
+  f32x4 o[D / 16];
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  const int kend = p.causal ? q0 + 16 : p.seq;
+  const float* kp = p.k + row0 * p.ldk + hk * D;
+  const float* vp = p.v + row0 * p.ldv + hk * D;
+  for (int k0 = wave * 16; k0 < kend; k0 += W * 16) {
+    Rows32<D> kr;
+    Cols32<D> vc;
+    kr.load(kp + k0 * p.ldk, p.ldk, c, g);
+    vc.load(vp + k0 * p.ldv, p.ldv, c, g);
+    f32x4 s = score32<D>(kr, q);
     float mx = m;
 #pragma unroll
-    for (int j = 0; j < 32; ++j) {
-      float t = 0.f;
-#pragma unroll
-      for (int d = 0; d < H; ++d) t = fmaf(q[d], Ks[j][half * H + d], t);
-      t = pair_sum(t) * p.scale;
-      if (p.causal && k0 + j > qi) t = -INFINITY;
-      s[j] = t;
-      mx = fmaxf(mx, t);
+    for (int r = 0; r < 4; ++r) {
+      s[r] *= p.scale;
+      if (p.causal && k0 + 4 * g + r > q0 + c) s[r] = -INFINITY;
+      mx = fmaxf(mx, s[r]);
     }
-    const float alpha = __expf(m - mx);   // m = -inf on the first tile: alpha = 0, o = l = 0
+    mx = quad_max(mx);
+    // (a row whose scores so far are all -inf keeps a sum of zero)
+    const float base = mx == -INFINITY ? 0.f : mx;
+    const float alpha = expf(m - base);
+    m = mx;
     l *= alpha;
 #pragma unroll
-    for (int d = 0; d < H; ++d) o[d] *= alpha;
-    m = mx;
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-      const float e = expf(s[j] - m);
-      l += e;
-#pragma unroll
-      for (int d = 0; d < H; ++d) o[d] = fmaf(e, Vs[j][half * H + d], o[d]);
+    for (int r = 0; r < 4; ++r) {
+      s[r] = expf(s[r] - base);
+      l += s[r];
     }
-  }
-  const float inv = 1.0f / l;
 #pragma unroll
-  for (int d = 0; d < H; ++d) p.o[(row0 + qi) * p.ldo + h * D + half * H + d] = o[d] * inv;
-  if (half == 0) p.lse[((long)b * p.n_heads + h) * p.seq + qi] = m + logf(l);
+    for (int i = 0; i < D / 16; ++i) o[i] *= alpha;
+    outer32<D>(o, vc, s);
+  }
+  l = quad_sum(l);
+  if (g == 0) {
+    ms[wave][c] = m;
+    ls[wave][c] = l;
+  }
+  __syncthreads();
+  float mall = ms[0][c];
+#pragma unroll
+  for (int w = 1; w < W; ++w) mall = fmaxf(mall, ms[w][c]);
+  const float base = mall == -INFINITY ? 0.f : mall;
+  float lall = 0.f;
+#pragma unroll
+  for (int w = 0; w < W; ++w) lall += ls[w][c] * expf(ms[w][c] - base);
+  const float f = expf(m - base) / lall;
+#pragma unroll
+  for (int i = 0; i < D / 16; ++i) o[i] *= f;
+  store_sum32<D, W>(o, buf, p.o + (row0 + q0) * p.ldo + h * D, p.ldo);
+  if (threadIdx.x < 16) p.lse[((long)b * p.n_heads + h) * p.seq + q0 + c] = mall + logf(lall);
 }
 
-// dQ (a pair of lanes per query), and delta = rowsum(dO o O) for the dK/dV kernel
+// dQ of 16 queries, and delta = rowsum(dO o O) for the dK/dV kernel
 template <int D>
-__global__ __launch_bounds__(128) void attn_dq32_kernel(Attn32 p) {
-  constexpr int H = D / 2;
-  __shared__ float Ks[32][D], Vs[32][D];
-  const int tid = threadIdx.x, r = tid >> 1, half = tid & 1;
+__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dq32_kernel(Attn32 p) {
+  constexpr int W = kAttnWaves32<D>;
+  __shared__ float buf[W * 16 * D];
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = blockIdx.y, b = blockIdx.z, hk = h / (p.n_heads / p.n_kv_heads);
-  const int qi = blockIdx.x * 64 + r;
+  const int q0 = blockIdx.x * 16;
   const long row0 = (long)b * p.seq;
-  float q[H], g[H], dq[H];
+  Rows32<D> q, go;
+  q.load(p.q + (row0 + q0) * p.ldq + h * D, p.ldq, c, g);
+  go.load(p.d_o + (row0 + q0) * p.lddo + h * D, p.lddo, c, g);
   float dl = 0.f;
+  {
+    Rows32<D> o;
+    o.load(p.o + (row0 + q0) * p.ldo + h * D, p.ldo, c, g);
 #pragma unroll
-  for (int d = 0; d < H; ++d) {
-    q[d] = p.q[(row0 + qi) * p.ldq + h * D + half * H + d];
-    g[d] = p.d_o[(row0 + qi) * p.lddo + h * D + half * H + d];
-    dl = fmaf(g[d], p.o[(row0 + qi) * p.ldo + h * D + half * H + d], dl);
-    dq[d] = 0.f;
+    for (int t = 0; t < D / 16; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dl = fmaf(go.v[t][e], o.v[t][e], dl);
   }
-  dl = pair_sum(dl);
-  const long stat = ((long)b * p.n_heads + h) * p.seq + qi;
-  if (half == 0) p.delta[stat] = dl;
+  dl = quad_sum(dl);
+  const long stat = ((long)b * p.n_heads + h) * p.seq + q0 + c;
+  if (wave == 0 && g == 0) p.delta[stat] = dl;
   const float lse = p.lse[stat];
-  const int kend = p.causal ? blockIdx.x * 64 + 64 : p.seq;
-  for (int k0 = 0; k0 < kend; k0 += 32) {
-    __syncthreads();
-    for (int e = tid; e < 32 * D; e += 128) {
-      const int kr = e / D, d = e % D;
-      Ks[kr][d] = p.k[(row0 + k0 + kr) * p.ldk + hk * D + d];
-      Vs[kr][d] = p.v[(row0 + k0 + kr) * p.ldv + hk * D + d];
-    }
-    __syncthreads();
-#pragma unroll 1
-    for (int j = 0; j < 32; ++j) {
-      float t = 0.f, dp = 0.f;
+  f32x4 dq[D / 16];
 #pragma unroll
-      for (int d = 0; d < H; ++d) {
-        t = fmaf(q[d], Ks[j][half * H + d], t);
-        dp = fmaf(g[d], Vs[j][half * H + d], dp);
-      }
-      t = pair_sum(t) * p.scale;
-      dp = pair_sum(dp);
-      const float pr = (p.causal && k0 + j > qi) ? 0.f : expf(t - lse);
-      const float ds = pr * (dp - dl) * p.scale;
+  for (int i = 0; i < D / 16; ++i) dq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int kend = p.causal ? q0 + 16 : p.seq;
+  const float* kp = p.k + row0 * p.ldk + hk * D;
+  const float* vp = p.v + row0 * p.ldv + hk * D;
+  for (int k0 = wave * 16; k0 < kend; k0 += W * 16) {
+    Rows32<D> kr, vr;
+    Cols32<D> kc;
+    kr.load(kp + k0 * p.ldk, p.ldk, c, g);
+    vr.load(vp + k0 * p.ldv, p.ldv, c, g);
+    kc.load(kp + k0 * p.ldk, p.ldk, c, g);
+    f32x4 s = score32<D>(kr, q);
+    const f32x4 dp = score32<D>(vr, go);
 #pragma unroll
-      for (int d = 0; d < H; ++d) dq[d] = fmaf(ds, Ks[j][half * H + d], dq[d]);
+    for (int r = 0; r < 4; ++r) {
+      const float pr = (p.causal && k0 + 4 * g + r > q0 + c) ? 0.f : expf(s[r] * p.scale - lse);
+      s[r] = pr * (dp[r] - dl) * p.scale;
     }
+    outer32<D>(dq, kc, s);
   }
-#pragma unroll
-  for (int d = 0; d < H; ++d) p.dq[(row0 + qi) * p.lddq + h * D + half * H + d] = dq[d];
+  store_sum32<D, W>(dq, buf, p.dq + (row0 + q0) * p.lddq + h * D, p.lddq);
 }
 
-// dK, dV (a pair of lanes per key): the queries of every head of the key's group, in order
+// dK, dV of 16 keys: the waves take the 16-query tiles of every head of the keys' group in turn
 template <int D>
-__global__ __launch_bounds__(128) void attn_dkv32_kernel(Attn32 p) {
-  constexpr int H = D / 2;
-  __shared__ float Qs[32][D], Gs[32][D], Ls[32], Ds[32];
-  const int tid = threadIdx.x, r = tid >> 1, half = tid & 1;
+__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dkv32_kernel(Attn32 p) {
+  constexpr int W = kAttnWaves32<D>;
+  __shared__ float buf[W * 16 * D];
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hk = blockIdx.y, b = blockIdx.z, grp = p.n_heads / p.n_kv_heads;
-  const int kj = blockIdx.x * 64 + r;
+  const int k0 = blockIdx.x * 16;
   const long row0 = (long)b * p.seq;
-  float k[H], v[H], dk[H], dv[H];
+  Rows32<D> kr, vr;
+  kr.load(p.k + (row0 + k0) * p.ldk + hk * D, p.ldk, c, g);
+  vr.load(p.v + (row0 + k0) * p.ldv + hk * D, p.ldv, c, g);
+  f32x4 dk[D / 16], dv[D / 16];
 #pragma unroll
-  for (int d = 0; d < H; ++d) {
-    k[d] = p.k[(row0 + kj) * p.ldk + hk * D + half * H + d];
-    v[d] = p.v[(row0 + kj) * p.ldv + hk * D + half * H + d];
-    dk[d] = dv[d] = 0.f;
-  }
-  const int qbeg = p.causal ? blockIdx.x * 64 : 0;
-  for (int h = hk * grp; h < (hk + 1) * grp; ++h) {
-    for (int q0 = qbeg; q0 < p.seq; q0 += 32) {
-      __syncthreads();
-      for (int e = tid; e < 32 * D; e += 128) {
-        const int qr = e / D, d = e % D;
-        Qs[qr][d] = p.q[(row0 + q0 + qr) * p.ldq + h * D + d];
-        Gs[qr][d] = p.d_o[(row0 + q0 + qr) * p.lddo + h * D + d];
-      }
-      if (tid < 32) {
-        const long stat = ((long)b * p.n_heads + h) * p.seq + q0 + tid;
-        Ls[tid] = p.lse[stat];
-        Ds[tid] = p.delta[stat];
-      }
-      __syncthreads();
-#pragma unroll 1
-      for (int i = 0; i < 32; ++i) {
-        float t = 0.f, dp = 0.f;
+  for (int i = 0; i < D / 16; ++i) dk[i] = dv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int first = p.causal ? k0 / 16 : 0, tiles = p.seq / 16 - first;
+  for (int i = wave; i < grp * tiles; i += W) {
+    const int h = hk * grp + i / tiles, q0 = (first + i % tiles) * 16;
+    const float* qp = p.q + (row0 + q0) * p.ldq + h * D;
+    const float* gp = p.d_o + (row0 + q0) * p.lddo + h * D;
+    Rows32<D> qr, gr;
+    Cols32<D> qc, gc;
+    qr.load(qp, p.ldq, c, g);
+    gr.load(gp, p.lddo, c, g);
+    gc.load(gp, p.lddo, c, g);
+    qc.load(qp, p.ldq, c, g);
+    const long stat = ((long)b * p.n_heads + h) * p.seq + q0 + 4 * g;
+    const f32x4 lse = *(const f32x4_u*)(p.lse + stat), dl = *(const f32x4_u*)(p.delta + stat);
+    f32x4 s = score32<D>(qr, kr);
+    const f32x4 dp = score32<D>(gr, vr);
+    f32x4 ds;
 #pragma unroll
-        for (int d = 0; d < H; ++d) {
-          t = fmaf(Qs[i][half * H + d], k[d], t);
-          dp = fmaf(Gs[i][half * H + d], v[d], dp);
-        }
-        t = pair_sum(t) * p.scale;
-        dp = pair_sum(dp);
-        const float pr = (p.causal && kj > q0 + i) ? 0.f : expf(t - Ls[i]);
-        const float ds = pr * (dp - Ds[i]) * p.scale;
-#pragma unroll
-        for (int d = 0; d < H; ++d) {
-          dv[d] = fmaf(pr, Gs[i][half * H + d], dv[d]);
-          dk[d] = fmaf(ds, Qs[i][half * H + d], dk[d]);
-        }
-      }
+    for (int r = 0; r < 4; ++r) {
+      s[r] = (p.causal && k0 + c > q0 + 4 * g + r) ? 0.f : expf(s[r] * p.scale - lse[r]);
+      ds[r] = s[r] * (dp[r] - dl[r]) * p.scale;
     }
+    outer32<D>(dv, gc, s);
+    outer32<D>(dk, qc, ds);
   }
-#pragma unroll
-  for (int d = 0; d < H; ++d) {
-    p.dk[(row0 + kj) * p.lddk + hk * D + half * H + d] = dk[d];
-    p.dv[(row0 + kj) * p.lddv + hk * D + half * H + d] = dv[d];
-  }
+  store_sum32<D, W>(dv, buf, p.dv + (row0 + k0) * p.lddv + hk * D, p.lddv);
+  __syncthreads();
+  store_sum32<D, W>(dk, buf, p.dk + (row0 + k0) * p.lddk + hk * D, p.lddk);
 }
 
 int attn_check(const jpp_attn_args* a, const char* who, Attn32& p) {
@@ -506,6 +758,24 @@ int attn_check(const jpp_attn_args* a, const char* who, Attn32& p) {
 }
 
 }  // namespace
+
+int jpp_colsum_f32_items(hipStream_t stream, int n, const jpp_colsum_item* items, int64_t rows) {
+  JPP_REQUIRE(n >= 1 && n <= 4, "colsum_f32: 1 to 4 matrices");
+  ColItems32 p;
+  int blocks = 0;
+  for (int i = 0; i < 4; ++i) {
+    const jpp_colsum_item& q = items[i < n ? i : 0];
+    p.x[i] = (const float*)q.x;
+    p.acc[i] = q.acc;
+    p.ld[i] = q.ld;
+    p.cols[i] = (int)q.cols;
+    p.first[i] = i < n ? blocks : 0x7fffffff;
+    if (i < n) blocks += (int)((q.cols + 15) / 16);
+  }
+  hipLaunchKernelGGL(colsum32_kernel, dim3((unsigned)blocks), dim3(1024), 0, stream, p, (long)rows);
+  JPP_LAUNCH_CHECK();
+  return JPP_OK;
+}
 
 extern "C" {
 
@@ -550,9 +820,11 @@ int jpp_gemm_f32(void* stream, const jpp_gemm_args* a) {
   p.ta = a->trans_a != 0; p.tb = a->trans_b != 0; p.epi = e; p.gelu_tanh = a->gelu_tanh;
   p.seg = a->seg; p.n_seg = a->n_seg; p.group_mode = a->group_mode;
   p.stride_b = a->stride_b; p.stride_c = a->stride_c;
-  hipLaunchKernelGGL(sgemm_kernel,
-                     dim3((unsigned)(a->n / 64), (unsigned)(a->m / 64), group_k ? (unsigned)a->n_seg : 1u),
-                     dim3(256), 0, (hipStream_t)stream, p);
+  // the tallest tile that still gives every CU one (a taller tile reads its B fewer times)
+  const long strips = (a->m / 16) * (a->n / 64) * (group_k ? a->n_seg : 1);
+  if (strips >= 4 * 256) sgemm_launch<64>((hipStream_t)stream, p);
+  else if (strips >= 2 * 256) sgemm_launch<32>((hipStream_t)stream, p);
+  else sgemm_launch<16>((hipStream_t)stream, p);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
@@ -590,14 +862,12 @@ int jpp_norm_bwd_f32(void* stream, const jpp_norm_args* a) {
   JPP_REQUIRE(a->rows > 0 && a->cols > 0, "norm_bwd_f32: empty");
   JPP_REQUIRE(!a->mean || a->dbeta, "norm_bwd_f32: LayerNorm needs dbeta");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(norm_bwd32_kernel, dim3((unsigned)((a->rows + 3) / 4)), dim3(256), 0, st,
+  const unsigned row_blocks = (unsigned)((a->rows + 15) / 16), col_blocks = (unsigned)((a->cols + 15) / 16);
+  hipLaunchKernelGGL(norm_bwd32_kernel, dim3(row_blocks + col_blocks), dim3(1024), 0, st,
                      (const float*)a->dy, (const float*)a->x, (const float*)a->mean,
                      (const float*)a->rstd, (const float*)a->gamma, (const float*)a->resid,
-                     (float*)a->dx, (long)a->rows, (int)a->cols);
-  hipLaunchKernelGGL(norm_wgrad32_kernel, dim3((unsigned)((a->cols + 63) / 64)), dim3(64), 0, st,
-                     (const float*)a->dy, (const float*)a->x, (const float*)a->mean,
-                     (const float*)a->rstd, a->dgamma, a->mean ? a->dbeta : nullptr, (long)a->rows,
-                     (int)a->cols);
+                     (float*)a->dx, a->dgamma, a->mean ? a->dbeta : nullptr, (long)a->rows,
+                     (int)a->cols, (int)row_blocks);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
@@ -605,16 +875,14 @@ int jpp_norm_bwd_f32(void* stream, const jpp_norm_args* a) {
 int jpp_colsum_accum_f32(void* stream, const float* x, int64_t ld, int64_t rows, int64_t cols,
                          float* acc) {
   JPP_REQUIRE(x && acc && rows > 0 && cols > 0 && ld >= cols, "colsum_accum_f32: bad arguments");
-  hipLaunchKernelGGL(colsum32_kernel, dim3((unsigned)((cols + 63) / 64)), dim3(64), 0,
-                     (hipStream_t)stream, x, (long)ld, (long)rows, (int)cols, acc);
-  JPP_LAUNCH_CHECK();
-  return JPP_OK;
+  const jpp_colsum_item item = {x, ld, cols, acc};
+  return jpp_colsum_f32_items((hipStream_t)stream, 1, &item, rows);
 }
 
 int jpp_mse_loss_f32(void* stream, const float* out, const float* target, int64_t count,
                      float scale, float* loss, float* dout) {
   JPP_REQUIRE(out && target && loss && count > 0, "mse_loss_f32: bad arguments");
-  hipLaunchKernelGGL(mse32_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, out, target,
+  hipLaunchKernelGGL(mse32_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, out, target,
                      (long)count, scale, loss, dout);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
@@ -623,11 +891,11 @@ int jpp_mse_loss_f32(void* stream, const float* out, const float* target, int64_
 int jpp_attn_fwd_f32(void* stream, const jpp_attn_args* a) {
   Attn32 p;
   if (int rc = attn_check(a, "attn_fwd_f32", p)) return rc;
-  const dim3 grid((unsigned)(a->seq / 64), (unsigned)a->n_heads, (unsigned)a->batch);
+  const dim3 grid((unsigned)(a->seq / 16), (unsigned)a->n_heads, (unsigned)a->batch);
   if (a->head_dim == 64)
-    hipLaunchKernelGGL(attn_fwd32_kernel<64>, grid, dim3(128), 0, (hipStream_t)stream, p);
+    hipLaunchKernelGGL(attn_fwd32_kernel<64>, grid, dim3(64 * kAttnWaves32<64>), 0, (hipStream_t)stream, p);
   else
-    hipLaunchKernelGGL(attn_fwd32_kernel<128>, grid, dim3(128), 0, (hipStream_t)stream, p);
+    hipLaunchKernelGGL(attn_fwd32_kernel<128>, grid, dim3(64 * kAttnWaves32<128>), 0, (hipStream_t)stream, p);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
@@ -641,14 +909,14 @@ int jpp_attn_bwd_f32(void* stream, const jpp_attn_args* a) {
                   a->lddv >= (int64_t)a->n_kv_heads * a->head_dim,
               "attn_bwd_f32: leading dimension too small");
   hipStream_t st = (hipStream_t)stream;
-  const dim3 gq((unsigned)(a->seq / 64), (unsigned)a->n_heads, (unsigned)a->batch);
-  const dim3 gk((unsigned)(a->seq / 64), (unsigned)a->n_kv_heads, (unsigned)a->batch);
+  const dim3 gq((unsigned)(a->seq / 16), (unsigned)a->n_heads, (unsigned)a->batch);
+  const dim3 gk((unsigned)(a->seq / 16), (unsigned)a->n_kv_heads, (unsigned)a->batch);
   if (a->head_dim == 64) {
-    hipLaunchKernelGGL(attn_dq32_kernel<64>, gq, dim3(128), 0, st, p);
-    hipLaunchKernelGGL(attn_dkv32_kernel<64>, gk, dim3(128), 0, st, p);
+    hipLaunchKernelGGL(attn_dq32_kernel<64>, gq, dim3(64 * kAttnWaves32<64>), 0, st, p);
+    hipLaunchKernelGGL(attn_dkv32_kernel<64>, gk, dim3(64 * kAttnWaves32<64>), 0, st, p);
   } else {
-    hipLaunchKernelGGL(attn_dq32_kernel<128>, gq, dim3(128), 0, st, p);
-    hipLaunchKernelGGL(attn_dkv32_kernel<128>, gk, dim3(128), 0, st, p);
+    hipLaunchKernelGGL(attn_dq32_kernel<128>, gq, dim3(64 * kAttnWaves32<128>), 0, st, p);
+    hipLaunchKernelGGL(attn_dkv32_kernel<128>, gk, dim3(64 * kAttnWaves32<128>), 0, st, p);
   }
   JPP_LAUNCH_CHECK();
   return JPP_OK;

@@ -195,11 +195,8 @@ int attn_b(jpp_stage* s, hipStream_t st, const jpp_attn_args* a) {
 
 // a layer's four bias gradients: column sums of the cotangents, added to the accumulators
 int bias_grads4(jpp_stage* s, hipStream_t st, const jpp_colsum_item* items, float* partial) {
-  if (!s->f32()) return jpp_colsum_accum_multi(st, 4, items, s->T, partial);
-  for (int i = 0; i < 4; ++i)
-    RC(jpp_colsum_accum_f32(st, (const float*)items[i].x, items[i].ld, s->T, items[i].cols,
-                            items[i].acc));
-  return JPP_OK;
+  return s->f32() ? jpp_colsum_f32_items(st, 4, items, s->T)
+                  : jpp_colsum_accum_multi(st, 4, items, s->T, partial);
 }
 
 // dW[rows, cols] (+)= X^T dY, X: [T, rows], dY: [T, cols]

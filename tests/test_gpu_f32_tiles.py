@@ -1,0 +1,140 @@
+"""The f32 operators at the edges of their tiles: contractions of fewer steps than waves or
+prefetch stages, each output tile height in each orientation, leading dimensions and addresses
+that are multiples of 4 bytes only, column sums over ragged rows and columns, attention whose
+key tiles are fewer than the waves that share them.
+
+Bounds are a sum's own: each of n products is rounded once on its way into an fp32 chain, so an
+element is within (n + 4) 2^-24 of the sum of its terms' magnitudes."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from jaxpp_amd import runtime as rt
+
+pytestmark = pytest.mark.gpu
+U = 2.0 ** -24
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    rt.require_gpu()
+
+
+def dev(a):
+    return rt.DeviceBuffer.from_numpy(np.ascontiguousarray(a, dtype=np.float32))
+
+
+def padded(x, pad):
+    """x in rows of a leading dimension `pad` larger, and a device copy one float past an
+    aligned address."""
+    ld = x.shape[1] + pad
+    h = np.zeros(x.shape[0] * ld + 1, np.float32)
+    h[1:].reshape(x.shape[0], ld)[:, :x.shape[1]] = x
+    return dev(h), ld
+
+
+# strips of 16 x 64: fewer than a CU each (16-row tiles), two each (32), four each (64)
+SHAPES = [(64, 64, 16), (64, 128, 48), (128, 64, 80), (512, 1024, 144), (1024, 1024, 64), (1024, 1088, 208)]
+
+
+@pytest.mark.parametrize("lay", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("m,n,k", SHAPES, ids=["x".join(map(str, s)) for s in SHAPES])
+def test_gemm_f32_tiles(lay, m, n, k):
+    print(f"gemm_f32 {lay} {m}x{n}x{k}", flush=True)
+    rng = np.random.default_rng(m * 7 + n * 3 + k)
+    ta, tb = {"nn": (0, 1), "nt": (0, 0), "tn": (1, 1), "tt": (1, 0)}[lay]
+    A, B = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
+    c0 = rng.standard_normal((m, n), dtype=np.float32)
+    da, lda = padded(A.T if ta else A, 3)
+    db, ldb = padded(B.T if tb else B, 5)
+    dc, ldc = padded(c0, 1)
+    rt.gemm(da.ptr + 4, db.ptr + 4, dc.ptr + 4, m, n, k, lda, ldb, ldc, ta, tb, rt.EPI_ACC_F32, f32=True)
+    rt.sync()
+    raw = dc.download(np.float32, (m * ldc + 1,))
+    got = raw[1:].reshape(m, ldc)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    bound = (k + 4) * U * (np.abs(A64) @ np.abs(B64).T + np.abs(c0))
+    assert (np.abs(got[:, :n] - (c0 + A64 @ B64.T)) <= bound).all()
+    assert raw[0] == 0 and (got[:, n:] == 0).all()      # nothing beside the output is written
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 17), (64, 16), (513, 100), (1000, 256)])
+def test_norm_bwd_and_column_sums_f32_ragged(rows, cols):
+    rng = np.random.default_rng(rows + cols)
+    x, dy, resid = (rng.standard_normal((rows, cols), dtype=np.float32) for _ in range(3))
+    gamma, dg0, db0 = (rng.standard_normal(cols, dtype=np.float32) for _ in range(3))
+    mean = rng.standard_normal(rows, dtype=np.float32)
+    rstd = rng.random(rows, dtype=np.float32) + np.float32(0.5)
+    bufs = {k: dev(v) for k, v in dict(x=x, dy=dy, resid=resid, gamma=gamma, mean=mean, rstd=rstd,
+                                       dgamma=dg0, dbeta=db0, dx=np.zeros_like(x)).items()}
+    lib = rt.load()
+    a = rt.NormArgs()
+    for k, v in bufs.items():
+        setattr(a, k, v.ptr)
+    a.rows, a.cols, a.eps = rows, cols, 1e-5
+    rt.check(lib.jpp_norm_bwd_f32(None, C.byref(a)))
+    acc = dev(db0)
+    rt.check(lib.jpp_colsum_accum_f32(None, bufs["dy"].ptr, cols, rows, cols, acc.ptr))
+    rt.sync()
+    d, xh = dy.astype(np.float64), (x.astype(np.float64) - mean[:, None]) * rstd[:, None]
+    n = rows + 4
+    # (a term of dgamma is itself rounded three times)
+    assert (np.abs(bufs["dgamma"].download(np.float32, (cols,)) - (dg0 + (d * xh).sum(0))) <=
+            (n + 3) * U * (np.abs(dg0) + np.abs(d * xh).sum(0) +
+                           (np.abs(d) * np.abs(mean)[:, None] * rstd[:, None]).sum(0))).all()
+    for got in (bufs["dbeta"], acc):
+        assert (np.abs(got.download(np.float32, (cols,)) - (db0 + d.sum(0))) <=
+                n * U * (np.abs(db0) + np.abs(d).sum(0))).all()
+    w = d * gamma
+    want = (w - w.mean(1, keepdims=True) - xh * (w * xh).mean(1, keepdims=True)) * rstd[:, None] + resid
+    mag = (np.abs(w) + np.abs(w).mean(1, keepdims=True) +
+           (np.abs(x) + np.abs(mean)[:, None]) * rstd[:, None] * (1 + np.abs(w * xh).mean(1, keepdims=True)) *
+           (1 + np.abs(xh))) * rstd[:, None] + np.abs(resid)
+    assert (np.abs(bufs["dx"].download(np.float32, (rows, cols)) - want) <= (cols + 12) * U * mag).all()
+
+
+@pytest.mark.parametrize("d,hq,hk,seq,causal", [(64, 2, 1, 64, 1), (64, 3, 3, 192, 0), (128, 4, 2, 64, 0),
+                                                (128, 2, 2, 320, 1)])
+def test_attention_f32_tiles(d, hq, hk, seq, causal):
+    """Against float64; a difference of 2^-24 (d + 4) of the largest score moves a probability by
+    that share, and a result is a sum of d or seq terms of that error: 1e-5 of the largest
+    magnitude covers the sizes here."""
+    print(f"attention_f32 d={d} heads={hq}/{hk} seq={seq} causal={causal}", flush=True)
+    rng = np.random.default_rng(d + seq)
+    B, g = 2, hq // hk
+    q, do = (rng.standard_normal((B, seq, hq, d), dtype=np.float32) for _ in range(2))
+    k, v = (rng.standard_normal((B, seq, hk, d), dtype=np.float32) for _ in range(2))
+    qd, kd, vd, dod = dev(q), dev(k), dev(v), dev(do)
+    o, dq = (rt.DeviceBuffer(q.nbytes) for _ in range(2))
+    dk, dv = (rt.DeviceBuffer(k.nbytes) for _ in range(2))
+    lse, delta = rt.DeviceBuffer(B * hq * seq * 4), rt.DeviceBuffer(B * hq * seq * 4)
+    a = rt.AttnArgs()
+    a.q, a.k, a.v, a.o, a.lse, a.d_o, a.dq, a.dk, a.dv, a.delta = (
+        qd.ptr, kd.ptr, vd.ptr, o.ptr, lse.ptr, dod.ptr, dq.ptr, dk.ptr, dv.ptr, delta.ptr)
+    a.ldq = a.ldo = a.lddo = a.lddq = hq * d
+    a.ldk = a.ldv = a.lddk = a.lddv = hk * d
+    a.batch, a.seq, a.n_heads, a.n_kv_heads, a.head_dim, a.causal = B, seq, hq, hk, d, causal
+    lib = rt.load()
+    rt.check(lib.jpp_attn_fwd_f32(None, C.byref(a)))
+    rt.check(lib.jpp_attn_bwd_f32(None, C.byref(a)))
+    rt.sync()
+    q, k, v, do = (x.astype(np.float64).transpose(0, 2, 1, 3) for x in (q, k, v, do))
+    k, v = k.repeat(g, 1), v.repeat(g, 1)
+    s = q @ k.transpose(0, 1, 3, 2) / np.sqrt(d)
+    if causal:
+        s = np.where(np.tril(np.ones((seq, seq), bool)), s, -np.inf)
+    mx = s.max(-1, keepdims=True)
+    e = np.exp(s - mx)
+    p = e / e.sum(-1, keepdims=True)
+    out = p @ v
+    dp = do @ v.transpose(0, 1, 3, 2)
+    ds = p * (dp - (do * out).sum(-1, keepdims=True)) / np.sqrt(d)
+    want = {"o": out, "dq": ds @ k}
+    want["dk"], want["dv"] = (x.reshape(B, hk, g, seq, d).sum(2) for x in
+                              (ds.transpose(0, 1, 3, 2) @ q, p.transpose(0, 1, 3, 2) @ do))
+    for name, buf in (("o", o), ("dq", dq), ("dk", dk), ("dv", dv)):
+        w = want[name].transpose(0, 2, 1, 3)
+        assert np.abs(buf.download(np.float32, w.shape) - w).max() <= 1e-5 * np.abs(w).max(), name
+    w = (mx + np.log(e.sum(-1, keepdims=True)))[..., 0]
+    assert np.abs(lse.download(np.float32, w.shape) - w).max() <= 1e-5 * np.abs(w).max()
