@@ -548,6 +548,41 @@ AttnParams make_params(const jpp_attn_args* a) {
   return p;
 }
 
+// Where 16 rows per workgroup (attention_small.hip) beat the blocks of this file.  Forward: while
+// they are at most one workgroup per CU (seq x heads of all sequences <= 4096); measured, times
+// of the two: 5.3 / 4.8 us at 2 heads x 128 positions x 64, 17.8 / 9.7 at 2 x 1024 x 64, 10.4 / 8.1
+// at 16 x 256 x 128 under a mask; at twice that many workgroups 7.5 / 7.9 (32 x 256 x 64) down to
+// 0.72 of the speed.
+bool small_fwd(const jpp_attn_args* a) { return (int64_t)a->batch * a->n_heads * a->seq <= 4096; }
+
+// Backward: at most a workgroup of 16 keys per CU and twice as many of 16 queries (13.6 / 6.3 us,
+// 43.6 / 20.2, 31.4 / 19.1 at the sizes above; twice as many keys: 19.0 / 24.2).  Under a mask
+// the kernels of their own are quicker with many query heads per key (4 heads x 512 positions x
+// 128: 57.2 / 58.0 us, 8 x 256: 0.94 of the speed; 4 x 256: 1.23, 8 x 256 x 64: 1.17): the one
+// workgroup of 16 keys then walks all of their queries.
+// One launch writes dQ, dK and dV while it reads everything else, where two read only part of it:
+// a caller whose results lie over the inputs keeps the two.
+bool small_bwd(const jpp_attn_args* a) {
+  const int64_t rows = (int64_t)a->batch * a->seq, grp = a->n_heads / a->n_kv_heads;
+  if (rows * a->n_heads > 8192 || rows * a->n_kv_heads > 4096) return false;
+  if (a->causal && grp > 1 && grp * a->seq * a->head_dim > 131072) return false;
+  struct Range {
+    uintptr_t lo, hi;
+  };
+  auto range = [&](const void* p, int64_t ld, int heads) {
+    return Range{(uintptr_t)p, (uintptr_t)p + (uintptr_t)(((rows - 1) * ld + heads * a->head_dim) * 2)};
+  };
+  const Range out[3] = {range(a->dq, a->lddq, a->n_heads), range(a->dk, a->lddk, a->n_kv_heads),
+                        range(a->dv, a->lddv, a->n_kv_heads)};
+  const Range in[5] = {range(a->q, a->ldq, a->n_heads), range(a->k, a->ldk, a->n_kv_heads),
+                       range(a->v, a->ldv, a->n_kv_heads), range(a->o, a->ldo, a->n_heads),
+                       range(a->d_o, a->lddo, a->n_heads)};
+  for (const Range& w : out)
+    for (const Range& r : in)
+      if (w.lo < r.hi && r.lo < w.hi) return false;
+  return true;
+}
+
 }  // namespace
 
 extern "C" int jpp_attn_fwd(void* stream, const jpp_attn_args* a) {
@@ -558,6 +593,7 @@ extern "C" int jpp_attn_fwd(void* stream, const jpp_attn_args* a) {
   const double fl = 4.0 * a->batch * a->seq * (double)a->seq * a->n_heads * a->head_dim *
                     (a->causal ? 0.5 : 1.0);
   ProbeScope probe(st, "attn_fwd", fl, 0);
+  if (small_fwd(a)) return launch_small_fwd(st, p, a->head_dim, a->causal != 0);
 #define JPP_AF(D_, C_)                                                                  \
   do {                                                                                  \
     if (int rc = set_smem(attn_fwd_kernel<D_, C_>, 4 * D_ * 128)) return rc;            \
@@ -589,6 +625,14 @@ extern "C" int jpp_attn_bwd(void* stream, const jpp_attn_args* a) {
   const bool fused_rope = a->rope_cos && a->causal;
   if (fused_rope) { p.rope_cos = a->rope_cos; p.rope_sin = a->rope_sin; }
   hipStream_t st = (hipStream_t)stream;
+  if (small_bwd(a)) {
+    p.rope_cos = a->rope_cos;
+    p.rope_sin = a->rope_sin;
+    const double flops = 8.0 * a->batch * a->seq * (double)a->seq * a->n_heads * a->head_dim *
+                         (a->causal ? 0.5 : 1.0);
+    ProbeScope probe(st, "attn_bwd_small", flops, 0);
+    return launch_small_bwd(st, p, a->head_dim, a->causal != 0);
+  }
   dim3 gq(a->seq / 128, a->n_heads, a->batch);
   // causal: 64-key blocks, a workgroup takes blocks x and n-1-x; else 128-key blocks
   dim3 gkv(a->seq / 128, a->n_kv_heads, a->batch);

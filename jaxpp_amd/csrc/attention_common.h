@@ -230,6 +230,9 @@ int set_smem(K kern, int bytes) {
 int launch_dq(hipStream_t stream, const AttnParams& p, int head_dim, bool causal);
 // dK/dV under a causal mask (attention_dkv.hip); grid (seq/128, kv heads, batch)
 int launch_dkv_causal(hipStream_t stream, const AttnParams& p, int head_dim, dim3 grid);
+// problems too small to fill the device with the blocks of the others (attention_small.hip)
+int launch_small_fwd(hipStream_t stream, const AttnParams& p, int head_dim, bool causal);
+int launch_small_bwd(hipStream_t stream, const AttnParams& p, int head_dim, bool causal);
 
 }  // namespace jpp_attn
 
