@@ -276,6 +276,25 @@ int run_wgrads(jpp_stage* s, hipStream_t st, WgradBatch& w) {
     std::stable_sort(order, order + w.n, [](const jpp_gemm_args& a, const jpp_gemm_args& b) {
       return a.m * a.n < b.m * b.n;
     });
+    // Less than a full grid: a group's microbatches go one by one, in order.  Their products are
+    // too small for the accumulators' traffic to matter, and the sums stay those of an ungrouped
+    // run to the last bit (Adam's first updates magnify a reassociated sum that is nearly zero).
+    const int pairs = order[0].k_parts > 1 ? order[0].k_parts : 1;
+    if (pairs > 1 && (!whole || total < kFullGrid)) {
+      for (int part = 0; part < pairs; ++part) {
+        jpp_gemm_args one[4];
+        for (int i = 0; i < w.n; ++i) {
+          one[i] = order[i];
+          one[i].k_parts = 1;
+          if (part > 0) {
+            one[i].a = order[i].a_more[part - 1];
+            one[i].b = order[i].b_more[part - 1];
+          }
+        }
+        RC(jpp_gemm_bf16_multi(st, one, w.n));
+      }
+      return JPP_OK;
+    }
     return jpp_gemm_bf16_multi(st, order, w.n);
   }
   for (int i = 0; i < w.n; ++i) {
