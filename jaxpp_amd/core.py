@@ -408,6 +408,15 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
     act_elems = tokens * hidden
     f32 = spec0.dtype == "f32"           # an f32 model runs through the f32 operators
     any_ex = execs[0, 0]
+    act_bytes = act_elems * (4 if f32 else 2)
+
+    # (small microbatches of a kind share a buffer and travel as one copy)
+    mb_runs = rt.copy_runs([act_elems] * n)
+
+    def in_runs(make):
+        bufs = [make(first, last) for first, last in mb_runs]
+        return [rt.BufferPart(buf, m * act_bytes, act_bytes)
+                for buf, (first, last) in zip(bufs, mb_runs) for m in range(last - first)]
 
     def microbatches(x):
         if x.shape[1:] != (tokens, hidden):
@@ -415,7 +424,7 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
                 raise ValueError(f"a microbatch of shape {x.shape[1:]} does not hold "
                                  f"{tokens} x {hidden} values")
             x = x.reshape(n, tokens, hidden)
-        return [any_ex.upload_activation(x[m]) for m in range(n)]
+        return in_runs(lambda first, last: any_ex.upload_activation(x[first:last]))
 
     xs_dev = microbatches(tr.inputs[body.input_index][0])
     tgt_dev = None
@@ -455,7 +464,8 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
     loss_dev = rt.DeviceBuffer(4 * n)
     partial = rt.DeviceBuffer(4 * rt.NORM_PARTIALS)
     want_pred = any(isinstance(v, tracing.Traced) and v.shape != () for v in tracing.tree_leaves(outputs))
-    preds = {}
+    # (fetched behind the loop: a copy after each forward task would drain the queue)
+    preds_dev = in_runs(lambda first, last: rt.DeviceBuffer((last - first) * act_bytes)) if want_pred else []
     # the scale of the value that is differentiated sets the cotangent; loss values returned
     # with another scale are rescaled from it
     diff = tr.differentiated
@@ -476,7 +486,7 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
                 t0 = time.perf_counter()
             if kind is TaskType.FWD:
                 src = xs_dev[m] if s == 0 else act.pop((s, m))
-                dst = take()
+                dst = preds_dev[m] if preds_dev and s + 1 == S else take()
                 run_fwd(s, m, src, dst)
                 if s > 0:
                     free.append(src)
@@ -495,9 +505,8 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
                                                   float(loss_scale), loss_dev.ptr + 4 * m, d.ptr,
                                                   partial.ptr))
                     cot[s, m] = d
-                    if want_pred:
-                        preds[m] = any_ex.download_activation(dst, (tokens, hidden))
-                    free.append(dst)
+                    if not preds_dev:
+                        free.append(dst)
             elif kind is TaskType.BWD_W:
                 for sg in reversed(stage_segs[s]):
                     sg.ex.run_task(kind, 0, m)
@@ -515,6 +524,8 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
                 _statistics[mk_task_name(s, t.fwd_or_bwd)].append((time.perf_counter() - t0) * 1e3)
     rt.sync()
     losses = loss_dev.download(np.float32, (n,))
+    preds = [p for (first, last), buf in zip(mb_runs, preds_dev and [preds_dev[a].owner for a, _ in mb_runs])
+             for p in any_ex.download_activation(buf, (last - first, tokens, hidden))]
     grads = {}
     for s_, segs in enumerate(stage_segs):
         grads[s_] = []

@@ -29,6 +29,31 @@ def _zip_map(f, *trees):
     return f(*trees)
 
 
+def _offsets(leaves):
+    """Places of a run's leaves in one vector, each on 64 bytes, and the vector's length."""
+    at, n = [], 0
+    for a in leaves:
+        at.append(n)
+        n += -(-a.size // 16) * 16
+    return at, n
+
+
+def _map_runs(f, *trees):
+    """A tree like the first of what ``f`` returns per leaf.  ``f`` takes the leaves of a run
+    (`runtime.copy_runs`), one list per tree, float32 and contiguous: leaf by leaf a step of four
+    small layers was 250 uploads and 200 downloads, and those 20 of its 24 ms."""
+    from jaxpp_amd import runtime as rt
+    leaves = []
+    _zip_map(lambda *ls: leaves.append([np.ascontiguousarray(a, dtype=np.float32) for a in ls]), *trees)
+    out = []
+    for first, last in rt.copy_runs([ls[0].size for ls in leaves]):
+        for ls in leaves[first:last]:
+            assert all(a.size >= ls[0].size for a in ls), [a.shape for a in ls]
+        out += f(*([ls[k] for ls in leaves[first:last]] for k in range(len(trees))))
+    results = iter(out)
+    return _zip_map(lambda *_: next(results), *trees)
+
+
 @dataclass(frozen=True)
 class adam:
     """``optax.adam(learning_rate, b1, b2, eps)``: no weight decay, bias-corrected moments."""
@@ -49,21 +74,26 @@ class adam:
         rt.require_gpu()
         step = int(state["count"]) + 1
 
-        def leaf(g, m, v):
-            g = np.ascontiguousarray(g, dtype=np.float32)
-            n = g.size
-            dg, dm, dv = (rt.DeviceBuffer.from_numpy(np.ascontiguousarray(a, dtype=np.float32))
-                          for a in (g, m, v))
-            du = rt.DeviceBuffer(4 * n)
-            du.zero()
+        def run(gs, ms, vs):
+            """The leaves of a run as one vector: gradients, moments and updates of `n` elements
+            each behind one another on the device, one copy each way."""
+            at, n = _offsets(gs)
+            host = np.empty(3 * n, np.float32)
+            for k, leaves in enumerate((gs, ms, vs)):
+                for i, a in enumerate(leaves):
+                    host[k * n + at[i]:k * n + at[i] + gs[i].size] = a.reshape(-1)[:gs[i].size]
+            buf = rt.DeviceBuffer(16 * n)
+            buf.upload(host)
             # weights that start at zero end as the update itself
-            rt.adam_step(n, dg.ptr, dm.ptr, dv.ptr, step, master=du.ptr, lr=self.learning_rate,
-                         b1=self.b1, b2=self.b2, eps=self.eps)
+            rt.check(rt.load().jpp_fill_u32(buf.ptr + 12 * n, 0, n, None))
+            rt.adam_step(n, buf.ptr, buf.ptr + 4 * n, buf.ptr + 8 * n, step, master=buf.ptr + 12 * n,
+                         lr=self.learning_rate, b1=self.b1, b2=self.b2, eps=self.eps)
             rt.sync()
-            return (du.download(np.float32, g.shape), dm.download(np.float32, g.shape),
-                    dv.download(np.float32, g.shape))
+            out = buf.download(np.float32, (3 * n,), 4 * n)
+            part = lambda k, i: out[k * n + at[i]:k * n + at[i] + gs[i].size].reshape(gs[i].shape)
+            return [(part(2, i), part(0, i), part(1, i)) for i in range(len(gs))]
 
-        trio = _zip_map(leaf, grads, state["mu"], state["nu"])
+        trio = _map_runs(run, grads, state["mu"], state["nu"])
         pick = lambda k: _zip_map(lambda g, t: t[k], grads, trio)
         return pick(0), {"count": step, "mu": pick(1), "nu": pick(2)}
 
@@ -73,12 +103,17 @@ def apply_updates(params, updates):
     from jaxpp_amd import runtime as rt
     rt.require_gpu()
 
-    def leaf(p, u):
-        p = np.ascontiguousarray(p, dtype=np.float32)
-        dp = rt.DeviceBuffer.from_numpy(p)
-        du = rt.DeviceBuffer.from_numpy(np.ascontiguousarray(u, dtype=np.float32))
-        rt.check(rt.load().jpp_grad_accum_f32(None, dp.ptr, du.ptr, p.size, 1))
+    def run(ps, us):
+        at, n = _offsets(ps)
+        host = np.empty(2 * n, np.float32)
+        for k, leaves in enumerate((ps, us)):
+            for i, a in enumerate(leaves):
+                host[k * n + at[i]:k * n + at[i] + ps[i].size] = a.reshape(-1)[:ps[i].size]
+        buf = rt.DeviceBuffer(8 * n)
+        buf.upload(host)
+        rt.check(rt.load().jpp_grad_accum_f32(None, buf.ptr, buf.ptr + 4 * n, n, 1))
         rt.sync()
-        return dp.download(np.float32, p.shape)
+        out = buf.download(np.float32, (n,))
+        return [out[at[i]:at[i] + p.size].reshape(p.shape) for i, p in enumerate(ps)]
 
-    return _zip_map(leaf, params, updates)
+    return _map_runs(run, params, updates)

@@ -340,6 +340,14 @@ class DeviceBuffer:
             pass
 
 
+class BufferPart:
+    """A piece of a `DeviceBuffer`, which it keeps alive."""
+
+    def __init__(self, owner: DeviceBuffer, offset: int, nbytes: int):
+        assert offset + nbytes <= owner.nbytes
+        self.owner, self.nbytes, self.ptr = owner, nbytes, owner.ptr + offset
+
+
 def upload_ptr(ptr: int, a: np.ndarray):
     a = np.ascontiguousarray(a)
     check(load().jpp_memcpy_h2d(ptr, a.ctypes.data, a.nbytes))
@@ -349,6 +357,28 @@ def download_ptr(ptr: int, dtype, shape) -> np.ndarray:
     out = np.empty(shape, dtype=dtype)
     check(load().jpp_memcpy_d2h(out.ctypes.data, ptr, out.nbytes))
     return out
+
+
+# Elements of small tensors that travel as one copy.  A copy between pageable host memory and the
+# device costs 14 us and more whatever its size, and up to 115 us at 64 - 256 KB; one of 8 MB
+# moves at 16 - 35 GB/s.  Larger tensors gain nothing and would only be copied once more on the
+# host.
+COPY_RUN = 1 << 21
+
+
+def copy_runs(sizes, adjacent=None, limit: int = COPY_RUN) -> list:
+    """Splits tensors of these sizes (elements), in order, into runs ``(first, last + 1)`` that
+    travel as one copy: at most `limit` elements together, a larger tensor by itself.
+    ``adjacent(i)`` says whether tensor i follows tensor i - 1 without a break (None: always)."""
+    runs, first, total = [], 0, 0
+    for i, n in enumerate(sizes):
+        if i > first and (total + n > limit or not (adjacent is None or adjacent(i))):
+            runs.append((first, i))
+            first, total = i, 0
+        total += n
+    if len(sizes):
+        runs.append((first, len(sizes)))
+    return runs
 
 
 def sync():
@@ -591,50 +621,59 @@ class StageExecutor:
         q, w = c // 64, c % 64
         return np.where(w < 32, 32 * q + w, f + 32 * q + w - 32)
 
+    def _runs(self, ptrs, itemsize: int) -> list:
+        """The layer's parameters in runs of small ones that lie one behind the other."""
+        sizes = [r * c for _, r, c in self.params]
+        return copy_runs(sizes, lambda i: ptrs[i] == ptrs[i - 1] + sizes[i - 1] * itemsize)
+
+    def _download_layer(self, ptrs, dtype, convert=None) -> dict:
+        """name -> host array (in the host's column order) of the tensors at `ptrs`."""
+        out = {}
+        for first, last in self._runs(ptrs, np.dtype(dtype).itemsize):
+            run = self.params[first:last]
+            flat = download_ptr(ptrs[first], dtype, (sum(r * c for _, r, c in run),))
+            if convert is not None:
+                flat = convert(flat)
+            at = 0
+            for name, rows, cols in run:
+                shape = (cols,) if rows == 1 and not name.startswith("W") else (rows, cols)
+                a = flat[at:at + rows * cols].reshape(shape)
+                at += rows * cols
+                order = self._device_columns(name, cols)
+                if order is not None:
+                    host = np.empty_like(a)
+                    host[:, order] = a
+                    a = host
+                out[name] = a
+        return out
+
     def set_params(self, chunk: int, layer: int, params: dict):
         """Upload float32 host arrays as device parameters (bf16, or f32 for an f32 stage)."""
-        for name, rows, cols in self.params:
-            a = np.asarray(params[name], dtype=np.float32)
-            assert a.size == rows * cols, (name, a.shape, rows, cols)
-            order = self._device_columns(name, cols)
-            if order is not None:
-                a = np.ascontiguousarray(a.reshape(rows, cols)[:, order])
-            upload_ptr(self._ptr(load().jpp_stage_param_ptr, chunk, layer, name),
-                       a if self.dtype == "f32" else to_bf16_bits(a))
+        ptrs = [self._ptr(load().jpp_stage_param_ptr, chunk, layer, name) for name, _, _ in self.params]
+        for first, last in self._runs(ptrs, 4 if self.dtype == "f32" else 2):
+            arrays = []
+            for name, rows, cols in self.params[first:last]:
+                a = np.asarray(params[name], dtype=np.float32)
+                assert a.size == rows * cols, (name, a.shape, rows, cols)
+                order = self._device_columns(name, cols)
+                if order is not None:
+                    a = np.ascontiguousarray(a.reshape(rows, cols)[:, order])
+                arrays.append(a)
+            a = arrays[0] if len(arrays) == 1 else np.concatenate([x.reshape(-1) for x in arrays])
+            upload_ptr(ptrs[first], a if self.dtype == "f32" else to_bf16_bits(a))
 
     def get_params(self, chunk: int, layer: int) -> dict:
         """The device parameters as float32 host arrays."""
         self.join()
-        out = {}
-        for name, rows, cols in self.params:
-            shape = (cols,) if rows == 1 and not name.startswith("W") else (rows, cols)
-            ptr = self._ptr(load().jpp_stage_param_ptr, chunk, layer, name)
-            if self.dtype == "f32":
-                a = download_ptr(ptr, np.float32, shape)
-            else:
-                a = from_bf16_bits(download_ptr(ptr, np.uint16, shape))
-            order = self._device_columns(name, cols)
-            if order is not None:
-                host = np.empty_like(a)
-                host[:, order] = a
-                a = host
-            out[name] = a
-        return out
+        ptrs = [self._ptr(load().jpp_stage_param_ptr, chunk, layer, name) for name, _, _ in self.params]
+        if self.dtype == "f32":
+            return self._download_layer(ptrs, np.float32)
+        return self._download_layer(ptrs, np.uint16, from_bf16_bits)
 
     def get_grads(self, chunk: int, layer: int) -> dict:
         self.join()          # the copies below run on the null stream
-        out = {}
-        for name, rows, cols in self.params:
-            shape = (cols,) if rows == 1 and not name.startswith("W") else (rows, cols)
-            g = download_ptr(self._ptr(load().jpp_stage_grad_ptr, chunk, layer, name),
-                             np.float32, shape)
-            order = self._device_columns(name, cols)
-            if order is not None:
-                host = np.empty_like(g)
-                host[:, order] = g
-                g = host
-            out[name] = g
-        return out
+        ptrs = [self._ptr(load().jpp_stage_grad_ptr, chunk, layer, name) for name, _, _ in self.params]
+        return self._download_layer(ptrs, np.float32)
 
     def upload_activation(self, a: np.ndarray) -> "DeviceBuffer":
         """A float32 host array as a device tensor of the stage's element type."""
