@@ -8,6 +8,8 @@
 
 #include <mutex>
 
+#include <type_traits>
+
 #include "common.h"
 
 // Scratch of jpp_norm_bwd_static (the entry point that allocates nothing): the per-block
@@ -445,6 +447,171 @@ __global__ __launch_bounds__(1024) void colsum_multi_reduce_kernel(const float* 
 }
 
 // ---------------------------------------------------------------------------
+// Few rows: column sums by one workgroup per 64 columns, without partial sums in memory.
+// Two launches over 256 blocks of rows, the second adding up what the first left, are two
+// launches' latency and 256 x columns floats on the way between them, which at a few hundred
+// rows is more than the tensors themselves.  A thread owns 8 columns of every (NT / 8)-th row; the
+// row groups of a column meet inside a wave first, then in wave order.
+// ---------------------------------------------------------------------------
+// Sums over `rows` of load(r, a, b), which adds 8 columns of row r into a (and b), for 64
+// adjacent columns; thread t < 64 returns column t's two sums.
+template <int NT, int UNROLL, class Load>
+__device__ __forceinline__ float2 column_sums64(long rows, Load load) {
+  __shared__ float2 red[NT / 64][64];
+  constexpr int G = NT / 8;
+  const int tid = threadIdx.x;
+  float a[8], b[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) a[e] = b[e] = 0.f;
+  long r = tid >> 3;
+  for (; r + (UNROLL - 1) * G < rows; r += UNROLL * G) load(r, G, std::integral_constant<int, UNROLL>{}, a, b);
+  for (; r < rows; r += G) load(r, G, std::integral_constant<int, 1>{}, a, b);
+#pragma unroll
+  for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      a[e] += __shfl_xor(a[e], o);
+      b[e] += __shfl_xor(b[e], o);
+    }
+  if ((tid & 63) < 8)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[tid >> 6][(tid & 7) * 8 + e] = make_float2(a[e], b[e]);
+  __syncthreads();
+  float2 t = make_float2(0.f, 0.f);
+  if (tid < 64)
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+      t.x += red[w][tid].x;
+      t.y += red[w][tid].y;
+    }
+  return t;
+}
+
+// the bias gradients of a layer: workgroups first[i] .. first[i + 1] - 1 take tensor i
+struct ColsumPanels {
+  ColsumBatch b;
+  int first[4];
+};
+__global__ __launch_bounds__(1024) void colsum_few_rows_kernel(ColsumPanels p, long rows) {
+  const int blk = blockIdx.x;
+  const bool s1 = blk >= p.first[1], s2 = blk >= p.first[2], s3 = blk >= p.first[3];
+#define JPP_PICK(f) (s3 ? f[3] : s2 ? f[2] : s1 ? f[1] : f[0])
+  const bf16_t* const x = JPP_PICK(p.b.x);
+  const long ld = JPP_PICK(p.b.ld);
+  float* const acc = JPP_PICK(p.b.acc);
+  const int c0 = (blk - JPP_PICK(p.first)) * 64;
+  const int cols = s3 ? p.b.start[4] - p.b.start[3] : s2 ? p.b.start[3] - p.b.start[2]
+                   : s1 ? p.b.start[2] - p.b.start[1] : p.b.start[1];
+#undef JPP_PICK
+  const int c = c0 + (threadIdx.x & 7) * 8;
+  const bf16_t* src = x + c;
+  const float2 t = column_sums64<1024, 8>(c < cols ? rows : 0, [&](long r, int g, auto u, float (&a)[8], float (&)[8]) {
+    constexpr int U = decltype(u)::value;
+    uint4 v[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) v[i] = *(const uint4*)(src + (r + i * g) * ld);
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      float f[8];
+      unpack8(v[i], f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] += f[e];
+    }
+  });
+  if (threadIdx.x < 64 && c0 + (int)threadIdx.x < cols) acc[c0 + threadIdx.x] += t.x;
+}
+
+// A norm's whole backward in one launch: the first row_blocks workgroups take NT / 64 rows each, a
+// wave per row, for dx; each of the others the scale and shift gradients of 64 columns.
+// (512 threads: with 1024 the launch itself takes 2 us longer at a few hundred rows)
+constexpr int kFewRowsThreads = 512;
+template <bool LN, int NCH>
+__global__ __launch_bounds__(kFewRowsThreads) void norm_bwd_few_rows_kernel(
+    const bf16_t* __restrict__ dy, const bf16_t* __restrict__ x, const float* __restrict__ mean_in,
+    const float* __restrict__ rstd_in, const bf16_t* __restrict__ gamma, const bf16_t* resid,
+    bf16_t* dx, float* dgamma, float* dbeta, long rows, int cols, int row_blocks) {
+  if ((int)blockIdx.x >= row_blocks) {
+    const int c0 = ((int)blockIdx.x - row_blocks) * 64, c = c0 + (threadIdx.x & 7) * 8;
+    const float2 t = column_sums64<kFewRowsThreads, 8>(c < cols ? rows : 0, [&](long r, int g, auto u, float (&a)[8], float (&b)[8]) {
+      constexpr int U = decltype(u)::value;
+      uint4 vd[U], vx[U];
+      float mean[U], rstd[U];
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const long row = r + i * g;
+        vd[i] = *(const uint4*)(dy + row * cols + c);
+        vx[i] = *(const uint4*)(x + row * cols + c);
+        rstd[i] = rstd_in[row];
+        mean[i] = LN ? mean_in[row] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        float fd[8], fx[8];
+        unpack8(vd[i], fd);
+        unpack8(vx[i], fx);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          a[e] += fd[e] * ((fx[e] - mean[i]) * rstd[i]);
+          if (LN) b[e] += fd[e];
+        }
+      }
+    });
+    if (threadIdx.x < 64 && c0 + (int)threadIdx.x < cols) {
+      dgamma[c0 + threadIdx.x] += t.x;
+      if (LN) dbeta[c0 + threadIdx.x] += t.y;
+    }
+    return;
+  }
+  const int lane = threadIdx.x & 63, nchunk = cols >> 3;
+  const long row = (long)blockIdx.x * (kFewRowsThreads / 64) + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const float rstd = rstd_in[row], mean = LN ? mean_in[row] : 0.f;
+  uint4 vx[NCH], vd[NCH], vg[NCH], vr[NCH];
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = lane + 64 * i;
+    const uint4 none = make_uint4(0, 0, 0, 0);
+    vx[i] = c < nchunk ? ((const uint4*)(x + row * cols))[c] : none;
+    vd[i] = c < nchunk ? ((const uint4*)(dy + row * cols))[c] : none;
+    vg[i] = c < nchunk ? ((const uint4*)gamma)[c] : none;
+    vr[i] = resid && c < nchunk ? ((const uint4*)(resid + row * cols))[c] : none;
+  }
+  float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    float fx[8], fd[8], g[8];
+    unpack8(vx[i], fx);
+    unpack8(vd[i], fd);
+    unpack8(vg[i], g);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float dg = fd[e] * g[e];
+      s1 += dg;
+      s2 += dg * ((fx[e] - mean) * rstd);
+    }
+  }
+  s2 = wave_sum(s2) / cols;
+  s1 = LN ? wave_sum(s1) / cols : 0.f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int c = lane + 64 * i;
+    if (c >= nchunk) continue;
+    float fx[8], fd[8], g[8], q[8];
+    unpack8(vx[i], fx);
+    unpack8(vd[i], fd);
+    unpack8(vg[i], g);
+    unpack8(vr[i], q);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float o = (fd[e] * g[e] - s1 - (fx[e] - mean) * rstd * s2) * rstd;
+      if (resid) o += q[e];
+      fx[e] = o;
+    }
+    ((uint4*)(dx + row * cols))[c] = pack8(fx);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // SwiGLU
 // ---------------------------------------------------------------------------
 // gate and up of 8 features starting at feature 8c of row t: halves layout [gate | up], or
@@ -651,9 +818,40 @@ int launch_norm_fwd(hipStream_t st, const jpp_norm_args* a) {
   return JPP_OK;
 }
 
+// Where one launch with sums by 64 columns beats partial sums of 256 blocks and a second launch.
+// A norm's backward reads dy and x a second time for its sums, 64 columns per workgroup: up to
+// 1024 rows (LayerNorm, us, two launches / one: 512 x 1024 9.0 / 5.4, 1024 x 128 6.7 / 6.3, 1536 x
+// 128 6.7 / 7.6), wider than 512 columns - more workgroups - up to 1536 (1536 x 768 9.0 / 8.1, 2048 x
+// 768 9.2 / 11.9), and not where a row is spread over a workgroup (512 x 4096 12.9 / 14.0).
+bool norm_few_rows(long rows, long cols) { return cols < 4096 && rows <= (cols > 512 ? 1536 : 1024); }
+// Column sums read their tensors once either way (a layer's four of 9 x 1024 columns: 512 rows
+// 11.4 / 4.9, 4096 rows 17.7 / 11.8); taller ones want the rows split as well.
+constexpr long kColsumFewRows = 4096;
+
 template <bool LN>
 int launch_norm_bwd(hipStream_t st, const jpp_norm_args* a) {
   const int nch = (int)((a->cols / 8 + 63) / 64);
+  // (dx over dy or x: the one launch would read what it has already overwritten)
+  const uintptr_t size = (uintptr_t)(a->rows * a->cols * 2), out = (uintptr_t)a->dx;
+  const bool apart = (out + size <= (uintptr_t)a->dy || (uintptr_t)a->dy + size <= out) &&
+                     (out + size <= (uintptr_t)a->x || (uintptr_t)a->x + size <= out);
+  if (norm_few_rows(a->rows, a->cols) && apart) {
+    const int per = kFewRowsThreads / 64;
+    const int row_blocks = (int)((a->rows + per - 1) / per), col_blocks = (int)((a->cols + 63) / 64);
+#define JPP_NBF(N)                                                                                  \
+  hipLaunchKernelGGL((norm_bwd_few_rows_kernel<LN, N>), dim3(row_blocks + col_blocks),              \
+                     dim3(kFewRowsThreads), 0, st,                                               \
+                     (const bf16_t*)a->dy, (const bf16_t*)a->x, a->mean, a->rstd,                   \
+                     (const bf16_t*)a->gamma, (const bf16_t*)a->resid, (bf16_t*)a->dx, a->dgamma,   \
+                     a->dbeta, (long)a->rows, (int)a->cols, row_blocks)
+    if (nch <= 1) JPP_NBF(1);
+    else if (nch <= 2) JPP_NBF(2);
+    else if (nch <= 4) JPP_NBF(4);
+    else JPP_NBF(8);
+#undef JPP_NBF
+    JPP_LAUNCH_CHECK();
+    return JPP_OK;
+  }
   const int blocks = JPP_NORM_PARTIALS;
 #define JPP_NB(N)                                                                             \
   hipLaunchKernelGGL((norm_bwd_kernel<LN, N>), dim3(blocks), dim3(kNormBwdWaves * 64), 0, st, \
@@ -845,6 +1043,19 @@ int jpp_colsum_accum_multi(void* stream, int n, const jpp_colsum_item* items, in
   b.start[n] = at;
   hipStream_t st = (hipStream_t)stream;
   ProbeScope probe(st, "colsum", 0, bytes);
+  if (rows <= kColsumFewRows) {
+    ColsumPanels p;
+    int blocks = 0;
+    for (int i = 0; i < 4; ++i) {
+      p.first[i] = i < n ? blocks : 0x7fffffff;
+      if (i < n) blocks += (b.start[i + 1] - b.start[i] + 63) / 64;
+      else { b.x[i] = b.x[0]; b.ld[i] = b.ld[0]; b.acc[i] = b.acc[0]; b.start[i + 1] = at; }
+    }
+    p.b = b;
+    hipLaunchKernelGGL(colsum_few_rows_kernel, dim3(blocks), dim3(1024), 0, st, p, (long)rows);
+    JPP_LAUNCH_CHECK();
+    return JPP_OK;
+  }
   const int nb = (int)(rows < JPP_NORM_PARTIALS ? rows : JPP_NORM_PARTIALS);
   const int panels = (at / 8 + 255) / 256;
   hipLaunchKernelGGL(colsum_multi_partial_kernel, dim3(nb, panels), dim3(256), 0, st, b, (long)rows,
