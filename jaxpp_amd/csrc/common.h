@@ -194,7 +194,7 @@ struct DmaTile {
   static constexpr int BYTES = ROWS * 128;
   static constexpr int INSTS = ROWS / (8 * NW);  // wave-level loads per wave (NW waves share a tile)
   static_assert(INSTS >= 1, "tile too small for this many waves");
-  static_assert(ROWS == 64 || ROWS >= 128, "the chunk permutations stay inside rows of these lengths");
+  static_assert(!MC || ROWS == 64 || ROWS >= 128, "the chunk permutations stay inside rows of these lengths");
   typedef uint32_t Offsets[INSTS];
 
   // per-lane byte offsets (from the tile's first element) of this wave's loads;

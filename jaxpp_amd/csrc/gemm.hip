@@ -26,7 +26,7 @@
 #include <mutex>
 #include <string>
 
-#include "common.h"
+#include "gemm_wave.h"
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -96,46 +96,6 @@ struct GemmArgs<true> {
   GemmParams p;          // problem 0 and everything the problems share
   GemmProblem more[3];   // problems 1..3; `first` past the grid for those not in use
 };
-
-// erf(u / sqrt 2) and exp(-u^2 / 2) for the exact GELU and its derivative: the rational
-// approximation 7.1.26 of Abramowitz & Stegun (one reciprocal, one exponential, five fused
-// multiply-adds; absolute error 6e-7 in fp32, that of a float erf 1e-7 - either is three
-// orders below half a bf16 ulp of the results, and on bf16-valued N(0, 1.5) inputs as many
-// of the rounded results differ from a float64 evaluation's as with the library's erff: 2e-3
-// of gelu's - tiny values of the negative tail -, 4e-4 of its derivative's).  The library
-// call costs about 35 instructions, and an epilogue of a 256 x 256 tile makes 128 of them per
-// lane: 17 - 23 us of a 52 - 58 us GEMM at 4096 x 4096 x 1024.
-__device__ __forceinline__ void erf_and_gauss(float u, float& erf_x, float& gauss) {
-  const float ax = fabsf(u) * 0.7071067811865476f;
-  const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, ax, 1.0f));
-  gauss = __expf(-ax * ax);
-  float poly = fmaf(1.061405429f, t, -1.453152027f);
-  poly = fmaf(poly, t, 1.421413741f);
-  poly = fmaf(poly, t, -0.284496736f);
-  poly = fmaf(poly, t, 0.254829592f);
-  erf_x = copysignf(fmaf(-poly * t, gauss, 1.0f), u);
-}
-
-__device__ __forceinline__ float gelu_f(float u, int tanh_form) {
-  if (tanh_form) {
-    float t = tanhf(0.7978845608028654f * (u + 0.044715f * u * u * u));
-    return 0.5f * u * (1.0f + t);
-  }
-  float e, g;
-  erf_and_gauss(u, e, g);
-  return 0.5f * u * (1.0f + e);
-}
-
-__device__ __forceinline__ float gelu_grad_f(float u, int tanh_form) {
-  if (tanh_form) {
-    float t = tanhf(0.7978845608028654f * (u + 0.044715f * u * u * u));
-    return 0.5f * (1.0f + t) +
-           0.5f * u * (1.0f - t * t) * 0.7978845608028654f * (1.0f + 0.134145f * u * u);
-  }
-  float e, g;
-  erf_and_gauss(u, e, g);
-  return 0.5f * (1.0f + e) + u * g * 0.3989422804014327f;
-}
 
 // (sigmoid through the hardware reciprocal, 1 ulp: a correctly rounded division is ten
 // instructions, and an epilogue evaluates 64 - 128 of these per lane)
@@ -1006,6 +966,18 @@ int choose_tile(const jpp_gemm_args* a) {
   return tile == kTile64 && a->rope_cos && a->rope_head_dim > 64 ? (int)kTile64x128 : tile;
 }
 
+// Products that run on waves of their own (gemm_wave.hip): while their 32x64 tiles are at most one
+// per CU.  Over 65 random shapes below that line (M, N, K 128 .. 8192; both orientations, plain and
+// GELU epilogues) they take 0.99 to 0.70 of the time of the best tile here, 0.8 in the median;
+// above it, two rounds of them, 1.01 to 1.45.  A plain forward product without bias and
+// residual stays: its bits are those a product with the rotary epilogue rotates.
+bool runs_on_waves(const jpp_gemm_args* a) {
+  const bool kind = a->epilogue == JPP_EPI_BF16 ? !a->trans_b || a->bias || a->resid
+                                                : a->epilogue == (a->trans_b ? JPP_EPI_GELU : JPP_EPI_DGELU);
+  return kind && !a->tile && !a->trans_a && a->group_mode == JPP_GROUP_NONE && a->k_parts <= 1 &&
+         !a->rope_cos && (a->m / 32) * (a->n / 64) <= kCus;
+}
+
 // sub-problem whose first row / column is (m_off, n_off) of the full one
 void shift_origin(GemmParams& p, bool ta, bool tb, int epi, long m_off, long n_off) {
   p.a += ta ? m_off : m_off * p.lda;
@@ -1155,6 +1127,13 @@ extern "C" int jpp_gemm_bf16(void* stream_, const jpp_gemm_args* a) {
   GemmParams p;
   if (int rc = prepare(a, p)) return rc;
   int tile = a->tile ? a->tile : choose_tile(a);
+  if (runs_on_waves(a)) {
+    const GemmWave d = {p.a, p.b, (bf16_t*)p.c, (bf16_t*)p.c2, p.bias, p.resid, p.aux, p.m, p.n, p.k,
+                        p.lda, p.ldb, p.ldc, p.ldc2, p.ldresid, p.ldaux, p.gelu_tanh};
+    ProbeScope probe(stream, a->trans_b ? "gemm_nn_wave" : "gemm_nt_wave", 2.0 * a->m * a->n * a->k,
+                     2.0 * (a->m * a->k + a->n * a->k + a->m * a->n));
+    return launch_gemm_wave(stream, d, a->trans_b != 0, a->epilogue);
+  }
   // several operand pairs of an ungrouped product: the 256-wide tiles whatever its size
   // (jpp_gemm_bf16_multi is the way to run small ones)
   if (a->k_parts > 1 && !a->tile && a->group_mode == JPP_GROUP_NONE) tile = kTile256;

@@ -1,0 +1,167 @@
+// bf16 products of few tiles: C[m,n] = epilogue(sum_k A[m,k] Bop[n,k]), A's contraction index
+// contiguous (forward and input-gradient products).
+//
+// A workgroup owns 32 x 64 outputs; its four waves each multiply the whole tile over every fourth
+// K-step of 64 and their sums meet in LDS, in wave order.  With fewer tiles than CUs a product's
+// time is one tile's, and a tile whose waves share their operands in LDS is a chain of
+// latencies: barrier, fragment reads, copies, K-step after K-step.  Here every wave copies its own
+// steps into LDS of its own and waits for nothing but them: no barrier before the sums, and the
+// copies of four waves keep the CU's path to memory (64 bytes a cycle) busy, which is then what
+// bounds the tile: 12 KB a K-step, 192 cycles.  512 x 1024 x 4096 (256 tiles) 17.4 -> 13.9 us,
+// 512 x 1024 x 1024 9.0 -> 7.4, 256 x 256 x 768 7.2 -> 5.7, 128 x 128 x 128 5.0 -> 4.3, against
+// 64 x 64 tiles shared by two wave groups.  (64 x 64 outputs this way: two stages are all that
+// fits, 15.8 us for the first; operands from L2 straight into fragments, without LDS: 28 us, a
+// load of 16 rows x 64 bytes holds the path far longer than its kilobyte.)
+//
+// The operands' LDS images and the fragments read from them are those of gemm.hip (DmaTile), the
+// n side on the MFMA's A port: lane (c = lane % 16, g = lane / 16) ends up with row 16 i + c and
+// columns 16 j + 4 g + r of tile (i, j).
+#include <math.h>
+
+#include "gemm_wave.h"
+
+namespace {
+
+constexpr int W = 4;     // waves, one per SIMD
+constexpr int BM = 32, TM = BM / 16, NS = 3;   // rows of a tile, stages of a wave
+constexpr int PITCH = 68;                      // floats of a row of the sums
+
+template <bool TB, int EPI>
+__global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
+  using TileA = DmaTile<BM, false, 1>;
+  using TileB = DmaTile<64, TB, 1>;
+  constexpr int STAGE = TileA::BYTES + TileB::BYTES, COPIES = TileA::INSTS + TileB::INSTS;
+  extern __shared__ __align__(1024) uint8_t smem[];   // [W][NS][STAGE]; then [W][BM][PITCH] floats
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Consecutive workgroups go to the eight XCDs in turn, each with an L2 of its own: every XCD
+  // takes a run of tiles, 256 rows at a time, so that it reads a part of both operands.
+  const int tiles_n = p.n / 64, tiles_m = p.m / BM;
+  int pid = blockIdx.x;
+  if ((gridDim.x & 7) == 0) pid = (pid & 7) * (gridDim.x >> 3) + (pid >> 3);
+  const int rows = 256 / BM, first = pid / (rows * tiles_n) * rows, rows_here = min(tiles_m - first, rows);
+  const int within = pid - first * tiles_n;
+  const long m0 = (long)(first + within % rows_here) * BM, n0 = (long)(within / rows_here) * 64;
+
+  // the epilogue's share of this thread: 8 columns of a row; what it adds or multiplies with
+  // arrives during the contraction
+  static_assert(BM * 8 == 64 * W, "one piece of a row per thread");
+  const long row = m0 + (tid >> 3), ocol = n0 + (tid & 7) * 8;
+  const bf16_t* const pre_src = EPI == JPP_EPI_DGELU ? p.aux : EPI == JPP_EPI_BF16 ? p.resid : nullptr;
+  const long pre_ld = EPI == JPP_EPI_DGELU ? p.ldaux : p.ldresid;
+  uint4 pre = make_uint4(0, 0, 0, 0), bias = pre;
+  if (pre_src) pre = *(const uint4*)(pre_src + row * pre_ld + ocol);
+  if (p.bias) bias = *(const uint4*)(p.bias + ocol);
+
+  f32x4 acc[TM][4];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = (p.k / 64 - wave + W - 1) / W;   // wave, wave + W, ...
+  if (steps > 0) {
+    typename TileA::Offsets offa;
+    typename TileB::Offsets offb;
+    TileA::offsets(offa, p.lda, 0, lane);
+    TileB::offsets(offb, p.ldb, 0, lane);
+    const long step_b = TB ? 64 * p.ldb : 64;
+    const bf16_t* const pa = p.a + m0 * p.lda + wave * 64;
+    const bf16_t* const pb = p.b + (TB ? n0 : n0 * p.ldb) + wave * step_b;
+    const uint8_t* const stages = smem + wave * (NS * STAGE);
+    const uint32_t lds0 = lds_address(stages);
+    auto copy = [&](int stage, int t) {
+      const long at = min(t, steps - 1);   // (past the end the last step again, unused)
+      TileA::template issue<0, TileA::INSTS>(uniform_ptr(pa + at * (W * 64)), offa, lds0 + stage * STAGE, 0);
+      TileB::template issue<0, TileB::INSTS>(uniform_ptr(pb + at * W * step_b), offb,
+                                             lds0 + stage * STAGE + TileA::BYTES, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < NS; ++s) copy(s, s);
+    int st = 0;
+    for (int t = 0; t < steps; ++t) {
+      dma_wait<(NS - 1) * COPIES>();   // (copies land in order: this step's have)
+      const uint8_t* const sa = stages + st * STAGE;
+      const uint8_t* const sb = sa + TileA::BYTES;
+      bf16x8 fa[2][TM], fb[2][4];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) fb[k][j] = TileB::frag16(sb, 16 * j, k, lane);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fa[k][i] = TileA::frag16(sa, 16 * i, k, lane);
+      }
+      // every fragment is in registers: the stage can be filled again, under the MFMAs
+      lds_wait_all();
+      copy(st, t + NS);
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[k][j], fa[k][i], acc[i][j], 0, 0, 0);
+      st = st + 1 == NS ? 0 : st + 1;
+    }
+  }
+  dma_wait_all();    // (the copies past the end must not land in what the sums are staged in)
+  __syncthreads();
+  float* const part = (float*)smem;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *(f32x4*)(part + (wave * BM + 16 * i + c) * PITCH + 16 * j + 4 * g) = acc[i][j];
+  __syncthreads();
+  const float* src = part + (tid >> 3) * PITCH + (tid & 7) * 8;
+  f32x4 lo = *(const f32x4*)src, hi = *(const f32x4*)(src + 4);
+#pragma unroll
+  for (int w = 1; w < W; ++w) {
+    lo += *(const f32x4*)(src + w * BM * PITCH);
+    hi += *(const f32x4*)(src + w * BM * PITCH + 4);
+  }
+  float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, q[8];
+  if (p.bias) {
+    unpack8(bias, q);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] += q[e];
+  }
+  unpack8(pre, q);
+  if constexpr (EPI == JPP_EPI_BF16) {
+    if (p.resid) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += q[e];
+    }
+  } else if constexpr (EPI == JPP_EPI_DGELU) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] *= gelu_grad_f(q[e], p.gelu_tanh);
+  } else {
+    float gl[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) gl[e] = gelu_f(v[e], p.gelu_tanh);
+    *(uint4*)(p.c2 + row * p.ldc2 + ocol) = pack8(gl);
+  }
+  *(uint4*)(p.c + row * p.ldc + ocol) = pack8(v);
+}
+
+template <bool TB, int EPI>
+int launch(hipStream_t st, const GemmWave& p) {
+  constexpr int LOOP = W * NS * (BM + 64) * 128, SUMS = W * BM * PITCH * 4, SMEM = LOOP > SUMS ? LOOP : SUMS;
+  static_assert(SMEM <= 160 * 1024, "LDS of one CU");
+  auto kern = gemm_wave_kernel<TB, EPI>;
+  static std::once_flag configured;   // (the limit is sticky per kernel)
+  static hipError_t configure_rc = hipSuccess;
+  std::call_once(configured, [&] {
+    configure_rc = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+  });
+  JPP_CHECK_HIP(configure_rc);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((p.m / BM) * (p.n / 64))), dim3(64 * W), SMEM, st, p);
+  JPP_LAUNCH_CHECK();
+  return JPP_OK;
+}
+
+}  // namespace
+
+int launch_gemm_wave(hipStream_t st, const GemmWave& p, bool tb, int epi) {
+  if (tb) return epi == JPP_EPI_BF16 ? launch<true, JPP_EPI_BF16>(st, p) : launch<true, JPP_EPI_GELU>(st, p);
+  return epi == JPP_EPI_BF16 ? launch<false, JPP_EPI_BF16>(st, p) : launch<false, JPP_EPI_DGELU>(st, p);
+}
