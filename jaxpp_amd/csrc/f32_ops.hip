@@ -8,6 +8,8 @@
 // order that the shapes fix.
 #include <math.h>
 
+#include <mutex>
+
 #include "common.h"
 
 namespace {
@@ -108,6 +110,9 @@ struct Frag32 {
   }
 };
 
+template <int BM>
+constexpr int kStages32 = BM == 16 ? 3 : 2;   // (what fits beside the sums)
+
 // A workgroup owns BM x 64 outputs; its four waves each multiply the whole tile over every
 // fourth step of 16 contraction elements, and their four sums meet in LDS in wave order.
 // These products are small (512 x 256 x 256 and a few times that): what bounds them is latency,
@@ -119,9 +124,18 @@ struct Frag32 {
 // 6.5 us, 512 x 256 x 1024 9.7 us; the 64 x 64 tile of 16 x 16 threads in its place, one barrier
 // pair per 16 contraction elements on 32 CUs, and attention with a pair of lanes per row made a
 // two-layer row of eight microbatches of 512 tokens 30.0 ms, now 2.30 ms.
-template <int BM, bool TA, bool TB>
+//
+// STAGED (both contraction indices contiguous): every wave copies its own steps, 32 elements of
+// the contraction at a time, into LDS of its own and reads the fragments there, with no barrier
+// either.  A fragment loaded from memory directly touches 16 rows with 64 bytes each, and the
+// CU's path takes such a load far longer than one of eight whole lines; of the operands of the
+// other orientations one is read along its rows anyway.  (A 32-element step is 128 bytes a row:
+// the LDS image is that of a bf16 tile of 64.)
+template <int BM, bool TA, bool TB, bool STAGED>
 __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
   constexpr int TM = BM / 16, TN = 4, D = BM == 64 ? 2 : 4, PITCH = 68;
+  static_assert(!STAGED || (!TA && !TB && BM <= 32), "staged: both operands [rows][k], two tiles' LDS");
+  extern __shared__ __align__(1024) uint8_t smem[];   // (STAGED) [4 waves][stages][BM + 64 rows of 128 bytes]
   __shared__ float part[2][4][16 * PITCH];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -162,7 +176,56 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int steps = (p.k / 16 - wave + 3) / 4;   // wave, wave + 4, ...
+  if constexpr (STAGED) {
+    constexpr int NS = kStages32<BM>, STAGE = (BM + 64) * 128;
+    using TileA = DmaTile<BM, false, 1>;
+    using TileB = DmaTile<64, false, 1>;
+    const int steps = (p.k / 32 - wave + 3) / 4;   // wave, wave + 4, ...
+    if (steps > 0) {
+      typename TileA::Offsets offa;
+      typename TileB::Offsets offb;
+      TileA::offsets(offa, 2 * p.lda, 0, lane);    // (in 2-byte elements)
+      TileB::offsets(offb, 2 * p.ldb, 0, lane);
+      const bf16_t* const pa = (const bf16_t*)(p.a + m0 * p.lda + wave * 32);
+      const bf16_t* const pb = (const bf16_t*)(p.b + n0 * p.ldb + wave * 32);
+      const uint8_t* const stages = smem + wave * (NS * STAGE);
+      const uint32_t lds0 = lds_address(stages);
+      auto copy = [&](int stage, int t) {
+        const long at = min(t, steps - 1) * 256L;  // (past the end the last step again, unused)
+        TileA::template issue<0, TileA::INSTS>(uniform_ptr(pa + at), offa, lds0 + stage * STAGE, 0);
+        TileB::template issue<0, TileB::INSTS>(uniform_ptr(pb + at), offb, lds0 + stage * STAGE + BM * 128, 0);
+      };
+#pragma unroll
+      for (int q = 0; q < NS; ++q) copy(q, q);
+      int st = 0;
+      for (int t = 0; t < steps; ++t) {
+        dma_wait<(NS - 1) * (TileA::INSTS + TileB::INSTS)>();
+        const uint8_t* const sa = stages + st * STAGE;
+        f32x4 fa[2][TM], fb[2][TN];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) fb[h][j] = *(const f32x4*)(sa + BM * 128 + slab_off(16 * j + c, 4 * h + g));
+#pragma unroll
+          for (int i = 0; i < TM; ++i) fa[h][i] = *(const f32x4*)(sa + slab_off(16 * i + c, 4 * h + g));
+        }
+        lds_wait_all();   // every fragment is in registers: the stage can be filled again
+        copy(st, t + NS);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+              for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[h][j][s], fa[h][i][s], acc[i][j], 0, 0, 0);
+        st = st + 1 == NS ? 0 : st + 1;
+      }
+    }
+    dma_wait_all();
+  }
+  const int steps = STAGED ? 0 : (p.k / 16 - wave + 3) / 4;   // wave, wave + 4, ...
   if (steps > 0) {
     const long step_a = TA ? 64 * p.lda : 64, step_b = TB ? 64 * p.ldb : 64;
     const float* pa = FA::lane_ptr(p.a + (TA ? m0 : m0 * p.lda), p.lda, c, g) + wave * (step_a / 4);
@@ -257,12 +320,32 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
 }
 
 template <int BM>
-void sgemm_launch(hipStream_t st, const SgemmParams& p) {
+int sgemm_launch(hipStream_t st, const SgemmParams& p) {
   const dim3 grid((unsigned)(p.m / BM * (p.n / 64)), 1u, p.group_mode == JPP_GROUP_K ? (unsigned)p.n_seg : 1u);
-  if (p.ta && p.tb) hipLaunchKernelGGL((sgemm_kernel<BM, true, true>), grid, dim3(256), 0, st, p);
-  else if (p.ta) hipLaunchKernelGGL((sgemm_kernel<BM, true, false>), grid, dim3(256), 0, st, p);
-  else if (p.tb) hipLaunchKernelGGL((sgemm_kernel<BM, false, true>), grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((sgemm_kernel<BM, false, false>), grid, dim3(256), 0, st, p);
+  // (copies of 16 bytes, whole steps)
+  const bool staged = BM <= 32 && !p.ta && !p.tb && p.k % 32 == 0 && (p.lda | p.ldb | p.stride_b) % 4 == 0 &&
+                      ((uintptr_t)p.a | (uintptr_t)p.b) % 16 == 0;
+  if constexpr (BM <= 32) {
+    if (staged) {
+      constexpr int SMEM = 4 * kStages32<BM> * (BM + 64) * 128;
+      auto kern = sgemm_kernel<BM, false, false, true>;
+      static std::once_flag configured;   // (the limit is sticky per kernel)
+      static hipError_t configure_rc = hipSuccess;
+      std::call_once(configured, [&] {
+        configure_rc = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM);
+      });
+      JPP_CHECK_HIP(configure_rc);
+      hipLaunchKernelGGL(kern, grid, dim3(256), SMEM, st, p);
+      JPP_LAUNCH_CHECK();
+      return JPP_OK;
+    }
+  }
+  if (p.ta && p.tb) hipLaunchKernelGGL((sgemm_kernel<BM, true, true, false>), grid, dim3(256), 0, st, p);
+  else if (p.ta) hipLaunchKernelGGL((sgemm_kernel<BM, true, false, false>), grid, dim3(256), 0, st, p);
+  else if (p.tb) hipLaunchKernelGGL((sgemm_kernel<BM, false, true, false>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((sgemm_kernel<BM, false, false, false>), grid, dim3(256), 0, st, p);
+  JPP_LAUNCH_CHECK();
+  return JPP_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -822,11 +905,9 @@ int jpp_gemm_f32(void* stream, const jpp_gemm_args* a) {
   p.stride_b = a->stride_b; p.stride_c = a->stride_c;
   // the tallest tile that still gives every CU one (a taller tile reads its B fewer times)
   const long strips = (a->m / 16) * (a->n / 64) * (group_k ? a->n_seg : 1);
-  if (strips >= 4 * 256) sgemm_launch<64>((hipStream_t)stream, p);
-  else if (strips >= 2 * 256) sgemm_launch<32>((hipStream_t)stream, p);
-  else sgemm_launch<16>((hipStream_t)stream, p);
-  JPP_LAUNCH_CHECK();
-  return JPP_OK;
+  if (strips >= 4 * 256) return sgemm_launch<64>((hipStream_t)stream, p);
+  if (strips >= 2 * 256) return sgemm_launch<32>((hipStream_t)stream, p);
+  return sgemm_launch<16>((hipStream_t)stream, p);
 }
 
 int jpp_rope_f32(void* stream, float* x, int64_t ld, const float* cos_tab, const float* sin_tab,

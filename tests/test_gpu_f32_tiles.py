@@ -25,31 +25,34 @@ def dev(a):
     return rt.DeviceBuffer.from_numpy(np.ascontiguousarray(a, dtype=np.float32))
 
 
-def padded(x, pad):
-    """x in rows of a leading dimension `pad` larger, and a device copy one float past an
+def padded(x, pad, at=4):
+    """x in rows of a leading dimension `pad` larger, and a device copy `at` bytes past an
     aligned address."""
     ld = x.shape[1] + pad
-    h = np.zeros(x.shape[0] * ld + 1, np.float32)
-    h[1:].reshape(x.shape[0], ld)[:, :x.shape[1]] = x
+    h = np.zeros(x.shape[0] * ld + at // 4, np.float32)
+    h[at // 4:].reshape(x.shape[0], ld)[:, :x.shape[1]] = x
     return dev(h), ld
 
 
 # strips of 16 x 64: fewer than a CU each (16-row tiles), two each (32), four each (64)
-SHAPES = [(64, 64, 16), (64, 128, 48), (128, 64, 80), (512, 1024, 144), (1024, 1024, 64), (1024, 1088, 208)]
+SHAPES = [(64, 64, 16), (64, 64, 32), (64, 128, 48), (128, 64, 80), (128, 128, 416), (512, 1024, 144),
+          (512, 1024, 160), (1024, 1024, 64), (1024, 1088, 208)]
 
 
+@pytest.mark.parametrize("aligned", [False, True])
 @pytest.mark.parametrize("lay", ["nn", "nt", "tn", "tt"])
 @pytest.mark.parametrize("m,n,k", SHAPES, ids=["x".join(map(str, s)) for s in SHAPES])
-def test_gemm_f32_tiles(lay, m, n, k):
+def test_gemm_f32_tiles(lay, m, n, k, aligned):
     print(f"gemm_f32 {lay} {m}x{n}x{k}", flush=True)
     rng = np.random.default_rng(m * 7 + n * 3 + k)
     ta, tb = {"nn": (0, 1), "nt": (0, 0), "tn": (1, 1), "tt": (1, 0)}[lay]
     A, B = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
     c0 = rng.standard_normal((m, n), dtype=np.float32)
-    da, lda = padded(A.T if ta else A, 3)
-    db, ldb = padded(B.T if tb else B, 5)
+    at = 0 if aligned else 4        # the operands' distance from an aligned address
+    da, lda = padded(A.T if ta else A, 4 if aligned else 3, at)
+    db, ldb = padded(B.T if tb else B, 8 if aligned else 5, at)
     dc, ldc = padded(c0, 1)
-    rt.gemm(da.ptr + 4, db.ptr + 4, dc.ptr + 4, m, n, k, lda, ldb, ldc, ta, tb, rt.EPI_ACC_F32, f32=True)
+    rt.gemm(da.ptr + at, db.ptr + at, dc.ptr + 4, m, n, k, lda, ldb, ldc, ta, tb, rt.EPI_ACC_F32, f32=True)
     rt.sync()
     raw = dc.download(np.float32, (m * ldc + 1,))
     got = raw[1:].reshape(m, ldc)
