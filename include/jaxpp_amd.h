@@ -96,7 +96,7 @@ int jpp_graph_destroy(void* graph_exec);
  *       nt: dx = dy W^T, tn: dW = x^T dy)
  *   (+ "w8" for 8-wave tiles, "s3" - "s5" for 3 to 5 LDS stages, "k2" for tiles shared by two
  *   wave groups, "_multi" for several products in one launch),
- *   attn_fwd, attn_bwd_dq, attn_bwd_dkv, norm_fwd, norm_bwd, swiglu_fwd,
+ *   gemm_{nn,nt}_wave, attn_fwd, attn_bwd_dq, attn_bwd_dkv, attn_bwd_small, norm_fwd, norm_bwd, swiglu_fwd,
  *   swiglu_bwd, rope, grad_accum, colsum, adam */
 int jpp_probe_begin(const char* kernel_class);
 int jpp_probe_end(int64_t* launches, double* total_ms, double* total_flops, double* total_bytes);
