@@ -120,16 +120,17 @@ constexpr int kStages32 = BM == 16 ? 3 : 2;   // (what fits beside the sums)
 // contraction, and operands go from L2 straight into MFMA fragments - no barrier and no LDS
 // before the sums, D steps of loads in flight per wave.  v_mfma_f32_16x16x4_f32 accumulates as
 // a chain of fused multiply-adds does, at twice the rate of v_fma_f32; the four shorter chains
-// halve the distance to a float64 sum (5.7e-7 -> 2.9e-7 at k = 1024).  512 x 256 x 256 takes
-// 6.5 us, 512 x 256 x 1024 9.7 us; the 64 x 64 tile of 16 x 16 threads in its place, one barrier
+// halve the distance to a float64 sum (5.7e-7 -> 2.9e-7 at k = 1024).  512 x 256 outputs, k = 256
+// and 1024, take 7.3 us on average; the 64 x 64 tile of 16 x 16 threads in its place, one barrier
 // pair per 16 contraction elements on 32 CUs, and attention with a pair of lanes per row made a
-// two-layer row of eight microbatches of 512 tokens 30.0 ms, now 2.30 ms.
+// two-layer row of eight microbatches of 512 tokens 30.0 ms, now 2.15 ms.
 //
 // STAGED (both contraction indices contiguous): every wave copies its own steps, 32 elements of
 // the contraction at a time, into LDS of its own and reads the fragments there, with no barrier
 // either.  A fragment loaded from memory directly touches 16 rows with 64 bytes each, and the
 // CU's path takes such a load far longer than one of eight whole lines; of the operands of the
-// other orientations one is read along its rows anyway.  (A 32-element step is 128 bytes a row:
+// other orientations one is read along its rows anyway (512 x 256, k = 256 to 1024: 10.3 -> 7.0 us
+// on average).  (A 32-element step is 128 bytes a row:
 // the LDS image is that of a bf16 tile of 64.)
 template <int BM, bool TA, bool TB, bool STAGED>
 __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
