@@ -148,7 +148,8 @@ typedef struct {
   int tile;          /* 0: choose (may run the last, half-empty round of 256x256 tiles as a second
                         launch of 128x256 tiles); 1: 128x128; 2: 256x128; 3: 128x256; 4: 256x256
                         (8 waves each); 5: 64x64 (two groups of 4 waves that take the K-steps in
-                        turn: the even and the odd steps are summed apart, then added) */
+                        turn: the even and the odd steps are summed apart, then added; not with
+                        a rotary epilogue of heads of 128, which such a tile splits) */
   /* grouped GEMM over experts (0 = plain).  seg: device int32 [n_seg + 1], row
    * offsets of the expert groups in the token-permuted buffers, multiples of 256.
    *   JPP_GROUP_M: rows of A and C are grouped; group e multiplies b + e * stride_b.

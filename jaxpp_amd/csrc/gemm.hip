@@ -1138,6 +1138,10 @@ extern "C" int jpp_gemm_bf16(void* stream_, const jpp_gemm_args* a) {
   // (jpp_gemm_bf16_multi is the way to run small ones)
   if (a->k_parts > 1 && !a->tile && a->group_mode == JPP_GROUP_NONE) tile = kTile256;
   JPP_REQUIRE(a->tile >= 0 && a->tile <= 5, "gemm: unknown tile %d", a->tile);
+  // (the rotary epilogue finds a column's partner in the staged row of its own tile)
+  JPP_REQUIRE(a->tile != kTile64 || !a->rope_cos || a->rope_head_dim <= 64,
+              "gemm: the rotary epilogue's heads of %d elements do not lie inside a 64x64 tile (tile 5)",
+              a->rope_head_dim);
   if ((tile == kTile256x128 || tile == kTile256) && a->m % 256) tile = a->n % 256 ? kTile128 : kTile128x256;
   if ((tile == kTile128x256 || tile == kTile256) && a->n % 256) tile = a->m % 256 ? kTile128 : kTile256x128;
 

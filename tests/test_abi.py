@@ -63,6 +63,18 @@ def test_error_convention_without_gpu():
     assert lib.jpp_stage_adam_step(None, None, 1, 0.0, 0.0, 0.0, 0.0, 0.0) == -1
 
 
+def test_a_tile_narrower_than_a_rotated_head_is_refused():
+    """The 64x64 tile (5) holds half of a head of 128, so its rotary epilogue would read a
+    column's partner outside the staged row.  (Host check: no device, no memory is touched.)"""
+    at = 1 << 20
+    a = rt.GemmArgs()
+    a.a = a.b = a.c = a.rope_cos = a.rope_sin = at
+    a.m, a.n, a.k, a.lda, a.ldb, a.ldc = 128, 256, 64, 64, 256, 256
+    a.trans_b, a.tile, a.rope_cols, a.rope_seq, a.rope_head_dim = 1, 5, 256, 128, 128
+    assert rt.load().jpp_gemm_bf16(None, ctypes.byref(a)) == -1
+    assert b"64x64 tile" in rt.load().jpp_last_error()
+
+
 def test_workspace_sizes():
     """jpp_workspace_bytes: what the tests allocate by hand for each operator's scratch."""
     lib = rt.load()

@@ -63,6 +63,24 @@ def test_rotated_heads_of_128_on_small_tiles(k):
     np.testing.assert_array_equal(fused.download_bf16((m, n)), plain.download_bf16((m, n)))
 
 
+@pytest.mark.parametrize("batch,heads,rot,k", [(1, 4, 2, 64), (2, 10, 7, 448), (9, 20, 20, 64)])
+def test_rotated_heads_of_64_on_64x64_tiles(batch, heads, rot, k):
+    """Tile 5 holds a head of 64 whole (odd tile columns and rows among them, more tiles than
+    CUs); a rotated head of 128 is refused, tests/test_abi.py."""
+    seq, d = 128, 64
+    print(f"gemm+rope on 64x64 tiles, {batch} x {heads}/{rot} heads, k={k}", flush=True)
+    rng = np.random.default_rng(batch + k)
+    m, n = batch * seq, heads * d
+    da, dw = dev_bf16(rnd(rng, m, k)), dev_bf16(rnd(rng, k, n, scale=0.1))
+    cos, sin = (rt.DeviceBuffer.from_numpy(t) for t in L.rope_tables(seq, d, 5e5, np.float32))
+    plain, fused = rt.DeviceBuffer(2 * m * n), rt.DeviceBuffer(2 * m * n)
+    rt.gemm(da.ptr, dw.ptr, plain.ptr, m, n, k, k, n, n, 0, 1, tile=5)
+    rt.check(rt.load().jpp_rope(None, plain.ptr, n, cos.ptr, sin.ptr, batch, seq, rot, d, 0))
+    rt.gemm(da.ptr, dw.ptr, fused.ptr, m, n, k, k, n, n, 0, 1, tile=5, rope=(cos.ptr, sin.ptr, rot * d, seq, d))
+    rt.sync()
+    np.testing.assert_array_equal(fused.download_bf16((m, n)), plain.download_bf16((m, n)))
+
+
 @pytest.mark.parametrize("parts,k,shapes", [
     (1, 64, [(128, 384), (128, 128), (128, 256), (256, 128)]),          # 28 tiles of 64x64
     (3, 192, [(384, 128), (128, 640)]),                                  # nine steps over three pairs
