@@ -249,60 +249,72 @@ struct WgradBatch {
   }
 };
 
+// A gathered weight gradient by itself.
+int run_apart(jpp_stage* s, hipStream_t st, const jpp_gemm_args& q) {
+  const int pairs = q.k_parts > 1 ? q.k_parts : 1;
+  const void* xs[4] = {q.a, q.a_more[0], q.a_more[1], q.a_more[2]};
+  const void* dys[4] = {q.b, q.b_more[0], q.b_more[1], q.b_more[2]};
+  return wgrad_n(s, st, pairs, xs, q.lda, dys, q.ldb, (float*)q.c, q.m, q.n);
+}
+
 // Runs a layer's gathered weight gradients.  As one grid of 256x256 tiles when that takes fewer
 // rounds of the 256 CUs than the launches one by one (whose last rounds stay partly empty: a
 // round of 128x256 tiles for a rest of at most 128 tiles costs about 0.77 of a full one).  When
-// together they are less than a round (kFullGrid tiles), or not all a multiple of 256 in both
-// directions, always: one by one each would leave most of the device idle - four products of
-// 768 .. 3072 x 768 on 1152 tokens were 80 us in six launches, BERT-large's four (192 tiles of
-// 256x256 together) 3.3 % of that stage's step.  Which way is taken depends on the shapes only.
+// together they are less than a round (kFullGrid tiles), always: one by one each would leave
+// most of the device idle - four products of 768 .. 3072 x 768 on 1152 tokens were 80 us in six
+// launches, BERT-large's four (192 tiles of 256x256 together) 3.3 % of that stage's step.
+// A layer with a matrix that is not a multiple of 256 in both directions has no such grid.  Its
+// whole matrices of a full grid go by themselves (a group's microbatches as one product), and
+// from 1024 tokens on also those that fill the rounds of their own tiles (of 512 tiles of
+// 128x128, two per CU: a single round to three quarters, several to two thirds), each on its best
+// tile; the rest go together on small ones.  Rows of 4096 tokens a microbatch, all together /
+// like this: Llama-shaped, hidden 2048 and feed-forward 5504 12.6 / 11.2 ms, 4096 and 11136 23.4 /
+// 18.5; encoder of 1408 and 5632 9.2 / 8.9; decoder blocks of 1536 and 4224 8.26 / 7.89.  On 512
+// tokens the last three are 0.99 of the speed with those matrices apart.
+// Which way is taken depends on the shapes only.
 int run_wgrads(jpp_stage* s, hipStream_t st, WgradBatch& w) {
   constexpr long kFullGrid = 192;
-  const bool multi = w.n >= 2 && !s->f32() && s->d.fused_wgrad_accum;
-  bool whole = true;
+  bool whole = true, full[4] = {};
   long total = 0;
   double apart = 0;
   for (int i = 0; i < w.n; ++i) {
     const jpp_gemm_args& q = w.g[i];
-    whole = whole && q.m % 256 == 0 && q.n % 256 == 0;
+    const bool in_256 = q.m % 256 == 0 && q.n % 256 == 0;
     const long t = (q.m / 256) * (q.n / 256), rest = t % 256;
+    whole = whole && in_256;
+    const long t128 = (q.m / 128) * (q.n / 128), rounds = (t128 + 511) / 512;
+    full[i] = (in_256 && t >= kFullGrid) || (s->T >= 1024 && t128 >= 384 && 3 * t128 >= 2 * 512 * rounds);
     total += t;
     apart += (double)(t / 256) + (rest == 0 ? 0.0 : (rest <= 128 && t > 256 ? 0.77 : 1.0));
   }
-  if (multi && (!whole || total < kFullGrid || (double)((total + 255) / 256) < apart - 0.25)) {
-    // smallest first: measured 1 % faster than largest first at the Llama-3-8B shapes
-    jpp_gemm_args order[4];
-    for (int i = 0; i < w.n; ++i) order[i] = w.g[i];
-    std::stable_sort(order, order + w.n, [](const jpp_gemm_args& a, const jpp_gemm_args& b) {
-      return a.m * a.n < b.m * b.n;
-    });
-    // Less than a full grid: a group's microbatches go one by one, in order.  Their products are
-    // too small for the accumulators' traffic to matter, and the sums stay those of an ungrouped
-    // run to the last bit (Adam's first updates magnify a reassociated sum that is nearly zero).
-    const int pairs = order[0].k_parts > 1 ? order[0].k_parts : 1;
-    if (pairs > 1 && (!whole || total < kFullGrid)) {
-      for (int part = 0; part < pairs; ++part) {
-        jpp_gemm_args one[4];
-        for (int i = 0; i < w.n; ++i) {
-          one[i] = order[i];
-          one[i].k_parts = 1;
-          if (part > 0) {
-            one[i].a = order[i].a_more[part - 1];
-            one[i].b = order[i].b_more[part - 1];
-          }
-        }
-        RC(jpp_gemm_bf16_multi(st, one, w.n));
+  const bool one_grid = total < kFullGrid || (double)((total + 255) / 256) < apart - 0.25;
+  const bool may_gather = !s->f32() && s->d.fused_wgrad_accum && (!whole || one_grid);
+  jpp_gemm_args grid[4];
+  int n = 0;
+  for (int i = 0; i < w.n; ++i)
+    if (may_gather && (whole || !full[i])) grid[n++] = w.g[i];
+    else RC(run_apart(s, st, w.g[i]));
+  if (n <= 1) return n ? run_apart(s, st, grid[0]) : JPP_OK;
+  // smallest first: measured 1 % faster than largest first at the Llama-3-8B shapes
+  std::stable_sort(grid, grid + n, [](const jpp_gemm_args& a, const jpp_gemm_args& b) {
+    return a.m * a.n < b.m * b.n;
+  });
+  // Less than a full grid: a group's microbatches go one by one, in order.  Their products are
+  // too small for the accumulators' traffic to matter, and the sums stay those of an ungrouped
+  // run to the last bit (Adam's first updates magnify a reassociated sum that is nearly zero).
+  const int pairs = grid[0].k_parts > 1 ? grid[0].k_parts : 1;
+  if (pairs == 1 || (whole && total >= kFullGrid)) return jpp_gemm_bf16_multi(st, grid, n);
+  for (int part = 0; part < pairs; ++part) {
+    jpp_gemm_args one[4];
+    for (int i = 0; i < n; ++i) {
+      one[i] = grid[i];
+      one[i].k_parts = 1;
+      if (part > 0) {
+        one[i].a = grid[i].a_more[part - 1];
+        one[i].b = grid[i].b_more[part - 1];
       }
-      return JPP_OK;
     }
-    return jpp_gemm_bf16_multi(st, order, w.n);
-  }
-  for (int i = 0; i < w.n; ++i) {
-    const jpp_gemm_args& q = w.g[i];
-    const int pairs = q.k_parts > 1 ? q.k_parts : 1;
-    const void* xs[4] = {q.a, q.a_more[0], q.a_more[1], q.a_more[2]};
-    const void* dys[4] = {q.b, q.b_more[0], q.b_more[1], q.b_more[2]};
-    RC(wgrad_n(s, st, pairs, xs, q.lda, dys, q.ldb, (float*)q.c, q.m, q.n));
+    RC(jpp_gemm_bf16_multi(st, one, n));
   }
   return JPP_OK;
 }
