@@ -55,7 +55,10 @@ LLAMA = dict(n_kv_heads=4, head_dim=128, causal=True, rope_theta=5e5, eps=1e-5)
     # one without a matrix that fills a round: everything in one launch per microbatch
     (LayerSpec("bert", 896, 14, 3584, 128, 1, eps=1e-12), 2,
      lambda c: sum(c.values()) == 2 and all(k.endswith("_multi") for k in c)),
-], ids=["wide", "narrow"])
+    # 160 whole tiles together: one launch over both microbatches; 90: one for each
+    (LayerSpec("bert", 1024, 16, 3072, 128, 1, eps=1e-12), 2, lambda c: list(c.values()) == [1]),
+    (LayerSpec("bert", 768, 12, 2304, 128, 1, eps=1e-12), 2, lambda c: list(c.values()) == [2]),
+], ids=["wide", "narrow", "half-round", "less"])
 def test_weight_gradient_launches(spec, group, check):
     print(f"weight gradients of {spec.family} {spec.hidden}/{spec.ffn}, group {group}", flush=True)
     params = init_layer_params(spec, 3, 0, perturb=True)
