@@ -177,8 +177,8 @@ typedef struct {
    * weight gradients of several microbatches accumulate this way with one read and one write
    * of the fp32 accumulator instead of one per microbatch.  0 or 1: one pair.  Built for
    * trans_a = trans_b = 1 with JPP_EPI_ACC_F32, on every tile but 256x128 (`tile` 0 takes
-   * 256x256, or 128x256 when M is not a multiple of 256; a grouped contraction goes by its
-   * size); anything else is JPP_ERR_INVALID. */
+   * 256x256, 128x256 when M is not a multiple of 256, 128x128 when N is not; a grouped
+   * contraction goes by its size); anything else is JPP_ERR_INVALID. */
   const void* a_more[3];
   const void* b_more[3];
   int k_parts;

@@ -1144,6 +1144,8 @@ extern "C" int jpp_gemm_bf16(void* stream_, const jpp_gemm_args* a) {
               a->rope_head_dim);
   if ((tile == kTile256x128 || tile == kTile256) && a->m % 256) tile = a->n % 256 ? kTile128 : kTile128x256;
   if ((tile == kTile128x256 || tile == kTile256) && a->n % 256) tile = a->m % 256 ? kTile128 : kTile256x128;
+  // (256x128 is the one tile not built for several pairs)
+  if (a->k_parts > 1 && !a->tile && tile == kTile256x128) tile = kTile128;
 
   // A grid of 256x256 tiles whose last round fills at most half of the 256 CUs runs that
   // round as a separate launch of 128x256 tiles over the last rows or columns: a full round

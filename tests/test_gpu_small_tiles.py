@@ -105,6 +105,23 @@ def test_small_weight_gradients_in_one_launch(parts, k, shapes):
         close(dc.download(np.float32, shape), want, 1e-4 * math.sqrt(k * parts), f"multi {shape}")
 
 
+@pytest.mark.parametrize("m,n", [(128, 128), (128, 256), (256, 128), (768, 384), (384, 768), (256, 512)])
+def test_operand_pairs_of_every_extent(m, n):
+    """A weight gradient over three operand pairs, tile left to the library, whichever of M and N
+    are multiples of 256."""
+    k, parts = 192, 3
+    print(f"{parts} operand pairs {m}x{n}x{k}", flush=True)
+    rng = np.random.default_rng(m + n)
+    As, Bs = [rnd(rng, k, m) for _ in range(parts)], [rnd(rng, k, n, scale=0.3) for _ in range(parts)]
+    prev = rng.standard_normal((m, n)).astype(np.float32)
+    dA, dB, dc = [dev_bf16(a) for a in As], [dev_bf16(b) for b in Bs], rt.DeviceBuffer.from_numpy(prev)
+    rt.gemm(dA[0].ptr, dB[0].ptr, dc.ptr, m, n, k, m, n, n, 1, 1, rt.EPI_ACC_F32,
+            more=[(a.ptr, b.ptr) for a, b in zip(dA[1:], dB[1:])])
+    rt.sync()
+    want = prev + sum(a.astype(np.float64).T @ b.astype(np.float64) for a, b in zip(As, Bs))
+    close(dc.download(np.float32, (m, n)), want, 1e-4 * math.sqrt(k * parts), "operand pairs")
+
+
 @pytest.mark.parametrize("counts", [[70, 0, 256, 3], [300, 1, 64, 129]])
 def test_small_grouped_products(counts):
     """Row-grouped and contraction-grouped products that state how many rows hold data: small
