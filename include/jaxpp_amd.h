@@ -166,8 +166,9 @@ typedef struct {
   int n_seg;
   int group_mode;
   int64_t stride_b, stride_c;
-  int64_t group_rows; /* non-padding rows over all groups, for the probe's FLOP and byte
-                       * accounting only (0: the padded extent is counted) */
+  int64_t group_rows; /* non-padding rows over all groups (an estimate will do): for the probe's
+                       * FLOP and byte accounting, and for the choice of a tile where `tile`
+                       * leaves it to the library (0: the padded extent is counted, 256x256) */
   const int32_t* seg_rows; /* device int32 [n_seg] or NULL: rows of each group that hold data;
                             * the rest of a group is zero padding, which JPP_GROUP_K then leaves
                             * out of the contraction (whole 64-row steps of it) */

@@ -869,16 +869,53 @@ int launch_multi(hipStream_t stream, GemmParams* ps, int n) {
 
 // The 128x128 tile runs with five LDS stages (one workgroup per CU) when every CU has at most
 // one tile, else with two (two workgroups per CU); the 64x64 tile, whose two wave groups share
-// it, with four or two by the same rule.
-bool deep_stages(long tiles, long ksteps, int tile) {
-  return tiles <= kCus && (tile == kTile128 || ksteps > 8);
+// it, with four or two by the same rule if the contraction is long enough for the longer prologue:
+// more than 8 K-steps, of a grouped contraction (8 experts of 256 x 256, four / two stages:
+// 600 rows each 6.7 / 6.2 us, 1024 7.9 / 7.3, 2048 12.1 / 15.2) 24.
+bool deep_stages(long tiles, long ksteps, int tile, bool group_k = false) {
+  return tiles <= kCus && (tile == kTile128 || ksteps > (group_k ? 24 : 8));
 }
 
+struct Extent { long m, n; };
+
+// What the choice of a tile and of its form go by: the extent of the grid (of a grouped contraction
+// an output per group), the part of it that holds data (of grouped rows, if the caller counted
+// them) and the K-steps (of a grouped contraction the groups' average, 0 if not counted).
+// The form follows the grid also where grouped rows fill only a part of it: consecutive tiles
+// belong to one XCD, so the workgroups that find work lie on the first ones, more than one
+// per CU there (top-2 of 8 experts, hidden 512, on 512 tokens: the row 5 % slower with the form
+// by the rows that hold data).
+Extent grid_extent(const jpp_gemm_args* a) {
+  return {a->group_mode == JPP_GROUP_K ? a->m * a->n_seg : a->m, a->n};
+}
+Extent work_extent(const jpp_gemm_args* a) {
+  Extent e = grid_extent(a);
+  if (a->group_mode == JPP_GROUP_M && a->group_rows)   // half of a segment's last 256 rows are padding on average
+    e.m = std::min<long>(e.m, (a->group_rows + 128L * a->n_seg + 255) / 256 * 256);
+  return e;
+}
+long work_ksteps(const jpp_gemm_args* a) {
+  if (a->group_mode == JPP_GROUP_K) return a->group_rows ? a->group_rows / (64L * a->n_seg) + 1 : 0;
+  return a->k / 64 * (a->k_parts > 1 ? a->k_parts : 1);
+}
+// tiles of bm x bn in all of the extents, -1 if one does not divide into them
+long count_tiles(const Extent* e, int n, int bm, int bn) {
+  long tiles = 0;
+  for (int i = 0; i < n; ++i) {
+    if (e[i].m % bm || e[i].n % bn) return -1;
+    tiles += (e[i].m / bm) * (e[i].n / bn);
+  }
+  return tiles;
+}
+bool deep_form(const jpp_gemm_args* a, int tile) {
+  const Extent e = grid_extent(a);
+  const int b = tile == kTile64 ? 64 : 128;
+  return deep_stages(count_tiles(&e, 1, b, b), work_ksteps(a), tile, a->group_mode == JPP_GROUP_K);
+}
+
+// `deep`: which form of the 64x64 and 128x128 tiles
 template <bool TA, bool TB, int EPI>
-int launch_tiled(hipStream_t stream, GemmParams& p, int tile) {
-  const int bm = tile == kTile64 ? 64 : 128;
-  const long tiles = (long)(p.m / bm) * (p.n / bm) * (p.group_mode == JPP_GROUP_K ? p.n_seg : 1);
-  const bool deep = deep_stages(tiles, p.k / 64, tile);
+int launch_tiled(hipStream_t stream, GemmParams& p, int tile, bool deep) {
   switch (tile) {
     case kTile256x128:  // 8 waves of 128x32; three stages where the accumulator rows leave room
       return launch<256, 128, TA, TB, EPI, 8, EPI == JPP_EPI_ACC_F32 ? 2 : 3>(stream, p);
@@ -924,44 +961,35 @@ constexpr TileForm kWeightGrad[] = {
     {kTile128, 128, 128, true, 0.f, 6.0f, 0.46f, 0.46f},  {kTile128, 128, 128, false, 0.f, 4.5f, 0.75f, 0.81f},
     {kTile128x256, 128, 256, true, 0.f, 6.6f, 0.95f, 0.95f}, {kTile256, 256, 256, true, 0.f, 10.f, 1.28f, 1.28f}};
 
-struct Extent { long m, n; };
-
-// tile with the smallest estimate for products of these extents in one grid; *us: the estimate
-int cheapest_tile(const Extent* e, int n, long ksteps, bool wgrad, bool may_64, bool may_128x256, float* us) {
+// tile with the smallest estimate for products of these extents in one grid (`grid`: the extents
+// that its form goes by)
+int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool wgrad, bool group_k,
+                  bool may_128x256) {
   int best = kTile128;
   float best_us = 0.f;
   for (const TileForm& f : wgrad ? kWeightGrad : kForward) {
-    if ((f.tile == kTile64 && !may_64) || (f.tile == kTile128x256 && !may_128x256)) continue;
-    long tiles = 0;
-    for (int i = 0; i < n && tiles >= 0; ++i)
-      tiles = e[i].m % f.bm || e[i].n % f.bn ? -1 : tiles + (e[i].m / f.bm) * (e[i].n / f.bn);
+    if (f.tile == kTile128x256 && !may_128x256) continue;
+    const long tiles = count_tiles(e, n, f.bm, f.bn);
     if (tiles < 0) continue;
-    if ((f.tile == kTile64 || f.tile == kTile128) && f.deep != deep_stages(tiles, ksteps, f.tile)) continue;
+    if ((f.tile == kTile64 || f.tile == kTile128) &&
+        f.deep != deep_stages(count_tiles(grid, n, f.bm, f.bn), ksteps, f.tile, group_k)) continue;
     const long w = (tiles + kCus - 1) / kCus;
     const float t = f.start + w * (f.tile_cost + ksteps * (w == 1 ? f.lone_step : f.step));
     if (best_us == 0.f || t < best_us) { best_us = t; best = f.tile; }
   }
-  if (us) *us = best_us;
   return best;
 }
 
 // The 256x256 tile run by 8 waves (two per SIMD, so one wave's LDS reads hide under the other's
 // MFMAs) is the fastest whenever it gives most CUs a tile; smaller problems go by the estimate.
-// Grouped problems (whole 256-row segments) are estimated from the rows that hold data.
 int choose_tile(const jpp_gemm_args* a) {
-  const bool group_m = a->group_mode == JPP_GROUP_M, group_k = a->group_mode == JPP_GROUP_K;
-  Extent e = {a->m, a->n};
-  long ksteps = a->k / 64;
-  if (group_m && a->group_rows)   // half of a segment's last 256 rows are padding on average
-    e.m = std::min<long>(a->m, (a->group_rows + 128L * a->n_seg + 255) / 256 * 256);
-  if (group_k) {
-    e.m *= a->n_seg;              // an output per group
-    if (a->group_rows) ksteps = a->group_rows / (64L * a->n_seg) + 1;
-    else return kTile256;
-  }
+  const Extent e = work_extent(a);
+  if (a->group_mode != JPP_GROUP_NONE && !a->group_rows) return kTile256;
   const long t256 = e.m % 256 == 0 && e.n % 256 == 0 ? (e.m / 256) * (e.n / 256) : 0;
-  if (t256 >= kMostCus || (group_m && !a->group_rows)) return kTile256;
-  const int tile = cheapest_tile(&e, 1, ksteps, a->trans_a && a->trans_b, true, true, nullptr);
+  if (t256 >= kMostCus) return kTile256;
+  const Extent grid = grid_extent(a);
+  const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), a->trans_a && a->trans_b,
+                                 a->group_mode == JPP_GROUP_K, true);
   // (a rotated head lies inside one tile)
   return tile == kTile64 && a->rope_cos && a->rope_head_dim > 64 ? (int)kTile64x128 : tile;
 }
@@ -1001,10 +1029,10 @@ void shift_origin(GemmParams& p, bool ta, bool tb, int epi, long m_off, long n_o
   if (p.aux) p.aux += m_off * p.ldaux + c_cols;
 }
 
-int dispatch(hipStream_t stream, const jpp_gemm_args* a, GemmParams& p, int tile) {
+int dispatch(hipStream_t stream, const jpp_gemm_args* a, GemmParams& p, int tile, bool deep = false) {
   const int ta = a->trans_a != 0, tb = a->trans_b != 0, e = a->epilogue;
 #define JPP_GEMM_CASE(TA_, TB_, E_) \
-  if (ta == TA_ && tb == TB_ && e == E_) return launch_tiled<TA_, TB_, E_>(stream, p, tile)
+  if (ta == TA_ && tb == TB_ && e == E_) return launch_tiled<TA_, TB_, E_>(stream, p, tile, deep)
   JPP_GEMM_CASE(0, 1, JPP_EPI_BF16);     // forward
   JPP_GEMM_CASE(0, 1, JPP_EPI_GELU);     // forward + GELU
   JPP_GEMM_CASE(0, 1, JPP_EPI_F32);      // forward, f32 out (router logits)
@@ -1185,11 +1213,11 @@ extern "C" int jpp_gemm_bf16(void* stream_, const jpp_gemm_args* a) {
       wide.tail_split = 3;
       wide.m = (int)std::min<long>(a->m, 128 / tn * 256);    // at most 128
       int rc = dispatch(stream, a, head, 4);
-      if (rc == JPP_OK && small.m > 0) rc = dispatch(stream, a, small, 1);
+      if (rc == JPP_OK && small.m > 0) rc = dispatch(stream, a, small, kTile128, true);  // (at most 256 tiles)
       return rc != JPP_OK ? rc : dispatch(stream, a, wide, 3);
     }
   }
-  return dispatch(stream, a, p, tile);
+  return dispatch(stream, a, p, tile, deep_form(a, tile));
 }
 
 extern "C" int jpp_gemm_bf16_multi(void* stream_, const jpp_gemm_args* problems, int n_problems) {
@@ -1217,7 +1245,7 @@ extern "C" int jpp_gemm_bf16_multi(void* stream_, const jpp_gemm_args* problems,
   JPP_REQUIRE(tiles < (1L << 30), "gemm_multi: too many tiles");
   const long ksteps = (long)ps[0].k / 64 * ps[0].k_parts;
   const int tile = whole && t256 >= kMostCus ? (int)kTile256
-                   : cheapest_tile(e, n_problems, ksteps, true, true, false, nullptr);
+                   : cheapest_tile(e, e, n_problems, ksteps, true, false, false);
   const bool deep = deep_stages(tile == kTile64 ? tiles : tiles / 4, ksteps, tile);
   if (tile == kTile256) return launch_multi<256, 256, 8, 2>(stream, ps, n_problems);
   if (tile == kTile64)

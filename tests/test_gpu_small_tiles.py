@@ -156,3 +156,30 @@ def test_small_grouped_products(counts):
             close(got[rows], want, 1e-2, f"rows of group {e}")
         want = acc[e] + 2 * x[rows].astype(np.float64).T @ dy[rows].astype(np.float64)
         close(dacc.download(np.float32, (E, h, f))[e], want, 1e-4 * math.sqrt(2 * max(c, 1)), f"dW of group {e}")
+
+
+@pytest.mark.parametrize("rows,form", [(1472, ""), (1536, "s4")])
+def test_grouped_contraction_runs_in_the_form_that_was_priced(rows, form):
+    """At most one 64x64 tile per CU takes the tile's four-stage form from 25 K-steps on - by the
+    groups' rows (and one step more), not by k, which is unused - as the choice of the tile
+    assumes."""
+    E, h, f = 8, 256, 256
+    print(f"grouped contraction of {rows} rows", flush=True)
+    rng = np.random.default_rng(2)
+    per = (rows + 255) // 256 * 256
+    seg, cnt = np.arange(E + 1, dtype=np.int32) * per, np.full(E, rows, np.int32)
+    x, dy = np.zeros((E * per, h), np.float32), np.zeros((E * per, f), np.float32)
+    for e in range(E):
+        x[seg[e]:seg[e] + rows], dy[seg[e]:seg[e] + rows] = rnd(rng, rows, h), rnd(rng, rows, f, scale=0.3)
+    dx, ddy, b_seg, b_cnt = dev_bf16(x), dev_bf16(dy), rt.DeviceBuffer.from_numpy(seg), rt.DeviceBuffer.from_numpy(cnt)
+    dacc = rt.DeviceBuffer(4 * E * h * f)
+    dacc.zero()
+    with rt.probe("*") as p:
+        rt.gemm(dx.ptr, ddy.ptr, dacc.ptr, h, f, 0, h, f, f, 1, 1, rt.EPI_ACC_F32, stride_c=h * f, seg=b_seg.ptr,
+                n_seg=E, group_mode=2, group_rows=E * rows, seg_rows=b_cnt.ptr)
+        rt.sync()
+    got = dacc.download(np.float32, (E, h, f))
+    for e in range(E):
+        r = slice(seg[e], seg[e] + rows)
+        close(got[e], x[r].astype(np.float64).T @ dy[r], 1e-4 * math.sqrt(rows), f"gradient {e}")
+    assert list(p.classes) == [f"gemm_tn_accf32_64x64{form}k2"], p.classes
