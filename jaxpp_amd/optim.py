@@ -13,6 +13,7 @@ double and rounded once.
 """
 from __future__ import annotations
 
+import math
 from dataclasses import dataclass
 
 import numpy as np
@@ -38,18 +39,45 @@ def _offsets(leaves):
     return at, n
 
 
+def _upload_run(buf, n, at, *kinds):
+    """The kinds of leaves of a run (gradients, moments, ...; one list each) behind one another
+    into `buf`, a vector of `n` elements per kind: one packed copy, or of a run of one leaf straight
+    from the leaves' own memory.  A leaf's kinds are read as far as the first one reaches."""
+    if len(at) == 1:
+        for k, (a,) in enumerate(kinds):
+            buf.upload(a.reshape(-1)[:kinds[0][0].size], 4 * n * k)
+        return
+    host = np.empty(n * len(kinds), np.float32)
+    for k, leaves in enumerate(kinds):
+        for i, a in enumerate(leaves):
+            size = kinds[0][i].size
+            host[k * n + at[i]:k * n + at[i] + size] = a.reshape(-1)[:size]
+    buf.upload(host)
+
+
+def _download_run(buf, n, at, leaves, *kinds):
+    """The kinds `kinds` (adjacent ones) of `buf`'s vectors as arrays of the leaves' shapes, one
+    list per kind: views of one array, or of a run of one leaf arrays of their own."""
+    if len(at) == 1:
+        return [[buf.download(np.float32, leaves[0].shape, 4 * n * k)] for k in kinds]
+    out = buf.download(np.float32, (n * len(kinds),), 4 * n * kinds[0])
+    return [[out[n * k + i:n * k + i + a.size].reshape(a.shape) for i, a in zip(at, leaves)]
+            for k in range(len(kinds))]
+
+
 def _map_runs(f, *trees):
     """A tree like the first of what ``f`` returns per leaf.  ``f`` takes the leaves of a run
     (`runtime.copy_runs`), one list per tree, float32 and contiguous: leaf by leaf a step of four
     small layers was 250 uploads and 200 downloads, and those 20 of its 24 ms."""
     from jaxpp_amd import runtime as rt
     leaves = []
-    _zip_map(lambda *ls: leaves.append([np.ascontiguousarray(a, dtype=np.float32) for a in ls]), *trees)
+    _zip_map(lambda *ls: leaves.append(ls), *trees)
     out = []
-    for first, last in rt.copy_runs([ls[0].size for ls in leaves]):
-        for ls in leaves[first:last]:
+    for first, last in rt.copy_runs([math.prod(np.shape(ls[0])) for ls in leaves]):
+        run = [[np.ascontiguousarray(a, dtype=np.float32) for a in ls] for ls in leaves[first:last]]
+        for ls in run:
             assert all(a.size >= ls[0].size for a in ls), [a.shape for a in ls]
-        out += f(*([ls[k] for ls in leaves[first:last]] for k in range(len(trees))))
+        out += f(*([ls[k] for ls in run] for k in range(len(trees))))
     results = iter(out)
     return _zip_map(lambda *_: next(results), *trees)
 
@@ -76,22 +104,17 @@ class adam:
 
         def run(gs, ms, vs):
             """The leaves of a run as one vector: gradients, moments and updates of `n` elements
-            each behind one another on the device, one copy each way."""
+            each behind one another on the device.  The updates come back as memory of their own:
+            the moments outlive the step, they do not."""
             at, n = _offsets(gs)
-            host = np.empty(3 * n, np.float32)
-            for k, leaves in enumerate((gs, ms, vs)):
-                for i, a in enumerate(leaves):
-                    host[k * n + at[i]:k * n + at[i] + gs[i].size] = a.reshape(-1)[:gs[i].size]
             buf = rt.DeviceBuffer(16 * n)
-            buf.upload(host)
+            _upload_run(buf, n, at, gs, ms, vs)
             # weights that start at zero end as the update itself
             rt.check(rt.load().jpp_fill_u32(buf.ptr + 12 * n, 0, n, None))
             rt.adam_step(n, buf.ptr, buf.ptr + 4 * n, buf.ptr + 8 * n, step, master=buf.ptr + 12 * n,
                          lr=self.learning_rate, b1=self.b1, b2=self.b2, eps=self.eps)
             rt.sync()
-            out = buf.download(np.float32, (3 * n,), 4 * n)
-            part = lambda k, i: out[k * n + at[i]:k * n + at[i] + gs[i].size].reshape(gs[i].shape)
-            return [(part(2, i), part(0, i), part(1, i)) for i in range(len(gs))]
+            return list(zip(*_download_run(buf, n, at, gs, 3), *_download_run(buf, n, at, gs, 1, 2)))
 
         trio = _map_runs(run, grads, state["mu"], state["nu"])
         pick = lambda k: _zip_map(lambda g, t: t[k], grads, trio)
@@ -105,15 +128,10 @@ def apply_updates(params, updates):
 
     def run(ps, us):
         at, n = _offsets(ps)
-        host = np.empty(2 * n, np.float32)
-        for k, leaves in enumerate((ps, us)):
-            for i, a in enumerate(leaves):
-                host[k * n + at[i]:k * n + at[i] + ps[i].size] = a.reshape(-1)[:ps[i].size]
         buf = rt.DeviceBuffer(8 * n)
-        buf.upload(host)
+        _upload_run(buf, n, at, ps, us)
         rt.check(rt.load().jpp_grad_accum_f32(None, buf.ptr, buf.ptr + 4 * n, n, 1))
         rt.sync()
-        out = buf.download(np.float32, (n,))
-        return [out[at[i]:at[i] + p.size].reshape(p.shape) for i, p in enumerate(ps)]
+        return _download_run(buf, n, at, ps, 0)[0]
 
     return _map_runs(run, params, updates)

@@ -359,20 +359,23 @@ def download_ptr(ptr: int, dtype, shape) -> np.ndarray:
     return out
 
 
-# Elements of small tensors that travel as one copy.  A copy between pageable host memory and the
-# device costs 14 us and more whatever its size, and up to 115 us at 64 - 256 KB; one of 8 MB
-# moves at 16 - 35 GB/s.  Larger tensors gain nothing and would only be copied once more on the
-# host.
+# Elements of small tensors that travel as one copy, and of one that travels by itself.  A copy
+# between pageable host memory and the device costs 14 us and more whatever its size, and up to 115
+# us at 64 - 256 KB; one of 8 MB moves at 16 - 35 GB/s.  Larger tensors gain nothing and would only
+# be copied once more on the host (an optimizer step over 16 leaves of 1024 x 1024: in runs of two
+# 37.8 ms, by themselves 32.7; over 64 of 256 x 1024: in runs 39.5, by themselves 42.9).
 COPY_RUN = 1 << 21
+COPY_ALONE = 1 << 19
 
 
-def copy_runs(sizes, adjacent=None, limit: int = COPY_RUN) -> list:
+def copy_runs(sizes, adjacent=None) -> list:
     """Splits tensors of these sizes (elements), in order, into runs ``(first, last + 1)`` that
-    travel as one copy: at most `limit` elements together, a larger tensor by itself.
+    travel as one copy: at most `COPY_RUN` elements together, one of `COPY_ALONE` by itself.
     ``adjacent(i)`` says whether tensor i follows tensor i - 1 without a break (None: always)."""
     runs, first, total = [], 0, 0
     for i, n in enumerate(sizes):
-        if i > first and (total + n > limit or not (adjacent is None or adjacent(i))):
+        if i > first and (total + n > COPY_RUN or max(n, sizes[i - 1]) >= COPY_ALONE or
+                          not (adjacent is None or adjacent(i))):
             runs.append((first, i))
             first, total = i, 0
         total += n

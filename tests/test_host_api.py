@@ -318,3 +318,16 @@ def test_schedule_task_fusion_switch(monkeypatch):
     monkeypatch.setenv("JAXPP_DISABLE_SCHEDULE_TASK_FUSION", "maybe")
     with pytest.raises(ValueError, match="Unsupported value JAXPP_DISABLE_SCHEDULE_TASK_FUSION=maybe"):
         make_rank_plan(sched, n, 0)
+
+
+def test_copy_runs_split_tensors_in_order():
+    """Every tensor in one run, in order; at most COPY_RUN elements together, tensors of COPY_ALONE
+    and more alone, no run across a break in memory."""
+    from jaxpp_amd import runtime as rt
+    A, R = rt.COPY_ALONE, rt.COPY_RUN
+    assert rt.copy_runs([]) == []
+    assert rt.copy_runs([10] * 5) == [(0, 5)]
+    assert rt.copy_runs([A, 1, 2, A, A, 3]) == [(0, 1), (1, 3), (3, 4), (4, 5), (5, 6)]
+    assert rt.copy_runs([A - 1] * 9) == [(0, 4), (4, 8), (8, 9)]
+    assert rt.copy_runs([5, R + 1, 5]) == [(0, 1), (1, 2), (2, 3)]
+    assert rt.copy_runs([1, 1, 1, 1], lambda i: i != 2) == [(0, 2), (2, 4)]
