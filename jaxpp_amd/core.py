@@ -365,6 +365,11 @@ def _stage_lifetimes(rows: list, num_stages: int) -> tuple:
     return peak, split
 
 
+# Device memory in which the predictions that a loop returns may wait for its end; where they
+# would take more, each is fetched behind its forward task.
+HELD_PREDICTIONS = 1 << 28
+
+
 def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
     from jaxpp_amd import runtime as rt
     fn = _active_function
@@ -464,8 +469,11 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
     loss_dev = rt.DeviceBuffer(4 * n)
     partial = rt.DeviceBuffer(4 * rt.NORM_PARTIALS)
     want_pred = any(isinstance(v, tracing.Traced) and v.shape != () for v in tracing.tree_leaves(outputs))
-    # (fetched behind the loop: a copy after each forward task would drain the queue)
-    preds_dev = in_runs(lambda first, last: rt.DeviceBuffer((last - first) * act_bytes)) if want_pred else []
+    preds = {}
+    # (fetched behind the loop: a copy after each forward task drains the queue)
+    preds_dev = []
+    if want_pred and n * act_bytes <= HELD_PREDICTIONS:
+        preds_dev = in_runs(lambda first, last: rt.DeviceBuffer((last - first) * act_bytes))
     # the scale of the value that is differentiated sets the cotangent; loss values returned
     # with another scale are rescaled from it
     diff = tr.differentiated
@@ -506,6 +514,8 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
                                                   partial.ptr))
                     cot[s, m] = d
                     if not preds_dev:
+                        if want_pred:
+                            preds[m] = any_ex.download_activation(dst, (tokens, hidden))
                         free.append(dst)
             elif kind is TaskType.BWD_W:
                 for sg in reversed(stage_segs[s]):
@@ -524,8 +534,10 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
                 _statistics[mk_task_name(s, t.fwd_or_bwd)].append((time.perf_counter() - t0) * 1e3)
     rt.sync()
     losses = loss_dev.download(np.float32, (n,))
-    preds = [p for (first, last), buf in zip(mb_runs, preds_dev and [preds_dev[a].owner for a, _ in mb_runs])
-             for p in any_ex.download_activation(buf, (last - first, tokens, hidden))]
+    if preds_dev:
+        for first, last in mb_runs:
+            run = any_ex.download_activation(preds_dev[first].owner, (last - first, tokens, hidden))
+            preds.update(zip(range(first, last), run))
     grads = {}
     for s_, segs in enumerate(stage_segs):
         grads[s_] = []

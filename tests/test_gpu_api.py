@@ -299,3 +299,55 @@ def test_the_example_script_runs_and_learns():
     for argv in (["--steps", "4"], ["--steps", "3", "--dtype", "f32", "--pp", "3", "--num-ubatches", "6"]):
         history = mod.main(argv)
         assert all(np.isfinite(history)) and history[-1] < history[0], history
+
+
+def test_predictions_wait_on_the_device_within_a_bound(monkeypatch):
+    """Predictions are fetched behind the loop while they fit in a bound; beyond it each is fetched
+    behind its forward task and its buffer used again.  The same numbers either way, and n - 1
+    activations less at the peak."""
+    rt.require_gpu()
+    from jaxpp_amd import core
+    spec, n_mb, pp = LayerSpec("bert", 256, 4, 512, 128, 1, eps=1e-12), 8, 2
+    model = jaxpp.nn.TransformerStack(spec, n_layers=pp, layers_per_stage=1)
+    params = model.init(seed=0, perturb=True)
+    batch = np.random.default_rng(3).standard_normal((n_mb, spec.tokens, spec.hidden), dtype=np.float32)
+    mesh = jaxpp.MpmdMesh(jaxpp.DeviceMesh(np.arange(pp).reshape(pp, 1), ("mpmd", "data")), "mpmd")
+
+    def loss_fn(pars, mb):
+        res = model.apply(pars, mb)
+        return jaxpp.nn.mse_loss(res, mb) / n_mb, res
+
+    @partial(jaxpp.mpmd_jit_with_loop, mpmd_mesh=mesh)
+    def train_step(pars, batch):
+        return jaxpp.treduce(partial(jaxpp.value_and_grad(loss_fn, has_aux=True), pars), batch,
+                             schedule=jaxpp.Std1F1B(pp))
+
+    live, peak = [0], [0]
+
+    class Counted(rt.DeviceBuffer):
+        def __init__(self, nbytes):
+            super().__init__(nbytes)
+            live[0] += self.nbytes
+            peak[0] = max(peak[0], live[0])
+
+        def free(self):
+            if self.ptr:
+                live[0] -= self.nbytes
+            super().free()
+
+    train_step(params, batch)               # (the executors and their memory)
+    monkeypatch.setattr(rt, "DeviceBuffer", Counted)
+    res, peaks = [], []
+    act = spec.tokens * spec.hidden * 2
+    for bound in (n_mb * act, n_mb * act - 1):
+        monkeypatch.setattr(core, "HELD_PREDICTIONS", bound)
+        live[0] = peak[0] = 0
+        res.append(train_step(params, batch))
+        peaks.append(peak[0])
+    assert peaks[0] - peaks[1] >= (n_mb - 1) * act, peaks
+    (losses, preds), grads = res[0]
+    (losses1, preds1), grads1 = res[1]
+    np.testing.assert_array_equal(losses, losses1)
+    np.testing.assert_array_equal(preds, preds1)
+    np.testing.assert_array_equal(grads["layers"][0]["W1"], grads1["layers"][0]["W1"])
+    train_step.close()
