@@ -105,6 +105,30 @@ def test_small_weight_gradients_in_one_launch(parts, k, shapes):
         close(dc.download(np.float32, shape), want, 1e-4 * math.sqrt(k * parts), f"multi {shape}")
 
 
+@pytest.mark.parametrize("rows,cols", [(1, c) for c in range(1, 18)] + [(9, 5), (10, 5), (17, 3), (3, 19)])
+def test_every_tile_of_a_grid_is_computed_once(rows, cols):
+    """Grids of every remainder by the 8 XCDs, fewer tiles than XCDs and groups of tile rows that do
+    not come out even, plain and as the second problem of a launch: C += A B with 0/1 operands is
+    exact, and a tile left out or taken twice shows."""
+    m, n, k = 128 * rows, 128 * cols, 64
+    print(f"{rows} x {cols} tiles", flush=True)
+    rng = np.random.default_rng(rows + cols)
+    a, b = (rng.integers(0, 2, s).astype(np.float32) for s in ((k, m), (k, n)))
+    c0 = rng.integers(0, 9, (m, n)).astype(np.float32)
+    da, db, want = dev_bf16(a), dev_bf16(b), c0 + a.T @ b
+    for tile in (1, 5):
+        dc = rt.DeviceBuffer.from_numpy(c0)
+        rt.gemm(da.ptr, db.ptr, dc.ptr, m, n, k, m, n, n, 1, 1, rt.EPI_ACC_F32, tile=tile)
+        rt.sync()
+        np.testing.assert_array_equal(dc.download(np.float32, (m, n)), want)
+    first, dc = rt.DeviceBuffer.from_numpy(c0[:128, :128]), rt.DeviceBuffer.from_numpy(c0)
+    rt.gemm_multi([dict(a=da.ptr, b=db.ptr, c=first.ptr, m=128, n=128, k=k, lda=m, ldb=n, ldc=128),
+                   dict(a=da.ptr, b=db.ptr, c=dc.ptr, m=m, n=n, k=k, lda=m, ldb=n, ldc=n)])
+    rt.sync()
+    np.testing.assert_array_equal(dc.download(np.float32, (m, n)), want)
+    np.testing.assert_array_equal(first.download(np.float32, (128, 128)), want[:128, :128])
+
+
 @pytest.mark.parametrize("m,n", [(128, 128), (128, 256), (256, 128), (768, 384), (384, 768), (256, 512)])
 def test_operand_pairs_of_every_extent(m, n):
     """A weight gradient over three operand pairs, tile left to the library, whichever of M and N
