@@ -112,13 +112,14 @@ __device__ __forceinline__ void swiglu_grad_f(float g, float u, float d, float& 
 // XCDs (8 of them, each with its own L2); give every XCD a contiguous range of
 // tiles, and inside a range walk GROUP tile-rows at a time so the B panels in
 // flight stay L2 resident.
-constexpr int kColumnSplitRows = 64;  // tile rows from which XCDs split by columns
+constexpr int kColumnSplitRows = 16384;  // rows from which XCDs split by columns
 
-template <bool WGRAD = false>
+template <bool WGRAD, int BM>
 __device__ __forceinline__ void tile_of_block(int pid, int tiles_m, int tiles_n, bool front_only, int& tm, int& tn) {
   const int nwg = tiles_m * tiles_n;
-  if ((tiles_n & 7) == 0 && tiles_m >= kColumnSplitRows) {
-    // Very tall outputs (the experts' row-grouped products: 16 384 token copies and more):
+  if ((tiles_n & 7) == 0 && tiles_m * BM >= kColumnSplitRows) {
+    // Very tall outputs (the experts' row-grouped products: 16 384 token copies and more; not
+    // by tile rows: 4096 rows of 64x64 tiles, N = 512, K = 7168 took 71 us this way, 43 the other):
     // every XCD owns an eighth of the tile columns and walks them 8 tile-rows at a time, so a
     // B panel - which changes from expert to expert - is fetched by one XCD only.  The split
     // below would hand whole row groups to single XCDs and have each of them stream every
@@ -251,7 +252,7 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
   const int wm = wave / WN, wn = wave % WN;
   int tm, tn;
   const int tiles = p.tiles_m * p.tiles_n;
-  tile_of_block<TA && TB>(p.group_mode == JPP_GROUP_K ? bid % tiles : bid, p.tiles_m, p.tiles_n,
+  tile_of_block<TA && TB, BM>(p.group_mode == JPP_GROUP_K ? bid % tiles : bid, p.tiles_m, p.tiles_n,
                           p.group_mode == JPP_GROUP_M, tm, tn);
   long m0 = (long)tm * BM;
   const long n0 = (long)tn * BN;

@@ -105,11 +105,12 @@ def test_small_weight_gradients_in_one_launch(parts, k, shapes):
         close(dc.download(np.float32, shape), want, 1e-4 * math.sqrt(k * parts), f"multi {shape}")
 
 
-@pytest.mark.parametrize("rows,cols", [(1, c) for c in range(1, 18)] + [(9, 5), (10, 5), (17, 3), (3, 19)])
+@pytest.mark.parametrize("rows,cols", [(1, c) for c in range(1, 18)] + [(9, 5), (10, 5), (17, 3), (3, 19),
+                                                                                 (32, 4), (128, 8)])
 def test_every_tile_of_a_grid_is_computed_once(rows, cols):
-    """Grids of every remainder by the 8 XCDs, fewer tiles than XCDs and groups of tile rows that do
-    not come out even, plain and as the second problem of a launch: C += A B with 0/1 operands is
-    exact, and a tile left out or taken twice shows."""
+    """Grids of every remainder by the 8 XCDs, fewer tiles than XCDs, groups of tile rows that do
+    not come out even, tall ones (columns split over the XCDs), plain and as the second problem
+    of a launch: C += A B with 0/1 operands is exact, and a tile left out or taken twice shows."""
     m, n, k = 128 * rows, 128 * cols, 64
     print(f"{rows} x {cols} tiles", flush=True)
     rng = np.random.default_rng(rows + cols)
