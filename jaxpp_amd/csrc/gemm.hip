@@ -880,11 +880,12 @@ int launch_multi(hipStream_t stream, GemmParams* ps, int n) {
 
 // The 128x128 tile runs with five LDS stages (one workgroup per CU) when every CU has at most
 // one tile, else with two (two workgroups per CU); the 64x64 tile, whose two wave groups share
-// it, with four or two by the same rule if the contraction is long enough for the longer prologue:
-// more than 8 K-steps, of a grouped contraction (8 experts of 256 x 256, four / two stages:
-// 600 rows each 6.7 / 6.2 us, 1024 7.9 / 7.3, 2048 12.1 / 15.2) 24.
-bool deep_stages(long tiles, long ksteps, int tile, bool group_k = false) {
-  return tiles <= kCus && (tile == kTile128 || ksteps > (group_k ? 24 : 8));
+// it, with four or two by the same rule - and if the contraction is long enough for the longer
+// prologue.  Time of the deep form over that of two stages, 96 to 256 tiles, operands out of L2 as
+// a layer finds them: 128x128 1.03 - 1.11 at 1 - 3 K-steps, 1.03 at 4, 0.96 at 6, 0.8 at 16;
+// 64x64 1.05 at 1 - 4, 1.02 at 6, 0.99 at 8, 0.91 at 12, 0.84 at 20.
+bool deep_stages(long tiles, long ksteps, int tile) {
+  return tiles <= kCus && ksteps > (tile == kTile128 ? 4 : 8);
 }
 
 struct Extent { long m, n; };
@@ -921,7 +922,7 @@ long count_tiles(const Extent* e, int n, int bm, int bn) {
 bool deep_form(const jpp_gemm_args* a, int tile) {
   const Extent e = grid_extent(a);
   const int b = tile == kTile64 ? 64 : 128;
-  return deep_stages(count_tiles(&e, 1, b, b), work_ksteps(a), tile, a->group_mode == JPP_GROUP_K);
+  return deep_stages(count_tiles(&e, 1, b, b), work_ksteps(a), tile);
 }
 
 // `deep`: which form of the 64x64 and 128x128 tiles
@@ -974,8 +975,7 @@ constexpr TileForm kWeightGrad[] = {
 
 // tile with the smallest estimate for products of these extents in one grid (`grid`: the extents
 // that its form goes by)
-int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool wgrad, bool group_k,
-                  bool may_128x256) {
+int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool wgrad, bool may_128x256) {
   int best = kTile128;
   float best_us = 0.f;
   for (const TileForm& f : wgrad ? kWeightGrad : kForward) {
@@ -983,7 +983,7 @@ int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool 
     const long tiles = count_tiles(e, n, f.bm, f.bn);
     if (tiles < 0) continue;
     if ((f.tile == kTile64 || f.tile == kTile128) &&
-        f.deep != deep_stages(count_tiles(grid, n, f.bm, f.bn), ksteps, f.tile, group_k)) continue;
+        f.deep != deep_stages(count_tiles(grid, n, f.bm, f.bn), ksteps, f.tile)) continue;
     const long w = (tiles + kCus - 1) / kCus;
     const float t = f.start + w * (f.tile_cost + ksteps * (w == 1 ? f.lone_step : f.step));
     if (best_us == 0.f || t < best_us) { best_us = t; best = f.tile; }
@@ -999,8 +999,7 @@ int choose_tile(const jpp_gemm_args* a) {
   const long t256 = e.m % 256 == 0 && e.n % 256 == 0 ? (e.m / 256) * (e.n / 256) : 0;
   if (t256 >= kMostCus) return kTile256;
   const Extent grid = grid_extent(a);
-  const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), a->trans_a && a->trans_b,
-                                 a->group_mode == JPP_GROUP_K, true);
+  const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), a->trans_a && a->trans_b, true);
   // (a rotated head lies inside one tile)
   return tile == kTile64 && a->rope_cos && a->rope_head_dim > 64 ? (int)kTile64x128 : tile;
 }
@@ -1256,7 +1255,7 @@ extern "C" int jpp_gemm_bf16_multi(void* stream_, const jpp_gemm_args* problems,
   JPP_REQUIRE(tiles < (1L << 30), "gemm_multi: too many tiles");
   const long ksteps = (long)ps[0].k / 64 * ps[0].k_parts;
   const int tile = whole && t256 >= kMostCus ? (int)kTile256
-                   : cheapest_tile(e, e, n_problems, ksteps, true, false, false);
+                   : cheapest_tile(e, e, n_problems, ksteps, true, false);
   const bool deep = deep_stages(tile == kTile64 ? tiles : tiles / 4, ksteps, tile);
   if (tile == kTile256) return launch_multi<256, 256, 8, 2>(stream, ps, n_problems);
   if (tile == kTile64)
