@@ -951,31 +951,35 @@ int launch_tiled(hipStream_t stream, GemmParams& p, int tile, bool deep) {
 }
 
 // Expected time of a product of `tiles` tiles, `ksteps` K-steps of 64 each, in us:
-//   start + w * (tile_cost + ksteps * step),   w = tiles of the busiest of the 256 CUs
+//   start + w * (tile_cost [+ gelu] + ksteps * step),   w = tiles of the busiest of the 256 CUs
 // (two workgroups fit on a CU in the two-stage forms: their steps overlap, so a CU's lone
-// workgroup takes a step cost of its own).  The constants are least-squares fits to 208 random
-// shapes (M, N 128 .. 8192, K 128 .. 8192) timed alone, 7 tile forms each, mean error 4 - 10 %;
-// choosing the smallest estimate costs 1.8 % against always choosing the measured best, where
-// the rule before (256x256 from 192 tiles on, else 128x128) cost 37 %: a 512 x 1024 x 4096
-// input gradient has 32 tiles of 128x128 for 256 CUs and took 28 us, 15 us as 128 tiles of
-// 64x64 with two wave groups each.
+// workgroup takes a step cost of its own; `gelu`: the arithmetic of a GELU epilogue).  The
+// constants are least-squares fits to 1300 random products (M, N 128 .. 16384, K 128 .. 16384, every
+// orientation and epilogue) timed in every form with the operands out of L2, as a layer finds
+// them, and accumulators out of every cache: mean error 4 - 10 %.  The two wide forward forms
+// stand 10 % above their fit: 128x128 is otherwise passed over where they are close.  Taking
+// the smallest estimate costs 0.3 % against always taking the measured best.  Against the rule
+// before (256x256 from 192 tiles on, else 128x128: 36 % on average) it is slower by more than 2 %
+// for 9 of the 1300, by 6 % at most: a 512 x 1024 x 4096 input gradient has 32 tiles of 128x128
+// for 256 CUs and took 28 us, 15 us as 128 tiles of 64x64 with two wave groups each.
 struct TileForm {
   int tile, bm, bn;
   bool deep;              // which of the tile's two forms (kTile128, kTile64)
-  float start, tile_cost, lone_step, step;
+  float start, tile_cost, gelu, lone_step, step;
 };
 constexpr TileForm kForward[] = {
-    {kTile64, 64, 64, true, 1.5f, 2.8f, 0.19f, 0.19f},    {kTile64, 64, 64, false, 2.1f, 1.4f, 0.285f, 0.19f},
-    {kTile128, 128, 128, true, 0.f, 5.2f, 0.41f, 0.41f},  {kTile128, 128, 128, false, 1.2f, 2.6f, 0.60f, 0.45f},
-    {kTile128x256, 128, 256, true, 0.f, 6.1f, 0.65f, 0.65f}, {kTile256, 256, 256, true, 0.f, 7.9f, 1.07f, 1.07f}};
+    {kTile64, 64, 64, true, 0.f, 4.8f, 0.5f, 0.18f, 0.18f},     {kTile64, 64, 64, false, 2.7f, 1.5f, 0.3f, 0.26f, 0.17f},
+    {kTile128, 128, 128, true, 0.f, 6.3f, 2.1f, 0.39f, 0.39f},  {kTile128, 128, 128, false, 3.4f, 2.3f, 1.7f, 0.49f, 0.365f},
+    {kTile128x256, 128, 256, true, 1.1f, 7.4f, 5.2f, 0.705f, 0.715f},
+    {kTile256, 256, 256, true, 0.2f, 11.2f, 11.f, 1.155f, 1.19f}};
 constexpr TileForm kWeightGrad[] = {
-    {kTile64, 64, 64, true, 1.0f, 3.2f, 0.23f, 0.23f},    {kTile64, 64, 64, false, 1.7f, 1.8f, 0.31f, 0.21f},
-    {kTile128, 128, 128, true, 0.f, 6.0f, 0.46f, 0.46f},  {kTile128, 128, 128, false, 0.f, 4.5f, 0.75f, 0.81f},
-    {kTile128x256, 128, 256, true, 0.f, 6.6f, 0.95f, 0.95f}, {kTile256, 256, 256, true, 0.f, 10.f, 1.28f, 1.28f}};
+    {kTile64, 64, 64, true, 0.f, 5.2f, 0.f, 0.28f, 0.28f},      {kTile64, 64, 64, false, 3.7f, 2.0f, 0.f, 0.19f, 0.22f},
+    {kTile128, 128, 128, true, 0.f, 8.6f, 0.f, 0.515f, 0.515f}, {kTile128, 128, 128, false, 2.2f, 6.8f, 0.f, 0.32f, 0.77f},
+    {kTile128x256, 128, 256, true, 0.f, 11.2f, 0.f, 1.13f, 1.02f}, {kTile256, 256, 256, true, 0.f, 15.5f, 0.f, 1.43f, 1.43f}};
 
 // tile with the smallest estimate for products of these extents in one grid (`grid`: the extents
 // that its form goes by)
-int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool wgrad, bool may_128x256) {
+int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool wgrad, bool gelu, bool may_128x256) {
   int best = kTile128;
   float best_us = 0.f;
   for (const TileForm& f : wgrad ? kWeightGrad : kForward) {
@@ -985,7 +989,7 @@ int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool 
     if ((f.tile == kTile64 || f.tile == kTile128) &&
         f.deep != deep_stages(count_tiles(grid, n, f.bm, f.bn), ksteps, f.tile)) continue;
     const long w = (tiles + kCus - 1) / kCus;
-    const float t = f.start + w * (f.tile_cost + ksteps * (w == 1 ? f.lone_step : f.step));
+    const float t = f.start + w * (f.tile_cost + (gelu ? f.gelu : 0.f) + ksteps * (w == 1 ? f.lone_step : f.step));
     if (best_us == 0.f || t < best_us) { best_us = t; best = f.tile; }
   }
   return best;
@@ -999,7 +1003,8 @@ int choose_tile(const jpp_gemm_args* a) {
   const long t256 = e.m % 256 == 0 && e.n % 256 == 0 ? (e.m / 256) * (e.n / 256) : 0;
   if (t256 >= kMostCus) return kTile256;
   const Extent grid = grid_extent(a);
-  const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), a->trans_a && a->trans_b, true);
+  const bool gelu = a->epilogue == JPP_EPI_GELU || a->epilogue == JPP_EPI_DGELU;
+  const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), a->trans_a && a->trans_b, gelu, true);
   // (a rotated head lies inside one tile)
   return tile == kTile64 && a->rope_cos && a->rope_head_dim > 64 ? (int)kTile64x128 : tile;
 }
@@ -1255,7 +1260,7 @@ extern "C" int jpp_gemm_bf16_multi(void* stream_, const jpp_gemm_args* problems,
   JPP_REQUIRE(tiles < (1L << 30), "gemm_multi: too many tiles");
   const long ksteps = (long)ps[0].k / 64 * ps[0].k_parts;
   const int tile = whole && t256 >= kMostCus ? (int)kTile256
-                   : cheapest_tile(e, e, n_problems, ksteps, true, false);
+                   : cheapest_tile(e, e, n_problems, ksteps, true, false, false);
   const bool deep = deep_stages(tile == kTile64 ? tiles : tiles / 4, ksteps, tile);
   if (tile == kTile256) return launch_multi<256, 256, 8, 2>(stream, ps, n_problems);
   if (tile == kTile64)
