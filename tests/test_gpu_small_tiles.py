@@ -11,6 +11,8 @@ import numpy as np
 import pytest
 
 from jaxpp_amd import runtime as rt
+import test_gpu_kernels as K
+import test_gpu_random_kernels as R
 from test_gpu_kernels import close, dev_bf16, rnd
 from oracle import layers as L
 
@@ -45,6 +47,27 @@ def test_small_tiles(lay, m, n, k, tile):
     rt.gemm(*args, dc.ptr, *dims, rt.EPI_BF16, tile=tile)
     rt.sync()
     close(dc.download_bf16((m, n)), want, 1e-2, "bf16")
+
+
+# (few tiles with two and with four stages; one K-step; more tiles than CUs)
+@pytest.mark.parametrize("m,n,k", [(128, 128, 64), (256, 384, 320), (384, 512, 704), (1152, 1280, 448)])
+@pytest.mark.parametrize("ta,tb,epi", K.GEMM_CASES)
+def test_every_epilogue_on_64x64_tiles(ta, tb, epi, m, n, k):
+    K.test_gemm(ta, tb, epi, 5, m, n, k)
+
+
+@pytest.mark.parametrize("m,f,k", [(128, 128, 64), (256, 640, 640), (1152, 640, 128)])
+def test_swiglu_epilogues_on_64x64_tiles(m, f, k):
+    K.test_gemm_swiglu_epilogues(5, m, f, k)
+
+
+@pytest.mark.parametrize("seed", range(24))
+def test_random_products_on_64x64_tiles(seed, monkeypatch):
+    """The random products (padded leading dimensions, bias and residual or not, operand pairs) with
+    tile 5 in the place of the tile drawn."""
+    gemm = rt.gemm
+    monkeypatch.setattr(rt, "gemm", lambda *a, **kw: gemm(*a, **{**kw, "tile": 5}))
+    R.test_random_gemm(100 + seed)
 
 
 @pytest.mark.parametrize("k", [64, 448])
