@@ -187,6 +187,9 @@ __device__ __forceinline__ int group_steps(const int* seg, const int* seg_rows, 
   return (rows + 63) / 64;
 }
 
+// Whether a form has room for the accumulator's rows beside its operand stages (C += A B).
+constexpr bool streams_accumulator(int stages, int wave_groups) { return wave_groups == 1 && stages <= 4; }
+
 template <int BM, int BN, bool TA, bool TB, int EPI, int NW, int NS, bool KP = false, bool MP = false,
           int KG = 1>
 __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
@@ -340,7 +343,8 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
   // loops too short for that add the old values in the epilogue, where rows are whole too.
   static_assert(BN * 4 <= 1024, "a row of the fp32 tile is one 64-lane copy");
   constexpr int NBT = BM / NW, C_LDS = NS * (BM + BN) * 128, C_PITCH = 1024 + 16;  // a copy is 1 KB
-  const bool stream_c = KG == 1 && NS <= 4 && EPI == JPP_EPI_ACC_F32 && kt_n >= NBT + NS;
+  constexpr bool STREAM_C = EPI == JPP_EPI_ACC_F32 && streams_accumulator(NS, KG);
+  const bool stream_c = STREAM_C && kt_n >= NBT + NS;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -441,7 +445,7 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
           else if (cin == 1) dma_wait<(NS - 2) * OPB + 1>();
           else if (cin == 2) dma_wait<(NS - 2) * OPB + 2>();
           else dma_wait<(NS - 2) * OPB + 3>();
-          
+          static_assert(!STREAM_C || NS <= 4, "the wait above distinguishes up to three rows in flight");
         }
         lds_wait_all();
         __syncthreads();
@@ -781,7 +785,7 @@ int launch(hipStream_t stream, GemmParams& p) {
   constexpr int SMEM_LOOP = KG * NS * (BM + BN) * 128,
                 SMEM_EPI = (KG > 1 ? BM : BM / 2) * (BN * 4 + 16);
   // + NS+1 buffers of NW rows of the fp32 tile (padded) for C += A B
-  constexpr int SMEM = EPI == JPP_EPI_ACC_F32 && KG == 1 && NS <= 4 ? SMEM_LOOP + (NS + 1) * NW * (1024 + 16)
+  constexpr int SMEM = EPI == JPP_EPI_ACC_F32 && streams_accumulator(NS, KG) ? SMEM_LOOP + (NS + 1) * NW * (1024 + 16)
                        : (EPI == JPP_EPI_F32 || SMEM_LOOP > SMEM_EPI) ? SMEM_LOOP : SMEM_EPI;
   if constexpr (!KP) {
     // several operand pairs: only the accumulating weight-gradient kernels are built for that
@@ -833,8 +837,7 @@ int launch(hipStream_t stream, GemmParams& p) {
 // Llama-3-8B-shaped layer are 13 full rounds together - and small ones share the device.
 template <int BM, int BN, int NW, int NS, int KG = 1>
 int launch_multi(hipStream_t stream, GemmParams* ps, int n) {
-  constexpr bool STREAM_C = KG == 1 && NS <= 4;
-  constexpr int SMEM = KG * NS * (BM + BN) * 128 + (STREAM_C ? (NS + 1) * NW * (1024 + 16) : 0);
+  constexpr int SMEM = KG * NS * (BM + BN) * 128 + (streams_accumulator(NS, KG) ? (NS + 1) * NW * (1024 + 16) : 0);
   static_assert(SMEM <= 160 * 1024, "LDS of one CU");
   GemmArgs<true> args;
   args.p = ps[0];
