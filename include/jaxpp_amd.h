@@ -211,7 +211,7 @@ int jpp_gemm_bf16(void* stream, const jpp_gemm_args* args);
  * into BWD_W): launched one by one, each leaves its last round of tiles partly empty (a 6144 x
  * 4096 gradient is 384 tiles on 256 CUs), small ones most of the device; together they close up.
  * Tiles are 256x256 when M and N are multiples of 256 and the problems are most of a round of
- * them, else 128x128 or 64x64.  Every output element is computed by one workgroup in a fixed
+ * them, else 256x256, 128x128 or 64x64 by an estimate of their time.  Every output element is computed by one workgroup in a fixed
  * order (deterministic), the same order as in a single launch on the same tile; a single launch
  * that runs its last round on 128x256 tiles adds the old accumulator value at another point of
  * the sum there, so the two agree to fp32 rounding.  n_problems = 1 is jpp_gemm_bf16. */
@@ -309,8 +309,8 @@ int jpp_sum_accum_f32(void* stream, float* acc, const float* parts, int n_parts,
 /* acc[j] += sum_t x[t,j] (bias gradients); partial: f32 [JPP_NORM_PARTIALS*cols]. */
 int jpp_colsum_accum(void* stream, const void* x, int64_t ld, int64_t rows, int64_t cols,
                      float* acc, float* partial);
-/* The same for up to 4 tensors of `rows` rows in one pair of launches (the bias gradients of
- * a layer); partial: f32 [JPP_NORM_PARTIALS * sum of cols]. */
+/* The same for up to 4 tensors of `rows` rows (the bias gradients of a layer), in one launch up to
+ * 4096 rows and a pair beyond; partial: f32 [JPP_NORM_PARTIALS * sum of cols]. */
 typedef struct {
   const void* x;     /* bf16 [rows, cols], leading dimension ld */
   int64_t ld, cols;  /* multiples of 8 */
