@@ -959,12 +959,13 @@ int launch_tiled(hipStream_t stream, GemmParams& p, int tile, bool deep) {
 // workgroup takes a step cost of its own; `gelu`: the arithmetic of a GELU epilogue).  The
 // constants are least-squares fits to 1300 random products (M, N 128 .. 16384, K 128 .. 16384, every
 // orientation and epilogue) timed in every form with the operands out of L2, as a layer finds
-// them, and accumulators out of every cache: mean error 4 - 10 %.  The two wide forward forms
-// stand 10 % above their fit: 128x128 is otherwise passed over where they are close.  Taking
-// the smallest estimate costs 0.3 % against always taking the measured best.  Against the rule
-// before (256x256 from 192 tiles on, else 128x128: 36 % on average) it is slower by more than 2 %
-// for 9 of the 1300, by 6 % at most: a 512 x 1024 x 4096 input gradient has 32 tiles of 128x128
-// for 256 CUs and took 28 us, 15 us as 128 tiles of 64x64 with two wave groups each.
+// them, and accumulators out of every cache: mean error 4 - 10 %.  The forward 128x256 stands 10 %
+// above its fit: 128x128 is otherwise passed over where they are close.  Taking the smallest
+// estimate costs 0.1 % against always taking the measured best.  Against the rule before (256x256
+// from 192 tiles on, else 128x128: 36 % on average) it is slower by more than 2 % for 12 of the
+// 1300, all but one by 6 % at most (180 tiles of 256x256, 3 K-steps: 14 %): a 512 x 1024 x 4096 input
+// gradient has 32 tiles of 128x128 for 256 CUs and took 28 us, 15 us as 128 tiles of 64x64 with two
+// wave groups each.
 struct TileForm {
   int tile, bm, bn;
   bool deep;              // which of the tile's two forms (kTile128, kTile64)
@@ -974,7 +975,7 @@ constexpr TileForm kForward[] = {
     {kTile64, 64, 64, true, 0.f, 4.8f, 0.5f, 0.18f, 0.18f},     {kTile64, 64, 64, false, 2.7f, 1.5f, 0.3f, 0.26f, 0.17f},
     {kTile128, 128, 128, true, 0.f, 6.3f, 2.1f, 0.39f, 0.39f},  {kTile128, 128, 128, false, 3.4f, 2.3f, 1.7f, 0.49f, 0.365f},
     {kTile128x256, 128, 256, true, 1.1f, 7.4f, 5.2f, 0.705f, 0.715f},
-    {kTile256, 256, 256, true, 0.2f, 11.2f, 11.f, 1.155f, 1.19f}};
+    {kTile256, 256, 256, true, 0.2f, 10.2f, 10.f, 1.05f, 1.08f}};
 constexpr TileForm kWeightGrad[] = {
     {kTile64, 64, 64, true, 0.f, 5.2f, 0.f, 0.28f, 0.28f},      {kTile64, 64, 64, false, 3.7f, 2.0f, 0.f, 0.19f, 0.22f},
     {kTile128, 128, 128, true, 0.f, 8.6f, 0.f, 0.515f, 0.515f}, {kTile128, 128, 128, false, 2.2f, 6.8f, 0.f, 0.32f, 0.77f},
