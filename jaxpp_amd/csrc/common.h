@@ -174,6 +174,14 @@ __device__ __forceinline__ void dma_wait() {
   static_assert(PENDING >= 0 && PENDING < 64, "vmcnt is a 6-bit counter");
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PENDING) : "memory");
 }
+// waits until at most `groups` (wave-uniform, at most MAX) groups of PER loads each are outstanding
+template <int PER, int MAX>
+__device__ __forceinline__ void dma_wait_groups(int groups) {
+  if constexpr (MAX > 0) {
+    if (groups < MAX) return dma_wait_groups<PER, MAX - 1>(groups);
+  }
+  dma_wait<PER * MAX>();
+}
 // waits for this wave's LDS reads, so that what they read may be overwritten
 __device__ __forceinline__ void lds_wait_all() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 

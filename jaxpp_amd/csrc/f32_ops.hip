@@ -192,7 +192,8 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
       const uint8_t* const stages = smem + wave * (NS * STAGE);
       const uint32_t lds0 = lds_address(stages);
       auto copy = [&](int stage, int t) {
-        const long at = min(t, steps - 1) * 256L;  // (past the end the last step again, unused)
+        if (t >= steps) return;
+        const long at = t * 256L;
         TileA::template issue<0, TileA::INSTS>(uniform_ptr(pa + at), offa, lds0 + stage * STAGE, 0);
         TileB::template issue<0, TileB::INSTS>(uniform_ptr(pb + at), offb, lds0 + stage * STAGE + BM * 128, 0);
       };
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
       for (int q = 0; q < NS; ++q) copy(q, q);
       int st = 0;
       for (int t = 0; t < steps; ++t) {
-        dma_wait<(NS - 1) * (TileA::INSTS + TileB::INSTS)>();
+        dma_wait_groups<TileA::INSTS + TileB::INSTS, NS - 1>(steps - 1 - t);
         const uint8_t* const sa = stages + st * STAGE;
         f32x4 fa[2][TM], fb[2][TN];
 #pragma unroll

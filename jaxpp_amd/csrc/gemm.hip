@@ -379,17 +379,19 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
   // NS-1 K-steps may stay in flight (where a stage's refill is split over two K-steps, see
   // LATE below, its second half is the youngest request and everything is waited for).
   constexpr int OPB = IA + IB;  // operand copies per wave and K-step
+  constexpr bool EXACT = NS == 2 && BM * BN <= 128 * 128;
   bf16x8 fw[2][TN], fx[2][TMH];
   if (kt_n > 0) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const int k = k_step(min(s, it_n - 1));
-      if (dma_wave) {
+      if (dma_wave && (!EXACT || s < it_n)) {
         TileA::template issue<0, IA>(uniform_ptr(a_at(k)), offa, lds0 + s * STAGE, wave);
         TileB::template issue<0, IB>(uniform_ptr(b_at(k)), offb, lds0 + s * STAGE + A_BYTES, wave);
       }
     }
-    dma_wait<(NS - 1) * OPB>();  // stage 0 has landed; the others may still be in flight
+    if constexpr (EXACT) dma_wait_groups<OPB, NS - 1>(it_n - 1);
+    else dma_wait<(NS - 1) * OPB>();  // stage 0 has landed; the others may still be in flight
   }
   __syncthreads();
 #pragma unroll
@@ -409,6 +411,10 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
   // the copies land too late.)
   constexpr int LATE = (NS == 2 && BM == 256 && BN == 256 && NW == 8) ? 2 : 0;
   constexpr bool SPLIT = LATE > 0;
+  // With two stages and two workgroups on a CU the last copies are not repeated: they would hold the
+  // CU's path while the other workgroup's are due and this one's end would wait for them (512 x 4096
+  // x 1024 with a GELU 15.1 -> 14.3 us, 512 x 3072 x 1024 12.5 -> 12.1).  Deep forms, alone on
+  // their CU, and the 256 x 256 tile lose as much by the branches around their copies (0 - 2 %).
   const bf16_t* ga_late = nullptr;
   const bf16_t* gb_late = nullptr;
   int st_late = 0;
@@ -418,7 +424,8 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
     const uint8_t* sb = sa + A_BYTES;
     const uint8_t* na = stages + nst * STAGE;
     const bool live = KG == 1 || kt * KG + grp < kt_n;
-    // past the end the last K-step is fetched again, unused
+    // past the end the last K-step is fetched again, unused (EXACT: nothing is)
+    const bool refill = dma_wave && (!EXACT || kt + NS < it_n);
     const int kn = k_step(min(kt + NS, it_n - 1));
     const bf16_t* ga = uniform_ptr(a_at(kn));
     const bf16_t* gb = uniform_ptr(b_at(kn));
@@ -488,7 +495,7 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
         if (!SPLIT && ks == NB - 1) {
 #pragma unroll
           for (int i = 2 * ib; i < 2 * ib + 2; ++i)
-            if (i % (TMH / PARTS) == 0 && dma_wave) {
+            if (i % (TMH / PARTS) == 0 && refill) {
               TileA::template issue_part<IA / PARTS>(i / (TMH / PARTS), ga, offa, lds0 + st * STAGE, wave);
               TileB::template issue_part<IB / PARTS>(i / (TMH / PARTS), gb, offb,
                                                      lds0 + st * STAGE + A_BYTES, wave);
@@ -502,7 +509,7 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
           const int slot = ks * 2 + ib;           // pair of MFMA rows within the K-step
           if (ks == NB - 1) {
             const int part = slot - (2 * NB - (4 - LATE));
-            if (part >= 0 && dma_wave) {
+            if (part >= 0 && refill) {
               TileA::template issue_part<IA / PARTS>(part, ga, offa, lds0 + st * STAGE, wave);
               TileB::template issue_part<IB / PARTS>(part, gb, offb, lds0 + st * STAGE + A_BYTES, wave);
             }
@@ -540,7 +547,7 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
     st = nst;
     cbi = cbi + 1 == NS + 1 ? 0 : cbi + 1;
   }
-  dma_wait_all();   // the refetches of the last two K-steps must not outlive the block's LDS
+  dma_wait_all();
 
   // the groups' sums, in group order: wave w of every group holds the same elements, so they
   // change hands through LDS lane by lane, 16 bytes at a time

@@ -70,7 +70,8 @@ __global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
     const uint8_t* const stages = smem + wave * (NS * STAGE);
     const uint32_t lds0 = lds_address(stages);
     auto copy = [&](int stage, int t) {
-      const long at = min(t, steps - 1);   // (past the end the last step again, unused)
+      if (t >= steps) return;
+      const long at = t;
       TileA::template issue<0, TileA::INSTS>(uniform_ptr(pa + at * (W * 64)), offa, lds0 + stage * STAGE, 0);
       TileB::template issue<0, TileB::INSTS>(uniform_ptr(pb + at * W * step_b), offb,
                                              lds0 + stage * STAGE + TileA::BYTES, 0);
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
     for (int s = 0; s < NS; ++s) copy(s, s);
     int st = 0;
     for (int t = 0; t < steps; ++t) {
-      dma_wait<(NS - 1) * COPIES>();   // (copies land in order: this step's have)
+      dma_wait_groups<COPIES, NS - 1>(steps - 1 - t);   // (copies land in order: this step's have)
       const uint8_t* const sa = stages + st * STAGE;
       const uint8_t* const sb = sa + TileA::BYTES;
       bf16x8 fa[2][TM], fb[2][4];
@@ -103,7 +104,6 @@ __global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
       st = st + 1 == NS ? 0 : st + 1;
     }
   }
-  dma_wait_all();    // (the copies past the end must not land in what the sums are staged in)
   __syncthreads();
   float* const part = (float*)smem;
 #pragma unroll
