@@ -36,7 +36,7 @@ namespace {
 enum { kTile128 = 1, kTile256x128 = 2, kTile128x256 = 3, kTile256 = 4, kTile64 = 5,
        kTile64x128 = 6 /* the library's own choice only */ };
 constexpr long kCus = 256;
-constexpr long kMostCus = 192;  // 256x256 tiles from which a grid of them is taken without asking
+constexpr long kMostCus = 192;  // 256x256 tiles from which a forward grid of them is taken without asking
 
 struct GemmParams {
   const bf16_t* a;
@@ -187,8 +187,10 @@ __device__ __forceinline__ int group_steps(const int* seg, const int* seg_rows, 
   return (rows + 63) / 64;
 }
 
-// Whether a form has room for the accumulator's rows beside its operand stages (C += A B).
-constexpr bool streams_accumulator(int stages, int wave_groups) { return wave_groups == 1 && stages <= 4; }
+// Whether a form streams the accumulator's rows through LDS beside its operand stages (C += A B): the
+// large tiles, alone on their CU.  (A 128x128 tile with room for the rows would be alone on its CU too: the
+// gradients of the epilogue's comment 115 us instead of 87.)
+constexpr bool streams_accumulator(int bm, int bn) { return bm * bn > 128 * 128; }
 
 template <int BM, int BN, bool TA, bool TB, int EPI, int NW, int NS, bool KP = false, bool MP = false,
           int KG = 1>
@@ -343,7 +345,7 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
   // loops too short for that add the old values in the epilogue, where rows are whole too.
   static_assert(BN * 4 <= 1024, "a row of the fp32 tile is one 64-lane copy");
   constexpr int NBT = BM / NW, C_LDS = NS * (BM + BN) * 128, C_PITCH = 1024 + 16;  // a copy is 1 KB
-  constexpr bool STREAM_C = EPI == JPP_EPI_ACC_F32 && streams_accumulator(NS, KG);
+  constexpr bool STREAM_C = EPI == JPP_EPI_ACC_F32 && streams_accumulator(BM, BN);
   const bool stream_c = STREAM_C && kt_n >= NBT + NS;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -579,10 +581,33 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
     // fp32 outputs leave through LDS as well (see below), a quarter of the tile per pass:
     // 16-byte stores of contiguous rows instead of 32-byte pieces of 32 rows
     constexpr int IPP = WHOLE ? TM : TM / 2, RP = WHOLE ? BM : IPP * 16, PITCH = BN * 4 + 16,
-                  NT = NW * KG * 64;
-    constexpr int TPR = BN / 4, RPI = NT / TPR;
-#pragma unroll 1
-    for (int pass = 0; pass < (WHOLE ? 1 : 2 * (TM / IPP)); ++pass) {
+                  NT = NW * KG * 64, PASSES = WHOLE ? 1 : 2 * (TM / IPP);
+    constexpr int TPR = BN / 4, RPI = NT / TPR, PER = RP / RPI;
+    static_assert(RP % RPI == 0, "rows of a pass split evenly over the threads");
+    const int c4 = (tid % TPR) * 4;
+    auto row_of = [&](int pass, int it) {
+      return m0 + (pass / (TM / IPP)) * (BM / 2) + (pass % (TM / IPP)) * IPP * 16 + tid / TPR + it * RPI;
+    };
+    // Old values that did not stream in are read here, by rows and past the caches: a small tile's
+    // all at once, a large one's (out of registers for that) a pass ahead, the next pass's while this
+    // one's leave.  Through the caches, and each pass's behind the one before it, a layer's four gradients
+    // of hidden 2048 and feed-forward 5632 on 512 tokens took 110 us as 256x256 tiles and 168 as
+    // 128x128; now 96 and 87 (what their accumulators' 352 MB alone take: 84).
+    const bool add_here = EPI == JPP_EPI_ACC_F32 && !stream_c;
+    constexpr int BUFS = PASSES * PER <= 8 ? PASSES : 1;
+    f32x4 old[BUFS][PER];
+    auto fetch = [&](int pass) {
+#pragma unroll
+      for (int it = 0; it < PER; ++it)
+        old[pass % BUFS][it] =
+            __builtin_nontemporal_load((const f32x4*)((const float*)p.c + row_of(pass, it) * p.ldc + n0 + c4));
+    };
+    if (add_here) {
+#pragma unroll
+      for (int pass = 0; pass < BUFS; ++pass) fetch(pass);
+    }
+#pragma unroll(BUFS)
+    for (int pass = 0; pass < PASSES; ++pass) {
       const int half = pass / (TM / IPP), i0 = (pass % (TM / IPP)) * IPP;
       __syncthreads();
       if (WHOLE ? grp == 0 : wm == half) {
@@ -596,37 +621,21 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
           }
       }
       __syncthreads();
-      const long mrow0 = m0 + half * (BM / 2) + i0 * 16;
-      const int c4 = (tid % TPR) * 4;
-      static_assert(RP % RPI == 0, "rows of a pass split evenly over the threads");
-      float4 v[RP / RPI];
-      if (EPI == JPP_EPI_ACC_F32 && !stream_c) {
-        // a K loop too short to stream the old values in: they are read here, by rows, all of
-        // a thread's rows before the first is used
-        float4 old[RP / RPI];
+      f32x4 v[PER];
 #pragma unroll
-        for (int it = 0; it < RP / RPI; ++it)
-          old[it] = *(const float4*)((const float*)p.c + (mrow0 + tid / TPR + it * RPI) * p.ldc +
-                                     n0 + c4);
+      for (int it = 0; it < PER; ++it) v[it] = *(const f32x4*)(smem + (tid / TPR + it * RPI) * PITCH + c4 * 4);
+      if (add_here) {
 #pragma unroll
-        for (int it = 0; it < RP / RPI; ++it) {
-          const float4 t = *(const float4*)(smem + (tid / TPR + it * RPI) * PITCH + c4 * 4);
-          v[it] = make_float4(old[it].x + t.x, old[it].y + t.y, old[it].z + t.z, old[it].w + t.w);
-        }
-      } else {
-#pragma unroll
-        for (int it = 0; it < RP / RPI; ++it)
-          v[it] = *(const float4*)(smem + (tid / TPR + it * RPI) * PITCH + c4 * 4);
+        for (int it = 0; it < PER; ++it) v[it] = old[pass % BUFS][it] + v[it];
+        if (BUFS == 1 && pass + 1 < PASSES) fetch(pass + 1);
       }
 #pragma unroll
-      for (int it = 0; it < RP / RPI; ++it) {
-        float* dst = (float*)p.c + (mrow0 + tid / TPR + it * RPI) * p.ldc + n0 + c4;
+      for (int it = 0; it < PER; ++it) {
+        float* dst = (float*)p.c + row_of(pass, it) * p.ldc + n0 + c4;
         // the accumulators are not read again before the next microbatch: stored past the
         // caches they leave L2 to the operand panels (+0.4 % on the Llama-8B-shaped stage)
-        if (EPI == JPP_EPI_ACC_F32)
-          __builtin_nontemporal_store(f32x4{v[it].x, v[it].y, v[it].z, v[it].w}, (f32x4*)dst);
-        else
-          *(float4*)dst = v[it];
+        if (EPI == JPP_EPI_ACC_F32) __builtin_nontemporal_store(v[it], (f32x4*)dst);
+        else *(f32x4*)dst = v[it];
       }
     }
   } else {
@@ -792,7 +801,7 @@ int launch(hipStream_t stream, GemmParams& p) {
   constexpr int SMEM_LOOP = KG * NS * (BM + BN) * 128,
                 SMEM_EPI = (KG > 1 ? BM : BM / 2) * (BN * 4 + 16);
   // + NS+1 buffers of NW rows of the fp32 tile (padded) for C += A B
-  constexpr int SMEM = EPI == JPP_EPI_ACC_F32 && streams_accumulator(NS, KG) ? SMEM_LOOP + (NS + 1) * NW * (1024 + 16)
+  constexpr int SMEM = EPI == JPP_EPI_ACC_F32 && streams_accumulator(BM, BN) ? SMEM_LOOP + (NS + 1) * NW * (1024 + 16)
                        : (EPI == JPP_EPI_F32 || SMEM_LOOP > SMEM_EPI) ? SMEM_LOOP : SMEM_EPI;
   if constexpr (!KP) {
     // several operand pairs: only the accumulating weight-gradient kernels are built for that
@@ -844,7 +853,7 @@ int launch(hipStream_t stream, GemmParams& p) {
 // Llama-3-8B-shaped layer are 13 full rounds together - and small ones share the device.
 template <int BM, int BN, int NW, int NS, int KG = 1>
 int launch_multi(hipStream_t stream, GemmParams* ps, int n) {
-  constexpr int SMEM = KG * NS * (BM + BN) * 128 + (streams_accumulator(NS, KG) ? (NS + 1) * NW * (1024 + 16) : 0);
+  constexpr int SMEM = KG * NS * (BM + BN) * 128 + (streams_accumulator(BM, BN) ? (NS + 1) * NW * (1024 + 16) : 0);
   static_assert(SMEM <= 160 * 1024, "LDS of one CU");
   GemmArgs<true> args;
   args.p = ps[0];
@@ -960,33 +969,41 @@ int launch_tiled(hipStream_t stream, GemmParams& p, int tile, bool deep) {
   }
 }
 
-// Expected time of a product of `tiles` tiles, `ksteps` K-steps of 64 each, in us:
-//   start + w * (tile_cost [+ gelu] + ksteps * step),   w = tiles of the busiest of the 256 CUs
-// (two workgroups fit on a CU in the two-stage forms: their steps overlap, so a CU's lone
-// workgroup takes a step cost of its own; `gelu`: the arithmetic of a GELU epilogue).  The
-// constants are least-squares fits to 1300 random products (M, N 128 .. 16384, K 128 .. 16384, every
-// orientation and epilogue) timed in every form with the operands out of L2, as a layer finds
-// them, and accumulators out of every cache: mean error 4 - 10 %.  The forward 128x256 stands 10 %
-// above its fit: 128x128 is otherwise passed over where they are close.  Taking the smallest
-// estimate costs 0.1 % against always taking the measured best.  Against the rule before (256x256
-// from 192 tiles on, else 128x128: 36 % on average) it is slower by more than 2 % for 12 of the
-// 1300, all but one by 6 % at most (180 tiles of 256x256, 3 K-steps: 14 %): a 512 x 1024 x 4096 input
-// gradient has 32 tiles of 128x128 for 256 CUs and took 28 us, 15 us as 128 tiles of 64x64 with two
-// wave groups each.
+// Expected time of a product of `tiles` tiles, `ksteps` K-steps of 64 each, in us, with w = tiles of the
+// busiest of the 256 CUs and s = tiles / 256 (`gelu`: the arithmetic of a GELU epilogue):
+//   w = 1:  start + tile_cost + gelu + s * share + ksteps * lone_step
+//   w > 1:  start + w * (tile_cost + gelu) + s * share + ksteps * (w * step + s * share_step)
+// (two workgroups of a two-stage form fit on a CU, their steps overlap; `share`: what the tiles wait for
+// together, the fp32 tile that a weight gradient's workgroup reads, adds to and writes).  The constants are
+// least-squares fits to random products in every form, with the operands out of L2, as a layer finds
+// them, and accumulators out of every cache.
+// Forward: 1300 products (M, N 128 .. 16384, K 128 .. 16384, every orientation and epilogue), mean error 4
+// - 10 %; the smallest estimate costs 0.1 % against the measured best.  128x256 stands 10 % above its
+// fit: 128x128 is otherwise passed over where they are close.  Against the rule before (256x256 from 192
+// tiles on, else 128x128: 36 % on average) it is slower by more than 2 % for 12 of the 1300, all but one by
+// 6 % at most (180 tiles of 256x256, 3 K-steps: 14 %): a 512 x 1024 x 4096 input gradient has 32 tiles of
+// 128x128 for 256 CUs and took 28 us, 15 us as 128 tiles of 64x64 with two wave groups each.
+// Weight gradients: 420 launches of 1 to 4 products (outputs 128 .. 8192 a side, 64 .. 8192 tokens), mean
+// error 2 - 11 %; the smallest estimate costs 0.3 % against the measured best.  256x256 from 192 tiles on
+// cost 9 % there and 36 % at worst (300 tiles, 2 K-steps: 44 us, 33 as 128x128; 1176 tiles, 4: 135 and 121): a
+// 256x256 tile, alone on its CU, waits for its fp32 tile apart from its K-steps, of two 128x128 tiles one's
+// wait falls on the other's steps.
 struct TileForm {
   int tile, bm, bn;
   bool deep;              // which of the tile's two forms (kTile128, kTile64)
-  float start, tile_cost, gelu, lone_step, step;
+  float start, tile_cost, gelu, lone_step, step, share, share_step;
 };
 constexpr TileForm kForward[] = {
-    {kTile64, 64, 64, true, 0.f, 4.8f, 0.5f, 0.18f, 0.18f},     {kTile64, 64, 64, false, 2.7f, 1.5f, 0.3f, 0.26f, 0.17f},
-    {kTile128, 128, 128, true, 0.f, 6.3f, 2.1f, 0.39f, 0.39f},  {kTile128, 128, 128, false, 3.4f, 2.3f, 1.7f, 0.49f, 0.365f},
-    {kTile128x256, 128, 256, true, 1.1f, 7.4f, 5.2f, 0.705f, 0.715f},
-    {kTile256, 256, 256, true, 0.2f, 10.2f, 10.f, 1.05f, 1.08f}};
+    {kTile64, 64, 64, true, 0.f, 4.8f, 0.5f, 0.18f, 0.18f, 0.f, 0.f},     {kTile64, 64, 64, false, 2.7f, 1.5f, 0.3f, 0.26f, 0.17f, 0.f, 0.f},
+    {kTile128, 128, 128, true, 0.f, 6.3f, 2.1f, 0.39f, 0.39f, 0.f, 0.f},  {kTile128, 128, 128, false, 3.4f, 2.3f, 1.7f, 0.49f, 0.365f, 0.f, 0.f},
+    {kTile128x256, 128, 256, true, 1.1f, 7.4f, 5.2f, 0.705f, 0.715f, 0.f, 0.f},
+    {kTile256, 256, 256, true, 0.2f, 10.2f, 10.f, 1.05f, 1.08f, 0.f, 0.f}};
 constexpr TileForm kWeightGrad[] = {
-    {kTile64, 64, 64, true, 0.f, 5.2f, 0.f, 0.28f, 0.28f},      {kTile64, 64, 64, false, 3.7f, 2.0f, 0.f, 0.19f, 0.22f},
-    {kTile128, 128, 128, true, 0.f, 8.6f, 0.f, 0.515f, 0.515f}, {kTile128, 128, 128, false, 2.2f, 6.8f, 0.f, 0.32f, 0.77f},
-    {kTile128x256, 128, 256, true, 0.f, 11.2f, 0.f, 1.13f, 1.02f}, {kTile256, 256, 256, true, 0.f, 15.5f, 0.f, 1.43f, 1.43f}};
+    {kTile64, 64, 64, true, 0.f, 3.8f, 0.f, 0.24f, 0.24f, 3.9f, 0.f},    {kTile64, 64, 64, false, 4.3f, 0.f, 0.f, 0.22f, 0.21f, 2.f, 0.f},
+    {kTile128, 128, 128, true, 0.f, 5.7f, 0.f, 0.485f, 0.485f, 6.4f, 0.f},
+    {kTile128, 128, 128, false, 5.1f, 0.45f, 0.f, 0.43f, 0.39f, 4.3f, 0.115f},
+    {kTile128x256, 128, 256, true, 3.f, 4.4f, 0.f, 0.9f, 0.83f, 7.8f, 0.08f},
+    {kTile256, 256, 256, true, 5.6f, 6.3f, 0.f, 1.28f, 1.08f, 16.f, 0.53f}};
 
 // tile with the smallest estimate for products of these extents in one grid (`grid`: the extents
 // that its form goes by)
@@ -1000,22 +1017,26 @@ int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool 
     if ((f.tile == kTile64 || f.tile == kTile128) &&
         f.deep != deep_stages(count_tiles(grid, n, f.bm, f.bn), ksteps, f.tile)) continue;
     const long w = (tiles + kCus - 1) / kCus;
-    const float t = f.start + w * (f.tile_cost + (gelu ? f.gelu : 0.f) + ksteps * (w == 1 ? f.lone_step : f.step));
+    const float share = (float)tiles / kCus;
+    const float t = f.start + w * (f.tile_cost + (gelu ? f.gelu : 0.f)) + share * f.share +
+                    ksteps * (w == 1 ? f.lone_step : w * f.step + share * f.share_step);
     if (best_us == 0.f || t < best_us) { best_us = t; best = f.tile; }
   }
   return best;
 }
 
 // The 256x256 tile run by 8 waves (two per SIMD, so one wave's LDS reads hide under the other's
-// MFMAs) is the fastest whenever it gives most CUs a tile; smaller problems go by the estimate.
+// MFMAs) is the fastest whenever it gives most CUs a tile; smaller problems go by the estimate, and
+// accumulated weight gradients all do.
 int choose_tile(const jpp_gemm_args* a) {
   const Extent e = work_extent(a);
   if (a->group_mode != JPP_GROUP_NONE && !a->group_rows) return kTile256;
   const long t256 = e.m % 256 == 0 && e.n % 256 == 0 ? (e.m / 256) * (e.n / 256) : 0;
-  if (t256 >= kMostCus) return kTile256;
+  const bool wgrad = a->trans_a && a->trans_b;
+  if (t256 >= kMostCus && !(wgrad && a->epilogue == JPP_EPI_ACC_F32)) return kTile256;
   const Extent grid = grid_extent(a);
   const bool gelu = a->epilogue == JPP_EPI_GELU || a->epilogue == JPP_EPI_DGELU;
-  const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), a->trans_a && a->trans_b, gelu, true);
+  const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), wgrad, gelu, true);
   // (a rotated head lies inside one tile)
   return tile == kTile64 && a->rope_cos && a->rope_head_dim > 64 ? (int)kTile64x128 : tile;
 }
@@ -1252,8 +1273,7 @@ extern "C" int jpp_gemm_bf16_multi(void* stream_, const jpp_gemm_args* problems,
   if (n_problems == 1) return jpp_gemm_bf16(stream_, problems);
   GemmParams ps[4];
   Extent e[4];
-  long tiles = 0, t256 = 0;
-  bool whole = true;
+  long tiles = 0;
   for (int i = 0; i < n_problems; ++i) {
     const jpp_gemm_args* a = problems + i;
     if (int rc = prepare(a, ps[i])) return rc;
@@ -1264,14 +1284,11 @@ extern "C" int jpp_gemm_bf16_multi(void* stream_, const jpp_gemm_args* problems,
     JPP_REQUIRE(a->k == problems[0].k && ps[i].k_parts == ps[0].k_parts,
                 "gemm_multi: problem %d differs from problem 0 in k or k_parts", i);
     e[i] = {a->m, a->n};
-    whole = whole && a->m % 256 == 0 && a->n % 256 == 0;
-    t256 += (a->m / 256) * (a->n / 256);
     tiles += (a->m / 64) * (a->n / 64);
   }
   JPP_REQUIRE(tiles < (1L << 30), "gemm_multi: too many tiles");
   const long ksteps = (long)ps[0].k / 64 * ps[0].k_parts;
-  const int tile = whole && t256 >= kMostCus ? (int)kTile256
-                   : cheapest_tile(e, e, n_problems, ksteps, true, false, false);
+  const int tile = cheapest_tile(e, e, n_problems, ksteps, true, false, false);
   const bool deep = deep_stages(tile == kTile64 ? tiles : tiles / 4, ksteps, tile);
   if (tile == kTile256) return launch_multi<256, 256, 8, 2>(stream, ps, n_problems);
   if (tile == kTile64)
