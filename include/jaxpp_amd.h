@@ -58,6 +58,20 @@ int jpp_malloc(void** ptr, size_t bytes);
 int jpp_free(void* ptr);
 int jpp_memcpy_h2d(void* dst, const void* src, size_t bytes);
 int jpp_memcpy_d2h(void* dst, const void* src, size_t bytes);
+/* Many tensors between pageable host memory and the device in one call, ordered as jpp_memcpy_*: behind
+ * everything queued on the null stream, complete when the call returns.  WORDS: 4-byte elements as they
+ * are.  BF16: float32 on the host, bf16 on the device (to the device rounded to nearest even, ties by the
+ * last bit kept).  Up to 8 host threads and 16 MiB of pinned memory work on a call; they are kept for the
+ * next one until jpp_copy_release or the end of the process's last stage object gives them back. */
+typedef enum { JPP_COPY_WORDS = 0, JPP_COPY_BF16 = 1 } jpp_copy_kind;
+typedef struct {
+  void* host;      /* 4-byte elements; only read by jpp_copy_h2d */
+  void* device;
+  int64_t count;   /* elements */
+} jpp_copy_item;
+int jpp_copy_h2d(int n, const jpp_copy_item* items, int kind);
+int jpp_copy_d2h(int n, const jpp_copy_item* items, int kind);
+int jpp_copy_release(void);
 int jpp_memcpy_d2d_async(void* dst, const void* src, size_t bytes, void* stream);
 int jpp_fill_u32(void* dst, uint32_t value, size_t count, void* stream);
 int jpp_stream_create(void** stream);

@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libjaxpp_amd.so")
-SOURCES = ["abi.hip", "gemm.hip", "gemm_wave.hip", "attention.hip", "attention_dq.hip", "attention_dkv.hip", "attention_small.hip", "elementwise.hip",
+SOURCES = ["abi.hip", "host_copy.hip", "gemm.hip", "gemm_wave.hip", "attention.hip", "attention_dq.hip", "attention_dkv.hip", "attention_small.hip", "elementwise.hip",
            "moe.hip", "optimizer.hip", "f32_ops.hip", "stage.hip"]
 # measurement aids: a library of their own beside the product library
 DIAG_LIB = os.path.join(LIBDIR, "libjaxpp_amd_diag.so")
@@ -69,7 +69,7 @@ def build(verbose: bool = True, jobs: int = 6) -> str:
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         all_objs = list(ex.map(compile_one, SOURCES + DIAG_SOURCES))
     objs, diag_objs = all_objs[:len(SOURCES)], all_objs[len(SOURCES):]
-    _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs])
+    _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-pthread", "-o", LIB, *objs])
     if verbose:
         print(f"[jaxpp_amd.build] linked {LIB}", flush=True)
     # resolves jpp_set_error from the product library next to it

@@ -405,9 +405,10 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
     for s_, segs in enumerate(stage_segs):
         for g, sg in enumerate(segs):
             sg.ex = execs[s_, g]
-            for li, params in enumerate(sg.layers):
-                sg.ex.set_params(0, li, params)
-            sg.ex.zero_grads()
+    segments = [sg for segs in stage_segs for sg in segs]
+    rt.set_params([(sg.ex, 0, li, params) for sg in segments for li, params in enumerate(sg.layers)])
+    for sg in segments:
+        sg.ex.zero_grads()
 
     tokens, hidden = spec0.tokens, spec0.hidden
     act_elems = tokens * hidden
@@ -538,11 +539,10 @@ def run_loop(tr, outputs, ops, n: int, schedule: BaseSchedule):
         for first, last in mb_runs:
             run = any_ex.download_activation(preds_dev[first].owner, (last - first, tokens, hidden))
             preds.update(zip(range(first, last), run))
-    grads = {}
-    for s_, segs in enumerate(stage_segs):
-        grads[s_] = []
-        for sg in segs:
-            grads[s_] += [sg.ex.get_grads(0, li) for li in range(len(sg.layers))]
+    places = [(s_, sg.ex, li) for s_, segs in enumerate(stage_segs) for sg in segs for li in range(len(sg.layers))]
+    grads = {s_: [] for s_ in range(S)}
+    for (s_, _, _), g in zip(places, rt.get_grads([(ex, 0, li) for _, ex, li in places])):
+        grads[s_].append(g)
 
     def reduce_leaf(v, op):
         if isinstance(v, tracing.GradOf):

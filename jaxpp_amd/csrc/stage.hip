@@ -18,6 +18,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <string>
 #include <utility>
@@ -26,6 +27,8 @@
 #include "common.h"
 
 namespace {
+
+std::atomic<int> g_stages{0};   // stage objects of the process
 
 struct ParamInfo {
   const char* name;
@@ -109,6 +112,7 @@ struct jpp_stage {
   // gradient half is done and whose weight-gradient half waits for the rest of its group.
   int wg = 1;
   std::vector<std::vector<std::pair<int, int>>> pend;
+  bool counted = false;  // among g_stages
   bool broken = false;   // a grouped weight-gradient launch failed half way: accumulators unusable
 
   bool f32() const { return d.dtype == JPP_DTYPE_F32; }
@@ -1013,11 +1017,14 @@ int jpp_stage_create(const jpp_stage_desc* d, jpp_stage** out) {
     return jpp_set_error(JPP_ERR_HIP, "stage_create: %s", hipGetErrorString(e5));
   }
   *out = s;
+  s->counted = true;
+  ++g_stages;
   return JPP_OK;
 }
 
 int jpp_stage_destroy(jpp_stage* s) {
   if (!s) return JPP_OK;
+  if (s->counted && --g_stages == 0) (void)jpp_copy_release();
   hipDeviceSynchronize();
   auto drop = [](hipEvent_t ev) { if (ev) hipEventDestroy(ev); };
   drop(s->ev_fork);

@@ -30,56 +30,78 @@ def _zip_map(f, *trees):
     return f(*trees)
 
 
+# Elements of the leaves that go through the device in one go.
+BATCH = 1 << 23
+
+
 def _offsets(leaves):
-    """Places of a run's leaves in one vector, each on 64 bytes, and the vector's length."""
+    """Places of leaves in one vector, one behind the other, and the vector's length (whole 64 bytes)."""
     at, n = [], 0
     for a in leaves:
         at.append(n)
-        n += -(-a.size // 16) * 16
-    return at, n
+        n += a.size
+    return at, -(-n // 16) * 16
 
 
-def _upload_run(buf, n, at, *kinds):
-    """The kinds of leaves of a run (gradients, moments, ...; one list each) behind one another
-    into `buf`, a vector of `n` elements per kind: one packed copy, or of a run of one leaf straight
-    from the leaves' own memory.  A leaf's kinds are read as far as the first one reaches."""
-    if len(at) == 1:
-        for k, (a,) in enumerate(kinds):
-            buf.upload(a.reshape(-1)[:kinds[0][0].size], 4 * n * k)
-        return
-    host = np.empty(n * len(kinds), np.float32)
-    for k, leaves in enumerate(kinds):
-        for i, a in enumerate(leaves):
-            size = kinds[0][i].size
-            host[k * n + at[i]:k * n + at[i] + size] = a.reshape(-1)[:size]
-    buf.upload(host)
-
-
-def _download_run(buf, n, at, leaves, *kinds):
-    """The kinds `kinds` (adjacent ones) of `buf`'s vectors as arrays of the leaves' shapes, one
-    list per kind: views of one array, or of a run of one leaf arrays of their own."""
-    if len(at) == 1:
-        return [[buf.download(np.float32, leaves[0].shape, 4 * n * k)] for k in kinds]
-    out = buf.download(np.float32, (n * len(kinds),), 4 * n * kinds[0])
-    return [[out[n * k + i:n * k + i + a.size].reshape(a.shape) for i, a in zip(at, leaves)]
-            for k in range(len(kinds))]
-
-
-def _map_runs(f, *trees):
-    """A tree like the first of what ``f`` returns per leaf.  ``f`` takes the leaves of a run
-    (`runtime.copy_runs`), one list per tree, float32 and contiguous: leaf by leaf a step of four
-    small layers was 250 uploads and 200 downloads, and those 20 of its 24 ms."""
+def _upload(ptr, n, at, *kinds):
+    """The kinds of leaves (gradients, moments, ...; one list each) behind one another to `ptr`, a vector
+    of `n` elements per kind, from the leaves' own memory.  A leaf's kinds are read as far as the
+    first one reaches."""
     from jaxpp_amd import runtime as rt
+    rt.copy_in([(a.reshape(-1)[:first.size], ptr + 4 * (n * k + i))
+                for k, leaves in enumerate(kinds) for a, first, i in zip(leaves, kinds[0], at)])
+
+
+def _download(ptr, n, at, leaves, *kinds):
+    """The kinds `kinds` of the vectors at `ptr` as arrays of the leaves' shapes, one list per kind:
+    views of one array per kind and run of small leaves (`runtime.copy_runs`)."""
+    from jaxpp_amd import runtime as rt
+    items, out = [], []
+    for k in kinds:
+        views = []
+        for first, last in rt.copy_runs([a.size for a in leaves]):
+            flat = np.empty(at[last - 1] + leaves[last - 1].size - at[first], np.float32)
+            items.append((flat, ptr + 4 * (n * k + at[first])))
+            views += [flat[i - at[first]:i - at[first] + a.size].reshape(a.shape)
+                      for i, a in zip(at[first:last], leaves[first:last])]
+        out.append(views)
+    rt.copy_out(items)
+    return out
+
+
+def _map_batches(f, *trees):
+    """A tree like the first of what ``f`` returns per leaf.  ``f`` takes consecutive leaves of at most
+    `BATCH` elements together (or one), one list per tree, float32 and contiguous."""
     leaves = []
     _zip_map(lambda *ls: leaves.append(ls), *trees)
-    out = []
-    for first, last in rt.copy_runs([math.prod(np.shape(ls[0])) for ls in leaves]):
-        run = [[np.ascontiguousarray(a, dtype=np.float32) for a in ls] for ls in leaves[first:last]]
-        for ls in run:
+    sizes = [math.prod(np.shape(ls[0])) for ls in leaves]
+    out, first = [], 0
+    while first < len(leaves):
+        last, total = first + 1, sizes[first]
+        while last < len(leaves) and total + sizes[last] <= BATCH:
+            total += sizes[last]
+            last += 1
+        batch = [[np.ascontiguousarray(a, dtype=np.float32) for a in ls] for ls in leaves[first:last]]
+        for ls in batch:
             assert all(a.size >= ls[0].size for a in ls), [a.shape for a in ls]
-        out += f(*([ls[k] for ls in run] for k in range(len(trees))))
+        out += f(*([ls[k] for ls in batch] for k in range(len(trees))))
+        first = last
     results = iter(out)
     return _zip_map(lambda *_: next(results), *trees)
+
+
+class _Scratch:
+    """Device memory that the batches of one call take in turn."""
+
+    def __init__(self):
+        self.buf = None
+
+    def take(self, nbytes: int) -> int:
+        from jaxpp_amd import runtime as rt
+        if self.buf is None or self.buf.nbytes < nbytes:
+            self.buf = None          # (freed before the larger one is taken)
+            self.buf = rt.DeviceBuffer(nbytes)
+        return self.buf.ptr
 
 
 @dataclass(frozen=True)
@@ -101,22 +123,22 @@ class adam:
         from jaxpp_amd import runtime as rt
         rt.require_gpu()
         step = int(state["count"]) + 1
+        scratch = _Scratch()
 
         def run(gs, ms, vs):
-            """The leaves of a run as one vector: gradients, moments and updates of `n` elements
+            """The leaves of a batch as one vector: gradients, moments and updates of `n` elements
             each behind one another on the device.  The updates come back as memory of their own:
             the moments outlive the step, they do not."""
             at, n = _offsets(gs)
-            buf = rt.DeviceBuffer(16 * n)
-            _upload_run(buf, n, at, gs, ms, vs)
+            ptr = scratch.take(16 * n)
             # weights that start at zero end as the update itself
-            rt.check(rt.load().jpp_fill_u32(buf.ptr + 12 * n, 0, n, None))
-            rt.adam_step(n, buf.ptr, buf.ptr + 4 * n, buf.ptr + 8 * n, step, master=buf.ptr + 12 * n,
+            rt.check(rt.load().jpp_fill_u32(ptr + 12 * n, 0, n, None))
+            _upload(ptr, n, at, gs, ms, vs)
+            rt.adam_step(n, ptr, ptr + 4 * n, ptr + 8 * n, step, master=ptr + 12 * n,
                          lr=self.learning_rate, b1=self.b1, b2=self.b2, eps=self.eps)
-            rt.sync()
-            return list(zip(*_download_run(buf, n, at, gs, 3), *_download_run(buf, n, at, gs, 1, 2)))
+            return list(zip(*_download(ptr, n, at, gs, 3, 1, 2)))
 
-        trio = _map_runs(run, grads, state["mu"], state["nu"])
+        trio = _map_batches(run, grads, state["mu"], state["nu"])
         pick = lambda k: _zip_map(lambda g, t: t[k], grads, trio)
         return pick(0), {"count": step, "mu": pick(1), "nu": pick(2)}
 
@@ -125,13 +147,13 @@ def apply_updates(params, updates):
     """``optax.apply_updates``: ``params + updates``, leaf by leaf, in f32 on the GPU."""
     from jaxpp_amd import runtime as rt
     rt.require_gpu()
+    scratch = _Scratch()
 
     def run(ps, us):
         at, n = _offsets(ps)
-        buf = rt.DeviceBuffer(8 * n)
-        _upload_run(buf, n, at, ps, us)
-        rt.check(rt.load().jpp_grad_accum_f32(None, buf.ptr, buf.ptr + 4 * n, n, 1))
-        rt.sync()
-        return _download_run(buf, n, at, ps, 0)[0]
+        ptr = scratch.take(8 * n)
+        _upload(ptr, n, at, ps, us)
+        rt.check(rt.load().jpp_grad_accum_f32(None, ptr, ptr + 4 * n, n, 1))
+        return _download(ptr, n, at, ps, 0)[0]
 
-    return _map_runs(run, params, updates)
+    return _map_batches(run, params, updates)

@@ -7,6 +7,7 @@ without a GPU every call raises.
 """
 from __future__ import annotations
 
+import atexit
 import ctypes as C
 import os
 from typing import Iterable
@@ -102,9 +103,14 @@ FAMILY = {"bert": 0, "llama": 1, "mixtral": 2, "decoder": 3}
 DTYPE = {"bf16": 0, "f32": 1}
 
 # every symbol include/jaxpp_amd.h declares
+class CopyItem(C.Structure):
+    _fields_ = [("host", C.c_void_p), ("device", C.c_void_p), ("count", C.c_int64)]
+
+
 EXPORTS = [
     "jpp_last_error", "jpp_version", "jpp_device_count", "jpp_set_device", "jpp_malloc",
     "jpp_free", "jpp_memcpy_h2d", "jpp_memcpy_d2h", "jpp_memcpy_d2d_async", "jpp_fill_u32",
+    "jpp_copy_h2d", "jpp_copy_d2h", "jpp_copy_release",
     "jpp_stream_create", "jpp_stream_destroy", "jpp_stream_sync", "jpp_stream_wait_event",
     "jpp_device_sync",
     "jpp_event_create", "jpp_event_destroy", "jpp_event_record", "jpp_event_sync",
@@ -212,6 +218,7 @@ def load():
                                    C.c_int64, C.c_int]
     lib.jpp_rope.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_int,
                              C.c_int, C.c_int, C.c_int, C.c_int]
+    lib.jpp_copy_h2d.argtypes = lib.jpp_copy_d2h.argtypes = [C.c_int, C.POINTER(CopyItem), C.c_int]
     lib.jpp_grad_accum_f32.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int]
     lib.jpp_colsum_accum.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int64,
                                      C.c_void_p, C.c_void_p]
@@ -258,6 +265,7 @@ def load():
     lib.jpp_stage_adam_step.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_double,
                                         C.c_double, C.c_double, C.c_double, C.c_double]
     _lib = lib
+    atexit.register(lib.jpp_copy_release)
     return lib
 
 
@@ -309,21 +317,25 @@ class DeviceBuffer:
 
     @classmethod
     def from_f32_as_bf16(cls, a: np.ndarray) -> "DeviceBuffer":
-        return cls.from_numpy(to_bf16_bits(a))
+        a = np.ascontiguousarray(a, dtype=np.float32)
+        buf = cls(2 * a.size)
+        copy_in([(a, buf.ptr)], bf16=True)
+        return buf
 
     def upload(self, a: np.ndarray, offset: int = 0):
         a = np.ascontiguousarray(a)
         assert offset + a.nbytes <= self.nbytes
-        check(load().jpp_memcpy_h2d(self.ptr + offset, a.ctypes.data, a.nbytes))
+        upload_ptr(self.ptr + offset, a)
 
     def download(self, dtype, shape, offset: int = 0) -> np.ndarray:
-        out = np.empty(shape, dtype=dtype)
-        assert offset + out.nbytes <= self.nbytes
-        check(load().jpp_memcpy_d2h(out.ctypes.data, self.ptr + offset, out.nbytes))
-        return out
+        assert offset + int(np.prod(shape)) * np.dtype(dtype).itemsize <= self.nbytes
+        return download_ptr(self.ptr + offset, dtype, shape)
 
     def download_bf16(self, shape) -> np.ndarray:
-        return from_bf16_bits(self.download(np.uint16, shape))
+        assert 2 * int(np.prod(shape)) <= self.nbytes
+        out = np.empty(shape, np.float32)
+        copy_out([(out, self.ptr)], bf16=True)
+        return out
 
     def zero(self, stream=None):
         check(load().jpp_fill_u32(self.ptr, 0, self.nbytes // 4, stream))
@@ -348,22 +360,49 @@ class BufferPart:
         self.owner, self.nbytes, self.ptr = owner, nbytes, owner.ptr + offset
 
 
+def _copy(fn, items, bf16: bool):
+    arr = (CopyItem * len(items))()
+    for q, (a, ptr) in zip(arr, items):
+        assert a.flags.c_contiguous and a.itemsize == 4, (a.shape, a.dtype, a.strides)
+        q.host, q.device, q.count = a.ctypes.data, ptr, a.size
+    check(fn(len(items), arr, int(bf16)))
+
+
+def copy_in(items, bf16: bool = False):
+    """Contiguous host arrays of 4-byte elements to the device, a list of (array, device pointer),
+    in one call of the library; `bf16`: float32 arrays, rounded to bf16 on the way."""
+    _copy(load().jpp_copy_h2d, items, bf16)
+
+
+def copy_out(items, bf16: bool = False):
+    """The other way, into the arrays; `bf16`: float32 arrays from bf16 tensors."""
+    _copy(load().jpp_copy_d2h, items, bf16)
+
+
+# Bytes from which a copy of one array goes through copy_in / copy_out (below: 14 us for a plain
+# one, 20 - 30 for those).
+COPY_LARGE = 1 << 16
+
+
 def upload_ptr(ptr: int, a: np.ndarray):
     a = np.ascontiguousarray(a)
-    check(load().jpp_memcpy_h2d(ptr, a.ctypes.data, a.nbytes))
+    if a.nbytes >= COPY_LARGE and a.nbytes % 4 == 0:
+        copy_in([(a.reshape(-1).view(np.uint32), ptr)])
+    else:
+        check(load().jpp_memcpy_h2d(ptr, a.ctypes.data, a.nbytes))
 
 
 def download_ptr(ptr: int, dtype, shape) -> np.ndarray:
     out = np.empty(shape, dtype=dtype)
-    check(load().jpp_memcpy_d2h(out.ctypes.data, ptr, out.nbytes))
+    if out.nbytes >= COPY_LARGE and out.nbytes % 4 == 0:
+        copy_out([(out.reshape(-1).view(np.uint32), ptr)])
+    else:
+        check(load().jpp_memcpy_d2h(out.ctypes.data, ptr, out.nbytes))
     return out
 
 
-# Elements of small tensors that travel as one copy, and of one that travels by itself.  A copy
-# between pageable host memory and the device costs 14 us and more whatever its size, and up to 115
-# us at 64 - 256 KB; one of 8 MB moves at 16 - 35 GB/s.  Larger tensors gain nothing and would only
-# be copied once more on the host (an optimizer step over 16 leaves of 1024 x 1024: in runs of two
-# 37.8 ms, by themselves 32.7; over 64 of 256 x 1024: in runs 39.5, by themselves 42.9).
+# Elements of small tensors whose results share one array, and of one that has an array of its own:
+# larger ones in an array together would keep each other alive for nothing.
 COPY_RUN = 1 << 21
 COPY_ALONE = 1 << 19
 
@@ -576,6 +615,28 @@ def adam_step(count, grad, m, v, step, master=None, param=None, lr=1e-3, b1=0.9,
     check(load().jpp_adam_step(stream, C.byref(a)))
 
 
+def set_params(layers):
+    """`StageExecutor.set_params` of several layers in one copy per element type: a list of (executor, chunk,
+    layer, params)."""
+    for bf16 in (False, True):
+        items = [it for ex, chunk, layer, params in layers if (ex.dtype != "f32") == bf16
+                 for it in ex._param_items(chunk, layer, params)]
+        if items:
+            copy_in(items, bf16)
+
+
+def get_grads(layers) -> list:
+    """`StageExecutor.get_grads` of several layers in one copy: a list of (executor, chunk, layer)."""
+    items, results = [], []
+    for ex, chunk, layer in layers:
+        ex.join()
+        more, result = ex._result_layer(ex._layer_ptrs(load().jpp_stage_grad_ptr, chunk, layer), False)
+        items += more
+        results.append(result)
+    copy_out(items)
+    return [result() for result in results]
+
+
 class StageExecutor:
     """One pipeline rank on one GPU: parameters, fp32 gradient accumulators,
     residual slots, and the FWD / BWD / BWD_I / BWD_W tasks."""
@@ -602,6 +663,7 @@ class StageExecutor:
                                               C.byref(c)))
             self.params.append((name.value.decode(), r.value, c.value))
         self.index = {n: i for i, (n, _, _) in enumerate(self.params)}
+        self._places = []
 
     @property
     def nbytes(self) -> int:
@@ -629,59 +691,75 @@ class StageExecutor:
         sizes = [r * c for _, r, c in self.params]
         return copy_runs(sizes, lambda i: ptrs[i] == ptrs[i - 1] + sizes[i - 1] * itemsize)
 
-    def _download_layer(self, ptrs, dtype, convert=None) -> dict:
-        """name -> host array (in the host's column order) of the tensors at `ptrs`."""
-        out = {}
-        for first, last in self._runs(ptrs, np.dtype(dtype).itemsize):
-            run = self.params[first:last]
-            flat = download_ptr(ptrs[first], dtype, (sum(r * c for _, r, c in run),))
-            if convert is not None:
-                flat = convert(flat)
-            at = 0
-            for name, rows, cols in run:
-                shape = (cols,) if rows == 1 and not name.startswith("W") else (rows, cols)
-                a = flat[at:at + rows * cols].reshape(shape)
-                at += rows * cols
-                order = self._device_columns(name, cols)
-                if order is not None:
-                    host = np.empty_like(a)
-                    host[:, order] = a
-                    a = host
-                out[name] = a
-        return out
+    def _result_layer(self, ptrs, bf16: bool):
+        """Host arrays for the tensors of a layer at `ptrs`: the items of a copy into them, and a function that
+        then gives name -> float32 array, in the host's column order."""
+        runs = []
+        for first, last in self._runs(ptrs, 2 if bf16 else 4):
+            runs.append((np.empty(sum(r * c for _, r, c in self.params[first:last]), np.float32), first, last))
+
+        def result() -> dict:
+            out = {}
+            for flat, first, last in runs:
+                at = 0
+                for name, rows, cols in self.params[first:last]:
+                    shape = (cols,) if rows == 1 and not name.startswith("W") else (rows, cols)
+                    a = flat[at:at + rows * cols].reshape(shape)
+                    at += rows * cols
+                    order = self._device_columns(name, cols)
+                    if order is not None:
+                        host = np.empty_like(a)
+                        host[:, order] = a
+                        a = host
+                    out[name] = a
+            return out
+
+        return [(flat, ptrs[first]) for flat, first, _ in runs], result
+
+    def _download_layer(self, ptrs, bf16: bool) -> dict:
+        items, result = self._result_layer(ptrs, bf16)
+        copy_out(items, bf16)
+        return result()
+
+    def _layer_ptrs(self, fn, chunk: int, layer: int) -> list:
+        """Device pointers of a layer's parameters (or gradients), by `fn`: the same number of elements apart
+        in every layer."""
+        if not self._places:
+            ptrs = [self._ptr(load().jpp_stage_grad_ptr, 0, 0, name) for name, _, _ in self.params]
+            self._places = [(p - ptrs[0]) // 4 for p in ptrs]
+        es = 2 if fn is load().jpp_stage_param_ptr and self.dtype != "f32" else 4
+        first = self._ptr(fn, chunk, layer, self.params[0][0])
+        return [first + es * d for d in self._places]
+
+    def _param_items(self, chunk: int, layer: int, params: dict) -> list:
+        items = []
+        ptrs = self._layer_ptrs(load().jpp_stage_param_ptr, chunk, layer)
+        for (name, rows, cols), ptr in zip(self.params, ptrs):
+            a = np.ascontiguousarray(params[name], dtype=np.float32)
+            assert a.size == rows * cols, (name, a.shape, rows, cols)
+            order = self._device_columns(name, cols)
+            if order is not None:
+                a = np.ascontiguousarray(a.reshape(rows, cols)[:, order])
+            items.append((a, ptr))
+        return items
 
     def set_params(self, chunk: int, layer: int, params: dict):
         """Upload float32 host arrays as device parameters (bf16, or f32 for an f32 stage)."""
-        ptrs = [self._ptr(load().jpp_stage_param_ptr, chunk, layer, name) for name, _, _ in self.params]
-        for first, last in self._runs(ptrs, 4 if self.dtype == "f32" else 2):
-            arrays = []
-            for name, rows, cols in self.params[first:last]:
-                a = np.asarray(params[name], dtype=np.float32)
-                assert a.size == rows * cols, (name, a.shape, rows, cols)
-                order = self._device_columns(name, cols)
-                if order is not None:
-                    a = np.ascontiguousarray(a.reshape(rows, cols)[:, order])
-                arrays.append(a)
-            a = arrays[0] if len(arrays) == 1 else np.concatenate([x.reshape(-1) for x in arrays])
-            upload_ptr(ptrs[first], a if self.dtype == "f32" else to_bf16_bits(a))
+        copy_in(self._param_items(chunk, layer, params), self.dtype != "f32")
 
     def get_params(self, chunk: int, layer: int) -> dict:
         """The device parameters as float32 host arrays."""
         self.join()
-        ptrs = [self._ptr(load().jpp_stage_param_ptr, chunk, layer, name) for name, _, _ in self.params]
-        if self.dtype == "f32":
-            return self._download_layer(ptrs, np.float32)
-        return self._download_layer(ptrs, np.uint16, from_bf16_bits)
+        return self._download_layer(self._layer_ptrs(load().jpp_stage_param_ptr, chunk, layer), self.dtype != "f32")
 
     def get_grads(self, chunk: int, layer: int) -> dict:
         self.join()          # the copies below run on the null stream
-        ptrs = [self._ptr(load().jpp_stage_grad_ptr, chunk, layer, name) for name, _, _ in self.params]
-        return self._download_layer(ptrs, np.float32)
+        return self._download_layer(self._layer_ptrs(load().jpp_stage_grad_ptr, chunk, layer), False)
 
     def upload_activation(self, a: np.ndarray) -> "DeviceBuffer":
         """A float32 host array as a device tensor of the stage's element type."""
         a = np.ascontiguousarray(a, dtype=np.float32)
-        return DeviceBuffer.from_numpy(a if self.dtype == "f32" else to_bf16_bits(a))
+        return DeviceBuffer.from_numpy(a) if self.dtype == "f32" else DeviceBuffer.from_f32_as_bf16(a)
 
     def new_activation(self) -> "DeviceBuffer":
         return DeviceBuffer(self.spec.tokens * self.spec.hidden * (4 if self.dtype == "f32" else 2))
