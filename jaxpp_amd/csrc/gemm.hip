@@ -1041,16 +1041,19 @@ int choose_tile(const jpp_gemm_args* a) {
   return tile == kTile64 && a->rope_cos && a->rope_head_dim > 64 ? (int)kTile64x128 : tile;
 }
 
-// Products that run on waves of their own (gemm_wave.hip): while their 32x64 tiles are at most one
-// per CU.  Over 65 random shapes below that line (M, N, K 128 .. 8192; both orientations, plain and
-// GELU epilogues) they take 0.99 to 0.70 of the time of the best tile here, 0.8 in the median;
-// above it, two rounds of them, 1.01 to 1.45.  A plain forward product without bias and
+// Products that run on waves of their own (gemm_wave.hip), by the rows of their tiles (0: they do
+// not).  32 while those tiles are at most one per CU: over 65 random shapes (M, N, K 128 .. 8192; both
+// orientations, plain and GELU epilogues) they take 0.99 to 0.70 of the time of the best tile
+// here, 0.8 in the median; above that line, two rounds of them, 1.01 to 1.45.  From there 64 while `tile`,
+// the choice among the tiles here, is the 64x64 one and those are at most one per CU, and with a GELU from
+// 9 K-steps on (gemm_wave.hip has the figures).  A plain forward product without bias and
 // residual stays: its bits are those a product with the rotary epilogue rotates.
-bool runs_on_waves(const jpp_gemm_args* a) {
+int rows_on_waves(const jpp_gemm_args* a, int tile) {
   const bool kind = a->epilogue == JPP_EPI_BF16 ? !a->trans_b || a->bias || a->resid
                                                 : a->epilogue == (a->trans_b ? JPP_EPI_GELU : JPP_EPI_DGELU);
-  return kind && !a->tile && !a->trans_a && a->group_mode == JPP_GROUP_NONE && a->k_parts <= 1 &&
-         !a->rope_cos && (a->m / 32) * (a->n / 64) <= kCus;
+  if (!kind || a->tile || a->trans_a || a->group_mode != JPP_GROUP_NONE || a->k_parts > 1 || a->rope_cos) return 0;
+  if ((a->m / 32) * (a->n / 64) <= kCus) return 32;
+  return tile == kTile64 && (a->m / 64) * (a->n / 64) <= kCus && (a->epilogue == JPP_EPI_BF16 || a->k > 8 * 64) ? 64 : 0;
 }
 
 // sub-problem whose first row / column is (m_off, n_off) of the full one
@@ -1202,12 +1205,12 @@ extern "C" int jpp_gemm_bf16(void* stream_, const jpp_gemm_args* a) {
   GemmParams p;
   if (int rc = prepare(a, p)) return rc;
   int tile = a->tile ? a->tile : choose_tile(a);
-  if (runs_on_waves(a)) {
+  if (const int rows = rows_on_waves(a, tile)) {
     const GemmWave d = {p.a, p.b, (bf16_t*)p.c, (bf16_t*)p.c2, p.bias, p.resid, p.aux, p.m, p.n, p.k,
                         p.lda, p.ldb, p.ldc, p.ldc2, p.ldresid, p.ldaux, p.gelu_tanh};
     ProbeScope probe(stream, a->trans_b ? "gemm_nn_wave" : "gemm_nt_wave", 2.0 * a->m * a->n * a->k,
                      2.0 * (a->m * a->k + a->n * a->k + a->m * a->n));
-    return launch_gemm_wave(stream, d, a->trans_b != 0, a->epilogue);
+    return launch_gemm_wave(stream, d, a->trans_b != 0, a->epilogue, rows);
   }
   // several operand pairs of an ungrouped product: the 256-wide tiles whatever its size
   // (jpp_gemm_bf16_multi is the way to run small ones)

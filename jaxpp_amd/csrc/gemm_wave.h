@@ -18,8 +18,8 @@ struct GemmWave {
   int gelu_tanh;
 };
 
-// tb: weight [k][n] (epilogues BF16, GELU) or [n][k] (BF16, DGELU)
-int launch_gemm_wave(hipStream_t stream, const GemmWave& p, bool tb, int epi);
+// tb: weight [k][n] (epilogues BF16, GELU) or [n][k] (BF16, DGELU); rows of a tile: 32 or 64
+int launch_gemm_wave(hipStream_t stream, const GemmWave& p, bool tb, int epi, int rows);
 
 namespace {
 

@@ -1,17 +1,23 @@
 // bf16 products of few tiles: C[m,n] = epilogue(sum_k A[m,k] Bop[n,k]), A's contraction index
 // contiguous (forward and input-gradient products).
 //
-// A workgroup owns 32 x 64 outputs; its four waves each multiply the whole tile over every fourth
-// K-step of 64 and their sums meet in LDS, in wave order.  With fewer tiles than CUs a product's
+// A workgroup owns BM x 64 outputs, 32 or 64 rows; its W waves each multiply the whole tile over every
+// W-th K-step of 64 and their sums meet in LDS, in wave order.  With fewer tiles than CUs a product's
 // time is one tile's, and a tile whose waves share their operands in LDS is a chain of
 // latencies: barrier, fragment reads, copies, K-step after K-step.  Here every wave copies its own
 // steps into LDS of its own and waits for nothing but them: no barrier before the sums, and the
-// copies of four waves keep the CU's path to memory (64 bytes a cycle) busy, which is then what
-// bounds the tile: 12 KB a K-step, 192 cycles.  512 x 1024 x 4096 (256 tiles) 17.4 -> 13.9 us,
-// 512 x 1024 x 1024 9.0 -> 7.4, 256 x 256 x 768 7.2 -> 5.7, 128 x 128 x 128 5.0 -> 4.3, against
-// 64 x 64 tiles shared by two wave groups.  (64 x 64 outputs this way: two stages are all that
-// fits, 15.8 us for the first; operands from L2 straight into fragments, without LDS: 28 us, a
-// load of 16 rows x 64 bytes holds the path far longer than its kilobyte.)
+// copies of the waves keep the CU's path to memory (64 bytes a cycle) busy, which is then what
+// bounds a tile of 32 rows: 12 KB a K-step, 192 cycles.  512 x 1024 x 4096 (256 tiles) 17.4 -> 13.9 us, 512 x
+// 1024 x 1024 9.0 -> 7.4, 256 x 256 x 768 7.2 -> 5.7, 128 x 128 x 128 5.0 -> 4.3, against 64 x 64 tiles
+// shared by two wave groups; without the copies past the end (3 of 7 at K = 1024) the first 10.3 where that
+// product runs by itself.  (Operands from L2 straight into fragments, without LDS: 28 us, a load of 16
+// rows x 64 bytes holds the path far longer than its kilobyte.)
+// Tiles of 64 rows, 16 KB a K-step, for up to twice the outputs: four waves with two stages each, which
+// is all that fits, and the copies between the MFMAs; 512 x 2048 outputs at K = 11264 / 5632 / 2048 46 -> 39 / 27
+// -> 25.7 / 9.6 -> 9.0 us against the tiles shared by two wave groups, 0.85 - 0.95 over 70 random shapes.
+// With a GELU or its derivative eight waves with one stage each, whose epilogue has twice the
+// threads: 0.85 - 0.95 (GELU) and 0.93 - 1.0 from 9 K-steps on, 1.0 - 1.1 below.  (Three stages of three waves 41.6 us
+// for the first, two of five 41.4, eight waves 37.8 but 12.1 instead of 11.8 at K = 3072.)
 //
 // The operands' LDS images and the fragments read from them are those of gemm.hip (DmaTile), the
 // n side on the MFMA's A port: lane (c = lane % 16, g = lane / 16) ends up with row 16 i + c and
@@ -22,12 +28,12 @@
 
 namespace {
 
-constexpr int W = 4;     // waves, one per SIMD
-constexpr int BM = 32, TM = BM / 16, NS = 3;   // rows of a tile, stages of a wave
 constexpr int PITCH = 68;                      // floats of a row of the sums
 
-template <bool TB, int EPI>
+// BM: rows of a tile; W: waves, at most one per SIMD; NS: stages of a wave
+template <bool TB, int EPI, int BM, int W, int NS>
 __global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
+  constexpr int TM = BM / 16;
   using TileA = DmaTile<BM, false, 1>;
   using TileB = DmaTile<64, TB, 1>;
   constexpr int STAGE = TileA::BYTES + TileB::BYTES, COPIES = TileA::INSTS + TileB::INSTS;
@@ -37,20 +43,33 @@ __global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
   // Consecutive workgroups go to the eight XCDs in turn, each with an L2 of its own: every XCD
   // takes a run of tiles, 256 rows at a time, so that it reads a part of both operands.
   const int tiles_n = p.n / 64, tiles_m = p.m / BM;
+  // (64 rows: the first XCDs one tile more where the number is not a multiple of 8 - 252 tiles as they come
+  // took 1.16 of the time of the tiles shared by wave groups, in runs 0.92.  The few scalar
+  // instructions more cost products of 32 rows 0.2 us each, a row of 512 tokens 1 %.)
   int pid = blockIdx.x;
-  if ((gridDim.x & 7) == 0) pid = (pid & 7) * (gridDim.x >> 3) + (pid >> 3);
+  if constexpr (BM == 64) {
+    const int nwg = gridDim.x, x = pid & 7;
+    pid = x * (nwg >> 3) + min(x, nwg & 7) + (pid >> 3);
+  } else if ((gridDim.x & 7) == 0) {
+    pid = (pid & 7) * (gridDim.x >> 3) + (pid >> 3);
+  }
   const int rows = 256 / BM, first = pid / (rows * tiles_n) * rows, rows_here = min(tiles_m - first, rows);
   const int within = pid - first * tiles_n;
   const long m0 = (long)(first + within % rows_here) * BM, n0 = (long)(within / rows_here) * 64;
 
-  // the epilogue's share of this thread: 8 columns of a row; what it adds or multiplies with
-  // arrives during the contraction
-  static_assert(BM * 8 == 64 * W, "one piece of a row per thread");
-  const long row = m0 + (tid >> 3), ocol = n0 + (tid & 7) * 8;
+  // the epilogue's share of this thread: 8 columns of a row, and of every STEP-th row behind it; what
+  // they are added to or multiplied with arrives during the contraction
+  constexpr int STEP = 8 * W, MINE = (BM + STEP - 1) / STEP;
+  const int row = tid >> 3;
+  const long ocol = n0 + (tid & 7) * 8;
   const bf16_t* const pre_src = EPI == JPP_EPI_DGELU ? p.aux : EPI == JPP_EPI_BF16 ? p.resid : nullptr;
   const long pre_ld = EPI == JPP_EPI_DGELU ? p.ldaux : p.ldresid;
-  uint4 pre = make_uint4(0, 0, 0, 0), bias = pre;
-  if (pre_src) pre = *(const uint4*)(pre_src + row * pre_ld + ocol);
+  uint4 pre[MINE], bias = make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int q = 0; q < MINE; ++q) {
+    pre[q] = make_uint4(0, 0, 0, 0);
+    if (pre_src && (BM % STEP == 0 || row + q * STEP < BM)) pre[q] = *(const uint4*)(pre_src + (m0 + row + q * STEP) * pre_ld + ocol);
+  }
   if (p.bias) bias = *(const uint4*)(p.bias + ocol);
 
   f32x4 acc[TM][4];
@@ -91,16 +110,41 @@ __global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
 #pragma unroll
         for (int i = 0; i < TM; ++i) fa[k][i] = TileA::frag16(sa, 16 * i, k, lane);
       }
-      // every fragment is in registers: the stage can be filled again, under the MFMAs
+      // every fragment is in registers: the stage can be filled again - of 32 rows at once, of 64
+      // between the MFMAs, which the copies would keep waiting for the path (a wave issues in
+      // order; with 32 rows that order costs a row of products of 512 tokens 1.5 %)
       lds_wait_all();
-      copy(st, t + NS);
+      constexpr int PARTS = BM == 32 ? 1 : 2 * TM, PER = COPIES / PARTS;
+      static_assert(COPIES % PARTS == 0, "copies split evenly over the rows of MFMAs");
+      auto refill = [&](int part) {
+        if (t + NS >= steps) return;
+        const bf16_t* const na = uniform_ptr(pa + (long)(t + NS) * (W * 64));
+        const bf16_t* const nb = uniform_ptr(pb + (long)(t + NS) * W * step_b);
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
+        for (int q = part * PER; q < part * PER + PER; ++q) {
+          if (q < TileA::INSTS) dma_load16(na, offa[min(q, TileA::INSTS - 1)], lds0 + st * STAGE + q * 1024);
+          else dma_load16(nb, offb[max(q - TileA::INSTS, 0)], lds0 + st * STAGE + q * 1024);
+        }
+      };
+      if (PARTS == 1) refill(0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+      for (int k = 0; k < 2; ++k) {
+        if constexpr (PARTS == 1) {
 #pragma unroll
-          for (int i = 0; i < TM; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[k][j], fa[k][i], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[k][j], fa[k][i], acc[i][j], 0, 0, 0);
+        } else {
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[k][j], fa[k][i], acc[i][j], 0, 0, 0);
+            refill(k * TM + i);
+          }
+        }
+      }
       st = st + 1 == NS ? 0 : st + 1;
     }
   }
@@ -112,42 +156,47 @@ __global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
     for (int j = 0; j < 4; ++j)
       *(f32x4*)(part + (wave * BM + 16 * i + c) * PITCH + 16 * j + 4 * g) = acc[i][j];
   __syncthreads();
-  const float* src = part + (tid >> 3) * PITCH + (tid & 7) * 8;
-  f32x4 lo = *(const f32x4*)src, hi = *(const f32x4*)(src + 4);
 #pragma unroll
-  for (int w = 1; w < W; ++w) {
-    lo += *(const f32x4*)(src + w * BM * PITCH);
-    hi += *(const f32x4*)(src + w * BM * PITCH + 4);
-  }
-  float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, q[8];
-  if (p.bias) {
-    unpack8(bias, q);
+  for (int q = 0; q < MINE; ++q) {
+    const int r = row + q * STEP;
+    if (BM % STEP && r >= BM) break;
+    const float* src = part + r * PITCH + (tid & 7) * 8;
+    f32x4 lo = *(const f32x4*)src, hi = *(const f32x4*)(src + 4);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] += q[e];
-  }
-  unpack8(pre, q);
-  if constexpr (EPI == JPP_EPI_BF16) {
-    if (p.resid) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] += q[e];
+    for (int w = 1; w < W; ++w) {
+      lo += *(const f32x4*)(src + w * BM * PITCH);
+      hi += *(const f32x4*)(src + w * BM * PITCH + 4);
     }
-  } else if constexpr (EPI == JPP_EPI_DGELU) {
+    float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, u[8];
+    if (p.bias) {
+      unpack8(bias, u);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] *= gelu_grad_f(q[e], p.gelu_tanh);
-  } else {
-    float gl[8];
+      for (int e = 0; e < 8; ++e) v[e] += u[e];
+    }
+    unpack8(pre[q], u);
+    if constexpr (EPI == JPP_EPI_BF16) {
+      if (p.resid) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) gl[e] = gelu_f(v[e], p.gelu_tanh);
-    *(uint4*)(p.c2 + row * p.ldc2 + ocol) = pack8(gl);
+        for (int e = 0; e < 8; ++e) v[e] += u[e];
+      }
+    } else if constexpr (EPI == JPP_EPI_DGELU) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= gelu_grad_f(u[e], p.gelu_tanh);
+    } else {
+      float gl[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) gl[e] = gelu_f(v[e], p.gelu_tanh);
+      *(uint4*)(p.c2 + (m0 + r) * p.ldc2 + ocol) = pack8(gl);
+    }
+    *(uint4*)(p.c + (m0 + r) * p.ldc + ocol) = pack8(v);
   }
-  *(uint4*)(p.c + row * p.ldc + ocol) = pack8(v);
 }
 
-template <bool TB, int EPI>
+template <bool TB, int EPI, int BM, int W, int NS>
 int launch(hipStream_t st, const GemmWave& p) {
   constexpr int LOOP = W * NS * (BM + 64) * 128, SUMS = W * BM * PITCH * 4, SMEM = LOOP > SUMS ? LOOP : SUMS;
   static_assert(SMEM <= 160 * 1024, "LDS of one CU");
-  auto kern = gemm_wave_kernel<TB, EPI>;
+  auto kern = gemm_wave_kernel<TB, EPI, BM, W, NS>;
   static std::once_flag configured;   // (the limit is sticky per kernel)
   static hipError_t configure_rc = hipSuccess;
   std::call_once(configured, [&] {
@@ -161,7 +210,13 @@ int launch(hipStream_t st, const GemmWave& p) {
 
 }  // namespace
 
-int launch_gemm_wave(hipStream_t st, const GemmWave& p, bool tb, int epi) {
-  if (tb) return epi == JPP_EPI_BF16 ? launch<true, JPP_EPI_BF16>(st, p) : launch<true, JPP_EPI_GELU>(st, p);
-  return epi == JPP_EPI_BF16 ? launch<false, JPP_EPI_BF16>(st, p) : launch<false, JPP_EPI_DGELU>(st, p);
+template <bool TB, int EPI>
+int launch_rows(hipStream_t st, const GemmWave& p, int rows) {
+  if (rows == 32) return launch<TB, EPI, 32, 4, 3>(st, p);
+  return EPI == JPP_EPI_BF16 ? launch<TB, EPI, 64, 4, 2>(st, p) : launch<TB, EPI, 64, 8, 1>(st, p);
+}
+
+int launch_gemm_wave(hipStream_t st, const GemmWave& p, bool tb, int epi, int rows) {
+  if (tb) return epi == JPP_EPI_BF16 ? launch_rows<true, JPP_EPI_BF16>(st, p, rows) : launch_rows<true, JPP_EPI_GELU>(st, p, rows);
+  return epi == JPP_EPI_BF16 ? launch_rows<false, JPP_EPI_BF16>(st, p, rows) : launch_rows<false, JPP_EPI_DGELU>(st, p, rows);
 }
