@@ -757,9 +757,16 @@ __global__ __launch_bounds__(256) void cast_bf16_f32_kernel(const bf16_t* __rest
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256)
     dst[i] = bf16_to_f32(src[i]);
 }
+// 64 bytes a thread in four runs of its workgroup, one trip each (12 GB 2120 us in strides through the whole
+// tensor, 1999 like this; past the caches 2040, and 32 us instead of 24 for a tensor of 184 MB).  `dst` need only
+// be aligned to its elements.
+typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* dst, uint32_t v, long n) {
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256)
-    dst[i] = v;
+  const long n4 = n / 4, at = (long)blockIdx.x * 1024 + threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (at + 256 * u < n4) ((u32x4_u*)dst)[at + 256 * u] = u32x4_u{v, v, v, v};
+  if (at < n - n4 * 4) dst[n4 * 4 + at] = v;
 }
 
 // loss of the last stage: mean((out - target)^2) * scale, and its cotangent
@@ -1104,8 +1111,10 @@ int jpp_fill_u32(void* dst, uint32_t value, size_t count, void* stream) {
   JPP_REQUIRE(dst || count == 0, "fill: null destination");
   if (count == 0) return JPP_OK;
   ProbeScope probe((hipStream_t)stream, "fill", 0, 4.0 * count);
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(grid_for((long)count)), dim3(256), 0,
-                     (hipStream_t)stream, (uint32_t*)dst, value, (long)count);
+  JPP_REQUIRE(count < (size_t)1 << 40, "fill: too large");
+  const unsigned blocks = (unsigned)(count / 4096 + 1);
+  hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, (uint32_t*)dst, value,
+                     (long)count);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
