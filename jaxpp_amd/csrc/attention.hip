@@ -548,24 +548,42 @@ AttnParams make_params(const jpp_attn_args* a) {
   return p;
 }
 
-// Where 16 rows per workgroup (attention_small.hip) beat the blocks of this file.  Forward: while
-// they are at most one workgroup per CU (seq x heads of all sequences <= 4096); measured, times
-// of the two: 5.3 / 4.8 us at 2 heads x 128 positions x 64, 17.8 / 9.7 at 2 x 1024 x 64, 10.4 / 8.1
-// at 16 x 256 x 128 under a mask; at twice that many workgroups 7.5 / 7.9 (32 x 256 x 64) down to
-// 0.72 of the speed.
+// Where 16 rows per workgroup (attention_small.hip) take the place of the blocks of this file.  Forward: while
+// they are at most one workgroup per CU (seq x heads of all sequences <= 4096); measured, times of the two: 4.5 /
+// 3.9 us at 2 heads x 128 positions x 64, 16.0 / 7.0 at 2 x 1024 x 64, 8.9 / 6.3 at 16 x 256 x 128 under a mask.  (At
+// twice that many workgroups they are still quicker, 9.6 / 7.8 at 16 x 512 x 64, but a row's maximum, whose
+// probability is 1 and has no rounding error, then counts once per 256 keys instead of once per 64: the output is 1 %
+// further from float64, 2.22e-3 instead of 2.19e-3.)
 bool small_fwd(const jpp_attn_args* a) { return (int64_t)a->batch * a->n_heads * a->seq <= 4096; }
 
-// Backward: at most a workgroup of 16 keys per CU and twice as many of 16 queries (13.6 / 6.3 us,
-// 43.6 / 20.2, 31.4 / 19.1 at the sizes above; twice as many keys: 19.0 / 24.2).  Under a mask
-// the kernels of their own are quicker with many query heads per key (4 heads x 512 positions x
-// 128: 57.2 / 58.0 us, 8 x 256: 0.94 of the speed; 4 x 256: 1.23, 8 x 256 x 64: 1.17): the one
-// workgroup of 16 keys then walks all of their queries.
+// Backward: where their expected time is shorter.  With x = workgroups of 16 queries per CU, g = query heads per key
+// head and S positions, in us:
+//   16 rows   c0 + c1 g S + x (c2 + c3 S)
+//   blocks    c0 + c1 S + c2 g S + c3 x S
+// (a workgroup's own walk - one of keys walks the queries of all of its heads - and what the others add).
+// Least squares of the relative error over 440 problems (128 .. 2048 positions, 1 .. 8 sequences, 2 .. 32 heads, all
+// key head counts, up to 4096 rows); mean error of the blocks 3 - 5 %, of the 16 rows 13 %.  The shorter estimate costs
+// 0.1 - 0.6 % over the shorter time; a workgroup of 16 keys and two of 16 queries per CU, the rule before these kernels
+// took their operands through LDS, 10 - 20 %.  16 query and 4 key heads x 512 positions x 128 under a mask: 57 us in
+// blocks, 31 in one launch of 16 rows; 16 heads x 512 x 64: 27.3 and 21.1; distances from float64 the same.
+struct SmallFit {
+  float rows16[4], blocks[4];
+};
+constexpr SmallFit kSmallBwd[2][2] = {   // [head 128][causal]
+    {{{3.81f, 0.00198f, 3.12f, 0.00784f}, {10.0f, 0.0101f, 0.0197f, 0.00116f}},
+     {{3.66f, 0.00254f, 3.25f, 0.00406f}, {15.5f, 0.0141f, 0.00793f, 0.00076f}}},
+    {{{5.37f, 0.00329f, 6.47f, 0.016f}, {16.2f, 0.0145f, 0.0405f, 0.003f}},
+     {{5.49f, 0.00447f, 6.39f, 0.00831f}, {23.6f, 0.0203f, 0.01f, 0.00129f}}}};
+
 // One launch writes dQ, dK and dV while it reads everything else, where two read only part of it:
 // a caller whose results lie over the inputs keeps the two.
 bool small_bwd(const jpp_attn_args* a) {
-  const int64_t rows = (int64_t)a->batch * a->seq, grp = a->n_heads / a->n_kv_heads;
-  if (rows * a->n_heads > 8192 || rows * a->n_kv_heads > 4096) return false;
-  if (a->causal && grp > 1 && grp * a->seq * a->head_dim > 131072) return false;
+  const int64_t rows = (int64_t)a->batch * a->seq;
+  const SmallFit& f = kSmallBwd[a->head_dim == 128][a->causal != 0];
+  const float S = a->seq, gS = S * (a->n_heads / a->n_kv_heads), x = (float)rows * a->n_heads / 4096.f;
+  if (f.rows16[0] + f.rows16[1] * gS + x * (f.rows16[2] + f.rows16[3] * S) >=
+      f.blocks[0] + f.blocks[1] * S + f.blocks[2] * gS + f.blocks[3] * x * S)
+    return false;
   struct Range {
     uintptr_t lo, hi;
   };

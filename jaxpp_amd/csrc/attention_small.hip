@@ -2,12 +2,19 @@
 //
 // A workgroup owns 16 rows of one head's queries (keys, for dK / dV) and its eight waves take
 // the other side 32 rows at a time in turn; their partial results meet in LDS, in wave order,
-// at the end (deterministic, no atomics).  Operands go from L2 straight into MFMA fragments:
-// there is no LDS and no barrier before the waves meet.  That reads the other side once per 16
-// rows instead of once per 64 to 256, which a large problem cannot afford and a small one does
-// not notice: here a kernel's time is how long one workgroup takes, and it takes an eighth of
-// the steps.  2 x 8 heads x 256 positions x 128 (32 workgroups of the kernels in attention.hip,
-// 16 to 32 in the backward): forward 10.3 us, backward 19.2 + 16.9 us there.
+// at the end (deterministic, no atomics).  That reads the other side once per 16 rows instead of once per
+// 64 to 256, which a large problem cannot afford and a small one does not notice: here a kernel's time is
+// how long one workgroup takes, and it takes an eighth of the steps.
+//
+// Every wave copies the 32 rows of its next step into LDS of its own, whole lines in flight under the
+// products of this one, and waits for nothing else: no barrier before the waves meet (but the forward's, which
+// share a row's maximum).  Row fragments are plain reads of that tile, column fragments transposing ones.
+// (Fragments loaded from memory directly take 16 rows x 64 bytes an instruction, which holds the CU's path
+// several times as long as its kilobyte, and the rows of both products once each: backward of 16 heads x 512 x 64
+// 35.3 us that way, 21.1 like this; of 16 and 4 heads x 512 x 128 without a mask 60 and 33; forward of 8 heads x 1024 x
+// 64 16.2 and 11.0.)  What is left of a step is latency: the copies of one tile cannot start before the
+// last fragment of the one before is out of it.  Tried: the rows of the output that dK / dV's row sums need a step
+// ahead in registers (0 - 8 % slower).
 //
 // With c = lane % 16 and g = lane / 16 the layouts fit each other unchanged
 // (v_mfma_f32_16x16x32_bf16: lane supplies row c, contraction elements 8 g .. 8 g + 7; a result
@@ -16,8 +23,7 @@
 //   score tiles    two results (u = 0, 1), rows 16 u + 4 g + r of the A side: rounded to bf16,
 //                  their eight values are the B operand of a product over those 32 rows, whose
 //                  contraction element 8 g + 4 u + r is row 16 u + 4 g + r
-//   column frag.   rows 16 u + 4 g + r, elements E c .. E c + E - 1 (E = head / 16) of a head:
-//                  one load per row; tile j takes element E c + j of the lane's eight rows
+//   column frag.   tile j: element 16 j + c of rows 16 u + 4 g + r, two transposing reads of four rows
 #include "attention_common.h"
 
 using namespace jpp_attn;
@@ -34,33 +40,40 @@ struct Rows {
 #pragma unroll
     for (int t = 0; t < D / 32; ++t) v[t] = *(const bf16x8*)(p + c * ld + 32 * t + 8 * g);
   }
+  // of rows row0 .. row0 + 15 of a tile in LDS
+  __device__ __forceinline__ void read(const uint8_t* tile, int row0, int c, int g) {
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t) v[t] = *(const bf16x8*)(tile + (t >> 1) * 4096 + slab_off(row0 + c, (t & 1) * 4 + g));
+  }
 };
 
-// column fragments of 32 rows
+// column fragments of a tile in LDS
 template <int D>
 struct Cols {
-  static constexpr int E = D / 16, DW = E / 2;   // elements, dwords of a lane's piece of a row
-  uint32_t v[8][DW];
-  __device__ __forceinline__ void load(const bf16_t* p, long ld, int c, int g) {
+  bf16x8 v[D / 16];
+  __device__ __forceinline__ void read(const uint8_t* tile, int c, int g) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const bf16_t* src = p + (16 * (e >> 2) + 4 * g + (e & 3)) * ld + E * c;
-      if constexpr (DW == 4) {
-        const uint4 q = *(const uint4*)src;
-        v[e][0] = q.x; v[e][1] = q.y; v[e][2] = q.z; v[e][3] = q.w;
-      } else {
-        const uint2 q = *(const uint2*)src;
-        v[e][0] = q.x; v[e][1] = q.y;
-      }
+    for (int j = 0; j < D / 16; ++j) {
+      const int n = 16 * j + ((c & 3) << 2);
+      const uint8_t* p = tile + (n >> 6) * 4096 + slab_off(4 * g + (c >> 2), (n & 63) >> 3) + ((n & 7) << 1);
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)JPP_LDS_PTR(p));
+      const s16x4 hi =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)JPP_LDS_PTR(p + 16 * 128));
+      v[j] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
   }
-  __device__ __forceinline__ bf16x8 tile(int j) const {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const uint32_t half = j & 1 ? 0x07060302u : 0x05040100u;
-    u32x4 f;
+};
+
+// A wave's copies of 32 rows of a head (D / 64 slabs of [32][64]) into a tile of LDS of its own.
+template <int D>
+struct TileCopy {
+  using Slab = DmaTile<32, false, 1>;
+  static constexpr int BYTES = 32 * D * 2, COPIES = D / 64 * Slab::INSTS;
+  typename Slab::Offsets off;
+  __device__ __forceinline__ TileCopy(long ld, int lane) { Slab::offsets(off, ld, 0, lane); }
+  __device__ __forceinline__ void issue(const bf16_t* src, uint32_t tile) const {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) f[e] = __builtin_amdgcn_perm(v[2 * e + 1][j >> 1], v[2 * e][j >> 1], half);
-    return __builtin_bit_cast(bf16x8, f);
+    for (int q = 0; q < D / 64; ++q) Slab::template issue<0, Slab::INSTS>(uniform_ptr(src + 64 * q), off, tile + q * 4096, 0);
   }
 };
 
@@ -80,7 +93,7 @@ __device__ __forceinline__ void outer(f32x4 (&acc)[D / 16], const Cols<D>& a, co
                    pack2(s[1][2], s[1][3])};
   const bf16x8 b = __builtin_bit_cast(bf16x8, q);
 #pragma unroll
-  for (int j = 0; j < D / 16; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.tile(j), b, acc[j], 0, 0, 0);
+  for (int j = 0; j < D / 16; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v[j], b, acc[j], 0, 0, 0);
 }
 
 __device__ __forceinline__ float quad_sum(float v) {   // over the four lanes that share c
@@ -97,23 +110,18 @@ __device__ __forceinline__ void clear(f32x4 (&acc)[D / 16]) {
 // The waves' accumulators, added in wave order and scaled, to 16 rows of `out` in bf16; with
 // tables they leave rotated back (element d pairs with d + D/2; rounded to bf16 first, as a
 // separate pass would read them back from memory), row i being position pos0 + i.  Register r
-// of tile j, lane (c, g) is element E (4 g + r) + j of row c.  `buf`: W x 16 x D floats of LDS.
+// of tile j, lane (c, g) is element 16 j + 4 g + r of row c.  `buf`: W x 16 x D floats of LDS.
 template <int D>
 __device__ __forceinline__ void store_sum(const f32x4 (&acc)[D / 16], float* buf, bf16_t* out, long ld,
                                           float scale, const float* cos_tab, const float* sin_tab, int pos0) {
-  constexpr int E = D / 16, QT = E / 4;   // quads of a lane's run of E elements
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __syncthreads();   // (the waves' tiles, or what was summed before, lie there)
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int q = 0; q < QT; ++q)
-      *(f32x4*)(buf + ((wave * 4 + r) * QT + q) * 256 + lane * 4) =
-          f32x4{acc[4 * q][r], acc[4 * q + 1][r], acc[4 * q + 2][r], acc[4 * q + 3][r]};
+  for (int j = 0; j < D / 16; ++j) *(f32x4*)(buf + (wave * (D / 16) + j) * 256 + lane * 4) = acc[j];
   __syncthreads();
-  // quad k of a row: elements 4 k .. 4 k + 3 = run k / QT (g = run / 4, r = run % 4), its quad k % QT
+  // quad k of a row: elements 4 k .. 4 k + 3
   auto quad = [&](int row, int k) {
-    const int run = k / QT;
-    const float* src = buf + ((run & 3) * QT + k % QT) * 256 + ((run >> 2) * 16 + row) * 4;
+    const float* src = buf + (k * 16 + row) * 4;
     f32x4 v = *(const f32x4*)src;
 #pragma unroll
     for (int w = 1; w < W; ++w) v += *(const f32x4*)(src + w * 16 * D);
@@ -162,21 +170,30 @@ __global__ __launch_bounds__(64 * W) void attn_small_fwd_kernel(AttnParams p) {
   const int kend = CAUSAL ? q0 + 16 : p.seq;
   const bf16_t* kp = p.k + row0 * p.ldk + hk * D;
   const bf16_t* vp = p.v + row0 * p.ldv + hk * D;
+  using Copy = TileCopy<D>;
+  const Copy ck(p.ldk, lane), cv(p.ldv, lane);
+  const uint8_t* const kt = (const uint8_t*)buf + wave * (2 * Copy::BYTES);
+  const uint8_t* const vt = kt + Copy::BYTES;
+  if (wave * 32 < kend) {
+    ck.issue(kp + (long)(wave * 32) * p.ldk, lds_address(kt));
+    cv.issue(vp + (long)(wave * 32) * p.ldv, lds_address(vt));
+  }
   // Rounds of W x 32 keys.  The waves share the running maximum: the probabilities are rounded
   // to bf16 for the second product, and against a reference other than the row's maximum they
   // round differently from a plain softmax's.
   int par = 0;
   for (int r0 = 0; r0 < kend; r0 += W * 32, par ^= 1) {
-    const int k0 = r0 + wave * 32;
+    const int k0 = r0 + wave * 32, kn = k0 + W * 32;
     const bool live = k0 < kend;   // (wave-uniform)
-    Cols<D> vc;
     f32x4 s[2];
     float mx = -INFINITY;
     if (live) {
       Rows<D> kr[2];
-      kr[0].load(kp + k0 * p.ldk, p.ldk, c, g);
-      kr[1].load(kp + (k0 + 16) * p.ldk, p.ldk, c, g);
-      vc.load(vp + k0 * p.ldv, p.ldv, c, g);
+      dma_wait<Copy::COPIES>();    // K is in (copies land in order)
+      kr[0].read(kt, 0, c, g);
+      kr[1].read(kt, 16, c, g);
+      lds_wait_all();
+      if (kn < kend) ck.issue(kp + (long)kn * p.ldk, lds_address(kt));
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         s[u] = score<D>(kr[u], q);
@@ -210,6 +227,12 @@ __global__ __launch_bounds__(64 * W) void attn_small_fwd_kernel(AttnParams p) {
           s[u][r] = fast_exp2(fmaf(s[u][r], sc, neg));
           l += s[u][r];
         }
+      Cols<D> vc;
+      if (kn < kend) dma_wait<Copy::COPIES>();   // V is in; the next keys may be on their way
+      else dma_wait_all();
+      vc.read(vt, c, g);
+      lds_wait_all();
+      if (kn < kend) cv.issue(vp + (long)kn * p.ldv, lds_address(vt));
       outer<D>(o, vc, s);
     }
   }
@@ -261,23 +284,27 @@ __global__ __launch_bounds__(64 * W) void attn_small_bwd_kernel(AttnParams p, in
     clear<D>(dk);
     clear<D>(dv);
     const int first = CAUSAL ? k0 / 32 : 0, steps = p.seq / 32 - first;
+    using Copy = TileCopy<D>;
+    const Copy cq(p.ldq, lane), cg(p.lddo, lane);
+    const uint8_t* const qt = (const uint8_t*)buf + wave * (2 * Copy::BYTES);
+    const uint8_t* const gt = qt + Copy::BYTES;
+    auto copy = [&](int i) {
+      const int h = hk * grp + i / steps, q0 = (first + i % steps) * 32;
+      cq.issue(p.q + (row0 + q0) * p.ldq + h * D, lds_address(qt));
+      cg.issue(p.d_o + (row0 + q0) * p.lddo + h * D, lds_address(gt));
+    };
+    if (wave < grp * steps) copy(wave);
     for (int i = wave; i < grp * steps; i += W) {
       const int h = hk * grp + i / steps, q0 = (first + i % steps) * 32;
-      const bf16_t* qp = p.q + (row0 + q0) * p.ldq + h * D;
-      const bf16_t* gp = p.d_o + (row0 + q0) * p.lddo + h * D;
       const bf16_t* op = p.o + (row0 + q0) * p.ldo + h * D;
       const float* lp = p.lse + ((long)b * p.n_heads + h) * p.seq + q0 + 4 * g;
-      Cols<D> qc, gc;
       f32x4 s[2], ds[2];
+      dma_wait_all();
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         Rows<D> qr, gr;
-        qr.load(qp + 16 * u * p.ldq, p.ldq, c, g);
-        gr.load(gp + 16 * u * p.lddo, p.lddo, c, g);
-        if (u == 0) {
-          gc.load(gp, p.lddo, c, g);
-          qc.load(qp, p.ldq, c, g);
-        }
+        qr.read(qt, 16 * u, c, g);
+        gr.read(gt, 16 * u, c, g);
         const f32x4 lse = *(const f32x4*)(lp + 16 * u);
         const float dl = row_delta<D>(gr, op + 16 * u * p.ldo, p.ldo, c, g);
         s[u] = score<D>(qr, kr);
@@ -290,11 +317,15 @@ __global__ __launch_bounds__(64 * W) void attn_small_bwd_kernel(AttnParams p, in
           ds[u][r] = pr * (ds[u][r] - __shfl(dl, 4 * g + r));
         }
       }
+      Cols<D> qc, gc;
+      gc.read(gt, c, g);
+      qc.read(qt, c, g);
+      lds_wait_all();
+      if (i + W < grp * steps) copy(i + W);
       outer<D>(dv, gc, s);
       outer<D>(dk, qc, ds);
     }
     store_sum<D>(dv, buf, p.dv + (row0 + k0) * p.lddv + hk * D, p.lddv, 1.0f, nullptr, nullptr, 0);
-    __syncthreads();
     store_sum<D>(dk, buf, p.dk + (row0 + k0) * p.lddk + hk * D, p.lddk, p.scale, p.rope_cos, p.rope_sin, k0);
     return;
   }
@@ -312,19 +343,24 @@ __global__ __launch_bounds__(64 * W) void attn_small_bwd_kernel(AttnParams p, in
   const int kend = CAUSAL ? q0 + 16 : p.seq;
   const bf16_t* kp = p.k + row0 * p.ldk + hk * D;
   const bf16_t* vp = p.v + row0 * p.ldv + hk * D;
+  using Copy = TileCopy<D>;
+  const Copy ck(p.ldk, lane), cv(p.ldv, lane);
+  const uint8_t* const kt = (const uint8_t*)buf + wave * (2 * Copy::BYTES);
+  const uint8_t* const vt = kt + Copy::BYTES;
+  auto copy = [&](int k0) {
+    ck.issue(kp + (long)k0 * p.ldk, lds_address(kt));
+    cv.issue(vp + (long)k0 * p.ldv, lds_address(vt));
+  };
+  if (wave * 32 < kend) copy(wave * 32);
   for (int k0 = wave * 32; k0 < kend; k0 += W * 32) {
-    Rows<D> kr[2], vr[2];
-    Cols<D> kc;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      kr[u].load(kp + (k0 + 16 * u) * p.ldk, p.ldk, c, g);
-      vr[u].load(vp + (k0 + 16 * u) * p.ldv, p.ldv, c, g);
-    }
-    kc.load(kp + k0 * p.ldk, p.ldk, c, g);
+    dma_wait_all();
     f32x4 ds[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const f32x4 s = score<D>(kr[u], q), dp = score<D>(vr[u], go);
+      Rows<D> kr, vr;
+      kr.read(kt, 16 * u, c, g);
+      vr.read(vt, 16 * u, c, g);
+      const f32x4 s = score<D>(kr, q), dp = score<D>(vr, go);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float pr = fast_exp2(fmaf(s[r], sc, -lse2));
@@ -332,17 +368,28 @@ __global__ __launch_bounds__(64 * W) void attn_small_bwd_kernel(AttnParams p, in
         ds[u][r] = pr * (dp[r] - dl);
       }
     }
+    Cols<D> kc;
+    kc.read(kt, c, g);
+    lds_wait_all();
+    if (k0 + W * 32 < kend) copy(k0 + W * 32);
     outer<D>(dq, kc, ds);
   }
   store_sum<D>(dq, buf, p.dq + (row0 + q0) * p.lddq + h * D, p.lddq, p.scale, p.rope_cos, p.rope_sin, q0);
 }
 
+// a tile of either operand per wave, over them the sums of 16 rows
+template <int D>
+constexpr int small_smem() {
+  return W * 2 * TileCopy<D>::BYTES;
+}
+static_assert(small_smem<64>() >= W * 16 * 64 * 4 && small_smem<128>() >= W * 16 * 128 * 4, "room for the sums");
+
 template <int D, bool CAUSAL>
 int fwd(hipStream_t st, const AttnParams& p) {
-  if (int rc = set_smem(attn_small_fwd_kernel<D, CAUSAL>, W * 16 * D * 4)) return rc;
+  if (int rc = set_smem(attn_small_fwd_kernel<D, CAUSAL>, small_smem<D>())) return rc;
   hipLaunchKernelGGL((attn_small_fwd_kernel<D, CAUSAL>),
                      dim3((unsigned)p.n_heads, (unsigned)(p.seq / 16), (unsigned)p.batch), dim3(64 * W),
-                     W * 16 * D * 4, st, p);
+                     small_smem<D>(), st, p);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
@@ -350,9 +397,9 @@ int fwd(hipStream_t st, const AttnParams& p) {
 template <int D, bool CAUSAL>
 int bwd(hipStream_t st, const AttnParams& p) {
   const int kv = p.seq / 16 * p.n_kv_heads * p.batch, q = p.seq / 16 * p.n_heads * p.batch;
-  if (int rc = set_smem(attn_small_bwd_kernel<D, CAUSAL>, W * 16 * D * 4)) return rc;
+  if (int rc = set_smem(attn_small_bwd_kernel<D, CAUSAL>, small_smem<D>())) return rc;
   hipLaunchKernelGGL((attn_small_bwd_kernel<D, CAUSAL>), dim3((unsigned)(kv + q)), dim3(64 * W),
-                     W * 16 * D * 4, st, p, kv);
+                     small_smem<D>(), st, p, kv);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
