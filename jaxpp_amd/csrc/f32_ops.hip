@@ -7,6 +7,7 @@
 // fp32 arithmetic throughout, the contractions on the fp32 matrix instruction, every sum in an
 // order that the shapes fix.
 #include <math.h>
+#include <string.h>
 
 #include <mutex>
 
@@ -133,7 +134,7 @@ constexpr int kStages32 = BM == 16 ? 3 : 2;   // (what fits beside the sums)
 // on average).  (A 32-element step is 128 bytes a row:
 // the LDS image is that of a bf16 tile of 64.)
 template <int BM, bool TA, bool TB, bool STAGED>
-__global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
+__device__ __forceinline__ void sgemm_tile(SgemmParams p, int blk) {
   constexpr int TM = BM / 16, TN = 4, D = BM == 64 ? 2 : 4, PITCH = 68;
   static_assert(!STAGED || (!TA && !TB && BM <= 32), "staged: both operands [rows][k], two tiles' LDS");
   extern __shared__ __align__(1024) uint8_t smem[];   // (STAGED) [4 waves][stages][BM + 64 rows of 128 bytes]
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tiles_n = p.n / 64;
-  const long m0 = (long)(blockIdx.x / tiles_n) * BM, n0 = (long)(blockIdx.x % tiles_n) * 64;
+  const long m0 = (long)(blk / tiles_n) * BM, n0 = (long)(blk % tiles_n) * 64;
   if (p.group_mode == JPP_GROUP_M) {
     // rows of A and C are grouped by expert; each group multiplies its own B
     if (m0 >= p.seg[p.n_seg]) return;
@@ -321,6 +322,11 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
   }
 }
 
+template <int BM, bool TA, bool TB, bool STAGED>
+__global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
+  sgemm_tile<BM, TA, TB, STAGED>(p, blockIdx.x);
+}
+
 template <int BM>
 int sgemm_launch(hipStream_t st, const SgemmParams& p) {
   const dim3 grid((unsigned)(p.m / BM * (p.n / 64)), 1u, p.group_mode == JPP_GROUP_K ? (unsigned)p.n_seg : 1u);
@@ -385,42 +391,45 @@ __global__ __launch_bounds__(256) void norm_fwd32_kernel(const float* __restrict
   }
 }
 
-// Column sums of 16 adjacent columns over all rows by one workgroup of 1024 threads: thread
-// (rg, c) = (tid / 16, tid % 16) adds rows rg, rg + 64, ... of column c, the 64 sums of a column
-// meet first inside a wave (4 of them), then in wave order.  These sums are latency and nothing
+// Column sums of 16 adjacent columns over all rows by one workgroup of NT threads: 64 sums a column, sum rg
+// over rows rg, rg + 64, ..., NT / 16 of them at a time; four adjacent ones meet first inside a wave, then the 16
+// fours in order (whatever NT, the same sums).  These sums are latency and nothing
 // else: one thread per column walks its rows one load after another, 4 to 16 waves on the whole
 // device.  Spread like this a thread's loads are in flight together: the four bias gradients of
 // a layer of hidden 256 on 512 tokens 4.8 us in one launch, a norm's backward 4.9 us.
 struct ColSum {
   float a, b;
 };
-template <typename Load>
+template <int NT, typename Load>
 __device__ __forceinline__ ColSum column_sums(long rows, Load load) {
   __shared__ ColSum red[16][16];
   const int tid = threadIdx.x, c = tid & 15, wave = tid >> 6;
-  ColSum s = {0.f, 0.f};
-  long r = tid >> 4;
-  for (; r + 7 * 64 < rows; r += 8 * 64) {
-    ColSum v[8];
+#pragma unroll 1
+  for (int part = 0; part < 1024 / NT; ++part) {
+    ColSum s = {0.f, 0.f};
+    long r = (tid >> 4) + part * (NT / 16);
+    for (; r + 7 * 64 < rows; r += 8 * 64) {
+      ColSum v[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = load(r + i * 64);
+      for (int i = 0; i < 8; ++i) v[i] = load(r + i * 64);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      s.a += v[i].a;
-      s.b += v[i].b;
+      for (int i = 0; i < 8; ++i) {
+        s.a += v[i].a;
+        s.b += v[i].b;
+      }
     }
-  }
-  for (; r < rows; r += 64) {
-    const ColSum v = load(r);
-    s.a += v.a;
-    s.b += v.b;
-  }
+    for (; r < rows; r += 64) {
+      const ColSum v = load(r);
+      s.a += v.a;
+      s.b += v.b;
+    }
 #pragma unroll
-  for (int o = 16; o < 64; o <<= 1) {
-    s.a += __shfl_xor(s.a, o);
-    s.b += __shfl_xor(s.b, o);
+    for (int o = 16; o < 64; o <<= 1) {
+      s.a += __shfl_xor(s.a, o);
+      s.b += __shfl_xor(s.b, o);
+    }
+    if ((tid & 63) < 16) red[wave + part * (NT / 64)][c] = s;
   }
-  if ((tid & 63) < 16) red[wave][c] = s;
   __syncthreads();
   ColSum t = {0.f, 0.f};
   if (tid < 16)
@@ -446,7 +455,7 @@ __global__ __launch_bounds__(1024) void norm_bwd32_kernel(const float* __restric
   if ((int)blockIdx.x >= row_blocks) {
     const int col = ((int)blockIdx.x - row_blocks) * 16 + (threadIdx.x & 15);
     const bool in = col < cols;
-    const ColSum s = column_sums(in ? rows : 0, [&](long r) {
+    const ColSum s = column_sums<1024>(in ? rows : 0, [&](long r) {
       const float d = dy[r * cols + col];
       const float mean = mean_in ? mean_in[r] : 0.f;
       return ColSum{d * (x[r * cols + col] - mean) * rstd_in[r], d};
@@ -487,8 +496,8 @@ struct ColItems32 {
   long ld[4];
   int cols[4], first[4];
 };
-__global__ __launch_bounds__(1024) void colsum32_kernel(ColItems32 p, long rows) {
-  const int blk = blockIdx.x;
+template <int NT>
+__device__ __forceinline__ void colsum_block(const ColItems32& p, int blk, long rows) {
   const bool s1 = blk >= p.first[1], s2 = blk >= p.first[2], s3 = blk >= p.first[3];
 #define JPP_PICK(field) (s3 ? p.field[3] : s2 ? p.field[2] : s1 ? p.field[1] : p.field[0])
   const float* const x = JPP_PICK(x);
@@ -497,8 +506,46 @@ __global__ __launch_bounds__(1024) void colsum32_kernel(ColItems32 p, long rows)
   const int cols = JPP_PICK(cols), col = (blk - JPP_PICK(first)) * 16 + (threadIdx.x & 15);
 #undef JPP_PICK
   const bool in = col < cols;
-  const ColSum s = column_sums(in ? rows : 0, [&](long r) { return ColSum{x[r * ld + col], 0.f}; });
+  const ColSum s = column_sums<NT>(in ? rows : 0, [&](long r) { return ColSum{x[r * ld + col], 0.f}; });
   if (threadIdx.x < 16 && in) acc[col] += s.a;
+}
+__global__ __launch_bounds__(1024) void colsum32_kernel(ColItems32 p, long rows) {
+  colsum_block<1024>(p, blockIdx.x, rows);
+}
+
+// A layer's weight gradients, up to four products C_i += A_i^T B_i over the same rows, and its bias gradients,
+// column sums over them, in one launch: workgroups first[i] .. first[i + 1] - 1 take product i, those from
+// col_first on the sums.  Apart, each fills a part of the device and is mostly latency: a layer of hidden 256 on
+// 512 tokens 31 us in five launches, 19 in one.
+struct SgemmWgrads {
+  SgemmParams p;        // what they share, and product 0
+  const float* a[4];
+  const float* b[4];
+  float* c[4];
+  long lda[4], ldb[4], ldc[4];
+  int n[4], first[4], col_first;
+  ColItems32 cols;
+};
+template <int BM>
+__global__ __launch_bounds__(256) void sgemm_wgrads_kernel(SgemmWgrads w) {
+  const int blk = blockIdx.x;
+  if (blk >= w.col_first) {
+    colsum_block<256>(w.cols, blk - w.col_first, w.p.k);
+    return;
+  }
+  const bool s1 = blk >= w.first[1], s2 = blk >= w.first[2], s3 = blk >= w.first[3];
+#define JPP_PICK(field) (s3 ? w.field[3] : s2 ? w.field[2] : s1 ? w.field[1] : w.field[0])
+  SgemmParams p = w.p;
+  p.a = JPP_PICK(a);
+  p.b = JPP_PICK(b);
+  p.c = JPP_PICK(c);
+  p.lda = JPP_PICK(lda);
+  p.ldb = JPP_PICK(ldb);
+  p.ldc = JPP_PICK(ldc);
+  p.n = JPP_PICK(n);
+  const int first = JPP_PICK(first);
+#undef JPP_PICK
+  sgemm_tile<BM, true, true, false>(p, blk - first);
 }
 
 // loss = scale * mean((out - target)^2), dout = scale * 2 (out - target) / count: one
@@ -844,9 +891,7 @@ int attn_check(const jpp_attn_args* a, const char* who, Attn32& p) {
 
 }  // namespace
 
-int jpp_colsum_f32_items(hipStream_t stream, int n, const jpp_colsum_item* items, int64_t rows) {
-  JPP_REQUIRE(n >= 1 && n <= 4, "colsum_f32: 1 to 4 matrices");
-  ColItems32 p;
+static int column_items(ColItems32& p, int n, const jpp_colsum_item* items) {
   int blocks = 0;
   for (int i = 0; i < 4; ++i) {
     const jpp_colsum_item& q = items[i < n ? i : 0];
@@ -857,7 +902,47 @@ int jpp_colsum_f32_items(hipStream_t stream, int n, const jpp_colsum_item* items
     p.first[i] = i < n ? blocks : 0x7fffffff;
     if (i < n) blocks += (int)((q.cols + 15) / 16);
   }
+  return blocks;
+}
+
+int jpp_colsum_f32_items(hipStream_t stream, int n, const jpp_colsum_item* items, int64_t rows) {
+  JPP_REQUIRE(n >= 1 && n <= 4, "colsum_f32: 1 to 4 matrices");
+  ColItems32 p;
+  const int blocks = column_items(p, n, items);
   hipLaunchKernelGGL(colsum32_kernel, dim3((unsigned)blocks), dim3(1024), 0, stream, p, (long)rows);
+  JPP_LAUNCH_CHECK();
+  return JPP_OK;
+}
+
+int jpp_wgrads_f32(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols, const jpp_colsum_item* items) {
+  JPP_REQUIRE(n >= 1 && n <= 4 && n_cols >= 0 && n_cols <= 4, "wgrads_f32: 1 to 4 products, up to 4 column sums");
+  SgemmWgrads w;
+  memset(&w, 0, sizeof(w));
+  long strips = 0;
+  for (int i = 0; i < 4; ++i) {
+    const jpp_gemm_args& q = g[i < n ? i : 0];
+    JPP_REQUIRE(q.k_parts <= 1 && q.k == g[0].k && q.k > 0 && q.m > 0 && q.n > 0 && q.m % 64 == 0 && q.n % 64 == 0 && q.k % 16 == 0 && q.lda >= q.m && q.ldb >= q.n &&
+                    q.ldc >= q.n, "wgrads_f32: product %d has a shape of its own or a bad one", i);
+    w.a[i] = (const float*)q.a; w.b[i] = (const float*)q.b; w.c[i] = (float*)q.c;
+    w.lda[i] = q.lda; w.ldb[i] = q.ldb; w.ldc[i] = q.ldc; w.n[i] = (int)q.n;
+    if (i < n) strips += (q.m / 16) * (q.n / 64);
+  }
+  w.p.k = (int)g[0].k;
+  w.p.ta = w.p.tb = 1;
+  w.p.epi = JPP_EPI_ACC_F32;
+  // 64-row tiles from a tile for every other CU on (a layer of hidden 256, 192 of them: 18.7 us, 32 rows 21.9,
+  // 16 rows 21.3): both operands' columns are read once per tile, and the narrow ones' loads repeat more
+  const int bm = strips >= 2 * 256 ? 64 : strips >= 256 ? 32 : 16;
+  int blocks = 0;
+  for (int i = 0; i < 4; ++i) {
+    w.first[i] = i < n ? blocks : 0x7fffffff;
+    if (i < n) blocks += (int)(g[i].m / bm * (g[i].n / 64));
+  }
+  w.col_first = blocks;
+  if (n_cols) blocks += column_items(w.cols, n_cols, items);
+  if (bm == 64) hipLaunchKernelGGL(sgemm_wgrads_kernel<64>, dim3((unsigned)blocks), dim3(256), 0, stream, w);
+  else if (bm == 32) hipLaunchKernelGGL(sgemm_wgrads_kernel<32>, dim3((unsigned)blocks), dim3(256), 0, stream, w);
+  else hipLaunchKernelGGL(sgemm_wgrads_kernel<16>, dim3((unsigned)blocks), dim3(256), 0, stream, w);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }

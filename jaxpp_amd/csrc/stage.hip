@@ -197,16 +197,27 @@ int attn_b(jpp_stage* s, hipStream_t st, const jpp_attn_args* a) {
   return s->f32() ? jpp_attn_bwd_f32(st, a) : jpp_attn_bwd(st, a);
 }
 
-// a layer's four bias gradients: column sums of the cotangents, added to the accumulators
-int bias_grads4(jpp_stage* s, hipStream_t st, const jpp_colsum_item* items, float* partial) {
+// A layer's four bias gradients that its input-gradient half has left to the weight-gradient half behind it.
+struct BiasGrads {
+  jpp_colsum_item item[4];
+  bool pending = false;
+};
+
+// a layer's four bias gradients: column sums of the cotangents, added to the accumulators (in f32 by `later`, if
+// given, beside the weight gradients of the same rows)
+int bias_grads4(jpp_stage* s, hipStream_t st, const jpp_colsum_item* items, float* partial, BiasGrads* later) {
+  if (later && s->f32()) {
+    std::copy(items, items + 4, later->item);
+    later->pending = true;
+    return JPP_OK;
+  }
   return s->f32() ? jpp_colsum_f32_items(st, 4, items, s->T)
                   : jpp_colsum_accum_multi(st, 4, items, s->T, partial);
 }
 
-// dW[rows, cols] (+)= X^T dY, X: [T, rows], dY: [T, cols]
+// dW[rows, cols] (+)= X^T dY (bf16), X: [T, rows], dY: [T, cols]
 int wgrad(jpp_stage* s, hipStream_t st, const void* x, int64_t ldx, const void* dy, int64_t lddy,
           float* acc, int64_t rows, int64_t cols) {
-  if (s->f32()) return gemm(s, st, x, ldx, 1, dy, lddy, 1, acc, cols, rows, cols, s->T, JPP_EPI_ACC_F32);
   if (s->d.fused_wgrad_accum)
     return gemm(s, st, x, ldx, 1, dy, lddy, 1, acc, cols, rows, cols, s->T, JPP_EPI_ACC_F32);
   void* g = s->S<>(s->s_wg);
@@ -219,7 +230,7 @@ int wgrad(jpp_stage* s, hipStream_t st, const void* x, int64_t ldx, const void* 
 int wgrad_n(jpp_stage* s, hipStream_t st, int n, const void* const* xs, int64_t ldx,
             const void* const* dys, int64_t lddy, float* acc, int64_t rows, int64_t cols) {
   const bool big = rows % 256 == 0 && cols % 256 == 0 && (rows / 256) * (cols / 256) >= 192;
-  if (n == 1 || !big || s->f32() || !s->d.fused_wgrad_accum) {
+  if (n == 1 || !big || !s->d.fused_wgrad_accum) {
     for (int i = 0; i < n; ++i) RC(wgrad(s, st, xs[i], ldx, dys[i], lddy, acc, rows, cols));
     return JPP_OK;
   }
@@ -237,6 +248,7 @@ int wgrad_n(jpp_stage* s, hipStream_t st, int n, const void* const* xs, int64_t 
 struct WgradBatch {
   jpp_gemm_args g[4];
   int n = 0;
+  const BiasGrads* bias = nullptr;   // to leave with them
   void add(jpp_stage* s, int pairs, const void* const* xs, int64_t ldx, const void* const* dys,
            int64_t lddy, float* acc, int64_t rows, int64_t cols) {
     jpp_gemm_args& q = g[n++];
@@ -278,6 +290,8 @@ int run_apart(jpp_stage* s, hipStream_t st, const jpp_gemm_args& q) {
 // Which way is taken depends on the shapes only.
 int run_wgrads(jpp_stage* s, hipStream_t st, WgradBatch& w) {
   constexpr long kFullGrid = 192;
+  // (f32: one microbatch's at a time)
+  if (s->f32()) return jpp_wgrads_f32(st, w.n, w.g, w.bias ? 4 : 0, w.bias ? w.bias->item : nullptr);
   bool whole = true, full[4] = {};
   long total = 0;
   double apart = 0;
@@ -292,7 +306,7 @@ int run_wgrads(jpp_stage* s, hipStream_t st, WgradBatch& w) {
     apart += (double)(t / 256) + (rest == 0 ? 0.0 : (rest <= 128 && t > 256 ? 0.77 : 1.0));
   }
   const bool one_grid = total < kFullGrid || (double)((total + 255) / 256) < apart - 0.25;
-  const bool may_gather = !s->f32() && s->d.fused_wgrad_accum && (!whole || one_grid);
+  const bool may_gather = s->d.fused_wgrad_accum && (!whole || one_grid);
   jpp_gemm_args grid[4];
   int n = 0;
   for (int i = 0; i < w.n; ++i)
@@ -457,8 +471,9 @@ int layer_fwd(jpp_stage* s, hipStream_t st, int chunk, int li, uint8_t* slot, vo
 // ---- one layer, input-gradient half -------------------------------------------
 // `w` holds the cotangents the weight-gradient half will read: the slot itself
 // when the backward is split, the shared scratch set otherwise.
+// With `later` the bias gradients are left to it where they can ride with the weight gradients.
 int layer_bwd_i(jpp_stage* s, hipStream_t st, int chunk, int li, uint8_t* slot, uint8_t* wbase,
-                const LayerStash& W, const void* dy, void* dx) {
+                const LayerStash& W, const void* dy, void* dx, BiasGrads* later) {
   const LayerStash& L = s->lay[li];
   const int64_t T = s->T, h = s->h, f = s->f;
   auto at = [&](const Buf& b) { return (void*)(slot + b.off); };
@@ -492,7 +507,7 @@ int layer_bwd_i(jpp_stage* s, hipStream_t st, int chunk, int li, uint8_t* slot, 
                                            {wt(W.du), f, f, s->G(chunk, li, B_b1)},
                                            {wt(W.da), h, h, s->G(chunk, li, B_bo)},
                                            {dqkv, 3 * h, 3 * h, s->G(chunk, li, B_bqkv)}};
-    RC(bias_grads4(s, st, bias_grads, partial));
+    RC(bias_grads4(s, st, bias_grads, partial, later));
     return JPP_OK;
   }
   void* dn = s->S<>(s->s_t2);   // dn2, later dn1
@@ -521,7 +536,7 @@ int layer_bwd_i(jpp_stage* s, hipStream_t st, int chunk, int li, uint8_t* slot, 
                                            {wt(W.du), f, f, s->G(chunk, li, B_b1)},
                                            {wt(W.dh1), h, h, s->G(chunk, li, B_bo)},
                                            {dqkv, 3 * h, 3 * h, s->G(chunk, li, B_bqkv)}};
-    RC(bias_grads4(s, st, bias_grads, partial));
+    RC(bias_grads4(s, st, bias_grads, partial, later));
     return JPP_OK;
   }
   // llama
@@ -572,7 +587,7 @@ int layer_bwd_i(jpp_stage* s, hipStream_t st, int chunk, int li, uint8_t* slot, 
 
 // ---- one layer, weight-gradient half --------------------------------------------
 int layer_bwd_w(jpp_stage* s, hipStream_t st, int chunk, int li, uint8_t* slot, uint8_t* wbase,
-                const LayerStash& W, const void* dy) {
+                const LayerStash& W, const void* dy, const BiasGrads* bias = nullptr) {
   // scratch for partial sums: the second stream has its own
   float* partial = s->S<float>(st == s->side && s->side ? s->s_partial_side : s->s_partial);
   const LayerStash& L = s->lay[li];
@@ -580,6 +595,7 @@ int layer_bwd_w(jpp_stage* s, hipStream_t st, int chunk, int li, uint8_t* slot, 
   auto at = [&](const Buf& b) { return (void*)(slot + b.off); };
   auto wt = [&](const Buf& b) { return (void*)(wbase + b.off); };
   WgradBatch wb;
+  if (bias && bias->pending) wb.bias = bias;
   if (s->d.family == JPP_FAMILY_BERT) {
     wb.add1(s, at(L.g), f, wt(W.dc), h, s->G(chunk, li, B_W2), f, h);
     wb.add1(s, at(L.x1), h, wt(W.du), f, s->G(chunk, li, B_W1), h, f);
@@ -1282,7 +1298,9 @@ int jpp_stage_run_task(jpp_stage* s, int kind, int chunk, int mb, const void* in
         JPP_CHECK_HIP(hipMemcpyAsync(keep, in, act, hipMemcpyDeviceToDevice, st));
         dy = keep;
       }
-      RC(layer_bwd_i(s, st, chunk, li, slot, wbase, W, dy, dx));
+      // (the halves run back to back on one stream: the bias gradients may go with the second)
+      BiasGrads bias;
+      RC(layer_bwd_i(s, st, chunk, li, slot, wbase, W, dy, dx, kind == JPP_BWD && s->wg == 1 && !two ? &bias : nullptr));
       if (kind == JPP_BWD && s->wg == 1) {
         if (two) {
           RC(fork());
@@ -1292,7 +1310,7 @@ int jpp_stage_run_task(jpp_stage* s, int kind, int chunk, int mb, const void* in
             s->set_pending[set_of(li)] = true;
           }
         } else {
-          RC(layer_bwd_w(s, st, chunk, li, slot, wbase, W, dy));
+          RC(layer_bwd_w(s, st, chunk, li, slot, wbase, W, dy, &bias));
         }
       }
       dy = dx;

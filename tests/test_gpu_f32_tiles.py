@@ -10,7 +10,12 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import parity
 from jaxpp_amd import runtime as rt
+from jaxpp_amd import schedules as S
+from jaxpp_amd.model import LayerSpec, init_layer_params
+from jaxpp_amd.plan import make_rank_plan
+from test_gpu_stage import run_on_gpu, run_on_oracle
 
 pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
@@ -141,3 +146,25 @@ def test_attention_f32_tiles(d, hq, hk, seq, causal):
         assert np.abs(buf.download(np.float32, w.shape) - w).max() <= 1e-5 * np.abs(w).max(), name
     w = (mx + np.log(e.sum(-1, keepdims=True)))[..., 0]
     assert np.abs(lse.download(np.float32, w.shape) - w).max() <= 1e-5 * np.abs(w).max()
+
+
+# 16 x 64 strips of a layer's weight gradients: 128 (16-row tiles), 384 (32), 768 and more (64), 400 (32)
+@pytest.mark.parametrize("family,h,heads,f,seq", [
+    ("bert", 128, 2, 256, 128), ("bert", 256, 4, 256, 256), ("bert", 256, 4, 1024, 384),
+    ("decoder", 384, 6, 640, 128), ("llama", 256, 4, 128, 128)])
+def test_layer_weight_and_bias_gradients_in_one_launch_f32(family, h, heads, f, seq):
+    """On one stream a layer's bias gradients go with its weight gradients, on two they go before them: the same
+    sums, whichever launch adds them up, and those of the oracle."""
+    print(f"wgrads_f32 {family} {h} {f} {seq}", flush=True)
+    spec = LayerSpec(family, h, heads, f, seq, 1, n_kv_heads=heads, head_dim=64, causal=family != "bert", eps=1e-5,
+                     dtype="f32")
+    sched = S.Std1F1B(1)
+    plan = make_rank_plan(sched, 2, 0)
+    params = {0: [init_layer_params(spec, 3, li, perturb=True) for li in range(2)]}
+    _, _, apart = run_on_gpu(spec, plan, 2, params, two_streams=True)
+    _, _, here = run_on_gpu(spec, plan, 2, params, two_streams=False)
+    _, _, want = run_on_oracle(spec, plan, params, S.preprocess_schedule_tasks(sched.tasks(2), 0, False)[0])
+    for li in range(2):
+        for name, w in want[0][li].items():
+            assert np.array_equal(here[0][li][name], apart[0][li][name]), name
+            parity.close(here[0][li][name], w.reshape(here[0][li][name].shape).astype(np.float64), 1e-4, name)
