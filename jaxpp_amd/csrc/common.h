@@ -62,6 +62,10 @@ int jpp_colsum_f32_items(hipStream_t stream, int n, const jpp_colsum_item* items
 // up to four accumulated weight gradients of the same k rows (plain ones: trans_a = trans_b = 1,
 // JPP_EPI_ACC_F32) and the column sums over those rows of up to four matrices, in one launch (f32_ops.hip)
 int jpp_wgrads_f32(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols, const jpp_colsum_item* items);
+// jpp_gemm_bf16_multi and jpp_colsum_accum_multi over the same rows, in one launch where the products take small
+// tiles and the rows are few (gemm.hip)
+int jpp_wgrads_bf16(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols, const jpp_colsum_item* items,
+                    int64_t rows, float* partial);
 
 // -- bf16 <-> f32 -------------------------------------------------------------
 __device__ __forceinline__ float bf16_to_f32(bf16_t b) {

@@ -10,6 +10,7 @@
 
 #include <type_traits>
 
+#include "colsum.h"
 #include "common.h"
 
 // Scratch of jpp_norm_bwd_static (the entry point that allocates nothing): the per-block
@@ -450,75 +451,11 @@ __global__ __launch_bounds__(1024) void colsum_multi_reduce_kernel(const float* 
 // Few rows: column sums by one workgroup per 64 columns, without partial sums in memory.
 // Two launches over 256 blocks of rows, the second adding up what the first left, are two
 // launches' latency and 256 x columns floats on the way between them, which at a few hundred
-// rows is more than the tensors themselves.  A thread owns 8 columns of every (NT / 8)-th row; the
-// row groups of a column meet inside a wave first, then in wave order.
+// rows is more than the tensors themselves.
 // ---------------------------------------------------------------------------
-// Sums over `rows` of load(r, a, b), which adds 8 columns of row r into a (and b), for 64
-// adjacent columns; thread t < 64 returns column t's two sums.
-template <int NT, int UNROLL, class Load>
-__device__ __forceinline__ float2 column_sums64(long rows, Load load) {
-  __shared__ float2 red[NT / 64][64];
-  constexpr int G = NT / 8;
-  const int tid = threadIdx.x;
-  float a[8], b[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) a[e] = b[e] = 0.f;
-  long r = tid >> 3;
-  for (; r + (UNROLL - 1) * G < rows; r += UNROLL * G) load(r, G, std::integral_constant<int, UNROLL>{}, a, b);
-  for (; r < rows; r += G) load(r, G, std::integral_constant<int, 1>{}, a, b);
-#pragma unroll
-  for (int o = 8; o < 64; o <<= 1)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      a[e] += __shfl_xor(a[e], o);
-      b[e] += __shfl_xor(b[e], o);
-    }
-  if ((tid & 63) < 8)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) red[tid >> 6][(tid & 7) * 8 + e] = make_float2(a[e], b[e]);
-  __syncthreads();
-  float2 t = make_float2(0.f, 0.f);
-  if (tid < 64)
-#pragma unroll
-    for (int w = 0; w < NT / 64; ++w) {
-      t.x += red[w][tid].x;
-      t.y += red[w][tid].y;
-    }
-  return t;
-}
-
-// the bias gradients of a layer: workgroups first[i] .. first[i + 1] - 1 take tensor i
-struct ColsumPanels {
-  ColsumBatch b;
-  int first[4];
-};
 __global__ __launch_bounds__(1024) void colsum_few_rows_kernel(ColsumPanels p, long rows) {
-  const int blk = blockIdx.x;
-  const bool s1 = blk >= p.first[1], s2 = blk >= p.first[2], s3 = blk >= p.first[3];
-#define JPP_PICK(f) (s3 ? f[3] : s2 ? f[2] : s1 ? f[1] : f[0])
-  const bf16_t* const x = JPP_PICK(p.b.x);
-  const long ld = JPP_PICK(p.b.ld);
-  float* const acc = JPP_PICK(p.b.acc);
-  const int c0 = (blk - JPP_PICK(p.first)) * 64;
-  const int cols = s3 ? p.b.start[4] - p.b.start[3] : s2 ? p.b.start[3] - p.b.start[2]
-                   : s1 ? p.b.start[2] - p.b.start[1] : p.b.start[1];
-#undef JPP_PICK
-  const int c = c0 + (threadIdx.x & 7) * 8;
-  const bf16_t* src = x + c;
-  const float2 t = column_sums64<1024, 8>(c < cols ? rows : 0, [&](long r, int g, auto u, float (&a)[8], float (&)[8]) {
-    constexpr int U = decltype(u)::value;
-    uint4 v[U];
-#pragma unroll
-    for (int i = 0; i < U; ++i) v[i] = *(const uint4*)(src + (r + i * g) * ld);
-#pragma unroll
-    for (int i = 0; i < U; ++i) {
-      float f[8];
-      unpack8(v[i], f);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) a[e] += f[e];
-    }
-  });
-  if (threadIdx.x < 64 && c0 + (int)threadIdx.x < cols) acc[c0 + threadIdx.x] += t.x;
+  __shared__ float2 red[16][64];
+  colsum_panel<1024>(p, blockIdx.x, rows, red);
 }
 
 // A norm's whole backward in one launch: the first row_blocks workgroups take NT / 64 rows each, a
@@ -532,7 +469,8 @@ __global__ __launch_bounds__(kFewRowsThreads) void norm_bwd_few_rows_kernel(
     bf16_t* dx, float* dgamma, float* dbeta, long rows, int cols, int row_blocks) {
   if ((int)blockIdx.x >= row_blocks) {
     const int c0 = ((int)blockIdx.x - row_blocks) * 64, c = c0 + (threadIdx.x & 7) * 8;
-    const float2 t = column_sums64<kFewRowsThreads, 8>(c < cols ? rows : 0, [&](long r, int g, auto u, float (&a)[8], float (&b)[8]) {
+    __shared__ float2 red[kFewRowsThreads / 64][64];
+    const float2 t = column_sums64<kFewRowsThreads, 8, 1>(c < cols ? rows : 0, red, [&](long r, int g, auto u, float (&a)[8], float (&b)[8]) {
       constexpr int U = decltype(u)::value;
       uint4 vd[U], vx[U];
       float mean[U], rstd[U];
@@ -889,6 +827,25 @@ int launch_norm_bwd(hipStream_t st, const jpp_norm_args* a) {
 
 }  // namespace
 
+int colsum_panels(int n, const jpp_colsum_item* items, int64_t rows, ColsumPanels* p, int* blocks) {
+  JPP_REQUIRE(items && n >= 1 && n <= 4 && rows > 0, "colsum_multi: 1 to 4 tensors are required");
+  *blocks = 0;
+  for (int i = 0; i < 4; ++i) {
+    const jpp_colsum_item& it = items[i < n ? i : 0];
+    JPP_REQUIRE(it.x && it.acc && it.cols > 0 && it.cols % 8 == 0 && it.ld % 8 == 0 &&
+                    it.ld >= it.cols && (uintptr_t)it.x % 16 == 0,
+                "colsum_multi: tensor %d: cols and ld must be multiples of 8, ld >= cols", i);
+    p->x[i] = (const bf16_t*)it.x;
+    p->ld[i] = it.ld;
+    p->acc[i] = it.acc;
+    p->cols[i] = (int)it.cols;
+    p->first[i] = i < n ? *blocks : 0x7fffffff;
+    if (i < n) *blocks += (int)((it.cols + 63) / 64);
+  }
+  if (rows > kColsumFewRows) *blocks = 0;
+  return JPP_OK;
+}
+
 extern "C" {
 
 int jpp_norm_fwd(void* stream, const jpp_norm_args* a) {
@@ -1029,40 +986,30 @@ int jpp_sum_accum_f32(void* stream, float* acc, const float* parts, int n_parts,
 
 int jpp_colsum_accum_multi(void* stream, int n, const jpp_colsum_item* items, int64_t rows,
                            float* partial) {
-  JPP_REQUIRE(items && partial && n >= 1 && n <= 4 && rows > 0,
-              "colsum_multi: 1 to 4 tensors and a partial-sum buffer are required");
-  ColsumBatch b;
-  b.n = n;
-  int at = 0;
-  double bytes = 0;
-  for (int i = 0; i < n; ++i) {
-    const jpp_colsum_item& it = items[i];
-    JPP_REQUIRE(it.x && it.acc && it.cols > 0 && it.cols % 8 == 0 && it.ld % 8 == 0 &&
-                    it.ld >= it.cols && (uintptr_t)it.x % 16 == 0,
-                "colsum_multi: tensor %d: cols and ld must be multiples of 8, ld >= cols", i);
-    b.x[i] = (const bf16_t*)it.x;
-    b.ld[i] = it.ld;
-    b.acc[i] = it.acc;
-    b.start[i] = at;
-    at += (int)it.cols;
-    bytes += 2.0 * rows * it.cols;
-  }
-  b.start[n] = at;
+  JPP_REQUIRE(partial, "colsum_multi: a partial-sum buffer is required");
   hipStream_t st = (hipStream_t)stream;
-  ProbeScope probe(st, "colsum", 0, bytes);
-  if (rows <= kColsumFewRows) {
-    ColsumPanels p;
-    int blocks = 0;
-    for (int i = 0; i < 4; ++i) {
-      p.first[i] = i < n ? blocks : 0x7fffffff;
-      if (i < n) blocks += (b.start[i + 1] - b.start[i] + 63) / 64;
-      else { b.x[i] = b.x[0]; b.ld[i] = b.ld[0]; b.acc[i] = b.acc[0]; b.start[i + 1] = at; }
-    }
-    p.b = b;
+  ColsumPanels p;
+  int blocks;
+  if (int rc = colsum_panels(n, items, rows, &p, &blocks)) return rc;
+  int at = 0;
+  for (int i = 0; i < n; ++i) at += p.cols[i];
+  ProbeScope probe(st, "colsum", 0, 2.0 * rows * at);
+  if (blocks) {
     hipLaunchKernelGGL(colsum_few_rows_kernel, dim3(blocks), dim3(1024), 0, st, p, (long)rows);
     JPP_LAUNCH_CHECK();
     return JPP_OK;
   }
+  ColsumBatch b;
+  b.n = n;
+  at = 0;
+  for (int i = 0; i < n; ++i) {
+    b.x[i] = p.x[i];
+    b.ld[i] = p.ld[i];
+    b.acc[i] = p.acc[i];
+    b.start[i] = at;
+    at += p.cols[i];
+  }
+  b.start[n] = at;
   const int nb = (int)(rows < JPP_NORM_PARTIALS ? rows : JPP_NORM_PARTIALS);
   const int panels = (at / 8 + 255) / 256;
   hipLaunchKernelGGL(colsum_multi_partial_kernel, dim3(nb, panels), dim3(256), 0, st, b, (long)rows,

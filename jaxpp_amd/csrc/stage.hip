@@ -203,10 +203,10 @@ struct BiasGrads {
   bool pending = false;
 };
 
-// a layer's four bias gradients: column sums of the cotangents, added to the accumulators (in f32 by `later`, if
-// given, beside the weight gradients of the same rows)
+// a layer's four bias gradients: column sums of the cotangents, added to the accumulators (by `later`, if
+// given, with the weight gradients of the same rows)
 int bias_grads4(jpp_stage* s, hipStream_t st, const jpp_colsum_item* items, float* partial, BiasGrads* later) {
-  if (later && s->f32()) {
+  if (later) {
     std::copy(items, items + 4, later->item);
     later->pending = true;
     return JPP_OK;
@@ -249,6 +249,7 @@ struct WgradBatch {
   jpp_gemm_args g[4];
   int n = 0;
   const BiasGrads* bias = nullptr;   // to leave with them
+  float* partial = nullptr;          // their scratch
   void add(jpp_stage* s, int pairs, const void* const* xs, int64_t ldx, const void* const* dys,
            int64_t lddy, float* acc, int64_t rows, int64_t cols) {
     jpp_gemm_args& q = g[n++];
@@ -312,7 +313,10 @@ int run_wgrads(jpp_stage* s, hipStream_t st, WgradBatch& w) {
   for (int i = 0; i < w.n; ++i)
     if (may_gather && (whole || !full[i])) grid[n++] = w.g[i];
     else RC(run_apart(s, st, w.g[i]));
-  if (n <= 1) return n ? run_apart(s, st, grid[0]) : JPP_OK;
+  if (n <= 1) {
+    if (w.bias) RC(jpp_colsum_accum_multi(st, 4, w.bias->item, s->T, w.partial));
+    return n ? run_apart(s, st, grid[0]) : JPP_OK;
+  }
   // smallest first: measured 1 % faster than largest first at the Llama-3-8B shapes
   std::stable_sort(grid, grid + n, [](const jpp_gemm_args& a, const jpp_gemm_args& b) {
     return a.m * a.n < b.m * b.n;
@@ -324,7 +328,8 @@ int run_wgrads(jpp_stage* s, hipStream_t st, WgradBatch& w) {
   // tiles, groups of four, apart / together: 512 tokens 2.73 / 2.50 ms, 4096 tokens 7.71 / 7.44).
   constexpr long kGroupTiles = 128;
   const int pairs = grid[0].k_parts > 1 ? grid[0].k_parts : 1;
-  if (pairs == 1 || (whole && total >= kGroupTiles)) return jpp_gemm_bf16_multi(st, grid, n);
+  if (pairs == 1 || (whole && total >= kGroupTiles))
+    return jpp_wgrads_bf16(st, n, grid, w.bias ? 4 : 0, w.bias ? w.bias->item : nullptr, s->T, w.partial);
   for (int part = 0; part < pairs; ++part) {
     jpp_gemm_args one[4];
     for (int i = 0; i < n; ++i) {
@@ -595,7 +600,10 @@ int layer_bwd_w(jpp_stage* s, hipStream_t st, int chunk, int li, uint8_t* slot, 
   auto at = [&](const Buf& b) { return (void*)(slot + b.off); };
   auto wt = [&](const Buf& b) { return (void*)(wbase + b.off); };
   WgradBatch wb;
-  if (bias && bias->pending) wb.bias = bias;
+  if (bias && bias->pending) {
+    wb.bias = bias;
+    wb.partial = partial;
+  }
   if (s->d.family == JPP_FAMILY_BERT) {
     wb.add1(s, at(L.g), f, wt(W.dc), h, s->G(chunk, li, B_W2), f, h);
     wb.add1(s, at(L.x1), h, wt(W.du), f, s->G(chunk, li, B_W1), h, f);

@@ -10,7 +10,11 @@ import numpy as np
 import pytest
 
 from jaxpp_amd import runtime as rt
+from jaxpp_amd import schedules as S
+from jaxpp_amd.model import LayerSpec, init_layer_params
+from jaxpp_amd.plan import make_rank_plan
 from oracle import layers as L
+from test_gpu_stage import run_on_gpu
 
 pytestmark = pytest.mark.gpu
 U = 2.0 ** -24
@@ -92,3 +96,23 @@ def test_column_sums(rows, cols):
         x = x[:, :c].astype(np.float64)
         assert (np.abs(a.download(np.float32, (c,)) - (a0 + x.sum(0))) <=
                 (rows + 8) * U * (np.abs(a0) + np.abs(x).sum(0))).all()
+
+
+# weight gradients on 64x64 tiles (few and many K-steps), on 128x128 ones, on 256x256 ones, some of them
+# apart; the last rows that are few and the first that are not
+@pytest.mark.parametrize("family,h,heads,f,seq,batch", [
+    ("bert", 128, 2, 512, 128, 1), ("decoder", 128, 2, 384, 384, 5), ("bert", 640, 10, 1280, 128, 3),
+    ("decoder", 1024, 8, 4096, 512, 1), ("bert", 768, 6, 3072, 512, 4), ("bert", 1024, 16, 4096, 512, 3),
+    ("decoder", 1408, 11, 5632, 128, 9), ("bert", 128, 2, 256, 512, 8), ("decoder", 128, 2, 256, 1408, 3)])
+def test_bias_gradients_beside_weight_gradients(family, h, heads, f, seq, batch):
+    """On one stream a layer's bias gradients go with its weight gradients, on two they go before them: the same
+    sums to the last bit, whichever launch adds them up."""
+    print(f"bias gradients {family} {h} {f} {seq} x {batch}", flush=True)
+    spec = LayerSpec(family, h, heads, f, seq, batch, head_dim=h // heads, causal=family == "decoder", eps=1e-5)
+    plan = make_rank_plan(S.Std1F1B(1), 2, 0)
+    params = {0: [init_layer_params(spec, 3, li, perturb=True) for li in range(2)]}
+    _, _, apart = run_on_gpu(spec, plan, 2, params, two_streams=True)
+    _, _, here = run_on_gpu(spec, plan, 2, params, two_streams=False)
+    for li in range(2):
+        for name, w in apart[0][li].items():
+            assert np.abs(w).max() > 0 and np.array_equal(here[0][li][name], w), name
