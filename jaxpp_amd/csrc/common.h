@@ -59,6 +59,10 @@ struct ProbeScope {
 
 // jpp_colsum_accum_f32 of up to four matrices with the same rows in one launch (f32_ops.hip)
 int jpp_colsum_f32_items(hipStream_t stream, int n, const jpp_colsum_item* items, int64_t rows);
+// jpp_norm_fwd(_f32) that also copies a tensor of the norm's shape, copy_src, to copy_dst (if not nullptr), which
+// overlaps none of the norm's operands
+int jpp_norm_fwd_copy(hipStream_t stream, const jpp_norm_args* a, const void* copy_src, void* copy_dst);
+int jpp_norm_fwd_copy_f32(hipStream_t stream, const jpp_norm_args* a, const void* copy_src, void* copy_dst);
 // up to four accumulated weight gradients of the same k rows (plain ones: trans_a = trans_b = 1,
 // JPP_EPI_ACC_F32) and the column sums over those rows of up to four matrices, in one launch (f32_ops.hip)
 int jpp_wgrads_f32(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols, const jpp_colsum_item* items);

@@ -55,7 +55,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 
 // ---------------------------------------------------------------------------
-// norm forward: one wave per row, the row cached in registers
+// norm forward: one wave per row, the row cached in registers.  With copy_dst it also carries a tensor of the same
+// shape, copy_src, there (copy_src = nullptr: x itself): a stage keeps its input like this instead of by a
+// copy of its own in front of the first layer.
 // ---------------------------------------------------------------------------
 template <bool LN, int NCH>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const bf16_t* __restrict__ x,
@@ -64,18 +66,34 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const bf16_t* __restrict_
                                                        bf16_t* __restrict__ y,
                                                        float* __restrict__ mean_out,
                                                        float* __restrict__ rstd_out, long rows,
-                                                       int cols, float eps) {
+                                                       int cols, float eps,
+                                                       const bf16_t* __restrict__ copy_src,
+                                                       bf16_t* __restrict__ copy_dst) {
   const int lane = threadIdx.x & 63;
   const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int nchunk = cols >> 3;
   const uint4* xr = (const uint4*)(x + row * cols);
   uint4 v[NCH];
-  float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int c = lane + 64 * i;
     v[i] = c < nchunk ? xr[c] : make_uint4(0, 0, 0, 0);
+  }
+  if (copy_dst) {
+    uint4* dst = (uint4*)(copy_dst + row * cols);
+    if (copy_src) {
+      const uint4* src = (const uint4*)(copy_src + row * cols);
+      for (int c = lane; c < nchunk; c += 64) dst[c] = src[c];
+    } else {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+        if (lane + 64 * i < nchunk) dst[lane + 64 * i] = v[i];
+    }
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
     float f[8];
     unpack8(v[i], f);
 #pragma unroll
@@ -746,13 +764,14 @@ int grid_for(long items, int per_block = 256, int cap = 256 * 32) {
 }
 
 template <bool LN>
-int launch_norm_fwd(hipStream_t st, const jpp_norm_args* a) {
+int launch_norm_fwd(hipStream_t st, const jpp_norm_args* a, const void* copy_src, void* copy_dst) {
   const int blocks = (int)((a->rows + 3) / 4);
   const int nch = (int)((a->cols / 8 + 63) / 64);
 #define JPP_NF(N)                                                                            \
   hipLaunchKernelGGL((norm_fwd_kernel<LN, N>), dim3(blocks), dim3(256), 0, st,               \
                      (const bf16_t*)a->x, (const bf16_t*)a->gamma, (const bf16_t*)a->beta,   \
-                     (bf16_t*)a->y, a->mean, a->rstd, (long)a->rows, (int)a->cols, a->eps)
+                     (bf16_t*)a->y, a->mean, a->rstd, (long)a->rows, (int)a->cols, a->eps,     \
+                     (const bf16_t*)copy_src, (bf16_t*)copy_dst)
   if (nch <= 1) JPP_NF(1);
   else if (nch <= 2) JPP_NF(2);
   else if (nch <= 4) JPP_NF(4);
@@ -827,6 +846,20 @@ int launch_norm_bwd(hipStream_t st, const jpp_norm_args* a) {
 
 }  // namespace
 
+int jpp_norm_fwd_copy(hipStream_t stream, const jpp_norm_args* a, const void* copy_src, void* copy_dst) {
+  JPP_REQUIRE(a && a->x && a->gamma && a->y && a->rstd, "norm_fwd: null operand");
+  JPP_REQUIRE(a->rows > 0 && a->cols > 0 && a->cols % 8 == 0 &&
+                  a->cols <= 8 * 64 * kMaxChunksPerLane,
+              "norm_fwd: cols must be a multiple of 8 and at most %d, got %ld",
+              8 * 64 * kMaxChunksPerLane, (long)a->cols);
+  JPP_REQUIRE((a->beta == nullptr) == (a->mean == nullptr),
+              "norm_fwd: beta and mean are both given (LayerNorm) or both NULL (RMSNorm)");
+  if (copy_src == a->x) copy_src = nullptr;
+  ProbeScope probe(stream, "norm_fwd", 0, (copy_dst ? copy_src ? 8.0 : 6.0 : 4.0) * a->rows * a->cols);
+  return a->beta ? launch_norm_fwd<true>(stream, a, copy_src, copy_dst)
+                 : launch_norm_fwd<false>(stream, a, copy_src, copy_dst);
+}
+
 int colsum_panels(int n, const jpp_colsum_item* items, int64_t rows, ColsumPanels* p, int* blocks) {
   JPP_REQUIRE(items && n >= 1 && n <= 4 && rows > 0, "colsum_multi: 1 to 4 tensors are required");
   *blocks = 0;
@@ -849,16 +882,7 @@ int colsum_panels(int n, const jpp_colsum_item* items, int64_t rows, ColsumPanel
 extern "C" {
 
 int jpp_norm_fwd(void* stream, const jpp_norm_args* a) {
-  JPP_REQUIRE(a && a->x && a->gamma && a->y && a->rstd, "norm_fwd: null operand");
-  JPP_REQUIRE(a->rows > 0 && a->cols > 0 && a->cols % 8 == 0 &&
-                  a->cols <= 8 * 64 * kMaxChunksPerLane,
-              "norm_fwd: cols must be a multiple of 8 and at most %d, got %ld",
-              8 * 64 * kMaxChunksPerLane, (long)a->cols);
-  JPP_REQUIRE((a->beta == nullptr) == (a->mean == nullptr),
-              "norm_fwd: beta and mean are both given (LayerNorm) or both NULL (RMSNorm)");
-  ProbeScope probe((hipStream_t)stream, "norm_fwd", 0, 4.0 * a->rows * a->cols);
-  return a->beta ? launch_norm_fwd<true>((hipStream_t)stream, a)
-                 : launch_norm_fwd<false>((hipStream_t)stream, a);
+  return jpp_norm_fwd_copy((hipStream_t)stream, a, nullptr, nullptr);
 }
 
 int jpp_norm_bwd(void* stream, const jpp_norm_args* a) {

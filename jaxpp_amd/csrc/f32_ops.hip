@@ -364,7 +364,8 @@ __global__ __launch_bounds__(256) void norm_fwd32_kernel(const float* __restrict
                                                          const float* __restrict__ beta,
                                                          float* __restrict__ y, float* mean_out,
                                                          float* rstd_out, long rows, int cols,
-                                                         float eps) {
+                                                         float eps, const float* __restrict__ copy_src,
+                                                         float* __restrict__ copy_dst) {
   const int lane = threadIdx.x & 63;
   const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -385,6 +386,8 @@ __global__ __launch_bounds__(256) void norm_fwd32_kernel(const float* __restrict
     const float v = (xr[c] - mean) * rstd * gamma[c];
     y[row * cols + c] = beta ? v + beta[c] : v;
   }
+  if (copy_dst)   // (as in the bf16 norm: the stage's input)
+    for (int c = lane; c < cols; c += 64) copy_dst[row * cols + c] = copy_src[row * cols + c];
   if (lane == 0) {
     if (mean_out) mean_out[row] = mean;
     rstd_out[row] = rstd;
@@ -947,6 +950,19 @@ int jpp_wgrads_f32(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols
   return JPP_OK;
 }
 
+int jpp_norm_fwd_copy_f32(hipStream_t stream, const jpp_norm_args* a, const void* copy_src, void* copy_dst) {
+  JPP_REQUIRE(a && a->x && a->gamma && a->y && a->rstd, "norm_fwd_f32: null operand");
+  JPP_REQUIRE(a->rows > 0 && a->cols > 0, "norm_fwd_f32: empty");
+  JPP_REQUIRE((a->beta == nullptr) == (a->mean == nullptr),
+              "norm_fwd_f32: beta and mean are both given (LayerNorm) or both NULL (RMSNorm)");
+  hipLaunchKernelGGL(norm_fwd32_kernel, dim3((unsigned)((a->rows + 3) / 4)), dim3(256), 0,
+                     stream, (const float*)a->x, (const float*)a->gamma,
+                     (const float*)a->beta, (float*)a->y, a->mean, a->rstd, (long)a->rows,
+                     (int)a->cols, a->eps, (const float*)copy_src, (float*)copy_dst);
+  JPP_LAUNCH_CHECK();
+  return JPP_OK;
+}
+
 extern "C" {
 
 int jpp_gemm_f32(void* stream, const jpp_gemm_args* a) {
@@ -1012,16 +1028,7 @@ int jpp_rope_f32(void* stream, float* x, int64_t ld, const float* cos_tab, const
 }
 
 int jpp_norm_fwd_f32(void* stream, const jpp_norm_args* a) {
-  JPP_REQUIRE(a && a->x && a->gamma && a->y && a->rstd, "norm_fwd_f32: null operand");
-  JPP_REQUIRE(a->rows > 0 && a->cols > 0, "norm_fwd_f32: empty");
-  JPP_REQUIRE((a->beta == nullptr) == (a->mean == nullptr),
-              "norm_fwd_f32: beta and mean are both given (LayerNorm) or both NULL (RMSNorm)");
-  hipLaunchKernelGGL(norm_fwd32_kernel, dim3((unsigned)((a->rows + 3) / 4)), dim3(256), 0,
-                     (hipStream_t)stream, (const float*)a->x, (const float*)a->gamma,
-                     (const float*)a->beta, (float*)a->y, a->mean, a->rstd, (long)a->rows,
-                     (int)a->cols, a->eps);
-  JPP_LAUNCH_CHECK();
-  return JPP_OK;
+  return jpp_norm_fwd_copy_f32((hipStream_t)stream, a, nullptr, nullptr);
 }
 
 int jpp_norm_bwd_f32(void* stream, const jpp_norm_args* a) {
