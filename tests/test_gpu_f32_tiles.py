@@ -102,6 +102,42 @@ def test_norm_bwd_and_column_sums_f32_ragged(rows, cols):
     assert (np.abs(bufs["dx"].download(np.float32, (rows, cols)) - want) <= (cols + 12) * U * mag).all()
 
 
+@pytest.mark.parametrize("ln", [True, False])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 63), (6, 64), (7, 65), (512, 256), (9, 257), (66, 512), (3, 513),
+                                       (130, 1024), (11, 1025), (65, 4100)])
+def test_norm_fwd_f32_row_lengths(rows, cols, ln):
+    """Rows a lane holds in 4, 8 or 16 registers, the last and first lengths of each, and longer ones.  The mean and
+    the mean square are sums of cols terms, each within (cols + 3) 2^-24 of its terms' magnitudes."""
+    rng = np.random.default_rng(rows * 3 + cols)
+    x = rng.standard_normal((rows, cols), dtype=np.float32) + np.float32(0.5)
+    gamma, beta = (rng.standard_normal(cols, dtype=np.float32) for _ in range(2))
+    bufs = dict(x=dev(x), gamma=dev(gamma), y=dev(np.zeros((rows + 1, cols))), rstd=dev(np.zeros(rows)))
+    if ln:
+        bufs.update(beta=dev(beta), mean=dev(np.zeros(rows)))
+    a = rt.NormArgs()
+    for k, b in bufs.items():
+        setattr(a, k, b.ptr)
+    a.rows, a.cols, a.eps = rows, cols, 1e-3
+    rt.check(rt.load().jpp_norm_fwd_f32(None, C.byref(a)))
+    rt.sync()
+    x64 = x.astype(np.float64)
+    mean = x64.mean(1, keepdims=True) if ln else np.zeros((rows, 1))
+    d = x64 - mean
+    var = (d * d).mean(1, keepdims=True) + a.eps
+    rstd = 1 / np.sqrt(var)
+    e = (cols + 3) * U                       # of the mean, of the variance, and half of it of rstd
+    em = e * np.abs(x64).mean(1, keepdims=True) if ln else 0.0
+    er = e + (2 * em * np.abs(d).mean(1, keepdims=True) + em * em) / var + 4 * U
+    y = bufs["y"].download(np.float32, (rows + 1, cols))
+    want = d * rstd * gamma + (beta if ln else 0)
+    mag = np.abs(gamma) * rstd
+    assert (np.abs(y[:rows] - want) <= mag * (em + np.abs(d) * (er + 4 * U)) + 2 * U * np.abs(want) + 1e-30).all()
+    assert (y[rows] == 0).all()
+    assert (np.abs(bufs["rstd"].download(np.float32, (rows,)) - rstd[:, 0]) <= (er * rstd)[:, 0]).all()
+    if ln:
+        assert (np.abs(bufs["mean"].download(np.float32, (rows,)) - mean[:, 0]) <= em[:, 0]).all()
+
+
 @pytest.mark.parametrize("d,hq,hk,seq,causal", [(64, 2, 1, 64, 1), (64, 3, 3, 192, 0), (128, 4, 2, 64, 0),
                                                 (128, 2, 2, 320, 1)])
 def test_attention_f32_tiles(d, hq, hk, seq, causal):
