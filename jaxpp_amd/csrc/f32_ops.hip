@@ -124,7 +124,7 @@ constexpr int kStages32 = BM == 16 ? 3 : 2;   // (what fits beside the sums)
 // halve the distance to a float64 sum (5.7e-7 -> 2.9e-7 at k = 1024).  512 x 256 outputs, k = 256
 // and 1024, take 7.3 us on average; the 64 x 64 tile of 16 x 16 threads in its place, one barrier
 // pair per 16 contraction elements on 32 CUs, and attention with a pair of lanes per row made a
-// two-layer row of eight microbatches of 512 tokens 30.0 ms, now 2.15 ms.
+// two-layer row of eight microbatches of 512 tokens 30.0 ms, now 1.70 ms.
 //
 // STAGED (both contraction indices contiguous): every wave copies its own steps, 32 elements of
 // the contraction at a time, into LDS of its own and reads the fragments there, with no barrier
@@ -821,29 +821,32 @@ __global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_fwd32_kernel(Attn32
   if (threadIdx.x < 16) p.lse[((long)b * p.n_heads + h) * p.seq + q0 + c] = mall + logf(lall);
 }
 
-// dQ of 16 queries, and delta = rowsum(dO o O) for the dK/dV kernel
+// this lane's share of delta = rowsum(dO o O) of row c, given the row's elements of dO
 template <int D>
-__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dq32_kernel(Attn32 p) {
+__device__ __forceinline__ float row_delta32(const Rows32<D>& go, const float* o_rows, long ldo, int c, int g) {
+  Rows32<D> o;
+  o.load(o_rows, ldo, c, g);
+  float dl = 0.f;
+#pragma unroll
+  for (int t = 0; t < D / 16; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dl = fmaf(go.v[t][e], o.v[t][e], dl);
+  return quad_sum(dl);
+}
+
+// dQ of 16 queries, and delta for the dK/dV kernel behind it
+template <int D>
+__device__ __forceinline__ void dq_tile32(const Attn32& p, float* buf, int qt, int h, int b) {
   constexpr int W = kAttnWaves32<D>;
-  __shared__ float buf[W * 16 * D];
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = blockIdx.y, b = blockIdx.z, hk = h / (p.n_heads / p.n_kv_heads);
-  const int q0 = blockIdx.x * 16;
+  const int hk = h / (p.n_heads / p.n_kv_heads);
+  const int q0 = qt * 16;
   const long row0 = (long)b * p.seq;
   Rows32<D> q, go;
   q.load(p.q + (row0 + q0) * p.ldq + h * D, p.ldq, c, g);
   go.load(p.d_o + (row0 + q0) * p.lddo + h * D, p.lddo, c, g);
-  float dl = 0.f;
-  {
-    Rows32<D> o;
-    o.load(p.o + (row0 + q0) * p.ldo + h * D, p.ldo, c, g);
-#pragma unroll
-    for (int t = 0; t < D / 16; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) dl = fmaf(go.v[t][e], o.v[t][e], dl);
-  }
-  dl = quad_sum(dl);
+  const float dl = row_delta32<D>(go, p.o + (row0 + q0) * p.ldo + h * D, p.ldo, c, g);
   const long stat = ((long)b * p.n_heads + h) * p.seq + q0 + c;
   if (wave == 0 && g == 0) p.delta[stat] = dl;
   const float lse = p.lse[stat];
@@ -871,15 +874,15 @@ __global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dq32_kernel(Attn32 
   store_sum32<D, W>(dq, buf, p.dq + (row0 + q0) * p.lddq + h * D, p.lddq);
 }
 
-// dK, dV of 16 keys: the waves take the 16-query tiles of every head of the keys' group in turn
-template <int D>
-__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dkv32_kernel(Attn32 p) {
+// dK, dV of 16 keys: the waves take the 16-query tiles of every head of the keys' group in turn.  ALONE: delta is not
+// there yet and is formed here too (the same value).
+template <int D, bool ALONE>
+__device__ __forceinline__ void dkv_tile32(const Attn32& p, float* buf, int kt, int hk, int b) {
   constexpr int W = kAttnWaves32<D>;
-  __shared__ float buf[W * 16 * D];
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int hk = blockIdx.y, b = blockIdx.z, grp = p.n_heads / p.n_kv_heads;
-  const int k0 = blockIdx.x * 16;
+  const int grp = p.n_heads / p.n_kv_heads;
+  const int k0 = kt * 16;
   const long row0 = (long)b * p.seq;
   Rows32<D> kr, vr;
   kr.load(p.k + (row0 + k0) * p.ldk + hk * D, p.ldk, c, g);
@@ -899,7 +902,15 @@ __global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dkv32_kernel(Attn32
     gc.load(gp, p.lddo, c, g);
     qc.load(qp, p.ldq, c, g);
     const long stat = ((long)b * p.n_heads + h) * p.seq + q0 + 4 * g;
-    const f32x4 lse = *(const f32x4_u*)(p.lse + stat), dl = *(const f32x4_u*)(p.delta + stat);
+    const f32x4 lse = *(const f32x4_u*)(p.lse + stat);
+    f32x4 dl;
+    if constexpr (ALONE) {
+      const float own = row_delta32<D>(gr, p.o + (row0 + q0) * p.ldo + h * D, p.ldo, c, g);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dl[r] = __shfl(own, 4 * g + r);
+    } else {
+      dl = *(const f32x4_u*)(p.delta + stat);
+    }
     f32x4 s = score32<D>(qr, kr);
     const f32x4 dp = score32<D>(gr, vr);
     f32x4 ds;
@@ -914,6 +925,52 @@ __global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dkv32_kernel(Attn32
   store_sum32<D, W>(dv, buf, p.dv + (row0 + k0) * p.lddv + hk * D, p.lddv);
   __syncthreads();
   store_sum32<D, W>(dk, buf, p.dk + (row0 + k0) * p.lddk + hk * D, p.lddk);
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dq32_kernel(Attn32 p) {
+  __shared__ float buf[kAttnWaves32<D> * 16 * D];
+  dq_tile32<D>(p, buf, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+template <int D>
+__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dkv32_kernel(Attn32 p) {
+  __shared__ float buf[kAttnWaves32<D> * 16 * D];
+  dkv_tile32<D, false>(p, buf, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+// both at once: the dK/dV workgroups, which take longer, in front (blockIdx.y: key heads, then query heads)
+template <int D>
+__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_bwd32_kernel(Attn32 p) {
+  __shared__ float buf[kAttnWaves32<D> * 16 * D];
+  if ((int)blockIdx.y < p.n_kv_heads) dkv_tile32<D, true>(p, buf, blockIdx.x, blockIdx.y, blockIdx.z);
+  else dq_tile32<D>(p, buf, blockIdx.x, blockIdx.y - p.n_kv_heads, blockIdx.z);
+}
+
+// Whether a backward is one launch: while its workgroups are at most one per CU (its registers allow one).  Either
+// half of a small one is a chain of latencies on part of the device, and they run beside each other in little more than
+// the longer one's time (us, two launches / one: 4 heads x 64, 4 x 128 rows 16.9 / 9.2; 1 x 512 rows under a
+// mask 34.3 / 19.1; 4 heads x 128, 4 x 128 rows 26.6 / 15.1); 384 and 512 workgroups 0.97 - 1.01 of the two's
+// time, 1024 1.08.  One launch writes dQ, dK and dV while it reads everything else, where two read only
+// part of it: a caller whose results lie over the inputs keeps the two.
+constexpr long kBwdAtOnce = 256;
+bool bwd32_at_once(const jpp_attn_args* a) {
+  const int64_t rows = (int64_t)a->batch * a->seq;
+  if (rows / 16 * (a->n_heads + a->n_kv_heads) > kBwdAtOnce) return false;
+  struct Range {
+    uintptr_t lo, hi;
+  };
+  auto range = [&](const void* p, int64_t ld, int heads) {
+    return Range{(uintptr_t)p, (uintptr_t)p + (uintptr_t)(((rows - 1) * ld + heads * a->head_dim) * 4)};
+  };
+  const Range out[3] = {range(a->dq, a->lddq, a->n_heads), range(a->dk, a->lddk, a->n_kv_heads),
+                        range(a->dv, a->lddv, a->n_kv_heads)};
+  const Range in[6] = {range(a->q, a->ldq, a->n_heads), range(a->k, a->ldk, a->n_kv_heads),
+                       range(a->v, a->ldv, a->n_kv_heads), range(a->o, a->ldo, a->n_heads),
+                       range(a->d_o, a->lddo, a->n_heads),
+                       {(uintptr_t)a->lse, (uintptr_t)a->lse + (uintptr_t)(rows * a->n_heads * 4)}};
+  for (const Range& w : out)
+    for (const Range& r : in)
+      if (w.lo < r.hi && r.lo < w.hi) return false;
+  return true;
 }
 
 int attn_check(const jpp_attn_args* a, const char* who, Attn32& p) {
@@ -1131,6 +1188,13 @@ int jpp_attn_bwd_f32(void* stream, const jpp_attn_args* a) {
                   a->lddv >= (int64_t)a->n_kv_heads * a->head_dim,
               "attn_bwd_f32: leading dimension too small");
   hipStream_t st = (hipStream_t)stream;
+  if (bwd32_at_once(a)) {
+    const dim3 grid((unsigned)(a->seq / 16), (unsigned)(a->n_heads + a->n_kv_heads), (unsigned)a->batch);
+    if (a->head_dim == 64) hipLaunchKernelGGL(attn_bwd32_kernel<64>, grid, dim3(64 * kAttnWaves32<64>), 0, st, p);
+    else hipLaunchKernelGGL(attn_bwd32_kernel<128>, grid, dim3(64 * kAttnWaves32<128>), 0, st, p);
+    JPP_LAUNCH_CHECK();
+    return JPP_OK;
+  }
   const dim3 gq((unsigned)(a->seq / 16), (unsigned)a->n_heads, (unsigned)a->batch);
   const dim3 gk((unsigned)(a->seq / 16), (unsigned)a->n_kv_heads, (unsigned)a->batch);
   if (a->head_dim == 64) {

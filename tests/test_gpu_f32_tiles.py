@@ -204,3 +204,37 @@ def test_layer_weight_and_bias_gradients_in_one_launch_f32(family, h, heads, f, 
         for name, w in want[0][li].items():
             assert np.array_equal(here[0][li][name], apart[0][li][name]), name
             parity.close(here[0][li][name], w.reshape(here[0][li][name].shape).astype(np.float64), 1e-4, name)
+
+
+# workgroups (rows / 16 x heads of both kinds): 16, 128, 192, 256, 384
+@pytest.mark.parametrize("d,hq,hk,seq,batch,causal", [(64, 2, 2, 64, 1, 0), (64, 6, 2, 128, 2, 1), (64, 4, 4, 128, 4, 0),
+                                                      (128, 2, 1, 128, 8, 1), (128, 3, 3, 64, 4, 0), (64, 8, 4, 256, 2, 0)])
+def test_attention_backward_f32_at_once_and_in_two(d, hq, hk, seq, batch, causal):
+    """Few workgroups: dQ, dK and dV in one launch, where they lie apart from the inputs; dK over K and dV over V keep
+    the two.  The same bits, with the results interleaved or not."""
+    print(f"attention_bwd_f32 d={d} heads={hq}/{hk} {batch}x{seq} causal={causal}", flush=True)
+    rng = np.random.default_rng(d + seq + hq)
+    T, W = batch * seq, (hq + 2 * hk) * d
+    qkv, o, do = (rng.standard_normal((T, w), dtype=np.float32) for w in (W, hq * d, hq * d))
+    lib = rt.load()
+    got = []
+    for over in (False, True):
+        bufs = dict(qkv=dev(qkv), o=dev(o), d_o=dev(do), lse=dev(np.zeros(batch * hq * seq)),
+                    delta=dev(np.zeros(2 * batch * hq * seq)), g=dev(np.zeros((T, W))))
+        a = rt.AttnArgs()
+        a.q, a.k, a.v = (bufs["qkv"].ptr + 4 * d * n for n in (0, hq, hq + hk))
+        a.dq, a.dk, a.dv = (bufs["g"].ptr + 4 * d * n for n in (0, hq, hq + hk))
+        a.ldq = a.ldk = a.ldv = a.lddq = a.lddk = a.lddv = W
+        a.ldo = a.lddo = hq * d
+        a.o, a.d_o, a.lse, a.delta = (bufs[k].ptr for k in ("o", "d_o", "lse", "delta"))
+        a.batch, a.seq, a.n_heads, a.n_kv_heads, a.head_dim, a.causal = batch, seq, hq, hk, d, causal
+        rt.check(lib.jpp_attn_fwd_f32(None, C.byref(a)))
+        if over:
+            a.dk, a.dv = a.k, a.v
+        rt.check(lib.jpp_attn_bwd_f32(None, C.byref(a)))
+        rt.sync()
+        g = bufs["g"].download(np.float32, (T, W))
+        if over:
+            g[:, hq * d:] = bufs["qkv"].download(np.float32, (T, W))[:, hq * d:]
+        got.append(g)
+    assert np.array_equal(*got) and np.isfinite(got[0]).all() and (got[0] != 0).mean() > 0.9
