@@ -224,9 +224,8 @@ int jpp_gemm_bf16(void* stream, const jpp_gemm_args* args);
  * dot_generals (one per parameter of the layer, src/jaxpp/jaxpr_utils.py:138-167 puts them all
  * into BWD_W): launched one by one, each leaves its last round of tiles partly empty (a 6144 x
  * 4096 gradient is 384 tiles on 256 CUs), small ones most of the device; together they close up.
- * Tiles are 256x256 when M and N are multiples of 256 and the problems are most of a round of
- * them, else 256x256, 128x128 or 64x64 by an estimate of their time.  Every output element is computed by one workgroup in a fixed
- * order (deterministic), the same order as in a single launch on the same tile; a single launch
+ * Tiles are 256x256, 128x128 or 64x64 by an estimate of their time, whatever the size.  Every output
+ * element is computed by one workgroup in a fixed order (deterministic), the same order as in a single launch on the same tile; a single launch
  * that runs its last round on 128x256 tiles adds the old accumulator value at another point of
  * the sum there, so the two agree to fp32 rounding.  n_problems = 1 is jpp_gemm_bf16. */
 int jpp_gemm_bf16_multi(void* stream, const jpp_gemm_args* problems, int n_problems);
