@@ -1027,8 +1027,9 @@ int jpp_wgrads_f32(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols
   long strips = 0;
   for (int i = 0; i < 4; ++i) {
     const jpp_gemm_args& q = g[i < n ? i : 0];
-    JPP_REQUIRE(q.k_parts <= 1 && q.k == g[0].k && q.k > 0 && q.m > 0 && q.n > 0 && q.m % 64 == 0 && q.n % 64 == 0 && q.k % 16 == 0 && q.lda >= q.m && q.ldb >= q.n &&
-                    q.ldc >= q.n, "wgrads_f32: product %d has a shape of its own or a bad one", i);
+    JPP_REQUIRE(q.k_parts <= 1 && q.k == g[0].k && q.k > 0 && q.k % 16 == 0 && q.m > 0 && q.m % 64 == 0 &&
+                    q.n > 0 && q.n % 64 == 0 && q.lda >= q.m && q.ldb >= q.n && q.ldc >= q.n,
+                "wgrads_f32: product %d has a shape of its own or a bad one", i);
     w.a[i] = (const float*)q.a; w.b[i] = (const float*)q.b; w.c[i] = (float*)q.c;
     w.lda[i] = q.lda; w.ldb[i] = q.ldb; w.ldc[i] = q.ldc; w.n[i] = (int)q.n;
     if (i < n) strips += (q.m / 16) * (q.n / 64);

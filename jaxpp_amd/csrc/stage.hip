@@ -351,7 +351,8 @@ int norm_f(jpp_stage* s, hipStream_t st, const void* x, const void* gamma, const
   memset(&a, 0, sizeof(a));
   a.x = x; a.gamma = gamma; a.beta = beta; a.y = y; a.mean = mean; a.rstd = rstd;
   a.rows = s->T; a.cols = s->h; a.eps = s->d.eps;
-  return s->f32() ? jpp_norm_fwd_copy_f32(st, &a, copy_src, copy_dst) : jpp_norm_fwd_copy(st, &a, copy_src, copy_dst);
+  return s->f32() ? jpp_norm_fwd_copy_f32(st, &a, copy_src, copy_dst)
+                  : jpp_norm_fwd_copy(st, &a, copy_src, copy_dst);
 }
 
 int norm_b(jpp_stage* s, hipStream_t st, const void* dy, const void* x, const float* mean,
@@ -1319,7 +1320,8 @@ int jpp_stage_run_task(jpp_stage* s, int kind, int chunk, int mb, const void* in
       }
       // (the halves run back to back on one stream: the bias gradients may go with the second)
       BiasGrads bias;
-      RC(layer_bwd_i(s, st, chunk, li, slot, wbase, W, dy, dx, kind == JPP_BWD && s->wg == 1 && !two ? &bias : nullptr));
+      const bool back_to_back = kind == JPP_BWD && s->wg == 1 && !two;
+      RC(layer_bwd_i(s, st, chunk, li, slot, wbase, W, dy, dx, back_to_back ? &bias : nullptr));
       if (kind == JPP_BWD && s->wg == 1) {
         if (two) {
           RC(fork());
