@@ -6,6 +6,7 @@
 // These kernels serve small problems whose results must hold 1e-4 against an fp32 CPU run:
 // fp32 arithmetic throughout, the contractions on the fp32 matrix instruction, every sum in an
 // order that the shapes fix.
+#include <limits.h>
 #include <math.h>
 #include <string.h>
 
@@ -327,6 +328,9 @@ __global__ __launch_bounds__(256) void sgemm_kernel(SgemmParams p) {
   sgemm_tile<BM, TA, TB, STAGED>(p, blockIdx.x);
 }
 
+// Rows of a product's tiles: the tallest that still give every CU one (a taller tile reads its B fewer times).
+int tile_rows32(long strips) { return strips >= 4 * 256 ? 64 : strips >= 2 * 256 ? 32 : 16; }
+
 template <int BM>
 int sgemm_launch(hipStream_t st, const SgemmParams& p) {
   const dim3 grid((unsigned)(p.m / BM * (p.n / 64)), 1u, p.group_mode == JPP_GROUP_K ? (unsigned)p.n_seg : 1u);
@@ -565,7 +569,7 @@ __global__ __launch_bounds__(1024) void colsum32_kernel(ColItems32 p, long rows)
 // A layer's weight gradients, up to four products C_i += A_i^T B_i over the same rows, and its bias gradients,
 // column sums over them, in one launch: workgroups first[i] .. first[i + 1] - 1 take product i, those from
 // col_first on the sums.  Apart, each fills a part of the device and is mostly latency: a layer of hidden 256 on
-// 512 tokens 31 us in five launches, 19 in one.
+// 512 tokens 27 us in five launches, 17 as one and the sums'.  Which products gain by it: kWgrads32 below.
 struct SgemmWgrads {
   SgemmParams p;        // what they share, and product 0
   const float* a[4];
@@ -997,6 +1001,73 @@ int attn_check(const jpp_attn_args* a, const char* who, Attn32& p) {
 
 }  // namespace
 
+// Ways to run a layer's weight gradients: one launch on tiles of 16, 32 or 64 rows, or a launch per product (each on
+// the tile that it takes by itself).  A CU takes one workgroup of any of them at a time.  Expected time, us, with
+// w = rounds of the 256 CUs, s = tiles / 256, k = rows of the contraction / 1024:
+//   w = 1   c0 + c1 k + s (c2 + c3 k)
+//   w > 1   c0 + w (c1 + c2 k) + s (c3 + c4 k)
+// (a round that all workgroups start together finds its operands in L2, later ones, out of step, do not: 512 x 2048
+// outputs are one round and 38 us at 2048 rows, two such products and 192 tiles more in one grid 58 a round).
+// Least squares of the relative error over 400 layers (hidden 64 .. 2048, feed-forward 1 .. 6 times that, 128 .. 8192
+// rows, post- and pre-norm and gated ones, also without a feed-forward), mean error 1 - 6 %.  The smallest estimate takes 0.4 % over
+// the best way, 9 % at worst; one launch always, on 64 rows from 512 strips of 16 on, 4 % and 82 %, and was slower than
+// a launch per product by up to 37 % (hidden 512, feed-forward 2048, 4096 rows: 336 us, 269 apart).
+struct Fit32 {
+  float one[4], more[5];
+};
+constexpr Fit32 kWgrads32[2][3] = {
+    {{{2.9f, 4.7f, 0.8f, 0.04f}, {0.f, 1.45f, 6.4f, 1.1f, 0.f}},     // a launch per product: 16, 32, 64 rows
+     {{4.1f, 8.0f, 0.f, 0.f}, {0.f, 2.2f, 11.8f, 1.1f, 0.8f}},
+     {{4.6f, 15.2f, 0.f, 0.f}, {5.7f, 0.f, 19.0f, 0.9f, 7.7f}}},
+    {{{3.8f, 4.5f, 0.8f, 0.9f}, {3.6f, 0.35f, 5.95f, 0.8f, 1.2f}},   // one launch
+     {{4.6f, 7.9f, 0.9f, 0.25f}, {3.9f, 1.35f, 9.0f, 0.3f, 5.4f}},
+     {{4.5f, 15.0f, 0.95f, 0.25f}, {7.5f, 0.f, 18.7f, 0.4f, 8.7f}}}};
+
+static float wgrads32_us(bool together, int rows, long strips, long contraction) {
+  const int i = rows / 32;   // 16, 32, 64
+  const Fit32& f = kWgrads32[together][i];
+  const long tiles = strips >> i;
+  const float k = contraction / 1024.f, s = tiles / 256.f, w = (float)((tiles + 255) / 256);
+  return tiles <= 256 ? f.one[0] + f.one[1] * k + s * (f.one[2] + f.one[3] * k)
+                      : f.more[0] + w * (f.more[1] + f.more[2] * k) + s * (f.more[3] + f.more[4] * k);
+}
+
+struct Wgrads32 {
+  int rows;    // of a tile of the one launch; 0: a launch per product
+  bool sums;   // the column sums go along
+};
+
+// The sums' workgroups cost next to nothing where they fit into the last round (0.05 of their own launch's time in the
+// median).  Where they do not, each holds a CU for as long as its walk over all rows takes: behind a single round that
+// is more than their own launch from 384 rows on (a layer of hidden 256 and 1024 on 512 tokens 18.8 us, 12.7 + 3.9
+// apart; on 4096 122 and 66 + 15), among several rounds, whose tiles are out of step, from 1024 rows on (0.99 of the
+// time up to there, 1.1 beyond).  Tiles of 16 rows leave room beside them: one round 0.7 - 0.9 up to 1024 rows, 1.17
+// beyond, several 0.98.
+static Wgrads32 wgrads32(int n, const jpp_gemm_args* g, int n_cols, const jpp_colsum_item* items) {
+  long strips = 0;
+  float best = 0.f;
+  for (int i = 0; i < n; ++i) {
+    const long own = (g[i].m / 16) * (g[i].n / 64);
+    strips += own;
+    best += wgrads32_us(false, tile_rows32(own), own, g[i].k);
+  }
+  Wgrads32 way = {0, false};
+  for (int rows : {16, 32, 64}) {
+    const float us = wgrads32_us(true, rows, strips, g[0].k);
+    if (us < best) {
+      best = us;
+      way.rows = rows;
+    }
+  }
+  if (!way.rows) return way;
+  long tiles = 0, blocks = 0;
+  for (int i = 0; i < n; ++i) tiles += (g[i].m / way.rows) * (g[i].n / 64);
+  for (int i = 0; i < n_cols; ++i) blocks += (items[i].cols + 15) / 16;
+  const long along = way.rows == 16 ? (tiles > 256 ? LONG_MAX : 1024) : tiles > 256 ? 768 : 256;   // rows
+  way.sums = g[0].k <= along || (tiles + blocks + 255) / 256 == (tiles + 255) / 256;
+  return way;
+}
+
 static int column_items(ColItems32& p, int n, const jpp_colsum_item* items) {
   int blocks = 0;
   for (int i = 0; i < 4; ++i) {
@@ -1024,7 +1095,7 @@ int jpp_wgrads_f32(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols
   JPP_REQUIRE(n >= 1 && n <= 4 && n_cols >= 0 && n_cols <= 4, "wgrads_f32: 1 to 4 products, up to 4 column sums");
   SgemmWgrads w;
   memset(&w, 0, sizeof(w));
-  long strips = 0;
+  double flops = 0;
   for (int i = 0; i < 4; ++i) {
     const jpp_gemm_args& q = g[i < n ? i : 0];
     JPP_REQUIRE(q.k_parts <= 1 && q.k == g[0].k && q.k > 0 && q.k % 16 == 0 && q.m > 0 && q.m % 64 == 0 &&
@@ -1032,14 +1103,22 @@ int jpp_wgrads_f32(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols
                 "wgrads_f32: product %d has a shape of its own or a bad one", i);
     w.a[i] = (const float*)q.a; w.b[i] = (const float*)q.b; w.c[i] = (float*)q.c;
     w.lda[i] = q.lda; w.ldb[i] = q.ldb; w.ldc[i] = q.ldc; w.n[i] = (int)q.n;
-    if (i < n) strips += (q.m / 16) * (q.n / 64);
+    if (i < n) flops += 2.0 * q.m * q.n * q.k;
   }
   w.p.k = (int)g[0].k;
   w.p.ta = w.p.tb = 1;
   w.p.epi = JPP_EPI_ACC_F32;
-  // 64-row tiles from a tile for every other CU on (a layer of hidden 256, 192 of them: 18.7 us, 32 rows 21.9,
-  // 16 rows 21.3): both operands' columns are read once per tile, and the narrow ones' loads repeat more
-  const int bm = strips >= 2 * 256 ? 64 : strips >= 256 ? 32 : 16;
+  const Wgrads32 way = wgrads32(n, g, n_cols, items);
+  if (!way.rows) {
+    for (int i = 0; i < n; ++i)
+      if (int rc = jpp_gemm_f32(stream, g + i)) return rc;
+    return n_cols ? jpp_colsum_f32_items(stream, n_cols, items, g[0].k) : JPP_OK;
+  }
+  if (n_cols && !way.sums) {
+    if (int rc = jpp_colsum_f32_items(stream, n_cols, items, g[0].k)) return rc;
+    n_cols = 0;
+  }
+  const int bm = way.rows;
   int blocks = 0;
   for (int i = 0; i < 4; ++i) {
     w.first[i] = i < n ? blocks : 0x7fffffff;
@@ -1047,6 +1126,7 @@ int jpp_wgrads_f32(hipStream_t stream, int n, const jpp_gemm_args* g, int n_cols
   }
   w.col_first = blocks;
   if (n_cols) blocks += column_items(w.cols, n_cols, items);
+  ProbeScope probe(stream, n_cols ? "wgrads_f32_sums" : "wgrads_f32", flops, 0);
   if (bm == 64) hipLaunchKernelGGL(sgemm_wgrads_kernel<64>, dim3((unsigned)blocks), dim3(256), 0, stream, w);
   else if (bm == 32) hipLaunchKernelGGL(sgemm_wgrads_kernel<32>, dim3((unsigned)blocks), dim3(256), 0, stream, w);
   else hipLaunchKernelGGL(sgemm_wgrads_kernel<16>, dim3((unsigned)blocks), dim3(256), 0, stream, w);
@@ -1111,10 +1191,9 @@ int jpp_gemm_f32(void* stream, const jpp_gemm_args* a) {
   p.ta = a->trans_a != 0; p.tb = a->trans_b != 0; p.epi = e; p.gelu_tanh = a->gelu_tanh;
   p.seg = a->seg; p.n_seg = a->n_seg; p.group_mode = a->group_mode;
   p.stride_b = a->stride_b; p.stride_c = a->stride_c;
-  // the tallest tile that still gives every CU one (a taller tile reads its B fewer times)
-  const long strips = (a->m / 16) * (a->n / 64) * (group_k ? a->n_seg : 1);
-  if (strips >= 4 * 256) return sgemm_launch<64>((hipStream_t)stream, p);
-  if (strips >= 2 * 256) return sgemm_launch<32>((hipStream_t)stream, p);
+  const int rows = tile_rows32((a->m / 16) * (a->n / 64) * (group_k ? a->n_seg : 1));
+  if (rows == 64) return sgemm_launch<64>((hipStream_t)stream, p);
+  if (rows == 32) return sgemm_launch<32>((hipStream_t)stream, p);
   return sgemm_launch<16>((hipStream_t)stream, p);
 }
 

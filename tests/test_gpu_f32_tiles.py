@@ -238,3 +238,28 @@ def test_attention_backward_f32_at_once_and_in_two(d, hq, hk, seq, batch, causal
             g[:, hq * d:] = bufs["qkv"].download(np.float32, (T, W))[:, hq * d:]
         got.append(g)
     assert np.array_equal(*got) and np.isfinite(got[0]).all() and (got[0] != 0).mean() > 0.9
+
+
+# a layer's ways: a launch per product; one launch, on tiles of 16 / 32 / 64 rows, with the sums along or behind
+@pytest.mark.parametrize("h,heads,f,seq,way", [
+    (512, 8, 2048, 1024, None), (128, 2, 256, 128, "along"), (128, 2, 512, 1152, "apart"), (256, 4, 512, 256, "along"),
+    (256, 4, 512, 1024, "apart"), (256, 4, 1024, 512, "apart"), (512, 8, 1024, 512, "along"), (384, 6, 768, 1024, "along"),
+    (512, 8, 1024, 1024, "apart")])
+def test_ways_of_a_layers_weight_gradients_f32(h, heads, f, seq, way):
+    """The way that the sizes choose, and the bits of the same gradients with the sums in front of them, on two
+    streams."""
+    print(f"wgrads_f32 {h} {f} {seq} {way}", flush=True)
+    spec = LayerSpec("bert", h, heads, f, seq, 1, n_kv_heads=heads, head_dim=64, causal=False, eps=1e-5, dtype="f32")
+    sched = S.Std1F1B(1)
+    plan = make_rank_plan(sched, 1, 0)
+    params = {0: [init_layer_params(spec, 3, 0, perturb=True)]}
+    _, _, two = run_on_gpu(spec, plan, 1, params, two_streams=True)
+    with rt.probe("*") as p:
+        _, _, one = run_on_gpu(spec, plan, 1, params, two_streams=False)
+    assert {k: v[0] for k, v in p.classes.items() if k.startswith("wgrads_f32")} == (
+        {} if way is None else {"wgrads_f32_sums" if way == "along" else "wgrads_f32": 1}), p.classes
+    _, _, want = run_on_oracle(spec, plan, params, S.preprocess_schedule_tasks(sched.tasks(1), 0, False)[0])
+    for name, w in want[0][0].items():
+        got = one[0][0][name]
+        assert np.array_equal(got, two[0][0][name]), name
+        parity.close(got, w.reshape(got.shape).astype(np.float64), 1e-4, name)
