@@ -556,33 +556,39 @@ AttnParams make_params(const jpp_attn_args* a) {
 // further from float64, 2.22e-3 instead of 2.19e-3.)
 bool small_fwd(const jpp_attn_args* a) { return (int64_t)a->batch * a->n_heads * a->seq <= 4096; }
 
-// Backward: where their expected time is shorter.  With x = workgroups of 16 queries per CU, g = query heads per key
-// head and S positions, in us:
-//   16 rows   c0 + c1 g S + x (c2 + c3 S)
+// Backward: where their expected time is shorter.  With x = workgroups of 16 queries per CU, y = workgroups of 16 keys
+// per CU, g = query heads per key head and S positions, in us:
+//   16 rows   c0 + c1 g S + x (c2 + c3 S) + c4 y
 //   blocks    c0 + c1 S + c2 g S + c3 x S
 // (a workgroup's own walk - one of keys walks the queries of all of its heads - and what the others add).
-// Least squares of the relative error over 440 problems (128 .. 2048 positions, 1 .. 8 sequences, 2 .. 32 heads, all
-// key head counts, up to 4096 rows); mean error of the blocks 3 - 5 %, of the 16 rows 13 %.  The shorter estimate costs
-// 0.1 - 0.6 % over the shorter time; a workgroup of 16 keys and two of 16 queries per CU, the rule before these kernels
-// took their operands through LDS, 10 - 20 %.  16 query and 4 key heads x 512 positions x 128 under a mask: 57 us in
-// blocks, 31 in one launch of 16 rows; 16 heads x 512 x 64: 27.3 and 21.1; distances from float64 the same.
+// Least squares of the relative error over 817 problems (128 .. 16384 positions, 1 .. 64 sequences, 1 .. 64 heads, all
+// key head counts, up to kSmallBwdRows rows in all; beyond those nothing is measured and the blocks stay); mean error of the
+// blocks 3 - 4 %, of the 16 rows 7 - 9 %.  The shorter estimate, the 16 rows' counted 2 % longer, costs 0.1 % over the
+// shorter time and is at worst 4 % slower than the blocks (16 % in one of 160 others: 5 sequences of 1152, 3 heads of
+// 64 under a mask, 43 us and 50 without the 2 %); without y, fitted up to 4096 rows, 22 % slower where many sequences have a head or two (64 x 256 positions, one head of 64: 22.4 us in blocks, 26.4).  A workgroup of 16
+// keys and two of 16 queries per CU, the rule before these kernels took their operands through LDS, costs 10 - 20 %.
+// 16 query and 4 key heads x 512 positions x 128 under a mask: 57 us in blocks, 31 in one launch of 16 rows; 16
+// heads x 512 x 64: 27.3 and 21.1; distances from float64 the same.
+constexpr int64_t kSmallBwdRows = 16384;
 struct SmallFit {
-  float rows16[4], blocks[4];
+  float rows16[5], blocks[4];
 };
 constexpr SmallFit kSmallBwd[2][2] = {   // [head 128][causal]
-    {{{3.81f, 0.00198f, 3.12f, 0.00784f}, {10.0f, 0.0101f, 0.0197f, 0.00116f}},
-     {{3.66f, 0.00254f, 3.25f, 0.00406f}, {15.5f, 0.0141f, 0.00793f, 0.00076f}}},
-    {{{5.37f, 0.00329f, 6.47f, 0.016f}, {16.2f, 0.0145f, 0.0405f, 0.003f}},
-     {{5.49f, 0.00447f, 6.39f, 0.00831f}, {23.6f, 0.0203f, 0.01f, 0.00129f}}}};
+    {{{3.54f, 0.00195f, 2.3f, 0.00709f, 2.39f}, {10.1f, 0.01f, 0.0198f, 0.000973f}},
+     {{3.27f, 0.00277f, 2.27f, 0.00327f, 2.6f}, {15.7f, 0.0149f, 0.00764f, 0.000348f}}},
+    {{{4.56f, 0.00395f, 5.14f, 0.0136f, 4.73f}, {16.2f, 0.0159f, 0.0407f, 0.00218f}},
+     {{4.37f, 0.006f, 4.53f, 0.00604f, 5.15f}, {24.f, 0.0203f, 0.00948f, 0.000991f}}}};
 
 // One launch writes dQ, dK and dV while it reads everything else, where two read only part of it:
 // a caller whose results lie over the inputs keeps the two.
 bool small_bwd(const jpp_attn_args* a) {
   const int64_t rows = (int64_t)a->batch * a->seq;
+  if (rows > kSmallBwdRows) return false;
   const SmallFit& f = kSmallBwd[a->head_dim == 128][a->causal != 0];
-  const float S = a->seq, gS = S * (a->n_heads / a->n_kv_heads), x = (float)rows * a->n_heads / 4096.f;
-  if (f.rows16[0] + f.rows16[1] * gS + x * (f.rows16[2] + f.rows16[3] * S) >=
-      f.blocks[0] + f.blocks[1] * S + f.blocks[2] * gS + f.blocks[3] * x * S)
+  const float S = a->seq, gS = S * (a->n_heads / a->n_kv_heads);
+  const float x = (float)rows * a->n_heads / 4096.f, y = (float)rows * a->n_kv_heads / 4096.f;
+  if (f.rows16[0] + f.rows16[1] * gS + x * (f.rows16[2] + f.rows16[3] * S) + f.rows16[4] * y >=
+      0.98f * (f.blocks[0] + f.blocks[1] * S + f.blocks[2] * gS + f.blocks[3] * x * S))
     return false;
   struct Range {
     uintptr_t lo, hi;
