@@ -35,14 +35,25 @@ __device__ __forceinline__ float adam_one(const AdamParams& p, float g, float w,
   return w - p.lr * mh / (sqrtf(vh) + p.eps);
 }
 
+template <bool CACHED, class T>
+__device__ __forceinline__ T fetch(const T* p) {
+  if constexpr (CACHED) return *p;
+  else return __builtin_nontemporal_load(p);
+}
+template <bool CACHED, class T>
+__device__ __forceinline__ void put(T v, T* p) {
+  if constexpr (CACHED) *p = v;
+  else __builtin_nontemporal_store(v, p);
+}
+
 // 8 parameters per lane: two 16-byte pieces of every f32 tensor, two of 8 bytes of the bf16, the second
 // 64 pieces behind the first, so that every access of a wave is one run of memory.  Ten streams of HBM
-// traffic and nothing else bound it.  Nothing is read again before the next step: all of it goes past the
-// caches (a tensor set that would fit the memory-side cache, 8.4e6 parameters, takes 50 us instead of 45,
-// 184e6 1253 instead of 1313).  One trip per wave: a grid that walks the tensors in strides has each
+// traffic and nothing else bound it.  One trip per wave: a grid that walks the tensors in strides has each
 // workgroup in ten far-apart places at a time (4.96 TB/s at 6e8 parameters, 5.53 without).  184e6 parameters
 // 1313 -> 1180 us, 6e8 4315 -> 3687.
-template <bool MASTER>
+// CACHED: through the caches, for tensors that the memory-side one may still hold from the gradients on (kCachedBytes).
+// Larger ones go past them: nothing is read again before the next step.
+template <bool MASTER, bool CACHED>
 __global__ __launch_bounds__(256) void adam_kernel(AdamParams p, long n8) {
   const int lane = threadIdx.x & 63;
   const long waves = (long)gridDim.x * 4;
@@ -54,13 +65,13 @@ __global__ __launch_bounds__(256) void adam_kernel(AdamParams p, long n8) {
     for (int u = 0; u < 2; ++u) {
       const long i = at + 64 * u;
       if (i >= end) continue;
-      g[u] = __builtin_nontemporal_load((const f32x4*)p.grad + i);
-      m[u] = __builtin_nontemporal_load((const f32x4*)p.m + i);
-      v[u] = __builtin_nontemporal_load((const f32x4*)p.v + i);
+      g[u] = fetch<CACHED>((const f32x4*)p.grad + i);
+      m[u] = fetch<CACHED>((const f32x4*)p.m + i);
+      v[u] = fetch<CACHED>((const f32x4*)p.v + i);
       if (MASTER) {
-        x[u] = __builtin_nontemporal_load((const f32x4*)p.master + i);
+        x[u] = fetch<CACHED>((const f32x4*)p.master + i);
       } else {
-        const u32x2 q = __builtin_nontemporal_load((const u32x2*)p.param + i);
+        const u32x2 q = fetch<CACHED>((const u32x2*)p.param + i);
         x[u] = f32x4{bf16lo_to_f32(q[0]), bf16hi_to_f32(q[0]), bf16lo_to_f32(q[1]), bf16hi_to_f32(q[1])};
       }
     }
@@ -75,13 +86,13 @@ __global__ __launch_bounds__(256) void adam_kernel(AdamParams p, long n8) {
         m[u][e] = me;
         v[u][e] = ve;
       }
-      __builtin_nontemporal_store(m[u], (f32x4*)p.m + i);
-      __builtin_nontemporal_store(v[u], (f32x4*)p.v + i);
-      if (MASTER) __builtin_nontemporal_store(x[u], (f32x4*)p.master + i);
+      put<CACHED>(m[u], (f32x4*)p.m + i);
+      put<CACHED>(v[u], (f32x4*)p.v + i);
+      if (MASTER) put<CACHED>(x[u], (f32x4*)p.master + i);
       if (p.param)
-        __builtin_nontemporal_store(u32x2{pack_bf16x2(x[u][0], x[u][1]), pack_bf16x2(x[u][2], x[u][3])},
+        put<CACHED>(u32x2{pack_bf16x2(x[u][0], x[u][1]), pack_bf16x2(x[u][2], x[u][3])},
                                     (u32x2*)p.param + i);
-      if (p.zero_grad) __builtin_nontemporal_store(f32x4{0.f, 0.f, 0.f, 0.f}, (f32x4*)p.grad + i);
+      if (p.zero_grad) put<CACHED>(f32x4{0.f, 0.f, 0.f, 0.f}, (f32x4*)p.grad + i);
     }
   }
 }
@@ -98,6 +109,12 @@ __global__ void adam_tail_kernel(AdamParams p, long start, long count) {
   if (p.param) p.param[i] = f32_to_bf16(w);
   if (p.zero_grad) p.grad[i] = 0.f;
 }
+
+// Bytes of all tensors of a step up to which it goes through the caches: three quarters of the memory-side one.  8.4e6
+// parameters (151 MB) again and again 38 us, past the caches 45; with 64 MB of other traffic between 39 and 48, with
+// 512 MB 60 and 49.  Rows with the step at their end (activations, weights and gradients between): 3.5e6 parameters
+// 607 us and 615, 7.1e6 699 and 710, 9.8e6 (177 MB) 3717 and 3720; 12.6e6 (227 MB) 3211 and 3157, 14.2e6 1821 and 1804.
+constexpr int64_t kCachedBytes = 192 << 20;
 
 }  // namespace
 
@@ -126,12 +143,15 @@ extern "C" int jpp_adam_step(void* stream, const jpp_adam_args* a) {
   hipStream_t st = (hipStream_t)stream;
   const double bytes = 12.0 + 8.0 + (a->master ? 8.0 : 2.0) + (a->param ? 2.0 : 0.0) +
                        (a->zero_grad ? 4.0 : 0.0);
+  const bool cached = a->count * (12 + (a->master ? 4 : 0) + (a->param ? 2 : 0)) <= kCachedBytes;
   ProbeScope probe(st, "adam", 0, bytes * a->count);
+  ProbeScope form(st, cached ? "adam_cached" : "adam_streamed", 0, bytes * a->count);   // (for a probe of one form alone)
   const long n8 = a->count / 8;
   const int grid = (int)std::min<long>(std::max<long>((n8 + 255) / 256, 1), 1 << 23);   // (2^31 threads)
   if (n8) {
-    if (a->master) hipLaunchKernelGGL(adam_kernel<true>, dim3(grid), dim3(256), 0, st, p, n8);
-    else hipLaunchKernelGGL(adam_kernel<false>, dim3(grid), dim3(256), 0, st, p, n8);
+    auto kern = a->master ? (cached ? adam_kernel<true, true> : adam_kernel<true, false>)
+                          : (cached ? adam_kernel<false, true> : adam_kernel<false, false>);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, st, p, n8);
   }
   if (a->count % 8) {
     if (a->master)

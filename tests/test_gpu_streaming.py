@@ -28,3 +28,38 @@ def test_fill_of_any_count_and_alignment(count, offset):
 @pytest.mark.parametrize("with_master", [True, False])
 def test_adam_of_partial_waves(count, with_master):
     optimizer.test_adam_flat(count, with_master)
+
+
+CACHED_BYTES = 192 << 20
+
+
+@pytest.mark.parametrize("with_master,with_param", [(True, True), (True, False), (False, True)])
+def test_adam_through_the_caches_and_past_them(with_master, with_param):
+    """Up to 192 MiB of tensors a step goes through the caches, larger ones past them: the form on either side of the
+    line, and the same bits from one call past them and two through them over the halves."""
+    per = 12 + 4 * with_master + 2 * with_param
+    line = CACHED_BYTES // per // 8 * 8
+    n = line + 8
+    print(f"adam {n} parameters, master {with_master}, param {with_param}", flush=True)
+    block = np.random.default_rng(per).standard_normal(1 << 20, dtype=np.float32)
+    long = np.resize(block, 4 * n)
+    start = {"grad": long[:n], "m": long[n // 2:n // 2 + n] * np.float32(0.1), "v": np.abs(long[7:7 + n]) * np.float32(0.01),
+             "master": long[n // 3:n // 3 + n], "param": rt.to_bf16_bits(long[n // 3:n // 3 + n])}
+
+    def run(parts):
+        b = {k: rt.DeviceBuffer.from_numpy(a) for k, a in start.items()}
+        for at, count, form in parts:
+            with rt.probe(form) as p:
+                rt.adam_step(count, b["grad"].ptr + 4 * at, b["m"].ptr + 4 * at, b["v"].ptr + 4 * at, 3,
+                             master=b["master"].ptr + 4 * at if with_master else None,
+                             param=b["param"].ptr + 2 * at if with_param else None, zero_grad=True)
+            assert p.launches == 1, (count, form)
+        return {k: b[k].download(a.dtype, a.shape) for k, a in start.items()}
+
+    half = n // 16 * 8
+    one = run([(0, n, "adam_streamed")])
+    two = run([(0, half, "adam_cached"), (half, n - half, "adam_cached")])
+    for k in start:
+        np.testing.assert_array_equal(one[k], two[k], err_msg=k)
+    assert (one["grad"] == 0).all() and not np.array_equal(one["m"], start["m"])
+    run([(0, line, "adam_cached")])
