@@ -61,8 +61,10 @@ int jpp_memcpy_d2h(void* dst, const void* src, size_t bytes);
 /* Many tensors between pageable host memory and the device in one call, ordered as jpp_memcpy_*: behind
  * everything queued on the null stream, complete when the call returns.  WORDS: 4-byte elements as they
  * are.  BF16: float32 on the host, bf16 on the device (to the device rounded to nearest even, ties by the
- * last bit kept).  Up to 8 host threads and 16 MiB of pinned memory work on a call; they are kept for the
- * next one until jpp_copy_release or the end of the process's last stage object gives them back. */
+ * last bit kept).  Up to 8 host threads and, per device, 16 MiB of pinned memory work on a call; they are kept
+ * for the next one until jpp_copy_release or the end of the process's last stage object gives them back.  One call at a
+ * time has them: one that finds them taken by another thread, or no pinned memory to be had, copies on its own
+ * thread. */
 typedef enum { JPP_COPY_WORDS = 0, JPP_COPY_BF16 = 1 } jpp_copy_kind;
 typedef struct {
   void* host;      /* 4-byte elements; only read by jpp_copy_h2d */

@@ -16,6 +16,7 @@
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
+#include <map>
 #include <mutex>
 #include <new>
 #include <thread>
@@ -30,6 +31,7 @@ namespace {
 constexpr int kLanes = 8;                 // at most; half of the process's CPUs
 constexpr size_t kSlot = 1 << 20;         // pinned bytes of a chunk, two per lane
 constexpr size_t kLeast = 256 << 10;      // no chunk smaller: an asynchronous copy takes 10 us to issue, one lane at a time
+constexpr size_t kAlone = 8 << 20;        // a chunk of a job without lanes
 
 struct Piece {   // consecutive elements of one item
   uint8_t* host;
@@ -46,6 +48,7 @@ struct Lane {
   uint8_t* slot[2] = {nullptr, nullptr};
 };
 struct Job {
+  Lane* lanes = nullptr;
   std::vector<Piece> pieces;
   std::vector<Chunk> chunks;
   bool up = false, bf16 = false;
@@ -79,6 +82,46 @@ void walk(const Job& j, const Chunk& c, uint8_t* slot) {
     else unpack(slot, j.pieces[i], j.bf16);
     slot += (size_t)j.pieces[i].count * es;
   }
+}
+
+// Cuts the items into chunks of at most `cut` bytes (a multiple of 4).
+void cut_items(Job& j, int n, const jpp_copy_item* items, size_t cut) {
+  const size_t es = j.bf16 ? 2 : 4;
+  j.pieces.clear();
+  j.chunks.clear();
+  for (int i = 0; i < n; ++i) {
+    int64_t left = items[i].count;
+    uint8_t *h = (uint8_t*)items[i].host, *d = (uint8_t*)items[i].device;
+    while (left > 0) {
+      if (j.chunks.empty() || j.chunks.back().bytes + es > cut || j.chunks.back().device + j.chunks.back().bytes != d)
+        j.chunks.push_back({d, 0, (int)j.pieces.size(), (int)j.pieces.size()});
+      Chunk& c = j.chunks.back();
+      const int64_t take = std::min(left, (int64_t)((cut - c.bytes) / es));
+      j.pieces.push_back({h, take});
+      c.last = (int)j.pieces.size();
+      c.bytes += (size_t)take * es;
+      h += take * 4;
+      d += (size_t)take * es;
+      left -= take;
+    }
+  }
+}
+
+// A whole job on the caller's thread and the null stream, without lanes: a chunk straight between host and device
+// where it is one tensor's words, else through pageable memory.
+hipError_t work_alone(const Job& j) {
+  std::vector<uint8_t> slot;
+  for (const Chunk& c : j.chunks) {
+    const bool direct = !j.bf16 && c.last - c.first == 1;
+    if (!direct && slot.size() < c.bytes) slot.resize(c.bytes);
+    uint8_t* const at = direct ? j.pieces[c.first].host : slot.data();
+    if (j.up && !direct) walk(j, c, at);
+    const hipError_t e = j.up ? hipMemcpy(c.device, at, c.bytes, hipMemcpyHostToDevice)
+                              : hipMemcpy(at, c.device, c.bytes, hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return e;
+    if (!j.up && !direct) walk(j, c, at);
+  }
+  return hipSuccess;
 }
 
 // One lane's share of a job.  Ends with nothing of it in flight, whatever failed.
@@ -120,9 +163,14 @@ void work(Job& j, Lane& l) {
   ok(hipStreamSynchronize(l.stream));
 }
 
-// The lanes' threads and pinned memory, made by the first copy that needs them and given back by
-// jpp_copy_release (at the latest; the last stage's end is one).  One job at a time: a second caller waits.
+// The lanes' threads, and for every device that is copied to or from the lanes' streams and pinned memory: made by the
+// first copy that needs them and given back by jpp_copy_release (at the latest; the last stage's end is one).  One job
+// has them at a time; who finds them taken copies without (work_alone).
 struct Pool {
+  struct Device {
+    Lane lanes[kLanes];
+    int n = 0;                     // those that are complete
+  };
   std::mutex call_mu;              // held for a whole job, and by release
   std::mutex mu;                   // guards what follows
   std::condition_variable wake, idle;
@@ -132,40 +180,48 @@ struct Pool {
   int lanes_wanted = 0, busy = 0;
   bool stop = false;
   Job* job = nullptr;
-  Lane lanes[kLanes];              // (call_mu) those of `device`
-  int device = -1, n_lanes = 0;
-  pid_t pid = 0;
+  std::map<int, Device> devices;   // (call_mu) by device
+  std::atomic<pid_t> pid{0};       // of the first copy
 
   static int most_lanes() {
     cpu_set_t set;
     const int cpus = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 2;
     return std::max(1, std::min(kLanes, cpus / 2));
   }
-  hipError_t open(int dev, int n) {
-    if (device != dev) close();
-    device = dev;
-    for (; n_lanes < n; ++n_lanes) {
-      Lane& l = lanes[n_lanes];
+  // Whether the pool is this process's own: the threads and streams of the one it was forked from are not here, and
+  // its locks may be held by nobody.
+  bool own() {
+    pid_t first = 0;
+    const pid_t here = getpid();
+    return pid.compare_exchange_strong(first, here) || first == here;
+  }
+  // the device's lanes, up to `n` of them: as many as there is memory for
+  Device& open(int dev, int n) {
+    Device& d = devices[dev];
+    for (; d.n < n; ++d.n) {
+      Lane& l = d.lanes[d.n];
       hipError_t e = l.stream ? hipSuccess : hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking);
       for (int s = 0; s < 2; ++s) {
         if (e == hipSuccess && !l.done[s]) e = hipEventCreateWithFlags(&l.done[s], hipEventDisableTiming);
         if (e == hipSuccess && !l.slot[s]) e = hipHostMalloc((void**)&l.slot[s], kSlot, hipHostMallocDefault);
       }
-      if (e != hipSuccess) return e;
+      if (e != hipSuccess) {
+        (void)hipGetLastError();   // (not for the next launch to report)
+        break;
+      }
     }
-    return hipSuccess;
+    return d;
   }
   void close() {
-    for (Lane& l : lanes) {
-      for (int s = 0; s < 2; ++s) {
-        if (l.done[s]) (void)hipEventDestroy(l.done[s]);
-        if (l.slot[s]) (void)hipHostFree(l.slot[s]);
+    for (auto& [dev, d] : devices)
+      for (Lane& l : d.lanes) {
+        for (int s = 0; s < 2; ++s) {
+          if (l.done[s]) (void)hipEventDestroy(l.done[s]);
+          if (l.slot[s]) (void)hipHostFree(l.slot[s]);
+        }
+        if (l.stream) (void)hipStreamDestroy(l.stream);
       }
-      if (l.stream) (void)hipStreamDestroy(l.stream);
-      l = Lane();
-    }
-    n_lanes = 0;
-    device = -1;
+    devices.clear();
   }
   void helper(int lane, uint64_t seen) {
     for (;;) {
@@ -182,7 +238,7 @@ struct Pool {
         if (lane >= lanes_wanted) continue;
         j = job;
       }
-      if (hipSetDevice(j->device) == hipSuccess) work(*j, lanes[lane]);
+      if (hipSetDevice(j->device) == hipSuccess) work(*j, j->lanes[lane]);
       std::lock_guard<std::mutex> lock(mu);
       if (--busy == 0) idle.notify_one();
     }
@@ -204,7 +260,7 @@ struct Pool {
       if (n > 1) hint = ++ticket;
     }
     if (n > 1) wake.notify_all();
-    work(j, lanes[0]);
+    work(j, j.lanes[0]);
     std::unique_lock<std::mutex> lock(mu);
     idle.wait(lock, [&] { return busy == 0; });
     job = nullptr;
@@ -241,38 +297,30 @@ int copy(int n, const jpp_copy_item* items, int kind, bool up) {
   if (total == 0) return JPP_OK;
   try {
     Pool& p = pool();
-    std::lock_guard<std::mutex> call(p.call_mu);
-    if (p.pid == 0) p.pid = getpid();
-    if (p.pid != getpid())
-      return jpp_set_error(JPP_ERR_STATE, "copy: the process was forked after its first copy");
-    const int most = Pool::most_lanes();
-    const size_t cut = std::min(kSlot, std::max(kLeast, (total / most + 4095) / 4096 * 4096));
+    if (!p.own()) return jpp_set_error(JPP_ERR_STATE, "copy: the process was forked after its first copy");
     Job j;
     j.up = up;
     j.bf16 = kind == JPP_COPY_BF16;
     JPP_CHECK_HIP(hipGetDevice(&j.device));
-    for (int i = 0; i < n; ++i) {
-      int64_t left = items[i].count;
-      uint8_t *h = (uint8_t*)items[i].host, *d = (uint8_t*)items[i].device;
-      while (left > 0) {
-        if (j.chunks.empty() || j.chunks.back().bytes + es > cut || j.chunks.back().device + j.chunks.back().bytes != d)
-          j.chunks.push_back({d, 0, (int)j.pieces.size(), (int)j.pieces.size()});
-        Chunk& c = j.chunks.back();
-        const int64_t take = std::min(left, (int64_t)((cut - c.bytes) / es));
-        j.pieces.push_back({h, take});
-        c.last = (int)j.pieces.size();
-        c.bytes += (size_t)take * es;
-        h += take * 4;
-        d += (size_t)take * es;
-        left -= take;
-      }
+    std::unique_lock<std::mutex> call(p.call_mu, std::try_to_lock);
+    Pool::Device* d = nullptr;
+    if (call.owns_lock()) {
+      const int most = Pool::most_lanes();
+      cut_items(j, n, items, std::min(kSlot, std::max(kLeast, (total / most + 4095) / 4096 * 4096)));
+      d = &p.open(j.device, (int)std::min<size_t>(most, j.chunks.size()));
     }
-    const int lanes = (int)std::min<size_t>(most, j.chunks.size());
-    JPP_CHECK_HIP(p.open(j.device, lanes));
-    // as a copy on the null stream: behind everything queued there, over when this returns
-    JPP_CHECK_HIP(hipStreamSynchronize(nullptr));
-    p.run(j, lanes);
-    const hipError_t e = (hipError_t)j.error.load();
+    hipError_t e;
+    if (d && d->n > 0) {
+      j.lanes = d->lanes;
+      // as a copy on the null stream: behind everything queued there, over when this returns
+      JPP_CHECK_HIP(hipStreamSynchronize(nullptr));
+      p.run(j, (int)std::min({(size_t)Pool::most_lanes(), (size_t)d->n, j.chunks.size()}));
+      e = (hipError_t)j.error.load();
+    } else {
+      if (d) call.unlock();
+      cut_items(j, n, items, kAlone);
+      e = work_alone(j);
+    }
     if (e != hipSuccess) return jpp_set_error(JPP_ERR_HIP, "copy: %s", hipGetErrorString(e));
     return JPP_OK;
   } catch (const std::exception& e) {
@@ -288,8 +336,9 @@ int jpp_copy_h2d(int n, const jpp_copy_item* items, int kind) { return copy(n, i
 int jpp_copy_d2h(int n, const jpp_copy_item* items, int kind) { return copy(n, items, kind, false); }
 int jpp_copy_release(void) {
   Pool& p = pool();
+  if (!p.pid || !p.own()) return JPP_OK;
   std::lock_guard<std::mutex> call(p.call_mu);
-  if (p.pid && p.pid == getpid()) p.release();
+  p.release();
   return JPP_OK;
 }
 
