@@ -615,26 +615,59 @@ def adam_step(count, grad, m, v, step, master=None, param=None, lr=1e-3, b1=0.9,
     check(load().jpp_adam_step(stream, C.byref(a)))
 
 
+# Elements of tensors that travel in one call, or one larger tensor (of a layer's results, the layer): what bounds the
+# host memory of arrays that are converted or reordered on the way.
+COPY_BATCH = 1 << 23
+
+
+def _copy_in_batches(items, bf16: bool):
+    """`copy_in` of the items that an iterator makes, some at a time."""
+    batch, total = [], 0
+    for item in items:
+        if batch and total + item[0].size > COPY_BATCH:
+            copy_in(batch, bf16)
+            batch, total = [], 0
+        batch.append(item)
+        total += item[0].size
+        del item
+    if batch:
+        copy_in(batch, bf16)
+
+
 def set_params(layers):
-    """`StageExecutor.set_params` of several layers in one copy per element type: a list of (executor, chunk,
-    layer, params)."""
+    """`StageExecutor.set_params` of several layers in as few copies as `COPY_BATCH` allows: a list of (executor,
+    chunk, layer, params)."""
     for bf16 in (False, True):
-        items = [it for ex, chunk, layer, params in layers if (ex.dtype != "f32") == bf16
-                 for it in ex._param_items(chunk, layer, params)]
-        if items:
-            copy_in(items, bf16)
+        _copy_in_batches((it for ex, chunk, layer, params in layers if (ex.dtype != "f32") == bf16
+                          for it in ex._param_items(chunk, layer, params)), bf16)
 
 
 def get_grads(layers) -> list:
-    """`StageExecutor.get_grads` of several layers in one copy: a list of (executor, chunk, layer)."""
-    items, results = [], []
+    """`StageExecutor.get_grads` of several layers in as few copies as `COPY_BATCH` allows: a list of (executor,
+    chunk, layer)."""
+    out, items, results = [], [], []
+
+    def flush():
+        copy_out(items)
+        items.clear()
+        while results:
+            out.append(results.pop(0)())
+
+    total = 0
     for ex, chunk, layer in layers:
         ex.join()
+        size = sum(r * c for _, r, c in ex.params)
+        if items and total + size > COPY_BATCH:
+            flush()
+            total = 0
         more, result = ex._result_layer(ex._layer_ptrs(load().jpp_stage_grad_ptr, chunk, layer), False)
         items += more
         results.append(result)
-    copy_out(items)
-    return [result() for result in results]
+        del more, result
+        total += size
+    if items:
+        flush()
+    return out
 
 
 class StageExecutor:
@@ -700,7 +733,8 @@ class StageExecutor:
 
         def result() -> dict:
             out = {}
-            for flat, first, last in runs:
+            while runs:           # (each run's array is given back before the next one's are reordered)
+                flat, first, last = runs.pop(0)
                 at = 0
                 for name, rows, cols in self.params[first:last]:
                     shape = (cols,) if rows == 1 and not name.startswith("W") else (rows, cols)
@@ -719,6 +753,7 @@ class StageExecutor:
     def _download_layer(self, ptrs, bf16: bool) -> dict:
         items, result = self._result_layer(ptrs, bf16)
         copy_out(items, bf16)
+        del items
         return result()
 
     def _layer_ptrs(self, fn, chunk: int, layer: int) -> list:
@@ -731,8 +766,8 @@ class StageExecutor:
         first = self._ptr(fn, chunk, layer, self.params[0][0])
         return [first + es * d for d in self._places]
 
-    def _param_items(self, chunk: int, layer: int, params: dict) -> list:
-        items = []
+    def _param_items(self, chunk: int, layer: int, params: dict):
+        """The items of a copy of a layer's parameters, one after the other."""
         ptrs = self._layer_ptrs(load().jpp_stage_param_ptr, chunk, layer)
         for (name, rows, cols), ptr in zip(self.params, ptrs):
             a = np.ascontiguousarray(params[name], dtype=np.float32)
@@ -740,12 +775,11 @@ class StageExecutor:
             order = self._device_columns(name, cols)
             if order is not None:
                 a = np.ascontiguousarray(a.reshape(rows, cols)[:, order])
-            items.append((a, ptr))
-        return items
+            yield a, ptr
 
     def set_params(self, chunk: int, layer: int, params: dict):
         """Upload float32 host arrays as device parameters (bf16, or f32 for an f32 stage)."""
-        copy_in(self._param_items(chunk, layer, params), self.dtype != "f32")
+        _copy_in_batches(self._param_items(chunk, layer, params), self.dtype != "f32")
 
     def get_params(self, chunk: int, layer: int) -> dict:
         """The device parameters as float32 host arrays."""
