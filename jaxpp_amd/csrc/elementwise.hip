@@ -714,15 +714,22 @@ __global__ __launch_bounds__(256) void cast_bf16_f32_kernel(const bf16_t* __rest
     dst[i] = bf16_to_f32(src[i]);
 }
 // 64 bytes a thread in four runs of its workgroup, one trip each (12 GB 2120 us in strides through the whole
-// tensor, 1999 like this; past the caches 2040, and 32 us instead of 24 for a tensor of 184 MB).  `dst` need only
-// be aligned to its elements.
+// tensor, 1999 like this; past the caches 2040, and 32 us instead of 24 for a tensor of 184 MB) up to the largest grid,
+// more beyond.  `dst` need only be aligned to its elements.
+constexpr long kFillMostBlocks = 1 << 23;   // (2^31 threads; 128 GiB in one trip)
+constexpr long fill_blocks(size_t count) {
+  return count / 4096 < (size_t)kFillMostBlocks ? (long)(count / 4096) + 1 : kFillMostBlocks;
+}
+static_assert(fill_blocks(1) == 1 && fill_blocks(4096) == 2 && fill_blocks(~(size_t)0) * 256 < 1L << 32, "grid limits");
+
 typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* dst, uint32_t v, long n) {
-  const long n4 = n / 4, at = (long)blockIdx.x * 1024 + threadIdx.x;
+  const long n4 = n / 4, first = (long)blockIdx.x * 1024 + threadIdx.x;
+  for (long at = first; at < n4; at += (long)gridDim.x * 1024)
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
-    if (at + 256 * u < n4) ((u32x4_u*)dst)[at + 256 * u] = u32x4_u{v, v, v, v};
-  if (at < n - n4 * 4) dst[n4 * 4 + at] = v;
+    for (int u = 0; u < 4; ++u)
+      if (at + 256 * u < n4) ((u32x4_u*)dst)[at + 256 * u] = u32x4_u{v, v, v, v};
+  if (first < n - n4 * 4) dst[n4 * 4 + first] = v;
 }
 
 // loss of the last stage: mean((out - target)^2) * scale, and its cotangent
@@ -1082,9 +1089,7 @@ int jpp_fill_u32(void* dst, uint32_t value, size_t count, void* stream) {
   JPP_REQUIRE(dst || count == 0, "fill: null destination");
   if (count == 0) return JPP_OK;
   ProbeScope probe((hipStream_t)stream, "fill", 0, 4.0 * count);
-  JPP_REQUIRE(count < (size_t)1 << 40, "fill: too large");
-  const unsigned blocks = (unsigned)(count / 4096 + 1);
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, (uint32_t*)dst, value,
+  hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)fill_blocks(count)), dim3(256), 0, (hipStream_t)stream, (uint32_t*)dst, value,
                      (long)count);
   JPP_LAUNCH_CHECK();
   return JPP_OK;

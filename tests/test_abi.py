@@ -4,6 +4,8 @@ import ctypes
 import os
 import re
 
+import pytest
+
 from jaxpp_amd import runtime as rt
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -61,6 +63,18 @@ def test_error_convention_without_gpu():
     assert lib.jpp_grad_accum_f32(None, None, None, 0, 0) == -1
     assert lib.jpp_adam_step(None, None) == -1
     assert lib.jpp_stage_adam_step(None, None, 1, 0.0, 0.0, 0.0, 0.0, 0.0) == -1
+
+
+def test_a_fill_of_any_size_is_left_to_the_device():
+    """No size is refused in advance (what there is no memory for cannot be a tensor): without a device the launch is
+    what fails."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("a launch would reach the device")
+    lib = rt.load()
+    for count in (1, 1 << 36, 1 << 41):
+        assert lib.jpp_fill_u32(64, 0, count, None) != 0
+        assert b"launch" in lib.jpp_last_error(), (count, lib.jpp_last_error())
 
 
 def test_a_tile_narrower_than_a_rotated_head_is_refused():

@@ -30,6 +30,20 @@ def test_adam_of_partial_waves(count, with_master):
     optimizer.test_adam_flat(count, with_master)
 
 
+def test_fill_of_more_than_the_largest_grid_takes_in_one_trip():
+    """128 GiB are a workgroup's single trip in the largest grid; 24 KB and 12 bytes more, a second trip for some."""
+    count = (1 << 35) + 6 * 1024 + 3
+    print(f"fill {count}", flush=True)
+    buf = rt.DeviceBuffer(4 * (count + 1))
+    rt.check(rt.load().jpp_fill_u32(buf.ptr, 5, count + 1, None))
+    rt.check(rt.load().jpp_fill_u32(buf.ptr, 0xabcd1234, count, None))
+    for at in (0, (1 << 34) - 4096, (1 << 35) - 8192, (1 << 35) - 4, count - 6000):
+        n = min(16384, count - at)
+        assert (buf.download(np.uint32, (n,), 4 * at) == 0xabcd1234).all(), at
+    assert buf.download(np.uint32, (1,), 4 * count)[0] == 5
+    buf.free()
+
+
 CACHED_BYTES = 192 << 20
 
 
