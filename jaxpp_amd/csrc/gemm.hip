@@ -1000,7 +1000,9 @@ int launch_tiled(hipStream_t stream, GemmParams& p, int tile, bool deep) {
 // tiles on, else 128x128: 36 % on average) it is slower by more than 2 % for 12 of the 1300, all but one by
 // 6 % at most (180 tiles of 256x256, 3 K-steps: 14 %): a 512 x 1024 x 4096 input gradient has 32 tiles of
 // 128x128 for 256 CUs and took 28 us, 15 us as 128 tiles of 64x64 with two wave groups each.
-// Weight gradients: 420 launches of 1 to 4 products (outputs 128 .. 8192 a side, 64 .. 8192 tokens), mean
+// 200 weight gradients that are not added to anything (written as bf16 or f32) are priced alike: 0.1 % over the measured
+// best, 10 % at worst; as accumulated ones 0.5 % and 22 % (2304 x 768 x 256: 7.0 us, 6.0 as 64x64).
+// Accumulated weight gradients: 420 launches of 1 to 4 products (outputs 128 .. 8192 a side, 64 .. 8192 tokens), mean
 // error 2 - 11 %; the smallest estimate costs 0.3 % against the measured best.  256x256 from 192 tiles on
 // cost 9 % there and 36 % at worst (300 tiles, 2 K-steps: 44 us, 33 as 128x128; 1176 tiles, 4: 135 and 121): a
 // 256x256 tile, alone on its CU, waits for its fp32 tile apart from its K-steps, of two 128x128 tiles one's
@@ -1024,7 +1026,8 @@ constexpr TileForm kWeightGrad[] = {
 
 // tile with the smallest estimate for products of these extents in one grid (`grid`: the extents
 // that its form goes by)
-int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool wgrad, bool gelu, bool may_128x256) {
+int cheapest_tile(const Extent* e, const Extent* grid, int n, long ksteps, bool wgrad /* accumulated */, bool gelu,
+                  bool may_128x256) {
   int best = kTile128;
   float best_us = 0.f;
   for (const TileForm& f : wgrad ? kWeightGrad : kForward) {
@@ -1049,8 +1052,8 @@ int choose_tile(const jpp_gemm_args* a) {
   const Extent e = work_extent(a);
   if (a->group_mode != JPP_GROUP_NONE && !a->group_rows) return kTile256;
   const long t256 = e.m % 256 == 0 && e.n % 256 == 0 ? (e.m / 256) * (e.n / 256) : 0;
-  const bool wgrad = a->trans_a && a->trans_b;
-  if (t256 >= kMostCus && !(wgrad && a->epilogue == JPP_EPI_ACC_F32)) return kTile256;
+  const bool wgrad = a->trans_a && a->trans_b && a->epilogue == JPP_EPI_ACC_F32;
+  if (t256 >= kMostCus && !wgrad) return kTile256;
   const Extent grid = grid_extent(a);
   const bool gelu = a->epilogue == JPP_EPI_GELU || a->epilogue == JPP_EPI_DGELU;
   const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), wgrad, gelu, true);

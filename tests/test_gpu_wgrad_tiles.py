@@ -48,3 +48,29 @@ def test_form_of_a_weight_gradient(m, n, k, form):
         rt.gemm(a.ptr, b.ptr, c.ptr, m, n, k, m, n, n, 1, 1, rt.EPI_ACC_F32)
         rt.sync()
     assert list(p.classes) == [f"gemm_tn_accf32_{form}"], p.classes
+
+
+@pytest.mark.parametrize("epi,name", [(rt.EPI_BF16, "bf16"), (rt.EPI_F32, "f32")])
+@pytest.mark.parametrize("m,n,k,form", [(2304, 768, 256, "64x64k2"), (6912, 1792, 704, "256x256w8"),
+                                        (640, 3200, 64, "64x64k2"), (1024, 1024, 1024, "64x64s4k2")])
+def test_form_of_a_weight_gradient_that_is_not_accumulated(m, n, k, form, epi, name):
+    """Products of the same layout without an old value go by the estimate of products without one; the bits are
+    those of the tile asked for by name, and the values float64's to a bf16 rounding (fp32 sums of terms of
+    size 0.3: 1e-4 sqrt(K))."""
+    print(f"weight gradient {m}x{n}x{k} {name}: {form}", flush=True)
+    rng = np.random.default_rng(m + k)
+    a, b = rnd(rng, k, m), rnd(rng, k, n, scale=0.3)
+    da, db = dev_bf16(a), dev_bf16(b)
+    es = 2 if epi == rt.EPI_BF16 else 4
+    own, named = rt.DeviceBuffer(es * m * n), rt.DeviceBuffer(es * m * n)
+    with rt.probe("*") as p:
+        rt.gemm(da.ptr, db.ptr, own.ptr, m, n, k, m, n, n, 1, 1, epi)
+        rt.sync()
+    assert list(p.classes) == [f"gemm_tn_{name}_{form}"], p.classes
+    rt.gemm(da.ptr, db.ptr, named.ptr, m, n, k, m, n, n, 1, 1, epi, tile={"64": 5, "128": 1, "256": 4}[form.split("x")[0]])
+    rt.sync()
+    dt = np.uint16 if es == 2 else np.uint32
+    np.testing.assert_array_equal(own.download(dt, (m, n)), named.download(dt, (m, n)))
+    got = own.download_bf16((m, n)) if es == 2 else own.download(np.float32, (m, n))
+    want = a.astype(np.float64).T @ b.astype(np.float64)
+    assert (np.abs(got - want) <= 1e-4 * math.sqrt(k) + (2.0 ** -8 * np.abs(want) if es == 2 else 0)).all()
