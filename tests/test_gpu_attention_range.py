@@ -21,9 +21,7 @@ def _gpu():
                                               (64, 0, 16, 4, 2, 512), (64, 0, 12, 12, 1, 384), (128, 1, 4, 1, 2, 128)])
 @pytest.mark.parametrize("pad,rope", [(0, False), (8, True)])
 def test_larger_problems_of_16_rows_equal_whole_blocks(d, causal, H, K, B, S, pad, rope):
-    with rt.probe("*") as p:
-        small.test_small_attention_equals_whole_blocks(d, causal, H, K, B, S, pad, rope)
-    assert p.classes["attn_bwd_small"][0] == 1 and p.classes["attn_bwd_dq"][0] == 1, p.classes
+    small.test_small_attention_equals_whole_blocks(d, causal, H, K, B, S, pad, rope)
 
 
 @pytest.mark.parametrize("d,causal,H,K,B,S,own", [

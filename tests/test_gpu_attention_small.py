@@ -56,11 +56,15 @@ def run(q, k, v, do, causal, pad, rope):
 def test_small_attention_equals_whole_blocks(d, causal, H, K, B, S, pad, rope):
     print(f"attention d={d} causal={causal} heads={H}/{K} b={B} s={S} pad={pad} rope={rope}", flush=True)
     rng = np.random.default_rng(d + S + H)
-    more = 16384 // (K * S) + 1                        # (past every limit of the 16-row kernels)
+    more = 16384 // (K * S) + 1     # (the blocks' side of both rules; the launches below are checked)
     draw = lambda h: L.bf16_round(rng.standard_normal((B + more, S, h, d), dtype=np.float32))
     q, k, v, do = draw(H), draw(K), draw(K), draw(H)
-    small = run(*(x[:B] for x in (q, k, v, do)), causal, pad, rope)
-    large = run(q, k, v, do, causal, pad, rope)
+    with rt.probe("*") as p:
+        small = run(*(x[:B] for x in (q, k, v, do)), causal, pad, rope)
+    assert "attn_bwd_small" in p.classes and "attn_bwd_dq" not in p.classes, p.classes
+    with rt.probe("*") as p:
+        large = run(q, k, v, do, causal, pad, rope)
+    assert "attn_bwd_small" not in p.classes and p.classes["attn_bwd_dq"][0] == 1, p.classes
     for name, s, g in zip(("o", "dqkv"), small, large):
         g = g[:B]
         assert np.abs(s - g).max() <= 2e-2 * np.abs(g).max(), name
