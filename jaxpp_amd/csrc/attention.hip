@@ -563,10 +563,13 @@ bool small_fwd(const jpp_attn_args* a) { return (int64_t)a->batch * a->n_heads *
 // (a workgroup's own walk - one of keys walks the queries of all of its heads - and what the others add).
 // Least squares of the relative error over 817 problems (128 .. 16384 positions, 1 .. 64 sequences, 1 .. 64 heads, all
 // key head counts, up to kSmallBwdRows rows in all; beyond those nothing is measured and the blocks stay); mean error of the
-// blocks 3 - 4 %, of the 16 rows 7 - 9 %.  The shorter estimate, the 16 rows' counted 2 % longer, costs 0.1 % over the
-// shorter time and is at worst 4 % slower than the blocks (16 % in one of 160 others: 5 sequences of 1152, 3 heads of
-// 64 under a mask, 43 us and 50 without the 2 %); without y, fitted up to 4096 rows, 22 % slower where many sequences have a head or two (64 x 256 positions, one head of 64: 22.4 us in blocks, 26.4).  A workgroup of 16
-// keys and two of 16 queries per CU, the rule before these kernels took their operands through LDS, costs 10 - 20 %.
+// blocks 3 - 4 %, of the 16 rows 7 - 9 %.  The 16 rows' are counted 5 % longer: their time goes up by steps, whole
+// rounds of workgroups, where the estimate is smooth.  Over 600 other problems, 366 of them near
+// or on the 16 rows' side, the choice costs 0.04 % over the shorter time and is at worst 4 % slower than the blocks (counted 2 % longer 0.2 % and 17 %: 3 sequences of 1536, 3 heads of 64
+// without a mask, 61.4 us in blocks and 72; 23 heads of 64 x 640 under one 32.4 and 35.6); without y, fitted up
+// to 4096 rows, 22 % slower where many sequences have a head or two (64 x 256 positions, one head of 64: 22.4 us in
+// blocks, 26.4).  A workgroup of 16 keys and two of 16 queries per CU, the rule before these kernels took their operands
+// through LDS, costs 10 - 20 %.
 // 16 query and 4 key heads x 512 positions x 128 under a mask: 57 us in blocks, 31 in one launch of 16 rows; 16
 // heads x 512 x 64: 27.3 and 21.1; distances from float64 the same.
 constexpr int64_t kSmallBwdRows = 16384;
@@ -588,7 +591,7 @@ bool small_bwd(const jpp_attn_args* a) {
   const float S = a->seq, gS = S * (a->n_heads / a->n_kv_heads);
   const float x = (float)rows * a->n_heads / 4096.f, y = (float)rows * a->n_kv_heads / 4096.f;
   if (f.rows16[0] + f.rows16[1] * gS + x * (f.rows16[2] + f.rows16[3] * S) + f.rows16[4] * y >=
-      0.98f * (f.blocks[0] + f.blocks[1] * S + f.blocks[2] * gS + f.blocks[3] * x * S))
+      0.95f * (f.blocks[0] + f.blocks[1] * S + f.blocks[2] * gS + f.blocks[3] * x * S))
     return false;
   struct Range {
     uintptr_t lo, hi;

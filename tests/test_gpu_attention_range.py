@@ -46,6 +46,8 @@ def test_side_of_the_estimate(d, causal, H, K, B, S, own):
     # many sequences of a head or two (more workgroups of keys than CUs), and beyond every measured size
     (64, 1, 1, 1, 64, 256, False), (128, 1, 2, 2, 16, 384, False), (128, 1, 1, 1, 32, 384, False),
     (64, 0, 1, 1, 130, 128, False),
+    # where the estimates are close and a round of workgroups more makes the 16 rows the slower side
+    (64, 0, 3, 3, 3, 1536, False), (128, 0, 5, 5, 2, 1280, False), (64, 1, 23, 23, 1, 640, False),
     # the sizes up to 4096 rows keep their side, and long sequences of one head theirs
     (64, 0, 2, 2, 8, 256, True), (128, 0, 4, 1, 1, 2048, True), (128, 1, 1, 1, 1, 8192, True)])
 def test_side_of_the_estimate_with_many_rows(d, causal, H, K, B, S, own):
