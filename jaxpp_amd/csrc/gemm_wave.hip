@@ -30,7 +30,7 @@ namespace {
 
 constexpr int PITCH = 68;                      // floats of a row of the sums
 
-// BM: rows of a tile; W: waves, at most one per SIMD; NS: stages of a wave
+// BM: rows of a tile; W: waves, one or two per SIMD; NS: stages of a wave
 template <bool TB, int EPI, int BM, int W, int NS>
 __global__ __launch_bounds__(64 * W) void gemm_wave_kernel(GemmWave p) {
   constexpr int TM = BM / 16;
@@ -208,15 +208,16 @@ int launch(hipStream_t st, const GemmWave& p) {
   return JPP_OK;
 }
 
-}  // namespace
-
 template <bool TB, int EPI>
 int launch_rows(hipStream_t st, const GemmWave& p, int rows) {
   if (rows == 32) return launch<TB, EPI, 32, 4, 3>(st, p);
   return EPI == JPP_EPI_BF16 ? launch<TB, EPI, 64, 4, 2>(st, p) : launch<TB, EPI, 64, 8, 1>(st, p);
 }
 
+}  // namespace
+
 int launch_gemm_wave(hipStream_t st, const GemmWave& p, bool tb, int epi, int rows) {
-  if (tb) return epi == JPP_EPI_BF16 ? launch_rows<true, JPP_EPI_BF16>(st, p, rows) : launch_rows<true, JPP_EPI_GELU>(st, p, rows);
-  return epi == JPP_EPI_BF16 ? launch_rows<false, JPP_EPI_BF16>(st, p, rows) : launch_rows<false, JPP_EPI_DGELU>(st, p, rows);
+  const bool plain = epi == JPP_EPI_BF16;
+  if (tb) return plain ? launch_rows<true, JPP_EPI_BF16>(st, p, rows) : launch_rows<true, JPP_EPI_GELU>(st, p, rows);
+  return plain ? launch_rows<false, JPP_EPI_BF16>(st, p, rows) : launch_rows<false, JPP_EPI_DGELU>(st, p, rows);
 }
