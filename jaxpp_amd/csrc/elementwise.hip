@@ -55,11 +55,13 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 
 // ---------------------------------------------------------------------------
-// norm forward: one wave per row, the row cached in registers.  With copy_dst it also carries a tensor of the same
-// shape, copy_src, there (copy_src = nullptr: x itself): a stage keeps its input like this instead of by a
-// copy of its own in front of the first layer.
+// norm forward: one wave per row, the row cached in registers.  COPY: it also carries a tensor of the same
+// shape, copy_src, to copy_dst (copy_src = nullptr: x itself): a stage keeps its input like this instead of by a
+// copy of its own in front of the first layer.  An instance of its own: as a branch, though not taken, it keeps the loads of
+// the scale and shift behind the row's sums (192 x 320 without a copy 3.1 us with it, 2.95 without; 5 % of rows of up to
+// 1024 columns, 1 % beyond).
 // ---------------------------------------------------------------------------
-template <bool LN, int NCH>
+template <bool LN, int NCH, bool COPY>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const bf16_t* __restrict__ x,
                                                        const bf16_t* __restrict__ gamma,
                                                        const bf16_t* __restrict__ beta,
@@ -75,12 +77,20 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const bf16_t* __restrict_
   const int nchunk = cols >> 3;
   const uint4* xr = (const uint4*)(x + row * cols);
   uint4 v[NCH];
+  float s = 0.f;
+  auto add = [&](int i) {
+    float f[8];
+    unpack8(v[i], f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += LN ? f[e] : f[e] * f[e];
+  };
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int c = lane + 64 * i;
     v[i] = c < nchunk ? xr[c] : make_uint4(0, 0, 0, 0);
+    if constexpr (!COPY) add(i);
   }
-  if (copy_dst) {
+  if constexpr (COPY) {
     uint4* dst = (uint4*)(copy_dst + row * cols);
     if (copy_src) {
       const uint4* src = (const uint4*)(copy_src + row * cols);
@@ -90,14 +100,8 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const bf16_t* __restrict_
       for (int i = 0; i < NCH; ++i)
         if (lane + 64 * i < nchunk) dst[lane + 64 * i] = v[i];
     }
-  }
-  float s = 0.f;
 #pragma unroll
-  for (int i = 0; i < NCH; ++i) {
-    float f[8];
-    unpack8(v[i], f);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s += LN ? f[e] : f[e] * f[e];
+    for (int i = 0; i < NCH; ++i) add(i);
   }
   s = wave_sum(s);
   float mean = 0.f, var;
@@ -775,9 +779,9 @@ int launch_norm_fwd(hipStream_t st, const jpp_norm_args* a, const void* copy_src
   const int blocks = (int)((a->rows + 3) / 4);
   const int nch = (int)((a->cols / 8 + 63) / 64);
 #define JPP_NF(N)                                                                            \
-  hipLaunchKernelGGL((norm_fwd_kernel<LN, N>), dim3(blocks), dim3(256), 0, st,               \
-                     (const bf16_t*)a->x, (const bf16_t*)a->gamma, (const bf16_t*)a->beta,   \
-                     (bf16_t*)a->y, a->mean, a->rstd, (long)a->rows, (int)a->cols, a->eps,     \
+  hipLaunchKernelGGL((copy_dst ? norm_fwd_kernel<LN, N, true> : norm_fwd_kernel<LN, N, false>), dim3(blocks), \
+                     dim3(256), 0, st, (const bf16_t*)a->x, (const bf16_t*)a->gamma, (const bf16_t*)a->beta, \
+                     (bf16_t*)a->y, a->mean, a->rstd, (long)a->rows, (int)a->cols, a->eps,   \
                      (const bf16_t*)copy_src, (bf16_t*)copy_dst)
   if (nch <= 1) JPP_NF(1);
   else if (nch <= 2) JPP_NF(2);
