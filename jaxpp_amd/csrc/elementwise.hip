@@ -727,12 +727,16 @@ constexpr long fill_blocks(size_t count) {
 static_assert(fill_blocks(1) == 1 && fill_blocks(4096) == 2 && fill_blocks(~(size_t)0) * 256 < 1L << 32, "grid limits");
 
 typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool STRIDES>
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* dst, uint32_t v, long n) {
   const long n4 = n / 4, first = (long)blockIdx.x * 1024 + threadIdx.x;
-  for (long at = first; at < n4; at += (long)gridDim.x * 1024)
+  long at = first;
+  do {
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (at + 256 * u < n4) ((u32x4_u*)dst)[at + 256 * u] = u32x4_u{v, v, v, v};
+    at += (long)gridDim.x * 1024;
+  } while (STRIDES && at < n4);
   if (first < n - n4 * 4) dst[n4 * 4 + first] = v;
 }
 
@@ -1093,8 +1097,9 @@ int jpp_fill_u32(void* dst, uint32_t value, size_t count, void* stream) {
   JPP_REQUIRE(dst || count == 0, "fill: null destination");
   if (count == 0) return JPP_OK;
   ProbeScope probe((hipStream_t)stream, "fill", 0, 4.0 * count);
-  hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)fill_blocks(count)), dim3(256), 0, (hipStream_t)stream, (uint32_t*)dst, value,
-                     (long)count);
+  const long blocks = fill_blocks(count);
+  hipLaunchKernelGGL((blocks < kFillMostBlocks ? fill_u32_kernel<false> : fill_u32_kernel<true>), dim3((unsigned)blocks), dim3(256), 0,
+                     (hipStream_t)stream, (uint32_t*)dst, value, (long)count);
   JPP_LAUNCH_CHECK();
   return JPP_OK;
 }
