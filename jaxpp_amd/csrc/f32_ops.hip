@@ -365,7 +365,7 @@ int sgemm_launch(hipStream_t st, const SgemmParams& p) {
 // ---------------------------------------------------------------------------
 // N > 0: rows of at most 64 N columns, which a lane holds in registers, with its share of the scale and shift: one
 // trip to memory instead of three loops of loads that wait for each other (512 x 256: 5.5 -> 3.2 us).
-template <int N>
+template <int N, bool COPY>
 __global__ __launch_bounds__(256) void norm_fwd32_kernel(const float* __restrict__ x,
                                                          const float* __restrict__ gamma,
                                                          const float* __restrict__ beta,
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(256) void norm_fwd32_kernel(const float* __restrict
     g[i] = in ? gamma[c] : 0.f;
     b[i] = in && beta ? beta[c] : 0.f;
   }
-  if (copy_dst) {   // (as in the bf16 norm: the stage's input)
+  if constexpr (COPY) {   // (as in the bf16 norm: the stage's input)
     if constexpr (N > 0) {
       float w[N];
 #pragma unroll
@@ -1139,8 +1139,9 @@ int jpp_norm_fwd_copy_f32(hipStream_t stream, const jpp_norm_args* a, const void
   JPP_REQUIRE(a->rows > 0 && a->cols > 0, "norm_fwd_f32: empty");
   JPP_REQUIRE((a->beta == nullptr) == (a->mean == nullptr),
               "norm_fwd_f32: beta and mean are both given (LayerNorm) or both NULL (RMSNorm)");
-  auto kern = a->cols <= 256 ? norm_fwd32_kernel<4> : a->cols <= 512 ? norm_fwd32_kernel<8>
-              : a->cols <= 1024 ? norm_fwd32_kernel<16> : norm_fwd32_kernel<0>;
+#define JPP_NF32(N) (copy_dst ? norm_fwd32_kernel<N, true> : norm_fwd32_kernel<N, false>)
+  auto kern = a->cols <= 256 ? JPP_NF32(4) : a->cols <= 512 ? JPP_NF32(8) : a->cols <= 1024 ? JPP_NF32(16) : JPP_NF32(0);
+#undef JPP_NF32
   hipLaunchKernelGGL(kern, dim3((unsigned)((a->rows + 3) / 4)), dim3(256), 0, stream, (const float*)a->x,
                      (const float*)a->gamma, (const float*)a->beta, (float*)a->y, a->mean, a->rstd, (long)a->rows,
                      (int)a->cols, a->eps, (const float*)copy_src, (float*)copy_dst);
