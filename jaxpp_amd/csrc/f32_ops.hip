@@ -878,15 +878,31 @@ __device__ __forceinline__ void dq_tile32(const Attn32& p, float* buf, int qt, i
   store_sum32<D, W>(dq, buf, p.dq + (row0 + q0) * p.lddq + h * D, p.lddq);
 }
 
-// dK, dV of 16 keys: the waves take the 16-query tiles of every head of the keys' group in turn.  ALONE: delta is not
-// there yet and is formed here too (the same value).
-template <int D, bool ALONE>
-__device__ __forceinline__ void dkv_tile32(const Attn32& p, float* buf, int kt, int hk, int b) {
+template <int D>
+__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dq32_kernel(Attn32 p) {
+  __shared__ float buf[kAttnWaves32<D> * 16 * D];
+  dq_tile32<D>(p, buf, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// dK, dV of 16 keys: the waves take the 16-query tiles of every head of the keys' group in turn.  WITH_DQ: the whole
+// backward in one launch (blockIdx.y: key heads, whose workgroups take longer, in front of the query heads).  delta is not
+// there yet then and is formed here too (the same value).  (As a function that two kernels call, the registers
+// of the one behind attn_dq32_kernel fall out worse: 7 heads of 128 on one key head, 2 x 640 rows under a mask 318 us, 305
+// like this.)
+template <int D, bool WITH_DQ>
+__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dkv32_kernel(Attn32 p) {
   constexpr int W = kAttnWaves32<D>;
+  __shared__ float buf[W * 16 * D];
+  if constexpr (WITH_DQ) {
+    if ((int)blockIdx.y >= p.n_kv_heads) {
+      dq_tile32<D>(p, buf, blockIdx.x, blockIdx.y - p.n_kv_heads, blockIdx.z);
+      return;
+    }
+  }
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int grp = p.n_heads / p.n_kv_heads;
-  const int k0 = kt * 16;
+  const int hk = blockIdx.y, b = blockIdx.z, grp = p.n_heads / p.n_kv_heads;
+  const int k0 = blockIdx.x * 16;
   const long row0 = (long)b * p.seq;
   Rows32<D> kr, vr;
   kr.load(p.k + (row0 + k0) * p.ldk + hk * D, p.ldk, c, g);
@@ -908,7 +924,7 @@ __device__ __forceinline__ void dkv_tile32(const Attn32& p, float* buf, int kt, 
     const long stat = ((long)b * p.n_heads + h) * p.seq + q0 + 4 * g;
     const f32x4 lse = *(const f32x4_u*)(p.lse + stat);
     f32x4 dl;
-    if constexpr (ALONE) {
+    if constexpr (WITH_DQ) {
       const float own = row_delta32<D>(gr, p.o + (row0 + q0) * p.ldo + h * D, p.ldo, c, g);
 #pragma unroll
       for (int r = 0; r < 4; ++r) dl[r] = __shfl(own, 4 * g + r);
@@ -929,24 +945,6 @@ __device__ __forceinline__ void dkv_tile32(const Attn32& p, float* buf, int kt, 
   store_sum32<D, W>(dv, buf, p.dv + (row0 + k0) * p.lddv + hk * D, p.lddv);
   __syncthreads();
   store_sum32<D, W>(dk, buf, p.dk + (row0 + k0) * p.lddk + hk * D, p.lddk);
-}
-
-template <int D>
-__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dq32_kernel(Attn32 p) {
-  __shared__ float buf[kAttnWaves32<D> * 16 * D];
-  dq_tile32<D>(p, buf, blockIdx.x, blockIdx.y, blockIdx.z);
-}
-template <int D>
-__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_dkv32_kernel(Attn32 p) {
-  __shared__ float buf[kAttnWaves32<D> * 16 * D];
-  dkv_tile32<D, false>(p, buf, blockIdx.x, blockIdx.y, blockIdx.z);
-}
-// both at once: the dK/dV workgroups, which take longer, in front (blockIdx.y: key heads, then query heads)
-template <int D>
-__global__ __launch_bounds__(64 * kAttnWaves32<D>) void attn_bwd32_kernel(Attn32 p) {
-  __shared__ float buf[kAttnWaves32<D> * 16 * D];
-  if ((int)blockIdx.y < p.n_kv_heads) dkv_tile32<D, true>(p, buf, blockIdx.x, blockIdx.y, blockIdx.z);
-  else dq_tile32<D>(p, buf, blockIdx.x, blockIdx.y - p.n_kv_heads, blockIdx.z);
 }
 
 // Whether a backward is one launch: while its workgroups are at most one per CU (its registers allow one).  Either
@@ -1271,8 +1269,8 @@ int jpp_attn_bwd_f32(void* stream, const jpp_attn_args* a) {
   hipStream_t st = (hipStream_t)stream;
   if (bwd32_at_once(a)) {
     const dim3 grid((unsigned)(a->seq / 16), (unsigned)(a->n_heads + a->n_kv_heads), (unsigned)a->batch);
-    if (a->head_dim == 64) hipLaunchKernelGGL(attn_bwd32_kernel<64>, grid, dim3(64 * kAttnWaves32<64>), 0, st, p);
-    else hipLaunchKernelGGL(attn_bwd32_kernel<128>, grid, dim3(64 * kAttnWaves32<128>), 0, st, p);
+    if (a->head_dim == 64) hipLaunchKernelGGL((attn_dkv32_kernel<64, true>), grid, dim3(64 * kAttnWaves32<64>), 0, st, p);
+    else hipLaunchKernelGGL((attn_dkv32_kernel<128, true>), grid, dim3(64 * kAttnWaves32<128>), 0, st, p);
     JPP_LAUNCH_CHECK();
     return JPP_OK;
   }
@@ -1280,10 +1278,10 @@ int jpp_attn_bwd_f32(void* stream, const jpp_attn_args* a) {
   const dim3 gk((unsigned)(a->seq / 16), (unsigned)a->n_kv_heads, (unsigned)a->batch);
   if (a->head_dim == 64) {
     hipLaunchKernelGGL(attn_dq32_kernel<64>, gq, dim3(64 * kAttnWaves32<64>), 0, st, p);
-    hipLaunchKernelGGL(attn_dkv32_kernel<64>, gk, dim3(64 * kAttnWaves32<64>), 0, st, p);
+    hipLaunchKernelGGL((attn_dkv32_kernel<64, false>), gk, dim3(64 * kAttnWaves32<64>), 0, st, p);
   } else {
     hipLaunchKernelGGL(attn_dq32_kernel<128>, gq, dim3(64 * kAttnWaves32<128>), 0, st, p);
-    hipLaunchKernelGGL(attn_dkv32_kernel<128>, gk, dim3(64 * kAttnWaves32<128>), 0, st, p);
+    hipLaunchKernelGGL((attn_dkv32_kernel<128, false>), gk, dim3(64 * kAttnWaves32<128>), 0, st, p);
   }
   JPP_LAUNCH_CHECK();
   return JPP_OK;
