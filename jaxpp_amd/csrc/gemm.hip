@@ -898,6 +898,9 @@ int launch_multi(hipStream_t stream, GemmParams* ps, int n, const ColsumPanels& 
   args.cols = cols;
   args.col_first = first;
   args.col_rows = col_rows;
+  if (col_blocks)   // (the sums that go along count here, not in a class of their own)
+    for (int i = 0; i < 4; ++i)
+      if (cols.first[i] < col_blocks) bytes += 2.0 * col_rows * cols.cols[i];
   static const std::string cls =
       std::string(class_name<BM, BN, true, true, JPP_EPI_ACC_F32, NW, NS, KG>()) + "_multi";
   ProbeScope probe(stream, cls.c_str(), flops, bytes);

@@ -116,3 +116,16 @@ def test_bias_gradients_beside_weight_gradients(family, h, heads, f, seq, batch)
     for li in range(2):
         for name, w in apart[0][li].items():
             assert np.abs(w).max() > 0 and np.array_equal(here[0][li][name], w), name
+
+
+@pytest.mark.parametrize("family,h,heads,f,seq", [("bert", 128, 2, 512, 128), ("decoder", 1024, 8, 4096, 512)])
+def test_probe_counts_the_sums_that_go_along(family, h, heads, f, seq):
+    """Their reads are bytes of the launch that they are part of."""
+    spec = LayerSpec(family, h, heads, f, seq, 1, head_dim=h // heads, causal=family == "decoder", eps=1e-5)
+    params = {0: [init_layer_params(spec, 3, 0, perturb=True)]}
+    with rt.probe("*") as p:
+        run_on_gpu(spec, make_rank_plan(S.Std1F1B(1), 1, 0), 1, params, two_streams=False)
+    (name, (launches, _, _, got)), = ((k, v) for k, v in p.classes.items() if k.endswith("_multi"))
+    shapes = [(f, h), (h, f), (h, h), (h, 3 * h)]
+    want = sum(2 * seq * (m + n) + 8 * m * n for m, n in shapes) + sum(2 * seq * n for _, n in shapes)
+    assert launches == 1 and "colsum" not in p.classes and got == want, (name, launches, got, want)
