@@ -605,8 +605,9 @@ __global__ __launch_bounds__(NW * KG * 64) void gemm_kernel(GemmArgs<MP> args) {
     // Old values that did not stream in are read here, by rows and past the caches: a small tile's
     // all at once, a large one's (out of registers for that) a pass ahead, the next pass's while this
     // one's leave.  Through the caches, and each pass's behind the one before it, a layer's four gradients
-    // of hidden 2048 and feed-forward 5632 on 512 tokens took 110 us as 256x256 tiles and 168 as
-    // 128x128; now 96 and 87 (what their accumulators' 352 MB alone take: 84).
+    // of hidden 2048 and gated feed-forward 5632 on 512 tokens took 112 us as 256x256 tiles, now 95.5 as 128x128, again and
+    // again by themselves; among the row's other kernels, under a profiler, 108 and 100 - 103.  Their accumulators' 361 MB
+    // alone are 66 us at 5.5 TB/s: the old values are asked for behind the contraction.
     const bool add_here = EPI == JPP_EPI_ACC_F32 && !stream_c;
     constexpr int BUFS = PASSES * PER <= 8 ? PASSES : 1;
     f32x4 old[BUFS][PER];
@@ -997,10 +998,10 @@ int launch_tiled(hipStream_t stream, GemmParams& p, int tile, bool deep) {
 // together, the fp32 tile that a weight gradient's workgroup reads, adds to and writes).  The constants are
 // least-squares fits to random products in every form, with the operands out of L2, as a layer finds
 // them, and accumulators out of every cache.
-// Forward: 1300 products (M, N 128 .. 16384, K 128 .. 16384, every orientation and epilogue), mean error 4
+// Forward: 969 products (M, N 128 .. 16384, K 128 .. 16384, every orientation and epilogue), mean error 4
 // - 10 %; the smallest estimate costs 0.1 % against the measured best.  128x256 stands 10 % above its
 // fit: 128x128 is otherwise passed over where they are close.  Against the rule before (256x256 from 192
-// tiles on, else 128x128: 36 % on average) it is slower by more than 2 % for 12 of the 1300, all but one by
+// tiles on, else 128x128: 36 % on average) it is slower by more than 2 % for 9 of the 969, all but one by
 // 6 % at most (180 tiles of 256x256, 3 K-steps: 14 %): a 512 x 1024 x 4096 input gradient has 32 tiles of
 // 128x128 for 256 CUs and took 28 us, 15 us as 128 tiles of 64x64 with two wave groups each.
 // 200 weight gradients that are not added to anything (written as bf16 or f32) are priced alike: 0.1 % over the measured
@@ -1060,7 +1061,9 @@ int choose_tile(const jpp_gemm_args* a) {
   const Extent grid = grid_extent(a);
   const bool gelu = a->epilogue == JPP_EPI_GELU || a->epilogue == JPP_EPI_DGELU;
   const int tile = cheapest_tile(&e, &grid, 1, work_ksteps(a), wgrad, gelu, true);
-  // (a rotated head lies inside one tile)
+  // A rotated head of 128 lies inside one tile: 64x128 at the price of 64x64, which it does not keep (512 x 3072 x 2048
+  // 16.6 us, 20 measured).  With the rotation the 128x128 tile does not keep its own either: where 64x128 is taken it
+  // needs 0.73 - 0.90 of that one's time (93 of 120 random products of 128 .. 2048 rows; in the others they are equal).
   return tile == kTile64 && a->rope_cos && a->rope_head_dim > 64 ? (int)kTile64x128 : tile;
 }
 

@@ -1,13 +1,13 @@
 // Copies between pageable host memory and the device: many tensors a call, converted on the way.
 //
-// hipMemcpy takes 14 - 115 us for a tensor of a few KB and moves 16 - 35 GB/s of a large one, on one host
-// thread; packing small tensors for it and converting to bf16 are more passes over host memory on the
+// hipMemcpy takes 10 - 20 us for a tensor of up to 256 KB and moves 25 GB/s of a large one to the device, 10 into a fresh
+// host array, on one host thread; packing small tensors for it and converting to bf16 are more passes over host memory on the
 // caller's thread, and fresh result arrays are paged in there.  Here a call's tensors are cut into chunks that are
 // contiguous on the device, and lanes - the caller's thread and up to seven more - take the next chunk each,
 // pack it into pinned memory of their own (or unpack it from there, converting) and run its copy on a
 // stream of their own, with a second chunk in flight meanwhile.  What is left is the link and the
-// host's memory: 256 KB 110 -> 18 us, 8 MB to the host 490 -> 250, 128 MB 29 -> 51 GB/s to the device and 10.5 -> 35 into a
-// fresh host array (1 MB to the device stays at 52 us).  A train step over host arrays of four layers of
+// host's memory: 8 MB 340 -> 275 us to the device and 495 -> 260 into a fresh host array, 128 MB 27 -> 37 - 49 GB/s and 10 -> 34
+// (a single tensor of up to 2 MB stays within 15 % of hipMemcpy).  A train step over host arrays of four layers of
 // hidden 256 (118 MB both ways) spent 9 of its 13 ms on these copies, now 4 of 7.
 #include <string.h>
 #include <unistd.h>

@@ -288,6 +288,12 @@ int run_apart(jpp_stage* s, hipStream_t st, const jpp_gemm_args& q) {
 // like this: Llama-shaped, hidden 2048 and feed-forward 5504 12.6 / 11.2 ms, 4096 and 11136 23.4 /
 // 18.5; encoder of 1408 and 5632 9.2 / 8.9; decoder blocks of 1536 and 4224 8.26 / 7.89.  On 512
 // tokens the last three are 0.99 of the speed with those matrices apart.
+// These lines count rounds of 256x256 tiles, and date from when full grids were made of them.  Now that accumulated
+// gradients take any tile by its estimate, on 320 random layers of one microbatch (hidden 128 .. 6144, 128 .. 8192
+// tokens) the lines cost 1.2 % over the best of all together and the largest one, two or all apart, 38 % at worst (hidden
+// 1152, gated 3072, 3712 tokens: 132 us together, 183 with the largest apart); all together would cost 0.4 % and 11 %.
+// None of the ways has become slower.  A group's microbatches one by one, where a matrix is not whole, cost more (hidden
+// 3456, gated 9472, groups of four x 128 tokens: 902 us, 273 as one grid over the operand pairs), for the sums' bits.
 // Which way is taken depends on the shapes only.
 int run_wgrads(jpp_stage* s, hipStream_t st, WgradBatch& w) {
   constexpr long kFullGrid = 192;
